@@ -358,10 +358,11 @@ def propagate_roofline(ctx, kt, workload_tag):
     avg_ms = kt["propagate_kernel"] / launches
     per_launch = alg_bytes / launches
     achieved = per_launch / (avg_ms * 1e-3) / 1e9 if avg_ms > 0 else 0.0
-    # one "launch" is the propagation step: k_propagate and, with one lane
-    # per link, the k_propagate_resume that continues its deferred links
-    # (the HIP events bracket both)
-    kernels = [f"k_propagate<{lanes}>"] + (["k_propagate_resume"] if lanes == 1 else [])
+    # one "launch" is the propagation step: k_propagate with one lane per
+    # link or, for steps of few links, a team of eight, and the
+    # k_propagate_resume that continues the deferred links of large steps
+    # (the HIP events bracket all)
+    kernels = [f"k_propagate<{lanes}>"] if lanes else ["k_propagate<1>", "k_propagate<8>", "k_propagate_resume"]
     kernel = " + ".join(kernels)
     traffic = None
     tpath = os.path.join(ROOT, "profiles", f"hbm_traffic_{workload_tag}.json")

@@ -45,8 +45,8 @@ ckf_status ckf_debug_propagate(const ckf_finding_config* cfg, const ckf_detector
 ckf_status ckf_debug_set_kernel_timing(ckf_algorithm* alg, int enable);
 
 /* Propagation schedule: lanes that navigate one link together in the
- * propagation kernel (1, 2, 4, 8 or 16; 0 = autotuned per seed-count class, the
- * default).  *lanes receives the schedule of the last call. */
+ * propagation kernel (1, 2, 4, 8 or 16; 0 = chosen for each step by how many
+ * links it has, the default).  *lanes receives the setting. */
 ckf_status ckf_debug_set_schedule(ckf_algorithm* alg, uint32_t lanes_per_link);
 ckf_status ckf_debug_get_schedule(const ckf_algorithm* alg, uint32_t* lanes_per_link);
 
@@ -62,7 +62,7 @@ ckf_status ckf_debug_kernel_times(const ckf_algorithm* alg, double* ms_find, dou
 ckf_status ckf_debug_find_split(const ckf_algorithm* alg, double* ms_find_kernel,
                                 double* ms_find_emit);
 /* The propagation group of the last timed call split into the propagation
- * kernel (k_propagate at the schedule's team size) and its compaction; their
+ * kernels (k_propagate, the deferred links of large steps) and their compaction; their
  * sum is ms_propagate. */
 ckf_status ckf_debug_propagate_split(const ckf_algorithm* alg, double* ms_propagate_kernel,
                                      double* ms_propagate_emit);

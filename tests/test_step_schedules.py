@@ -1,0 +1,49 @@
+"""Which kernels a step runs is chosen by how much of it there is; the tracks
+do not depend on it (GPU).
+
+The sizes lie on both sides of every line of the choice: one branch per
+surface bounds a step's links by the seeds, so 5,000 muons take one launch of
+16-lane teams, 16,000 one of 8-lane teams, 30,000 a 4 / 16 pair, 50,000 a 2 / 8
+pair and 60,000 a 1 / 8 pair; their later steps, with ever fewer links, cross
+from the first launch of a pair to the second.
+"""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from traccc_amd import _ffi as F
+from traccc_amd import ckf
+from traccc_amd import simulation as S
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _gpu(gpu_available):
+    return gpu_available
+
+
+def _columns(tracks):
+    return [tracks.offsets, tracks.constituents, tracks.chi2, tracks.ndf, tracks.pval, tracks.nholes]
+
+
+@pytest.mark.parametrize("n,branches", [(1, 1), (5120, 1), (5121, 1), (16384, 1), (16385, 1), (32769, 1),
+                                        (57345, 1), (3000, 3)])
+def test_propagation_launches_by_size(n, branches):
+    """The chosen launches and a fixed team give the same tracks, bit for bit."""
+    det, fld, gun = S.workload("C2", n_particles=n, seed=29)
+    ev = S.generate_event(det, fld, gun)
+    cfg = S.finding_config_for("C2")
+    cfg.max_num_branches_per_surface = branches
+    lib = F.load_library(ckf.LIB)
+    lib.ckf_debug_set_schedule.argtypes = [C.c_void_p, C.c_uint32]
+    ddet = ckf.DeviceDetector(det, fld)
+    dev = ckf.DeviceEvents(ddet, ev)
+    alg = ckf.combinatorial_kalman_filter_algorithm(cfg)
+    got = _columns(alg.run_device(ddet, dev).download())
+    assert lib.ckf_debug_set_schedule(alg._h, 4) == 0
+    want = _columns(alg.run_device(ddet, dev).download())
+    assert len(want[2]) > 0.9 * ev.n_seeds
+    for a, b in zip(got, want):
+        assert np.array_equal(a, b)

@@ -87,6 +87,12 @@ static_assert(sizeof(line_u32) == 128 && sizeof(line_u64) == 128, "one counter p
 // A deferred propagation: link, visited layers (2 words), RK steps, path,
 // the free state (11 words), the transport Jacobian (31 words), state ref.
 constexpr uint32_t kDeferWords = 48u;
+// Links of a step from which on second layer searches are deferred: below it
+// the continuing kernel's own chain (50-80 us for a few waves) costs more than
+// the divergence it takes out of the others: 84,815 links 124 us in place, 101
+// + 72 deferred; 285,989 268 and 229 + 74; 323,274 285 and 245 + 79 (the 40 us
+// grow with the links, the 80 do not).
+constexpr uint32_t kDeferLinks = 700000u;
 
 struct step_ctl {
     uint32_t step;        // current CKF step

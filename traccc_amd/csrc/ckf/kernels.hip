@@ -1150,21 +1150,32 @@ __device__ inline uint8_t finish_link(const ckf_params& P, const navigator<float
 
 // kT lanes propagate one link together (team navigator); 64 / kT links per
 // wave partition.  The team leader writes the results.  With one lane per
-// link, a propagation that needs a second layer search (a few % of them, but
-// nearly every wave has one) is written to the defer buffer and continued by
-// k_propagate_resume, so the wave does not run a second search, approach and
-// window for one or two of its lanes.
+// link and kDeferLinks links or more, a propagation that needs a second layer
+// search (a few % of them, but nearly every wave has one) is written to the
+// defer buffer and continued by k_propagate_resume, so the wave does not run a
+// second search, approach and window for one or two of its lanes.
+//
+// A propagation is a serial chain of ~100 us on one lane (Runge-Kutta steps,
+// layer search, module windows): a step whose waves all fit on the chip is
+// bound by that chain, which a team shortens, a larger one by the lanes, which
+// a team spends on redundant steps.  So a launch runs only when its step has
+// [from, below) links: two launches with different teams share the steps of a
+// call (propagate_schedule, runtime.hip); the other one's blocks leave at once.
 template <int kT>
-__global__ __launch_bounds__(kBlock) void k_propagate(ckf_params P) {
+__global__ __launch_bounds__(kBlock) void k_propagate(ckf_params P, uint32_t from, uint32_t below) {
     step_ctl* ctl = P.ctl;
     if (ctl->done) {
+        return;
+    }
+    const uint32_t n = links_this_step(P, ctl);
+    // the grid is sized for the largest step: a block without a partition leaves
+    if (n < from || n >= below || static_cast<uint64_t>(blockIdx.x) * kBlock >= static_cast<uint64_t>(n) * kT) {
         return;
     }
     // the navigation layers and groups live in LDS for the whole kernel
     __shared__ nav_tables s_nav;
     stage_nav_tables(s_nav, P.layers, P.n_layers, P.groups, P.n_groups, P.nav.mask_tol_max);
     const uint32_t step = ctl->step;
-    const uint32_t n = links_this_step(P, ctl);
     const uint32_t base = ctl->link_base;
     constexpr uint32_t kLinksPerWave = kWave / kT;
     const uint32_t n_parts = (n + kLinksPerWave - 1) / kLinksPerWave;
@@ -1172,7 +1183,7 @@ __global__ __launch_bounds__(kBlock) void k_propagate(ckf_params P) {
     const bool dedup = step >= P.dup_min_len;
     const uint32_t tl = lane() % kT;
     const bool leader = (tl == 0u);
-    const bool defer = (kT == 1) && P.defer_cap > 0u;
+    const bool defer = (kT == 1) && P.defer_cap > 0u && n >= kDeferLinks;
 
     xcd_ticket_run queue(&ctl->xcd_ticket[2][0].v, n_parts, 1u);
     for (;;) {
@@ -1945,24 +1956,24 @@ hipError_t launch_prop_emit(const ckf_params& P, const launch_shape& s, hipStrea
     return hipGetLastError();
 }
 
+template <int kT>
+void launch_team(const ckf_params& P, const prop_launch& l, hipStream_t stream) {
+    hipLaunchKernelGGL(k_propagate<kT>, dim3(l.blocks), dim3(kBlock), 0, stream, P, l.from, l.below);
+}
+
 hipError_t launch_propagate_work(const ckf_params& P, const launch_shape& s, hipStream_t stream) {
-    switch (s.prop_team) {
-        case 16:
-            hipLaunchKernelGGL(k_propagate<16>, dim3(s.prop_blocks), dim3(kBlock), 0, stream, P);
-            break;
-        case 8:
-            hipLaunchKernelGGL(k_propagate<8>, dim3(s.prop_blocks), dim3(kBlock), 0, stream, P);
-            break;
-        case 4:
-            hipLaunchKernelGGL(k_propagate<4>, dim3(s.prop_blocks), dim3(kBlock), 0, stream, P);
-            break;
-        case 2:
-            hipLaunchKernelGGL(k_propagate<2>, dim3(s.prop_blocks), dim3(kBlock), 0, stream, P);
-            break;
-        default:
-            hipLaunchKernelGGL(k_propagate<1>, dim3(s.prop_blocks), dim3(kBlock), 0, stream, P);
-            hipLaunchKernelGGL(k_propagate_resume, dim3(s.resume_blocks), dim3(kBlock), 0, stream, P);
-            break;
+    for (const prop_launch& l : s.prop) {
+        switch (l.team) {
+            case 16u: launch_team<16>(P, l, stream); break;
+            case 8u: launch_team<8>(P, l, stream); break;
+            case 4u: launch_team<4>(P, l, stream); break;
+            case 2u: launch_team<2>(P, l, stream); break;
+            case 1u: launch_team<1>(P, l, stream); break;
+            default: break;  // an unused entry
+        }
+    }
+    if (s.resume_blocks > 0u) {
+        hipLaunchKernelGGL(k_propagate_resume, dim3(s.resume_blocks), dim3(kBlock), 0, stream, P);
     }
     return hipGetLastError();
 }

@@ -7,16 +7,21 @@
 
 namespace tamd {
 
+// One launch of k_propagate: `team` lanes per link (1, 2, 4, 8 or 16; 0: no
+// launch) for steps of [from, below) links.
+struct prop_launch {
+    uint32_t team, from, below, blocks;
+};
+
 struct launch_shape {
     uint32_t find_blocks;
     uint32_t dedup_blocks;
-    uint32_t prop_blocks;
     uint32_t build_blocks;
-    uint32_t prop_team;  // lanes per link in k_propagate: 1, 2, 4, 8 or 16
+    prop_launch prop[2];
     uint32_t list_blocks;   // scorer-pruned finding: candidate lists
     uint32_t score_blocks;  // and the MLP + updates over them (64 inputs per wave)
     uint32_t emit_blocks;   // the compaction kernels (k_*_emit)
-    uint32_t resume_blocks; // deferred propagations (k_propagate_resume)
+    uint32_t resume_blocks; // deferred propagations (k_propagate_resume); 0: none deferred
 };
 
 // One CKF step: find_tracks, duplicate removal (active from
@@ -36,7 +41,7 @@ hipError_t launch_find_emit(const ckf_params& P, const launch_shape& s, hipStrea
 hipError_t launch_dedup(const ckf_params& P, const launch_shape& s, hipStream_t stream);
 hipError_t launch_propagate(const ckf_params& P, const launch_shape& s, hipStream_t stream,
                             bool fused_advance);
-// launch_propagate = the propagation kernel (at the schedule's team size),
+// launch_propagate = the propagation kernels (the schedule's launches),
 // then its compaction (k_prop_emit)
 hipError_t launch_propagate_work(const ckf_params& P, const launch_shape& s, hipStream_t stream);
 hipError_t launch_prop_emit(const ckf_params& P, const launch_shape& s, hipStream_t stream,

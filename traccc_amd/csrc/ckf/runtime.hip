@@ -11,9 +11,7 @@
 
 #include <algorithm>
 #include <cmath>
-#include <chrono>
 #include <cstdio>
-#include <map>
 #include <mutex>
 #include <cstring>
 #include <new>
@@ -116,9 +114,7 @@ struct ckf_algorithm {
     std::vector<char> graph_key;
     // per-kernel event timing (diagnostics; the step loop then runs uncaptured)
     uint32_t last_steps = 0;  // steps the previous call ran (sizes the first launch)
-    uint32_t prop_team = 1;   // lanes per link in k_propagate (chosen per call)
-    uint32_t schedule_override = 0;   // fixed lanes per link, 0 = autotuned
-    std::map<uint32_t, uint32_t> tuned;  // log2(seeds) -> lanes per link
+    uint32_t schedule_override = 0;   // fixed lanes per link, 0 = by each step's links
     bool timing = false;
     double t_find = 0.0, t_dedup = 0.0, t_prop = 0.0, t_other = 0.0, t_find_work = 0.0,
            t_find_emit = 0.0, t_prop_work = 0.0, t_prop_emit = 0.0;
@@ -150,6 +146,8 @@ struct ckf_algorithm {
 namespace {
 
 constexpr uint32_t kStepsPerChunk = 4u;
+// k_propagate's registers allow two waves per SIMD, four SIMDs per CU
+constexpr uint32_t kPropWavesPerCu = 8u;
 
 uint32_t parts(uint32_t n) { return (n + 63u) / 64u; }
 
@@ -172,8 +170,10 @@ void ensure_buffers(ckf_algorithm& A, const ckf_device_event& ev) {
     A.find_count.ensure(4u * size_t(A.in_cap));
     A.prop_flag.ensure(size_t(A.state_cap));
     // a propagation that needs a second layer search (a few % of them)
-    // continues in its own kernel; beyond the buffer it continues in place
-    A.defer_cap = std::max<uint32_t>(A.state_cap / 8u, 1024u);
+    // continues in its own kernel where a step may hold enough links for that
+    // to pay (some seeds branch: half of kDeferLinks seeds); beyond the buffer
+    // it continues in place
+    A.defer_cap = ev.n_seeds >= tamd::kDeferLinks / 2u ? std::max<uint32_t>(A.state_cap / 8u, 1024u) : 0u;
     A.defer.ensure(4u * size_t(tamd::kDeferWords) * A.defer_cap);
     A.tips.ensure(4u * size_t(A.tip_cap));
     A.seed_first.ensure(4u * size_t(std::max(ev.n_seeds, 1u)));
@@ -351,22 +351,58 @@ tamd::ckf_params make_params(ckf_algorithm& A, const ckf_device_detector& D,
     return P;
 }
 
-tamd::launch_shape make_shape(const ckf_algorithm& A) {
+// The launches of k_propagate in a step, by how many links a step of this call
+// can have (`bound`; with one branch per surface a step never has more links
+// than seeds).  W = the waves the chip holds (two per SIMD, what the kernel's
+// registers allow): a team is worth its redundant steps while its waves all
+// run at once.  us per step (1 without deferral / 2 / 4 / 8 / 16 lanes):
+// 285,989 links 268 / 416 / 518 / 693 / 1011; 84,815 124 / 156 / 188 / 288 /
+// 416; 54,417 117 / 106 / 131 / 187 / 264; 29,559 107 / 93 / 75 / 107 / 176;
+// 11,089 89 / 86 / 60 / 54 / 68; 3,435 93 / 79 / 55 / 44 / 40; 335 66 / 73 /
+// 48 / 36 / 30.  A call whose steps all fit one team's range runs one launch
+// (a second one costs ~3 us a step to find that it has nothing to do).
+void propagate_schedule(const ckf_algorithm& A, uint64_t bound, tamd::launch_shape& s) {
+    const uint64_t lanes = uint64_t(A.n_cu) * kPropWavesPerCu * 64u;
+    const uint32_t max_blocks = static_cast<uint32_t>(A.n_cu) * kPropWavesPerCu / 4u;
+    auto entry = [&](int k, uint32_t team, uint32_t from, uint32_t below) {
+        const uint64_t most = std::min<uint64_t>(bound, below);
+        const uint64_t blocks = (most * team + 255u) / 256u;
+        s.prop[k] = tamd::prop_launch{team, from, below, static_cast<uint32_t>(std::max<uint64_t>(
+                                                             1u, std::min<uint64_t>(blocks, max_blocks)))};
+    };
+    constexpr uint32_t kAll = 0xffffffffu;
+    s.prop[0] = s.prop[1] = tamd::prop_launch{};
+    if (A.schedule_override != 0u) {
+        entry(0, A.schedule_override, 0u, kAll);  // fixed (diagnostics)
+    } else if (bound * 16u <= lanes * 5u / 8u) {
+        entry(0, 16u, 0u, kAll);
+    } else if (bound * 8u <= lanes) {
+        entry(0, 8u, 0u, kAll);
+    } else if (bound * 4u <= lanes) {
+        const uint32_t t = static_cast<uint32_t>(lanes / 16u);  // 8,192 on 256 CUs
+        entry(0, 4u, t, kAll);
+        entry(1, 16u, 0u, t);
+    } else {
+        const uint32_t t = static_cast<uint32_t>(lanes * 27u / 128u);  // 27,648 on 256 CUs
+        entry(0, bound * 2u <= lanes * 7u / 8u ? 2u : 1u, t, kAll);
+        entry(1, 8u, 0u, t);
+    }
+}
+
+tamd::launch_shape make_shape(const ckf_algorithm& A, uint32_t n_seeds) {
     const uint32_t max_blocks = static_cast<uint32_t>(A.n_cu) * 8u;
     auto blocks = [&](uint32_t cap) {
         const uint32_t b = (parts(cap) + 3u) / 4u;
         return std::max(1u, std::min(b, max_blocks));
     };
-    tamd::launch_shape s;
+    tamd::launch_shape s{};
     // grids are upper bounds for the largest step: a wave beyond a step's
     // partitions leaves at once.  The find is sized for 16 inputs per wave
     // (its two-lane teams hold 32, the scored update 64).
     s.find_blocks = std::max(1u, std::min((((A.in_cap + 15u) / 16u) + 3u) / 4u, max_blocks));
     s.dedup_blocks = blocks(A.state_cap);
-    s.prop_team = A.prop_team;
-    const uint32_t prop_parts = (A.state_cap + 64u / s.prop_team - 1u) / (64u / s.prop_team);
-    s.prop_blocks = std::max(1u, std::min((prop_parts + 3u) / 4u, max_blocks));
-    s.resume_blocks = std::max(1u, std::min((parts(A.defer_cap) + 3u) / 4u, max_blocks));
+    propagate_schedule(A, A.cfg.max_num_branches_per_surface == 1u ? n_seeds : A.state_cap, s);
+    s.resume_blocks = A.defer_cap == 0u ? 0u : std::max(1u, std::min((parts(A.defer_cap) + 3u) / 4u, max_blocks));
     // scorer-pruned finding: 16 inputs per wave listing, 64 per scoring wave
     s.list_blocks = std::max(1u, std::min((((A.in_cap + 15u) / 16u) + 3u) / 4u, max_blocks));
     s.score_blocks = std::max(1u, std::min((((A.in_cap + 63u) / 64u) + 3u) / 4u, max_blocks));
@@ -594,46 +630,6 @@ void run_votes(ckf_algorithm& A, const tamd::ckf_params& P, const ckf_device_eve
     for (int i = 0; i < 10; ++i) std::swap(T.track_bytes[i], K2.track_bytes[i]);
 }
 
-// Propagation schedule autotuner: lanes per link in k_propagate.  Every
-// schedule gives the same tracks; which is fastest depends on how many links
-// a step holds against the machine's lanes (one lane per link fills the chip
-// once tens of thousands of links are live; a small event runs its links'
-// navigation on teams of lanes instead).  The first call of each size class
-// (log2 of the seed count) times the step loop once per schedule on its own
-// input and keeps the fastest; later calls of the class reuse it.  A fixed
-// schedule (ckf_debug_set_schedule) bypasses the tuner.
-template <typename Loop>
-uint32_t choose_schedule(ckf_algorithm& A, uint32_t n_seeds, Loop& step_loop) {
-    if (A.schedule_override != 0u) {
-        return A.schedule_override;
-    }
-    uint32_t cls = 0u;
-    while ((1u << cls) < n_seeds && cls < 31u) ++cls;
-    const auto it = A.tuned.find(cls);
-    if (it != A.tuned.end()) {
-        return it->second;
-    }
-    const uint32_t teams[5] = {1u, 2u, 4u, 8u, 16u};
-    uint32_t best = 1u;
-    double best_s = 1e300;
-    for (uint32_t t : teams) {
-        A.prop_team = t;
-        // the faster of two runs: a schedule's first run also captures its
-        // step graph, which would bias the choice against whichever runs first
-        for (int rep = 0; rep < 2; ++rep) {
-            const auto t0 = std::chrono::steady_clock::now();
-            step_loop();  // ends with a stream synchronisation
-            const double dt = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
-            if (dt < best_s) {
-                best_s = dt;
-                best = t;
-            }
-        }
-    }
-    A.tuned[cls] = best;
-    return best;
-}
-
 // The operator's dispatch (core/src/finding/combinatorial_kalman_filter_algorithm.cpp:47-57):
 // the progressive filter runs when asked for and at most one branch is kept.
 bool use_pkf(const ckf_finding_config& c) {
@@ -785,7 +781,7 @@ ckf_device_tracks* find_tracks(ckf_algorithm& A, const ckf_device_detector& D,
         for (int attempt = 0;; ++attempt) {
             ensure_buffers(A, ev);
             P = make_params(A, D, ev);
-            shape = make_shape(A);
+            shape = make_shape(A, ev.n_seeds);
             const uint32_t ovf = run_steps(A, P, shape, ev);
             if (ovf == 0u) {
                 break;
@@ -797,7 +793,6 @@ ckf_device_tracks* find_tracks(ckf_algorithm& A, const ckf_device_detector& D,
             A.stats.n_regrows += 1u;
         }
     };
-    A.prop_team = choose_schedule(A, ns, step_loop);
     step_loop();
     const tamd::step_ctl done = *A.h_ctl;
     A.stats.n_steps = done.n_steps_run;
@@ -1446,7 +1441,7 @@ ckf_status ckf_debug_get_schedule(const ckf_algorithm* alg, uint32_t* lanes_per_
         if (alg == nullptr || lanes_per_link == nullptr) {
             throw ckf_error(CKF_ERR_INVALID_ARGUMENT, "null argument");
         }
-        *lanes_per_link = alg->prop_team;
+        *lanes_per_link = alg->schedule_override;
     });
 }
 
