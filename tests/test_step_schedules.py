@@ -8,6 +8,7 @@ pair and 60,000 a 1 / 8 pair; their later steps, with ever fewer links, cross
 from the first launch of a pair to the second.
 """
 import ctypes as C
+import dataclasses
 
 import numpy as np
 import pytest
@@ -47,3 +48,26 @@ def test_propagation_launches_by_size(n, branches):
     assert len(want[2]) > 0.9 * ev.n_seeds
     for a, b in zip(got, want):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("n", [255, 256, 257, 1024, 1025, 32768, 65537])
+def test_compaction_partition_edges(n):
+    """Compaction works on partitions of 256 items, of 512 from 32,768 items on
+    and so up to 1,024 from 65,536 on: a batch of small events with that many
+    seeds in all gives each event the tracks the CPU oracle finds in it."""
+    import oracle
+    from concurrent.futures import ThreadPoolExecutor
+    det, fld, gun = S.workload("C1", n_particles=512, seed=31)
+    sizes = [512] * (n // 512) + ([n % 512] if n % 512 else [])
+    guns = [dataclasses.replace(gun, n_particles=k, seed=700 + e) for e, k in enumerate(sizes)]
+    events = S.generate_events(det, fld, guns)
+    cfg = S.finding_config_for("C1")
+    ddet = ckf.DeviceDetector(det, fld)
+    got = ckf.combinatorial_kalman_filter_algorithm(cfg).run_device(ddet, ckf.DeviceEvents(ddet, events)).download()
+    with ThreadPoolExecutor(8) as pool:
+        want = list(pool.map(lambda ev: oracle.run(cfg, det, fld, ev, 64), events))
+    assert sum(e.n_seeds for e in events) == n
+    for e, w in enumerate(want):
+        g = got.event(e)
+        assert np.array_equal(g.offsets, w.offsets), e
+        assert np.array_equal(g.constituents, w.constituents), e

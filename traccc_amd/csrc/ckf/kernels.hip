@@ -404,19 +404,82 @@ __device__ inline dlink staged_link(const stage_head& h, const stage_cand& c, ui
     return L;
 }
 
-// Compaction partitions of the emit kernels: a wave takes kEmitChunks
-// consecutive 64-item chunks per ticket, counts them, runs one decoupled
-// look-back for the whole partition, then writes.  Large partitions keep the
-// look-back chain short (its round trips, not the bytes, bound these kernels).
-constexpr uint32_t kEmitChunks = 16;
+// Compaction partitions of the emit kernels: a block takes up to kEmitChunks
+// consecutive chunks of kBlock items per ticket, counts them, runs one
+// decoupled look-back for the whole partition (its first wave), then writes.
+// A partition's items are in flight together, one per thread and chunk: with
+// one wave walking a partition of 1,024 items chunk by chunk, a step of 90,000
+// inputs kept 88 waves of the chip busy and its compaction took 50 us, four
+// times what the bytes and one look-back cost.
+constexpr uint32_t kEmitChunks = 4;
+constexpr uint32_t kEmitWaves = kBlock / kWave;
 
-// Chunks per partition for n items: one per 64 chunks of work, at most
-// kEmitChunks -- a look-back round trip covers 64 partitions, so the chain
-// any partition waits on stays at a round or two, while small steps still
-// spread over many waves.
+// Chunks per partition for n items: one per 64 partitions' worth of work, at
+// most kEmitChunks -- a look-back round trip covers 64 partitions, so the
+// chain any partition waits on stays at a round or two, while small steps
+// still spread over many blocks.
 __device__ inline uint32_t emit_chunks(uint32_t n) {
-    const uint32_t c = n / (kWave * 64u);
+    const uint32_t c = n / (kBlock * 64u);
     return c < 1u ? 1u : (c > kEmitChunks ? kEmitChunks : c);
+}
+
+struct emit_shared {
+    uint32_t ticket;
+    uint32_t tot[2][kEmitChunks * kEmitWaves];  // per channel: each wave's items of a chunk
+    uint64_t base;
+};
+
+// The block's next partition (every thread).  The two barriers also keep the
+// shared words of the last partition from being overwritten too early.
+__device__ inline uint32_t block_ticket(uint32_t* counter, emit_shared& S) {
+    __syncthreads();
+    if (threadIdx.x == 0u) {
+        S.ticket = atomicAdd(counter, 1u);
+    }
+    __syncthreads();
+    return S.ticket;
+}
+
+// Exclusive prefixes of v[chunk] over the partition's items in order (chunk
+// by chunk, thread by thread), in place; returns the partition's total.  Ends
+// with a barrier behind it.
+__device__ inline uint32_t block_prefix(uint32_t (&v)[kEmitChunks], int channel, emit_shared& S) {
+    const uint32_t w = threadIdx.x / kWave;
+#pragma unroll
+    for (uint32_t ch = 0; ch < kEmitChunks; ++ch) {
+        const uint32_t incl = wave_inclusive_scan(v[ch]);
+        if (lane() == kWave - 1) {
+            S.tot[channel][ch * kEmitWaves + w] = incl;
+        }
+        v[ch] = incl - v[ch];
+    }
+    __syncthreads();
+    uint32_t run = 0u;
+#pragma unroll
+    for (uint32_t ch = 0; ch < kEmitChunks; ++ch) {
+#pragma unroll
+        for (uint32_t q = 0; q < kEmitWaves; ++q) {
+            if (q == w) {
+                v[ch] += run;
+            }
+            run += S.tot[channel][ch * kEmitWaves + q];
+        }
+    }
+    return run;
+}
+
+// The partition's look-back by the block's first wave; every thread gets the
+// exclusive prefix of both channels.
+__device__ inline uint64_t block_lookback(uint64_t* lo_words, uint64_t* hi_words, uint32_t p, uint32_t epoch,
+                                          uint64_t agg, emit_shared& S) {
+    if (threadIdx.x < kWave) {
+        const uint64_t b = wave_lookback(lo_words, hi_words, p, epoch, agg);
+        if (threadIdx.x == 0u) {
+            S.base = b;
+        }
+    }
+    __syncthreads();
+    return S.base;
 }
 
 // A listed candidate's MLP row (16 shorts, 32 B): features 0-8, 10 and 11
@@ -843,6 +906,7 @@ __global__ __launch_bounds__(kBlock) void k_find(ckf_params P) {
 // chain of every later partition while it works.
 template <bool kLogging>
 __global__ __launch_bounds__(kBlock) void k_find_emit(ckf_params P) {
+    __shared__ emit_shared S;
     step_ctl* ctl = P.ctl;
     if (ctl->done) {
         return;
@@ -852,82 +916,77 @@ __global__ __launch_bounds__(kBlock) void k_find_emit(ckf_params P) {
     const uint32_t link_base = ctl->link_base;
     const uint32_t epoch = ctl->epoch;
     const uint32_t kc = emit_chunks(n_in);
-    const uint32_t part = kWave * kc;
+    const uint32_t part = kBlock * kc;
     const uint32_t n_parts = (n_in + part - 1u) / part;
-    auto input_seed = [&](uint32_t j) -> uint32_t { return P.stage_in[j].seed; };
-    const bool takes = wave_takes_tickets(n_parts);
+    if (blockIdx.x == 0u && threadIdx.x == 0u) {
+        // k_prop_emit's queue is cleared here, between its launches: a block
+        // of it that starts after the step's advance then still finds it spent
+        ctl->ticket[5].v = 0u;
+    }
+    if (blockIdx.x >= n_parts) {
+        return;
+    }
     for (;;) {
-        const uint32_t p = takes ? wave_ticket(&ctl->ticket[4].v) : n_parts;
+        const uint32_t p = block_ticket(&ctl->ticket[4].v, S);
         if (p >= n_parts) {
             break;
         }
-        const uint32_t i0 = p * part;
-        uint32_t n_out[kEmitChunks];
-        uint32_t total = 0u;
+        const uint32_t i0 = p * part + threadIdx.x;
+        uint32_t n_out[kEmitChunks], first[kEmitChunks];
 #pragma unroll
-        for (int ch = 0; ch < static_cast<int>(kEmitChunks); ++ch) {
-            const uint32_t i = i0 + static_cast<uint32_t>(ch) * kWave + lane();
-            const uint32_t count = (static_cast<uint32_t>(ch) < kc && i < n_in) ? P.find_count[i] : 0u;
-            n_out[ch] = (static_cast<uint32_t>(ch) < kc && i < n_in) ? (count > 0u ? count : 1u) : 0u;
-            total += wave_broadcast(wave_inclusive_scan(n_out[ch]), kWave - 1);
+        for (uint32_t ch = 0; ch < kEmitChunks; ++ch) {
+            const uint32_t i = i0 + ch * kBlock;
+            const bool valid = ch < kc && i < n_in;
+            const uint32_t count = valid ? P.find_count[i] : 0u;
+            n_out[ch] = valid ? (count > 0u ? count : 1u) : 0u;
+            first[ch] = n_out[ch];
         }
-        const uint64_t base = wave_lookback(P.lb_lo[0], nullptr, p, epoch,
-                                            pack2(total, 0u));
-        if (p == n_parts - 1u && lane() == 0u) {
-            ctl->n_links = lo32(base) + total;
+        const uint32_t total = block_prefix(first, 0, S);
+        const uint32_t base = lo32(block_lookback(P.lb_lo[0], nullptr, p, epoch, pack2(total, 0u), S));
+        if (p == n_parts - 1u && threadIdx.x == 0u) {
+            ctl->n_links = base + total;
         }
-        uint32_t run = lo32(base);
-        uint32_t last_seed = (i0 > 0u && lane() == 0u) ? input_seed(i0 - 1u) : kInvalid;
-        last_seed = wave_broadcast(last_seed, 0);
-#pragma unroll 1
-        for (uint32_t ch = 0; ch < kc; ++ch) {
-            if (i0 + ch * kWave >= n_in) {
-                break;  // uniform
-            }
-            const uint32_t i = i0 + ch * kWave + lane();
-            const bool valid = i < n_in;
-            // select n_out[ch] without a runtime index into the array
-            uint32_t no = 0u;
 #pragma unroll
-            for (int q = 0; q < static_cast<int>(kEmitChunks); ++q) {
-                if (static_cast<uint32_t>(q) == ch) no = n_out[q];
-            }
-            const uint32_t incl = wave_inclusive_scan(no);
-            const uint32_t first = run + incl - no;
-            run += wave_broadcast(incl, kWave - 1);
+        for (uint32_t ch = 0; ch < kEmitChunks; ++ch) {
+            const uint32_t i = i0 + ch * kBlock;
+            const bool valid = ch < kc && i < n_in;
             const stage_head h = valid ? P.stage_in[i] : stage_head{};
             const uint32_t seed = valid ? h.seed : kInvalid;
             // head of the seed's contiguous run of inputs
             uint32_t prev_seed = __shfl(seed, (lane() + kWave - 1u) % kWave, kWave);
             if (lane() == 0u) {
-                prev_seed = last_seed;
+                prev_seed = valid && i > 0u ? P.stage_in[i - 1u].seed : kInvalid;
             }
-            last_seed = wave_broadcast(seed, kWave - 1);
             if (!valid) {
                 continue;
             }
+            const uint32_t at = base + first[ch];
             if (i == 0u || prev_seed != seed) {
-                P.seed_first[seed] = first;
+                P.seed_first[seed] = at;
             }
-            for (uint32_t k = 0; k < no; ++k) {
+            for (uint32_t k = 0; k < n_out[ch]; ++k) {
                 const uint32_t slot = flt_slot(P, i, k);
                 if (slot >= P.flt_cap) {
                     break;  // k_find raised the overflow that discards this step
                 }
                 const dlink L = staged_link(h, P.stage_slot[slot], step, slot);
-                const uint32_t g = link_base + first + k;
-                if (g < P.link_cap && first + k < P.state_cap) {
+                const uint32_t g = link_base + at + k;
+                if (g < P.link_cap && at + k < P.state_cap) {
                     P.links[g] = L;
                     if constexpr (kLogging) {
                         if (L.meas != kInvalid) {
-#pragma unroll
-                            for (int q = 0; q < kFeatures; ++q) {
-                                float v = P.feat_slot[static_cast<size_t>(slot) * kFeatures + q];
-                                if (q == kFeatStanding) {
-                                    v = standing_of(P.seed_run_min, seed, epoch, v);
-                                }
-                                P.log_feat[static_cast<size_t>(g) * kFeatures + q] = v;
-                            }
+                            // a row is 48 B: three 16-byte pieces each way
+                            const float4* src = reinterpret_cast<const float4*>(
+                                P.feat_slot + static_cast<size_t>(slot) * kFeatures);
+                            float4* dst = reinterpret_cast<float4*>(
+                                P.log_feat + static_cast<size_t>(g) * kFeatures);
+                            const float4 f0 = src[0], f1 = src[1];
+                            float4 f2 = src[2];
+                            static_assert(kFeatures == 12 && kFeatStanding == 9, "feature 9 is .y of the third piece");
+                            f2.y = standing_of(P.seed_run_min, seed, epoch, f2.y);
+                            dst[0] = f0;
+                            dst[1] = f1;
+                            dst[2] = f2;
                         }
                     }
                 } else {
@@ -1055,6 +1114,7 @@ __global__ __launch_bounds__(kBlock) void k_dedup_mark(ckf_params P) {
 // After k_dedup_mark: each link's rank among the step's surviving links
 // (alive_prefix = alive bit | rank) and, per seed, the rank of its first link.
 __global__ __launch_bounds__(kBlock) void k_dedup_emit(ckf_params P) {
+    __shared__ emit_shared S;
     step_ctl* ctl = P.ctl;
     if (ctl->done || ctl->step < P.dup_min_len || (ctl->overflow & kFindOverflow) != 0u) {
         return;
@@ -1063,40 +1123,36 @@ __global__ __launch_bounds__(kBlock) void k_dedup_emit(ckf_params P) {
     const uint32_t base = ctl->link_base;
     const uint32_t epoch = ctl->epoch;
     const uint32_t kc = emit_chunks(n);
-    const uint32_t part = kWave * kc;
+    const uint32_t part = kBlock * kc;
     const uint32_t n_parts = (n + part - 1u) / part;
-    const bool takes = wave_takes_tickets(n_parts);
+    if (blockIdx.x >= n_parts) {
+        return;
+    }
     for (;;) {
-        const uint32_t p = takes ? wave_ticket(&ctl->ticket[6].v) : n_parts;
+        const uint32_t p = block_ticket(&ctl->ticket[6].v, S);
         if (p >= n_parts) {
             break;
         }
-        const uint32_t i0 = p * part;
-        uint64_t am[kEmitChunks];
-        uint32_t total = 0u;
+        const uint32_t i0 = p * part + threadIdx.x;
+        uint32_t alive[kEmitChunks], rank[kEmitChunks];
 #pragma unroll
-        for (int ch = 0; ch < static_cast<int>(kEmitChunks); ++ch) {
-            const uint32_t i = i0 + static_cast<uint32_t>(ch) * kWave + lane();
-            const bool a = static_cast<uint32_t>(ch) < kc && i < n && (P.alive_prefix[i] >> 31) != 0u;
-            am[ch] = wave_ballot(a);
-            total += static_cast<uint32_t>(__popcll(am[ch]));
+        for (uint32_t ch = 0; ch < kEmitChunks; ++ch) {
+            const uint32_t i = i0 + ch * kBlock;
+            alive[ch] = (ch < kc && i < n) ? P.alive_prefix[i] & 0x80000000u : 0u;
+            rank[ch] = alive[ch] >> 31;
         }
-        const uint64_t b = wave_lookback(P.lb_lo[1], nullptr, p, epoch,
-                                         pack2(total, 0u));
-        uint32_t run = lo32(b);
+        const uint32_t total = block_prefix(rank, 0, S);
+        const uint32_t run = lo32(block_lookback(P.lb_lo[1], nullptr, p, epoch, pack2(total, 0u), S));
 #pragma unroll
-        for (int ch = 0; ch < static_cast<int>(kEmitChunks); ++ch) {
-            const uint32_t i = i0 + static_cast<uint32_t>(ch) * kWave + lane();
-            if (static_cast<uint32_t>(ch) < kc && i < n) {
-                const bool a = ((am[ch] >> lane()) & 1ull) != 0ull;
-                const uint32_t before = run + prefix_count(am[ch]);
-                P.alive_prefix[i] = (a ? 0x80000000u : 0u) | before;
+        for (uint32_t ch = 0; ch < kEmitChunks; ++ch) {
+            const uint32_t i = i0 + ch * kBlock;
+            if (ch < kc && i < n) {
+                P.alive_prefix[i] = alive[ch] | (run + rank[ch]);
                 const uint32_t seed = load_link(P, base + i).seed;
                 if (P.seed_first[seed] == i) {
-                    P.seed_base[seed] = before;
+                    P.seed_base[seed] = run + rank[ch];
                 }
             }
-            run += static_cast<uint32_t>(__popcll(am[ch]));
         }
     }
 }
@@ -1334,115 +1390,96 @@ __global__ __launch_bounds__(kBlock) void k_propagate_resume(ckf_params P) {
 }
 
 // After k_propagate: the next step's inputs (links that reached a surface)
-// and the tips, compacted in link order (partitions of up to 1024 links); the
-// last block to leave runs the step advance (fused_advance) so the step loop
-// never waits on the host.
+// and the tips, compacted in link order (partitions of up to 1,024 links); the
+// block that finishes the step's last partition runs the step advance
+// (fused_advance) so the step loop never waits on the host.
 __global__ __launch_bounds__(kBlock) void k_prop_emit(ckf_params P, int fused_advance) {
-    __shared__ uint32_t s_exit;  // waves of this block past the queue
+    __shared__ emit_shared S;
     step_ctl* ctl = P.ctl;
     if (ctl->done) {
-        return;  // the whole grid returns
+        return;
     }
-    if (threadIdx.x == 0u) {
-        s_exit = 0u;
-    }
-    __syncthreads();
     const uint32_t n = links_this_step(P, ctl);
     const uint32_t base = ctl->link_base;
     const uint32_t epoch = ctl->epoch;
     const uint32_t tip_base = ctl->n_tips;
     const uint32_t kc = emit_chunks(n);
-    const uint32_t part = kWave * kc;
+    const uint32_t part = kBlock * kc;
     const uint32_t n_parts = (n + part - 1u) / part;
-    const bool takes = wave_takes_tickets(n_parts);
+    if (blockIdx.x >= n_parts) {
+        // a step abandoned by an overflow has no links and no partition that
+        // could end it
+        if (blockIdx.x == 0u && threadIdx.x == 0u && fused_advance && (ctl->overflow & kFindOverflow) != 0u) {
+            ctl->n_live = 0u;
+            ctl->n_tips_step = 0u;
+            advance_step(P, ctl);
+        }
+        return;
+    }
     for (;;) {
-        const uint32_t p = takes ? wave_ticket(&ctl->ticket[5].v) : n_parts;
+        const uint32_t p = block_ticket(&ctl->ticket[5].v, S);
         if (p >= n_parts) {
             break;
         }
-        const uint32_t i0 = p * part;
-        uint32_t fl[kEmitChunks];
-        uint32_t s_tot = 0u, t_tot = 0u;
+        const uint32_t i0 = p * part + threadIdx.x;
+        uint32_t fl[kEmitChunks], live_at[kEmitChunks], tip_at[kEmitChunks];
 #pragma unroll
-        for (int ch = 0; ch < static_cast<int>(kEmitChunks); ++ch) {
-            const uint32_t i = i0 + static_cast<uint32_t>(ch) * kWave + lane();
-            fl[ch] = (static_cast<uint32_t>(ch) < kc && i < n) ? P.prop_flag[i] : 0u;
-            s_tot += static_cast<uint32_t>(__popcll(wave_ballot((fl[ch] & 1u) != 0u)));
-            t_tot += static_cast<uint32_t>(__popcll(wave_ballot((fl[ch] >> 1) >= 1u)) +
-                                           __popcll(wave_ballot((fl[ch] >> 1) >= 2u)));
+        for (uint32_t ch = 0; ch < kEmitChunks; ++ch) {
+            const uint32_t i = i0 + ch * kBlock;
+            fl[ch] = (ch < kc && i < n) ? P.prop_flag[i] : 0u;
+            live_at[ch] = fl[ch] & 1u;
+            tip_at[ch] = fl[ch] >> 1;
         }
-        const uint64_t b = wave_lookback(P.lb_lo[2], P.lb_hi[2], p, epoch,
-                                         pack2(s_tot, t_tot));
-        uint32_t s_run = lo32(b), t_run = hi32(b);
+        const uint32_t s_tot = block_prefix(live_at, 0, S);
+        const uint32_t t_tot = block_prefix(tip_at, 1, S);
+        const uint64_t b = block_lookback(P.lb_lo[2], P.lb_hi[2], p, epoch, pack2(s_tot, t_tot), S);
 #pragma unroll
-        for (int ch = 0; ch < static_cast<int>(kEmitChunks); ++ch) {
-            const uint32_t i = i0 + static_cast<uint32_t>(ch) * kWave + lane();
-            const uint32_t f = fl[ch];
-            const bool succ = (f & 1u) != 0u;
-            const uint32_t ntip = f >> 1;
-            const uint64_t ms = wave_ballot(succ);
-            const uint64_t m1 = wave_ballot(ntip >= 1u);
-            const uint64_t m2 = wave_ballot(ntip >= 2u);
-            if (succ) {
-                const uint32_t pos = s_run + prefix_count(ms);
+        for (uint32_t ch = 0; ch < kEmitChunks; ++ch) {
+            const uint32_t i = i0 + ch * kBlock;
+            if ((fl[ch] & 1u) != 0u) {
+                const uint32_t pos = lo32(b) + live_at[ch];
                 if (pos < P.in_cap) {
                     P.live[pos] = i;
                 } else {
                     set_overflow(ctl, 16u);
                 }
             }
-            if (ntip > 0u) {
-                uint32_t pos = tip_base + t_run + prefix_count(m1) + prefix_count(m2);
-                for (uint32_t k = 0; k < ntip; ++k, ++pos) {
-                    if (pos < P.tip_cap) {
-                        P.tips[pos] = base + i;
-                    } else {
-                        set_overflow(ctl, 8u);
-                    }
+            uint32_t pos = tip_base + hi32(b) + tip_at[ch];
+            for (uint32_t k = 0; k < (fl[ch] >> 1); ++k, ++pos) {
+                if (pos < P.tip_cap) {
+                    P.tips[pos] = base + i;
+                } else {
+                    set_overflow(ctl, 8u);
                 }
             }
-            s_run += static_cast<uint32_t>(__popcll(ms));
-            t_run += static_cast<uint32_t>(__popcll(m1) + __popcll(m2));
         }
-        if (p == n_parts - 1u && lane() == 0u && !fused_advance) {
-            ctl->n_live = lo32(b) + s_tot;
-            ctl->n_tips_step = hi32(b) + t_tot;
-        }
-    }
-    if (fused_advance) {
-        // The last block to leave runs the step advance.  Every wave of the
-        // grid (ticket holder or not) counts itself once it has read the
-        // control block -- in LDS, then the block's last wave with one device
-        // atomic -- so no wave can start on the advanced control block.  The
-        // step's totals come from the last partition's look-back words, which
-        // carry their own visibility; the overflow bits that other blocks of
-        // this kernel raise are read with a device-scope atomic load (the
-        // bits they set with atomicOr live at the device's coherence point);
-        // everything else the advance reads was written by earlier kernels,
-        // and its own stores reach the next kernel at the launch boundary.
-        uint32_t in_block = 0u;
-        if (lane() == 0u) {
-            in_block = atomicAdd(&s_exit, 1u) + 1u;
-        }
-        in_block = wave_broadcast(in_block, 0);
-        if (in_block == blockDim.x / kWave) {
-            uint32_t before = 0u;
-            if (lane() == 0u) {
-                before = atomicAdd(&ctl->exit_count.v, 1u);
+        if (!fused_advance) {
+            if (p == n_parts - 1u && threadIdx.x == 0u) {
+                ctl->n_live = lo32(b) + s_tot;
+                ctl->n_tips_step = hi32(b) + t_tot;
             }
-            before = wave_broadcast(before, 0);
-            if (before + 1u == gridDim.x) {
-                uint32_t live = 0u, tips = 0u;
-                if (n_parts > 0u) {
-                    live = lookback_inclusive(P.lb_lo[2], n_parts - 1u, epoch);
-                    tips = lookback_inclusive(P.lb_hi[2], n_parts - 1u, epoch);
-                }
-                if (lane() == 0u) {
-                    ctl->n_live = live;
-                    ctl->n_tips_step = tips;
-                    advance_step(P, ctl);
-                    ctl->exit_count.v = 0u;
-                }
+            continue;
+        }
+        // The block that finishes the last partition advances the step: every
+        // partition counts itself once it is written (counting every block of
+        // the grid instead cost a 1,024-block grid 15 us of atomics on one
+        // word).  A block that starts after the advance does nothing: it finds
+        // done, or no links, or (with the step's old counts) a spent queue,
+        // which k_find_emit clears in the next step.  The step's totals come
+        // from the last partition's look-back words, which carry their own
+        // visibility; the overflow bits that other blocks raise are read with a
+        // device-scope atomic load (the bits they set with atomicOr live at the
+        // device's coherence point); everything else the advance reads was
+        // written by earlier kernels, and its own stores reach the next kernel
+        // at the launch boundary.
+        __syncthreads();
+        if (threadIdx.x == 0u) {
+            const uint32_t before = atomicAdd(&ctl->exit_count.v, 1u);
+            if (before + 1u == n_parts) {
+                ctl->exit_count.v = 0u;
+                ctl->n_live = lookback_inclusive(P.lb_lo[2], n_parts - 1u, epoch);
+                ctl->n_tips_step = lookback_inclusive(P.lb_hi[2], n_parts - 1u, epoch);
+                advance_step(P, ctl);
             }
         }
     }
@@ -1466,7 +1503,9 @@ __device__ void advance_step(const ckf_params& P, step_ctl* ctl) {
     ctl->step += 1u;
     ctl->n_steps_run = ctl->step;
     ctl->epoch += 1u;
-    for (int k = 0; k < kTickets; ++k) ctl->ticket[k].v = 0u;
+    for (int k = 0; k < kTickets; ++k) {
+        if (k != 5) ctl->ticket[k].v = 0u;  // [5] is still being taken from: see k_find_emit
+    }
     ctl->n_defer.v = 0u;
     for (int q = 0; q < 4; ++q) {
         for (uint32_t x = 0; x < kXcds; ++x) ctl->xcd_ticket[q][x].v = 0u;
@@ -1491,94 +1530,80 @@ __global__ void k_advance(ckf_params P) {
 // ---------------------------------------------------------------------------
 // Tips in (step, event) segments: each tip's kept rank and constituent
 // prefix, and every segment's bounds.  A partition is emit_chunks(n) chunks
-// of 64 tips with one look-back, so the look-back chain stays short when
-// there are millions of tips; the (event, step) key of a tip is
+// of kBlock tips with one look-back; the (event, step) key of a tip is
 // ev * max_cands + step (the host keeps n_events * max_cands below 2^31).
 __global__ __launch_bounds__(kBlock) void k_build_scan(ckf_params P) {
+    __shared__ emit_shared S;
     step_ctl* ctl = P.ctl;
     const uint32_t n = ctl->n_tips < P.tip_cap ? ctl->n_tips : P.tip_cap;
     const uint32_t epoch = ctl->epoch;
     const uint32_t kc = emit_chunks(n);
-    const uint32_t part = kWave * kc;
+    const uint32_t part = kBlock * kc;
     const uint32_t n_parts = (n + part - 1u) / part;
-    const uint32_t S = P.max_cands;
-    auto seg_key = [&](uint32_t g) -> uint32_t {
-        const dlink L = load_link(P, g);
-        return P.seed_event[L.seed] * S + link_step(L);
-    };
-    const bool takes = wave_takes_tickets(n_parts);
+    const uint32_t n_steps = P.max_cands;
+    if (blockIdx.x >= n_parts) {
+        return;
+    }
     for (;;) {
-        const uint32_t p = takes ? wave_ticket(&ctl->ticket[3].v) : n_parts;
+        const uint32_t p = block_ticket(&ctl->ticket[3].v, S);
         if (p >= n_parts) {
             break;
         }
-        const uint32_t t0 = p * part;
-        uint32_t kn[kEmitChunks];   // keep << 31 | n_cands
-        uint32_t key[kEmitChunks];  // segment key
-        uint32_t k_tot = 0u, c_tot = 0u;
+        const uint32_t t0 = p * part + threadIdx.x;
+        uint32_t kn[kEmitChunks];    // keep << 31 | n_cands
+        uint32_t key[kEmitChunks];   // segment key
+        uint32_t prev[kEmitChunks];  // segment key of the tip before
+        uint32_t kp[kEmitChunks], cp[kEmitChunks];
 #pragma unroll
-        for (int ch = 0; ch < static_cast<int>(kEmitChunks); ++ch) {
-            const uint32_t t = t0 + static_cast<uint32_t>(ch) * kWave + lane();
-            kn[ch] = 0u;
-            key[ch] = 0u;
-            if (static_cast<uint32_t>(ch) < kc && t < n) {
+        for (uint32_t ch = 0; ch < kEmitChunks; ++ch) {
+            const uint32_t t = t0 + ch * kBlock;
+            kn[ch] = key[ch] = prev[ch] = 0u;
+            if (ch < kc && t < n) {
                 const dlink L = load_link(P, P.tips[t]);
                 const uint32_t st = link_step(L);
                 const uint32_t nc = st + 1u - link_skipped(L);
                 const bool keep = nc >= P.min_cands && nc <= P.max_cands;
                 kn[ch] = (keep ? 0x80000000u : 0u) | nc;
-                key[ch] = P.seed_event[L.seed] * S + st;
+                key[ch] = P.seed_event[L.seed] * n_steps + st;
+                if (lane() == 0u && t > 0u) {
+                    const dlink B = load_link(P, P.tips[t - 1u]);
+                    prev[ch] = P.seed_event[B.seed] * n_steps + link_step(B);
+                }
             }
-            const bool keep = (kn[ch] >> 31) != 0u;
-            k_tot += static_cast<uint32_t>(__popcll(wave_ballot(keep)));
-            c_tot += wave_broadcast(wave_inclusive_scan(keep ? (kn[ch] & 0x7fffffffu) : 0u), kWave - 1);
-        }
-        const uint64_t b = wave_lookback(P.lb_lo[3], P.lb_hi[3], p, epoch,
-                                         pack2(k_tot, c_tot));
-        uint32_t k_run = lo32(b), c_run = hi32(b);
-        // segment key of the tip before this partition's first
-        uint32_t key_before = 0u;
-        if (t0 > 0u && t0 < n) {
-            key_before = seg_key(P.tips[t0 - 1u]);
-        }
-#pragma unroll
-        for (int ch = 0; ch < static_cast<int>(kEmitChunks); ++ch) {
-            if (static_cast<uint32_t>(ch) >= kc) {
-                continue;  // kc is wave-uniform
-            }
-            const uint32_t t = t0 + static_cast<uint32_t>(ch) * kWave + lane();
-            const bool keep = (kn[ch] >> 31) != 0u;
-            const uint32_t nc = kn[ch] & 0x7fffffffu;
-            const uint32_t w = keep ? nc : 0u;
-            const uint32_t cincl = wave_inclusive_scan(w);
-            const uint64_t mk = wave_ballot(keep);
-            // the previous tip's key: the lane below, across chunk boundaries
             const uint32_t below = __shfl(key[ch], static_cast<int>((lane() + kWave - 1u) % kWave), kWave);
-            const uint32_t prev_key = lane() == 0u ? key_before : below;
-            if (t < n) {
-                const uint32_t kp = k_run + prefix_count(mk);
-                const uint32_t cp = c_run + cincl - w;
-                P.tip_keep[t] = kn[ch];
-                P.tip_rank[t] = kp;
-                P.tip_cprefix[t] = cp;
-                const uint32_t seg = key[ch];
-                if (t == 0u || prev_key != seg) {
-                    P.seg_base[seg] = kp;
-                    P.seg_cbase[seg] = cp;
-                    // the previous segment ends where this one starts
-                    if (t > 0u) {
-                        P.seg_count[prev_key] = kp;
-                        P.seg_ccount[prev_key] = cp;
-                    }
-                }
-                if (t + 1u == n) {
-                    P.seg_count[seg] = kp + (keep ? 1u : 0u);
-                    P.seg_ccount[seg] = cp + w;
+            prev[ch] = lane() == 0u ? prev[ch] : below;
+            kp[ch] = kn[ch] >> 31;
+            cp[ch] = (kn[ch] >> 31) != 0u ? kn[ch] & 0x7fffffffu : 0u;
+        }
+        const uint32_t k_tot = block_prefix(kp, 0, S);
+        const uint32_t c_tot = block_prefix(cp, 1, S);
+        const uint64_t b = block_lookback(P.lb_lo[3], P.lb_hi[3], p, epoch, pack2(k_tot, c_tot), S);
+#pragma unroll
+        for (uint32_t ch = 0; ch < kEmitChunks; ++ch) {
+            const uint32_t t = t0 + ch * kBlock;
+            if (ch >= kc || t >= n) {
+                continue;
+            }
+            const bool keep = (kn[ch] >> 31) != 0u;
+            const uint32_t kr = lo32(b) + kp[ch];
+            const uint32_t cr = hi32(b) + cp[ch];
+            P.tip_keep[t] = kn[ch];
+            P.tip_rank[t] = kr;
+            P.tip_cprefix[t] = cr;
+            const uint32_t seg = key[ch];
+            if (t == 0u || prev[ch] != seg) {
+                P.seg_base[seg] = kr;
+                P.seg_cbase[seg] = cr;
+                // the previous segment ends where this one starts
+                if (t > 0u) {
+                    P.seg_count[prev[ch]] = kr;
+                    P.seg_ccount[prev[ch]] = cr;
                 }
             }
-            key_before = wave_broadcast(key[ch], kWave - 1);
-            k_run += static_cast<uint32_t>(__popcll(mk));
-            c_run += wave_broadcast(cincl, kWave - 1);
+            if (t + 1u == n) {
+                P.seg_count[seg] = kr + (keep ? 1u : 0u);
+                P.seg_ccount[seg] = cr + (keep ? kn[ch] & 0x7fffffffu : 0u);
+            }
         }
     }
 }
