@@ -71,3 +71,25 @@ def test_compaction_partition_edges(n):
         g = got.event(e)
         assert np.array_equal(g.offsets, w.offsets), e
         assert np.array_equal(g.constituents, w.constituents), e
+
+
+@pytest.mark.parametrize("minimum", [0, 1, 2, 3, 4, 7])
+def test_duplicate_removal_lengths(minimum):
+    """Links are compared by the hash of the measurements that duplicates must
+    share, which are fewer than four for a small minimum length: the tracks are
+    the oracle's for every minimum (dense enough that some links are dropped)."""
+    import oracle
+    det, fld, gun = S.workload("C4", n_particles=2500, seed=37)
+    ev = S.generate_event(det, fld, gun)
+    # every second seed again: identical histories from different seeds
+    again = np.concatenate([np.arange(ev.n_seeds), np.arange(0, ev.n_seeds, 2)])
+    ev = S.with_seeds(ev, ev.seed_surface_link[again], ev.seed_vector[again], ev.seed_covariance[again],
+                      ev.seed_particle[again])
+    cfg = S.finding_config_for("C4")
+    cfg.max_num_branches_per_surface = 3
+    cfg.duplicate_removal_minimum_length = minimum
+    got = ckf.combinatorial_kalman_filter_algorithm(cfg)(det, fld, ev)
+    want = oracle.run(cfg, det, fld, ev, 64)
+    assert len(want) < 1.5 * len(again)
+    assert np.array_equal(got.offsets, want.offsets)
+    assert np.array_equal(got.constituents, want.constituents)

@@ -60,6 +60,22 @@ struct stage_cand {
 };
 static_assert(sizeof(stage_head) == 32 && sizeof(stage_cand) == 8, "stage record sizes");
 
+// A link's measurement history in short: its four latest measurements, a hash
+// of all, the first two and how many (a root's: zeros).
+struct alignas(16) link_history {
+    uint4 last;
+    uint32_t all, first, second, count;
+};
+
+// A link in its duplicate-removal list.
+struct alignas(16) dedup_node {
+    uint32_t next;  // the list's next link of the step, kInvalid at its end
+    float p;        // the link's p-value
+    uint32_t hash;  // of its latest measurements
+    uint32_t head;  // its list
+    uint32_t all, first, second, count;  // of its history
+};
+
 TAMD_HD uint32_t link_step(const dlink& l) { return l.packed & 0xffffu; }
 TAMD_HD uint32_t link_skipped(const dlink& l) { return (l.packed >> 16) & 0xffu; }
 TAMD_HD uint32_t link_consec(const dlink& l) { return (l.packed >> 24) & 0xffu; }
@@ -113,7 +129,7 @@ struct step_ctl {
     uint64_t n_scored;        // scorer rows of the finished steps
     line_u32 ticket[kTickets];  // work-queue tickets: [0] progressive filter, [1] votes /
                                 // progressive filter, [2] free, [3] build, [4] find emit,
-                                // [5] propagate emit, [6] dedup emit, [7] free, [8] free
+                                // [5] propagate emit, [6] free, [7] resume, [8] free
     line_u32 exit_count;  // blocks of k_prop_emit that have finished this step
     line_u32 n_rows;      // scorer rows scored this step (added up by k_score_update)
     line_u64 n_props;     // propagations so far
@@ -170,10 +186,10 @@ struct ckf_params {
     uint32_t* tips;               // [tip_cap] global link indices
     uint32_t tip_cap;
     uint32_t* seed_first;         // [n_seeds] local index of the seed's first link this step
-    uint32_t* seed_base;          // [n_seeds] alive-prefix at that link (dedup steps)
-    uint32_t* alive_prefix;       // [state_cap] bit 31 = alive, low bits = exclusive alive prefix
+    link_history* history[2];     // [state_cap] each link's history, by step parity
+    uint64_t* alive_bits;         // [state_cap / 64 + 1] surviving links, a bit each (dedup steps)
     uint64_t* dedup_head;         // [n_meas + 1] epoch << 32 | link (epoch-tagged list heads)
-    uint32_t* dedup_next;         // [state_cap]
+    dedup_node* dedup_nodes;      // [state_cap]
     uint64_t* lb_lo[kLookbacks];  // look-back words per compaction: low counter channel
     uint64_t* lb_hi[kLookbacks];  // and high counter channel
     uint32_t lb_cap;

@@ -6,7 +6,8 @@
 //                 gain-matrix update, hole links; links are compacted in input
 //                 order with a wave scan + decoupled look-back
 //                 (traccc host: details/combinatorial_kalman_filter.hpp:174-364)
-//   k_dedup_*     duplicate removal grouped by last measurement
+//   k_dedup_mark  duplicate removal grouped by last measurement (the groups'
+//                 lists are made where the links are, in k_find_emit)
 //                 (traccc host :371-488)
 //   k_propagate   one lane per link: per-seed cap, hole limits, RK4 transport
 //                 to the next sensitive surface, tips; next-step inputs and
@@ -414,12 +415,14 @@ __device__ inline dlink staged_link(const stage_head& h, const stage_cand& c, ui
 constexpr uint32_t kEmitChunks = 4;
 constexpr uint32_t kEmitWaves = kBlock / kWave;
 
-// Chunks per partition for n items: one per 64 partitions' worth of work, at
-// most kEmitChunks -- a look-back round trip covers 64 partitions, so the
-// chain any partition waits on stays at a round or two, while small steps
-// still spread over many blocks.
-__device__ inline uint32_t emit_chunks(uint32_t n) {
-    const uint32_t c = n / (kBlock * 64u);
+// Chunks per partition for n items: one until there are `parts` partitions,
+// then more, at most kEmitChunks.  A look-back round trip covers 64 partitions,
+// so that many keep its chain at a round (k_prop_emit, 200,000 links: 12 us, 24
+// with 512); k_find_emit, whose items cost more than the chain, takes two for
+// every CU (with duplicate lists to make, 160,000 inputs: 38 us, 60 with 64).
+constexpr uint32_t kLightParts = 64u, kHeavyParts = 512u;
+__device__ inline uint32_t emit_chunks(uint32_t n, uint32_t parts) {
+    const uint32_t c = n / (kBlock * parts);
     return c < 1u ? 1u : (c > kEmitChunks ? kEmitChunks : c);
 }
 
@@ -900,6 +903,75 @@ __global__ __launch_bounds__(kBlock) void k_find(ckf_params P) {
     }
 }
 
+// Duplicate removal drops a link when another one has its measurement
+// history.  Both are longer than dup_min_len measurements, so they agree in
+// that many of their latest ones: every link carries a summary of its history
+// (from its previous link's), links enter a list by the hash of those that must
+// agree, and k_dedup_mark walks the histories of two links of a list only where
+// their summaries allow it.  (Lists by the last measurement alone, as the rule
+// states it, held 50 and more links in dense events, and the branches of a seed
+// that parted early agree in all that follows: a chain of dependent loads of
+// 50-110 us a step, however few links the step had.)
+__device__ inline link_history extend_history(const link_history& h, uint32_t meas) {
+    link_history r = h;
+    if (meas != kInvalid) {
+        r.last = make_uint4(meas, h.last.x, h.last.y, h.last.z);
+        uint32_t f = (h.all ^ meas) * 0x9e3779b1u;
+        r.all = f ^ (f >> 15);
+        r.first = h.count == 0u ? meas : h.first;
+        r.second = h.count == 1u ? meas : h.second;
+        r.count = h.count + 1u;
+    }
+    return r;
+}
+
+__device__ inline uint32_t latest_hash(const ckf_params& P, const uint4& r) {
+    uint32_t h = r.x * 0x9e3779b1u;
+    h ^= h >> 15;
+    if (P.dup_min_len >= 1u) h = (h ^ r.y) * 0x85ebca77u;
+    h ^= h >> 13;
+    if (P.dup_min_len >= 2u) h = (h ^ r.z) * 0xc2b2ae3du;
+    h ^= h >> 16;
+    if (P.dup_min_len >= 3u) h = (h ^ r.w) * 0x27d4eb2fu;
+    return h ^ (h >> 15);
+}
+
+// Enter link i of the step (L, with its history) into its list, with its
+// p-value, computed once per link instead of once per pair (the series and the
+// continued fraction take ~50 divisions).  A link that is too short neither
+// drops another one nor is dropped: kDedupShort stands for it.
+constexpr uint32_t kDedupShort = 0xffffffffu;
+
+__device__ inline void dedup_insert(const ckf_params& P, const dlink& L, const link_history& r, uint32_t i,
+                                    uint32_t step, uint32_t epoch) {
+    if (step + 1u - link_skipped(L) <= P.dup_min_len) {
+        P.dedup_nodes[i].head = kDedupShort;
+        return;
+    }
+    dedup_node node;
+    node.hash = latest_hash(P, r.last);
+    node.head = static_cast<uint32_t>((static_cast<uint64_t>(node.hash) * (P.n_meas + 1u)) >> 32);
+    // list heads carry the step's epoch: a head from an earlier step reads as empty
+    const unsigned long long tagged = (static_cast<unsigned long long>(epoch) << 32) | i;
+    const unsigned long long old =
+        atomicExch(reinterpret_cast<unsigned long long*>(&P.dedup_head[node.head]), tagged);
+    node.next = (static_cast<uint32_t>(old >> 32) == epoch) ? static_cast<uint32_t>(old) : kInvalid;
+    node.p = prob_chi2(L.chi2_sum, static_cast<float>(L.ndf_sum - 5u));
+    node.all = r.all;
+    node.first = r.first;
+    node.second = r.second;
+    node.count = r.count;
+    P.dedup_nodes[i] = node;
+}
+
+// Can a's history be contained in b's?  Equal numbers of measurements: the
+// whole histories agree.  One more in b: a's first is b's second.
+__device__ inline bool may_contain(const dedup_node& a, const dedup_node& b) {
+    if (a.count == b.count) return a.all == b.all;
+    if (a.count + 1u == b.count) return a.first == b.second;
+    return a.count < b.count;
+}
+
 // Links of the step, after k_find: the inputs' link counts (kept branches, or
 // one hole link) laid out in input order, then the links written.  Kept apart
 // from k_find so a partition with heavy inputs never holds the look-back
@@ -915,7 +987,8 @@ __global__ __launch_bounds__(kBlock) void k_find_emit(ckf_params P) {
     const uint32_t n_in = ctl->n_in < P.in_cap ? ctl->n_in : P.in_cap;
     const uint32_t link_base = ctl->link_base;
     const uint32_t epoch = ctl->epoch;
-    const uint32_t kc = emit_chunks(n_in);
+    const bool dedup = step >= P.dup_min_len;
+    const uint32_t kc = emit_chunks(n_in, kHeavyParts);
     const uint32_t part = kBlock * kc;
     const uint32_t n_parts = (n_in + part - 1u) / part;
     if (blockIdx.x == 0u && threadIdx.x == 0u) {
@@ -964,6 +1037,11 @@ __global__ __launch_bounds__(kBlock) void k_find_emit(ckf_params P) {
             if (i == 0u || prev_seed != seed) {
                 P.seed_first[seed] = at;
             }
+            // the previous link's history (a hole's state reference names its slot)
+            link_history before{};
+            if (step > 0u) {
+                before = P.history[(step + 1u) & 1u][h.hole_ref & kRefMask];
+            }
             for (uint32_t k = 0; k < n_out[ch]; ++k) {
                 const uint32_t slot = flt_slot(P, i, k);
                 if (slot >= P.flt_cap) {
@@ -973,6 +1051,11 @@ __global__ __launch_bounds__(kBlock) void k_find_emit(ckf_params P) {
                 const uint32_t g = link_base + at + k;
                 if (g < P.link_cap && at + k < P.state_cap) {
                     P.links[g] = L;
+                    const link_history r = extend_history(before, L.meas);
+                    P.history[step & 1u][at + k] = r;
+                    if (dedup) {
+                        dedup_insert(P, L, r, at + k, step, epoch);
+                    }
                     if constexpr (kLogging) {
                         if (L.meas != kInvalid) {
                             // a row is 48 B: three 16-byte pieces each way
@@ -1014,55 +1097,36 @@ __device__ inline uint32_t links_this_step(const ckf_params& P, const step_ctl* 
     return n < room ? n : room;
 }
 
-__global__ __launch_bounds__(kBlock) void k_dedup_insert(ckf_params P) {
-    const step_ctl* ctl = P.ctl;
-    if (ctl->done || ctl->step < P.dup_min_len || (ctl->overflow & kFindOverflow) != 0u) {
-        return;
-    }
-    const uint32_t n = links_this_step(P, ctl);
-    const uint32_t base = ctl->link_base;
-    const uint32_t epoch = ctl->epoch;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        dlink L = load_link(P, base + i);
-        while (L.meas == kInvalid && link_step(L) != 0u) {
-            L = load_link(P, L.prev);
-        }
-        const uint32_t key = (L.meas == kInvalid) ? P.n_meas : L.meas;
-        P.alive_prefix[i] = key;
-        // list heads carry the step's epoch: a head from an earlier step reads as empty
-        const unsigned long long tagged = (static_cast<unsigned long long>(epoch) << 32) | i;
-        const unsigned long long old = atomicExch(
-            reinterpret_cast<unsigned long long*>(&P.dedup_head[key]), tagged);
-        P.dedup_next[i] = (static_cast<uint32_t>(old >> 32) == epoch) ? static_cast<uint32_t>(old)
-                                                                       : kInvalid;
-    }
-}
-
 namespace {
 // Is track `a` dominated by `b` (identical measurement history down to a's
-// first link)?  traccc host :431-471.
+// first link)?  traccc host :431-471.  Two links with the same previous link
+// have the same history from there on, which ends the walk: the branches of a
+// seed mostly part a few links back.
 __device__ inline bool history_contained(const ckf_params& P, dlink a, dlink b) {
     for (;;) {
         while (a.meas == kInvalid && link_step(a) != 0u) a = load_link(P, a.prev);
         while (b.meas == kInvalid && link_step(b) != 0u) b = load_link(P, b.prev);
-        if (a.meas == b.meas) {
-            if (link_step(a) == 0u) return true;
-            if (link_step(b) == 0u) return false;
-            a = load_link(P, a.prev);
-            b = load_link(P, b.prev);
-        } else {
-            return false;
-        }
+        if (a.meas != b.meas) return false;
+        if (link_step(a) == 0u) return true;
+        if (link_step(b) == 0u) return false;
+        if (a.prev == b.prev) return true;
+        a = load_link(P, a.prev);
+        b = load_link(P, b.prev);
     }
 }
 }  // namespace
 
+// Which links survive: one bit each, a 64-bit word per partition of 64.  A
+// link is dropped when another has its history and a higher p-value (the lower
+// index on equal ones).  The list's nodes carry the p-values and what the
+// histories must agree in, so a pair costs one 32-byte load, and the histories
+// are walked only for the pairs that they decide.  k_propagate counts the bits of a seed's links for the
+// branch cap.
 __global__ __launch_bounds__(kBlock) void k_dedup_mark(ckf_params P) {
     step_ctl* ctl = P.ctl;
     if (ctl->done || ctl->step < P.dup_min_len || (ctl->overflow & kFindOverflow) != 0u) {
         return;
     }
-    const uint32_t step = ctl->step;
     const uint32_t n = links_this_step(P, ctl);
     const uint32_t base = ctl->link_base;
     const uint32_t epoch = ctl->epoch;
@@ -1074,87 +1138,48 @@ __global__ __launch_bounds__(kBlock) void k_dedup_mark(ckf_params P) {
             break;
         }
         const uint32_t i = p * kWave + lane();
-        const bool valid = i < n;
-        bool alive = true;
-        uint32_t seed = 0u;
-        if (valid) {
-            const dlink Li = load_link(P, base + i);
-            seed = Li.seed;
-            const uint32_t key = P.alive_prefix[i];
-            if (step + 1u - link_skipped(Li) > P.dup_min_len && Li.ndf_sum > 5u) {
-                const float p_this = prob_chi2(Li.chi2_sum, static_cast<float>(Li.ndf_sum - 5u));
-                const uint64_t h = P.dedup_head[key];
-                const uint32_t first = (static_cast<uint32_t>(h >> 32) == epoch)
-                                           ? static_cast<uint32_t>(h) : kInvalid;
-                for (uint32_t j = first; j != kInvalid; j = P.dedup_next[j]) {
-                    if (j == i) continue;
-                    const dlink Lj = load_link(P, base + j);
-                    if (step + 1u - link_skipped(Lj) <= P.dup_min_len || Li.ndf_sum <= 5u) continue;
-                    bool dominated = history_contained(P, Li, Lj);
-                    const float p_that = prob_chi2(Lj.chi2_sum, static_cast<float>(Lj.ndf_sum - 5u));
-                    if (p_this != p_that) {
-                        dominated = dominated && (p_that >= p_this);
-                    } else {
-                        dominated = dominated && (j < i);
-                    }
-                    if (dominated) {
+        bool alive = i < n;
+        dedup_node own{};
+        if (alive) {
+            own = P.dedup_nodes[i];
+        }
+        if (alive && own.head != kDedupShort) {
+            const uint64_t h = P.dedup_head[own.head];
+            uint32_t j = (static_cast<uint32_t>(h >> 32) == epoch) ? static_cast<uint32_t>(h) : kInvalid;
+            while (j != kInvalid) {
+                const dedup_node node = P.dedup_nodes[j];
+                const bool better = own.p != node.p ? node.p >= own.p : j < i;
+                if (j != i && node.hash == own.hash && better && may_contain(own, node)) {
+                    const dlink Li = load_link(P, base + i);
+                    if (Li.ndf_sum > 5u && history_contained(P, Li, load_link(P, base + j))) {
                         alive = false;
                         break;
                     }
                 }
+                j = node.next;
             }
         }
-        if (valid) {
-            P.alive_prefix[i] = alive ? 0x80000000u : 0u;  // ranks: k_dedup_emit
+        const uint64_t bits = wave_ballot(alive);
+        if (lane() == 0u) {
+            P.alive_bits[p] = bits;
         }
-        (void)seed;
     }
 }
 
-// After k_dedup_mark: each link's rank among the step's surviving links
-// (alive_prefix = alive bit | rank) and, per seed, the rank of its first link.
-__global__ __launch_bounds__(kBlock) void k_dedup_emit(ckf_params P) {
-    __shared__ emit_shared S;
-    step_ctl* ctl = P.ctl;
-    if (ctl->done || ctl->step < P.dup_min_len || (ctl->overflow & kFindOverflow) != 0u) {
-        return;
-    }
-    const uint32_t n = links_this_step(P, ctl);
-    const uint32_t base = ctl->link_base;
-    const uint32_t epoch = ctl->epoch;
-    const uint32_t kc = emit_chunks(n);
-    const uint32_t part = kBlock * kc;
-    const uint32_t n_parts = (n + part - 1u) / part;
-    if (blockIdx.x >= n_parts) {
-        return;
-    }
-    for (;;) {
-        const uint32_t p = block_ticket(&ctl->ticket[6].v, S);
-        if (p >= n_parts) {
-            break;
+// Surviving links among the step's links [from, to).
+__device__ inline uint32_t count_alive(const uint64_t* bits, uint32_t from, uint32_t to) {
+    uint32_t count = 0u;
+    for (uint32_t w = from / 64u; w * 64u < to; ++w) {
+        uint64_t b = bits[w];
+        if (w == from / 64u) {
+            b &= ~0ull << (from % 64u);
         }
-        const uint32_t i0 = p * part + threadIdx.x;
-        uint32_t alive[kEmitChunks], rank[kEmitChunks];
-#pragma unroll
-        for (uint32_t ch = 0; ch < kEmitChunks; ++ch) {
-            const uint32_t i = i0 + ch * kBlock;
-            alive[ch] = (ch < kc && i < n) ? P.alive_prefix[i] & 0x80000000u : 0u;
-            rank[ch] = alive[ch] >> 31;
+        if (to - w * 64u < 64u) {
+            b &= (1ull << (to % 64u)) - 1ull;
         }
-        const uint32_t total = block_prefix(rank, 0, S);
-        const uint32_t run = lo32(block_lookback(P.lb_lo[1], nullptr, p, epoch, pack2(total, 0u), S));
-#pragma unroll
-        for (uint32_t ch = 0; ch < kEmitChunks; ++ch) {
-            const uint32_t i = i0 + ch * kBlock;
-            if (ch < kc && i < n) {
-                P.alive_prefix[i] = alive[ch] | (run + rank[ch]);
-                const uint32_t seed = load_link(P, base + i).seed;
-                if (P.seed_first[seed] == i) {
-                    P.seed_base[seed] = run + rank[ch];
-                }
-            }
-        }
+        count += static_cast<uint32_t>(__popcll(b));
     }
+    return count;
 }
 
 __device__ void advance_step(const ckf_params& P, step_ctl* ctl);
@@ -1254,14 +1279,15 @@ __global__ __launch_bounds__(kBlock) void k_propagate(ckf_params P, uint32_t fro
         uint8_t flag = 0u;
         if (valid) {
             const dlink L = load_link(P, base + i);
+            // its place among the seed's (surviving) links, for the branch cap
+            const uint32_t first = P.seed_first[L.seed];
             bool alive = true;
-            uint32_t rank = 0u;
+            uint32_t rank = i - first;
             if (dedup) {
-                const uint32_t ap = P.alive_prefix[i];
-                alive = (ap >> 31) != 0u;
-                rank = (ap & 0x7fffffffu) - P.seed_base[L.seed];
-            } else {
-                rank = i - P.seed_first[L.seed];
+                alive = ((P.alive_bits[i / 64u] >> (i % 64u)) & 1ull) != 0ull;
+                if (rank >= P.n_branch_seed) {
+                    rank = count_alive(P.alive_bits, first, i);
+                }
             }
             if (alive && rank < P.n_branch_seed) {
                 if (link_skipped(L) > P.max_skip || link_consec(L) > P.max_consec) {
@@ -1403,7 +1429,7 @@ __global__ __launch_bounds__(kBlock) void k_prop_emit(ckf_params P, int fused_ad
     const uint32_t base = ctl->link_base;
     const uint32_t epoch = ctl->epoch;
     const uint32_t tip_base = ctl->n_tips;
-    const uint32_t kc = emit_chunks(n);
+    const uint32_t kc = emit_chunks(n, kLightParts);
     const uint32_t part = kBlock * kc;
     const uint32_t n_parts = (n + part - 1u) / part;
     if (blockIdx.x >= n_parts) {
@@ -1537,7 +1563,7 @@ __global__ __launch_bounds__(kBlock) void k_build_scan(ckf_params P) {
     step_ctl* ctl = P.ctl;
     const uint32_t n = ctl->n_tips < P.tip_cap ? ctl->n_tips : P.tip_cap;
     const uint32_t epoch = ctl->epoch;
-    const uint32_t kc = emit_chunks(n);
+    const uint32_t kc = emit_chunks(n, kLightParts);
     const uint32_t part = kBlock * kc;
     const uint32_t n_parts = (n + part - 1u) / part;
     const uint32_t n_steps = P.max_cands;
@@ -1959,9 +1985,7 @@ hipError_t launch_log_write(const ckf_params& P, uint32_t n, const uint32_t* blo
 }
 
 hipError_t launch_dedup(const ckf_params& P, const launch_shape& s, hipStream_t stream) {
-    hipLaunchKernelGGL(k_dedup_insert, dim3(s.dedup_blocks), dim3(kBlock), 0, stream, P);
     hipLaunchKernelGGL(k_dedup_mark, dim3(s.dedup_blocks), dim3(kBlock), 0, stream, P);
-    hipLaunchKernelGGL(k_dedup_emit, dim3(s.emit_blocks), dim3(kBlock), 0, stream, P);
     return hipGetLastError();
 }
 

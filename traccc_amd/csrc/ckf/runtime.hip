@@ -87,8 +87,8 @@ struct ckf_algorithm {
     uint32_t in_cap = 0, state_cap = 0, flt_cap = 0, link_cap = 0, tip_cap = 0, lb_cap = 0;
     uint32_t seed_cap = 0, meas_cap = 0, seg_cap = 0, ev_cap = 0;
     // work buffers
-    dbuf state[2], flt, stage_in, stage_slot, links, live, tips, seed_first, seed_base;
-    dbuf alive_prefix, dedup_head, dedup_next, lb_lo[tamd::kLookbacks], lb_hi[tamd::kLookbacks], ctl;
+    dbuf state[2], flt, stage_in, stage_slot, links, live, tips, seed_first;
+    dbuf history[2], alive_bits, dedup_head, dedup_nodes, lb_lo[tamd::kLookbacks], lb_hi[tamd::kLookbacks], ctl;
     dbuf tip_keep, tip_rank, tip_cprefix, seg_count, seg_ccount, seg_base, seg_cbase, seg_off,
         seg_coff, ev_toff, ev_coff;
     // measurement votes (max_num_tracks_per_measurement > 0)
@@ -125,7 +125,7 @@ struct ckf_algorithm {
             if (g) (void)hipGraphExecDestroy(g);
         }
         dbuf* all[] = {&state[0], &state[1], &flt, &stage_in, &stage_slot, &links, &live, &tips,
-                       &seed_first, &seed_base, &alive_prefix, &dedup_head, &dedup_next, &ctl,
+                       &seed_first, &history[0], &history[1], &alive_bits, &dedup_head, &dedup_nodes, &ctl,
                        &tip_keep, &tip_rank, &tip_cprefix, &seg_count, &seg_ccount, &seg_base,
                        &seg_cbase, &seg_off, &seg_coff, &ev_toff, &ev_coff, &vote_slots,
                        &vote_key, &vote_keep, &vote_rank, &vote_cpos, &vote_misc,
@@ -177,8 +177,9 @@ void ensure_buffers(ckf_algorithm& A, const ckf_device_event& ev) {
     A.defer.ensure(4u * size_t(tamd::kDeferWords) * A.defer_cap);
     A.tips.ensure(4u * size_t(A.tip_cap));
     A.seed_first.ensure(4u * size_t(std::max(ev.n_seeds, 1u)));
-    A.seed_base.ensure(4u * size_t(std::max(ev.n_seeds, 1u)));
-    A.alive_prefix.ensure(4u * size_t(A.state_cap));
+    A.history[0].ensure(sizeof(tamd::link_history) * size_t(A.state_cap));
+    A.history[1].ensure(sizeof(tamd::link_history) * size_t(A.state_cap));
+    A.alive_bits.ensure(8u * (size_t(A.state_cap) / 64u + 1u));
     {
         const size_t old = A.dedup_head.bytes;
         A.dedup_head.ensure(8u * (size_t(ev.n_meas) + 1u));
@@ -187,7 +188,7 @@ void ensure_buffers(ckf_algorithm& A, const ckf_device_event& ev) {
             hip_check(hipMemsetAsync(A.dedup_head.p, 0, A.dedup_head.bytes, A.stream), "memset");
         }
     }
-    A.dedup_next.ensure(4u * size_t(A.state_cap));
+    A.dedup_nodes.ensure(sizeof(tamd::dedup_node) * size_t(A.state_cap));
     for (int k = 0; k < tamd::kLookbacks; ++k) {
         for (dbuf* w : {&A.lb_lo[k], &A.lb_hi[k]}) {
             const size_t old = w->bytes;
@@ -298,10 +299,11 @@ tamd::ckf_params make_params(ckf_algorithm& A, const ckf_device_detector& D,
     P.tips = A.tips.as<uint32_t>();
     P.tip_cap = A.tip_cap;
     P.seed_first = A.seed_first.as<uint32_t>();
-    P.seed_base = A.seed_base.as<uint32_t>();
-    P.alive_prefix = A.alive_prefix.as<uint32_t>();
+    P.history[0] = A.history[0].as<tamd::link_history>();
+    P.history[1] = A.history[1].as<tamd::link_history>();
+    P.alive_bits = A.alive_bits.as<uint64_t>();
     P.dedup_head = A.dedup_head.as<uint64_t>();
-    P.dedup_next = A.dedup_next.as<uint32_t>();
+    P.dedup_nodes = A.dedup_nodes.as<tamd::dedup_node>();
     for (int k = 0; k < tamd::kLookbacks; ++k) {
         P.lb_lo[k] = A.lb_lo[k].as<uint64_t>();
         P.lb_hi[k] = A.lb_hi[k].as<uint64_t>();
