@@ -59,8 +59,15 @@
 namespace tamd {
 namespace {
 
-constexpr uint32_t kAmbBlock = 256;
+// Blocks of 1,024: appending to a list or adding to a counter takes one
+// atomic per block and pass.  All waves of a grid end on the same few words, so
+// with an atomic per wave of 64 those words bounded every kernel here (1 M
+// tracks, 5 M identifiers: k_amb_hot0 629 us for 20 MB, k_amb_output 179 us).
+constexpr uint32_t kAmbBlock = 1024;
+constexpr uint32_t kAmbWaves = kAmbBlock / kWave;
 constexpr uint32_t kSeqBlock = 1024;
+// identifiers of a track held in registers at a time
+constexpr uint32_t kIdChunk = 8;
 constexpr uint32_t kDead = 0u, kAlive = 1u;
 constexpr uint32_t kNone = 0xffffffffu;
 
@@ -78,6 +85,16 @@ struct amb_ctl {
     uint32_t pad[5];
 };
 
+// What the order of two tracks needs of each: one 16-byte load (as columns --
+// two offsets, count, p-value, state -- it was five scattered ones per entry of
+// every shared identifier's list).
+struct alignas(16) track_rec {
+    uint32_t n_shared;
+    uint32_t n_meas;
+    float pk;  // p-value, NaN as the lowest
+    uint32_t status;
+};
+
 struct amb_params {
     uint32_t n_tracks;
     uint32_t id_base;   // identifiers are in [id_base, id_base + id_bound)
@@ -87,8 +104,7 @@ struct amb_params {
     const uint32_t* off;   // [n_tracks + 1]
     const uint32_t* ids;   // absolute constituent positions off[t] ..
     const float* pval;
-    uint32_t* status;      // [n_tracks]
-    uint32_t* n_shared;    // [n_tracks]
+    track_rec* rec;        // [n_tracks]
     uint32_t* protect;     // [n_tracks] round tag (r + 1) of the tracks best on some identifier
     uint32_t* cand[2];     // [n_tracks]
     uint32_t* n_acc;       // [id_bound] accepted tracks holding the identifier
@@ -108,13 +124,10 @@ struct track_key {
     uint32_t t;
 };
 
-__device__ inline track_key key_of(const amb_params& P, uint32_t t) {
-    const uint32_t nm = P.off[t + 1] - P.off[t];
-    const uint32_t ns = P.n_shared[t];
+__device__ inline track_key key_of(const track_rec& r, uint32_t t) {
     track_key k;
-    k.rel = nm == 0u ? 0.f : __fdiv_rn(static_cast<float>(ns), static_cast<float>(nm));
-    const float p = P.pval[t];
-    k.pk = isnan(p) ? -INFINITY : p;
+    k.rel = r.n_meas == 0u ? 0.f : __fdiv_rn(static_cast<float>(r.n_shared), static_cast<float>(r.n_meas));
+    k.pk = r.pk;
     k.t = t;
     return k;
 }
@@ -140,87 +153,161 @@ __device__ inline uint32_t multiplicity(const amb_params& P, uint32_t t, uint32_
     return c;
 }
 
-// Append `value` for the lanes with `take` (called by the whole wave).
-__device__ inline void wave_append(uint32_t* counter, uint32_t* list, bool take, uint32_t value) {
+struct append_shared {
+    uint32_t tot[kAmbWaves];
+    uint32_t base;
+};
+
+// Append `value` for the threads with `take` (called by the whole block).
+__device__ inline void block_append(uint32_t* counter, uint32_t* list, bool take, uint32_t value,
+                                    append_shared& S) {
     const uint64_t m = wave_ballot(take);
-    if (m == 0ull) return;
-    const int leader = __builtin_ctzll(m);
-    uint32_t base = 0u;
-    if (lane() == static_cast<uint32_t>(leader)) base = atomicAdd(counter, __popcll(m));
-    base = __shfl(base, leader, kWave);
-    if (take) list[base + prefix_count(m)] = value;
+    const uint32_t w = threadIdx.x / kWave;
+    if (lane() == 0u) S.tot[w] = static_cast<uint32_t>(__popcll(m));
+    __syncthreads();
+    uint32_t before = 0u, total = 0u;
+#pragma unroll
+    for (uint32_t q = 0; q < kAmbWaves; ++q) {
+        before += q < w ? S.tot[q] : 0u;
+        total += S.tot[q];
+    }
+    if (threadIdx.x == 0u) S.base = total > 0u ? atomicAdd(counter, total) : 0u;
+    __syncthreads();
+    if (take) list[S.base + before + prefix_count(m)] = value;
 }
 
-__device__ inline void wave_count(uint32_t* counter, bool p) {
-    const uint64_t m = wave_ballot(p);
-    if (m != 0ull && lane() == static_cast<uint32_t>(__builtin_ctzll(m))) {
-        atomicAdd(counter, __popcll(m));
+// Add the threads' counts to a counter (called by the whole block).
+__device__ inline void block_count(uint32_t* counter, uint32_t n, append_shared& S) {
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) n += __shfl_xor(n, d, kWave);
+    __syncthreads();
+    if (lane() == 0u) S.tot[threadIdx.x / kWave] = n;
+    __syncthreads();
+    if (threadIdx.x == 0u) {
+        uint32_t total = 0u;
+        for (uint32_t q = 0; q < kAmbWaves; ++q) total += S.tot[q];
+        if (total > 0u) atomicAdd(counter, total);
     }
+}
+
+// The identifiers [j0, e) of a track whose constituents start at b, up to
+// kIdChunk of them, with a bit for each that is its first occurrence there.
+struct id_chunk {
+    uint32_t id[kIdChunk];
+    uint32_t n;
+    uint32_t fresh;
+};
+
+__device__ inline id_chunk load_ids(const uint32_t* ids, uint32_t b, uint32_t j0, uint32_t e) {
+    id_chunk c;
+    c.n = e - j0 < kIdChunk ? e - j0 : kIdChunk;
+    c.fresh = 0u;
+#pragma unroll
+    for (uint32_t k = 0; k < kIdChunk; ++k) c.id[k] = k < c.n ? ids[j0 + k] : 0u;
+#pragma unroll
+    for (uint32_t k = 0; k < kIdChunk; ++k) {
+        bool first = k < c.n;
+#pragma unroll
+        for (uint32_t q = 0; q < k; ++q) first = first && c.id[q] != c.id[k];
+        c.fresh |= first ? 1u << k : 0u;
+    }
+    for (uint32_t q = b; q < j0; ++q) {  // tracks longer than a chunk
+        const uint32_t id = ids[q];
+#pragma unroll
+        for (uint32_t k = 0; k < kIdChunk; ++k) {
+            if (c.id[k] == id) c.fresh &= ~(1u << k);
+        }
+    }
+    return c;
 }
 
 // Offsets non-decreasing and every identifier in range; a bad input leaves
 // the flag and takes no part in the counts (no access out of bounds).
 __global__ __launch_bounds__(kAmbBlock) void k_amb_count(amb_params P) {
+    __shared__ append_shared S;
+    uint32_t cands = 0u;
     for (uint32_t b0 = blockIdx.x * blockDim.x; b0 < P.n_tracks; b0 += gridDim.x * blockDim.x) {
         const uint32_t t = b0 + threadIdx.x;
-        bool cand = false;
-        if (t < P.n_tracks) {
-            const uint32_t b = P.off[t], e = P.off[t + 1];
-            P.n_shared[t] = 0u;
-            P.protect[t] = 0u;
-            if (e < b || e > P.n_entries) {
-                atomicOr(&P.ctl->bad_input, 1u);
-                P.status[t] = kDead;
-            } else {
-                cand = e - b >= P.min_meas;
-                P.status[t] = cand ? kAlive : kDead;
-                for (uint32_t j = b; cand && j < e; ++j) {
-                    const uint32_t id = P.ids[j] - P.id_base;
-                    if (P.ids[j] < P.id_base || id >= P.id_bound) {
+        if (t >= P.n_tracks) continue;
+        const uint32_t b = P.off[t], e = P.off[t + 1];
+        const float p = P.pval[t];
+        track_rec r{0u, e - b, isnan(p) ? -INFINITY : p, kDead};
+        P.protect[t] = 0u;
+        if (e < b || e > P.n_entries) {
+            atomicOr(&P.ctl->bad_input, 1u);
+        } else if (e - b >= P.min_meas) {
+            ++cands;
+            r.status = kAlive;
+            for (uint32_t j = b; j < e; j += kIdChunk) {
+                const id_chunk c = load_ids(P.ids, b, j, e);
+#pragma unroll
+                for (uint32_t k = 0; k < kIdChunk; ++k) {
+                    if (k >= c.n) continue;
+                    const uint32_t id = c.id[k] - P.id_base;
+                    if (c.id[k] < P.id_base || id >= P.id_bound) {
                         atomicOr(&P.ctl->bad_input, 2u);
-                        continue;
+                    } else if ((c.fresh >> k) & 1u) {
+                        atomicAdd(&P.n_acc[id], 1u);
                     }
-                    if (first_occurrence(P.ids, b, j)) atomicAdd(&P.n_acc[id], 1u);
                 }
             }
         }
-        wave_count(&P.ctl->n_candidates, cand);
+        P.rec[t] = r;
     }
+    block_count(&P.ctl->n_candidates, cands, S);
 }
 
 // The identifiers' track lists, each track's n_shared, and the first
 // candidate list (accepted tracks with n_shared >= 1).
 __global__ __launch_bounds__(kAmbBlock) void k_amb_fill(amb_params P) {
+    __shared__ append_shared S;
     for (uint32_t b0 = blockIdx.x * blockDim.x; b0 < P.n_tracks; b0 += gridDim.x * blockDim.x) {
         const uint32_t t = b0 + threadIdx.x;
         bool shared = false;
-        if (t < P.n_tracks && P.status[t] == kAlive) {
+        if (t < P.n_tracks && P.rec[t].status == kAlive) {
             const uint32_t b = P.off[t], e = P.off[t + 1];
             uint32_t ns = 0u;
-            for (uint32_t j = b; j < e; ++j) {
-                const uint32_t id = P.ids[j] - P.id_base;
-                if (P.ids[j] < P.id_base || id >= P.id_bound) continue;
-                if (first_occurrence(P.ids, b, j)) {
-                    P.list[P.list_off[id] + atomicAdd(&P.fill[id], 1u)] = t;
+            for (uint32_t j = b; j < e; j += kIdChunk) {
+                const id_chunk c = load_ids(P.ids, b, j, e);
+                // a chunk's counters, list places and offsets are in flight together
+                uint32_t acc[kIdChunk], at[kIdChunk], off[kIdChunk];
+                uint32_t good = 0u;
+#pragma unroll
+                for (uint32_t k = 0; k < kIdChunk; ++k) {
+                    const uint32_t id = c.id[k] - P.id_base;
+                    const bool in = k < c.n && c.id[k] >= P.id_base && id < P.id_bound;
+                    good |= in ? 1u << k : 0u;
+                    acc[k] = in ? P.n_acc[id] : 0u;
+                    // the list of an identifier that one track holds is never read
+                    const bool put = in && acc[k] >= 2u && ((c.fresh >> k) & 1u) != 0u;
+                    off[k] = put ? P.list_off[id] : 0u;
+                    at[k] = put ? atomicAdd(&P.fill[id], 1u) : 0u;
                 }
-                ns += P.n_acc[id] >= 2u ? 1u : 0u;
+#pragma unroll
+                for (uint32_t k = 0; k < kIdChunk; ++k) {
+                    if (((good >> k) & 1u) == 0u || acc[k] < 2u) continue;
+                    if ((c.fresh >> k) & 1u) P.list[off[k] + at[k]] = t;
+                    ++ns;
+                }
             }
-            P.n_shared[t] = ns;
+            P.rec[t].n_shared = ns;
             shared = ns >= 1u;
         }
-        wave_append(&P.ctl->n_cand[0], P.cand[0], shared, t);
+        block_append(&P.ctl->n_cand[0], P.cand[0], shared, t, S);
     }
 }
 
 __global__ __launch_bounds__(kAmbBlock) void k_amb_hot0(amb_params P) {
+    __shared__ append_shared S;
     for (uint32_t b0 = blockIdx.x * blockDim.x; b0 < P.id_bound; b0 += gridDim.x * blockDim.x) {
         const uint32_t m = b0 + threadIdx.x;
-        wave_append(&P.ctl->n_hot[0], P.hot[0], m < P.id_bound && P.n_acc[m] >= 2u, m);
+        block_append(&P.ctl->n_hot[0], P.hot[0], m < P.id_bound && P.n_acc[m] >= 2u, m, S);
     }
 }
 
 // Round r, first kernel: the best track of every shared identifier.
 __global__ __launch_bounds__(kAmbBlock) void k_amb_best(amb_params P, uint32_t r) {
+    __shared__ append_shared S;
     amb_ctl* c = P.ctl;
     if (c->done != 0u) return;
     if (r > 0u && c->removed[(r - 1u) & 1u] == 0u) {
@@ -245,23 +332,29 @@ __global__ __launch_bounds__(kAmbBlock) void k_amb_best(amb_params P, uint32_t r
             if (P.n_acc[m] >= 2u) {
                 keep = true;
                 track_key best{0.f, 0.f, kNone};
-                bool have = false;
-                for (uint32_t q = P.list_off[m]; q < P.list_off[m + 1u]; ++q) {
-                    const uint32_t u = P.list[q];
-                    if (P.status[u] != kAlive) continue;
-                    const track_key k = key_of(P, u);
-                    if (!have || worse(best, k)) {
-                        best = k;
-                        have = true;
+                const uint32_t q1 = P.list_off[m + 1u];
+                // four entries and their records in flight at a time
+                for (uint32_t q = P.list_off[m]; q < q1; q += 4u) {
+                    uint32_t u[4];
+                    track_rec rec[4];
+#pragma unroll
+                    for (uint32_t k = 0; k < 4u; ++k) u[k] = P.list[q + k < q1 ? q + k : q];
+#pragma unroll
+                    for (uint32_t k = 0; k < 4u; ++k) rec[k] = P.rec[u[k]];
+#pragma unroll
+                    for (uint32_t k = 0; k < 4u; ++k) {
+                        if (q + k >= q1 || rec[k].status != kAlive) continue;
+                        const track_key key = key_of(rec[k], u[k]);
+                        if (best.t == kNone || worse(best, key)) best = key;
                     }
                 }
-                if (have) {
+                if (best.t != kNone) {
                     P.best_of[m] = best.t;
                     P.protect[best.t] = r + 1u;
                 }
             }
         }
-        wave_append(&c->n_hot[(r + 1u) & 1u], P.hot[(r + 1u) & 1u], keep, m);
+        block_append(&c->n_hot[(r + 1u) & 1u], P.hot[(r + 1u) & 1u], keep, m, S);
     }
 }
 
@@ -269,6 +362,7 @@ __global__ __launch_bounds__(kAmbBlock) void k_amb_best(amb_params P, uint32_t r
 // identifiers.  Only protected tracks have n_shared lowered here, and a
 // protected track is never removed, so the removal test reads stable values.
 __global__ __launch_bounds__(kAmbBlock) void k_amb_remove(amb_params P, uint32_t r) {
+    __shared__ append_shared S;
     amb_ctl* c = P.ctl;
     if (c->done != 0u) return;
     if (blockIdx.x == 0u && threadIdx.x == 0u) {
@@ -276,13 +370,15 @@ __global__ __launch_bounds__(kAmbBlock) void k_amb_remove(amb_params P, uint32_t
     }
     const uint32_t nt = c->n_cand[r & 1u];
     const uint32_t* T = P.cand[r & 1u];
+    uint32_t removed = 0u;
     for (uint32_t b0 = blockIdx.x * blockDim.x; b0 < nt; b0 += gridDim.x * blockDim.x) {
         const uint32_t i = b0 + threadIdx.x;
         bool keep = false, removing = false;
         uint32_t t = 0u;
         if (i < nt) {
             t = T[i];
-            if (P.status[t] == kAlive && P.n_shared[t] >= 1u) {
+            const track_rec rec = P.rec[t];
+            if (rec.status == kAlive && rec.n_shared >= 1u) {
                 if (P.protect[t] == r + 1u) {
                     keep = true;
                 } else {
@@ -290,23 +386,31 @@ __global__ __launch_bounds__(kAmbBlock) void k_amb_remove(amb_params P, uint32_t
                 }
             }
         }
-        wave_append(&c->n_cand[(r + 1u) & 1u], P.cand[(r + 1u) & 1u], keep, t);
-        wave_count(&c->removed[r & 1u], removing);
-        wave_count(&c->total_removed, removing);
+        block_append(&c->n_cand[(r + 1u) & 1u], P.cand[(r + 1u) & 1u], keep, t, S);
         if (removing) {
-            P.status[t] = kDead;
+            ++removed;
+            P.rec[t].status = kDead;
             const uint32_t b = P.off[t], e = P.off[t + 1];
-            for (uint32_t j = b; j < e; ++j) {
-                if (!first_occurrence(P.ids, b, j)) continue;
-                const uint32_t id = P.ids[j] - P.id_base;
-                if (atomicSub(&P.n_acc[id], 1u) == 2u) {
-                    // the identifier's one remaining track is its best
-                    const uint32_t s = P.best_of[id];
-                    if (s < P.n_tracks) atomicSub(&P.n_shared[s], multiplicity(P, s, P.ids[j]));
+            for (uint32_t j = b; j < e; j += kIdChunk) {
+                const id_chunk ch = load_ids(P.ids, b, j, e);
+                uint32_t before[kIdChunk];
+#pragma unroll
+                for (uint32_t k = 0; k < kIdChunk; ++k) {
+                    before[k] = ((ch.fresh >> k) & 1u) != 0u ? atomicSub(&P.n_acc[ch.id[k] - P.id_base], 1u) : 0u;
+                }
+#pragma unroll
+                for (uint32_t k = 0; k < kIdChunk; ++k) {
+                    if (before[k] == 2u) {
+                        // the identifier's one remaining track is its best
+                        const uint32_t s = P.best_of[ch.id[k] - P.id_base];
+                        if (s < P.n_tracks) atomicSub(&P.rec[s].n_shared, multiplicity(P, s, ch.id[k]));
+                    }
                 }
             }
         }
     }
+    block_count(&c->removed[r & 1u], removed, S);
+    block_count(&c->total_removed, removed, S);
 }
 
 // One workgroup, one removal per iteration, as the reference iterates:
@@ -324,11 +428,12 @@ __global__ __launch_bounds__(kSeqBlock) void k_amb_sequential(amb_params P, uint
         track_key wk{0.f, 0.f, kNone};
         for (uint32_t i = tid; i < nt; i += kSeqBlock) {
             const uint32_t t = T[i];
-            if (P.status[t] != kAlive) continue;
-            const uint32_t ns = P.n_shared[t];
+            const track_rec rec = P.rec[t];
+            if (rec.status != kAlive) continue;
+            const uint32_t ns = rec.n_shared;
             if (ns == 0u) continue;
             mx = ns > mx ? ns : mx;
-            const track_key k = key_of(P, t);
+            const track_key k = key_of(rec, t);
             if (wt == kNone || worse(k, wk)) {
                 wk = k;
                 wt = t;
@@ -340,7 +445,7 @@ __global__ __launch_bounds__(kSeqBlock) void k_amb_sequential(amb_params P, uint
         for (uint32_t s = kSeqBlock / 2u; s > 0u; s >>= 1u) {
             if (tid < s) {
                 const uint32_t a = s_t[tid], b = s_t[tid + s];
-                if (b != kNone && (a == kNone || worse(key_of(P, b), key_of(P, a)))) {
+                if (b != kNone && (a == kNone || worse(key_of(P.rec[b], b), key_of(P.rec[a], a)))) {
                     s_t[tid] = b;
                 }
                 s_max[tid] = s_max[tid + s] > s_max[tid] ? s_max[tid + s] : s_max[tid];
@@ -359,16 +464,16 @@ __global__ __launch_bounds__(kSeqBlock) void k_amb_sequential(amb_params P, uint
                 uint32_t s = kNone;
                 for (uint32_t q = P.list_off[id]; q < P.list_off[id + 1u]; ++q) {
                     const uint32_t u = P.list[q];
-                    if (u != W && P.status[u] == kAlive) {
+                    if (u != W && P.rec[u].status == kAlive) {
                         s = u;
                         break;
                     }
                 }
-                if (s != kNone) atomicSub(&P.n_shared[s], multiplicity(P, s, P.ids[j]));
+                if (s != kNone) atomicSub(&P.rec[s].n_shared, multiplicity(P, s, P.ids[j]));
             }
         }
         __syncthreads();
-        if (tid == 0u) P.status[W] = kDead;
+        if (tid == 0u) P.rec[W].status = kDead;
         ++removed;
         __syncthreads();
     }
@@ -376,12 +481,14 @@ __global__ __launch_bounds__(kSeqBlock) void k_amb_sequential(amb_params P, uint
 }
 
 __global__ __launch_bounds__(kAmbBlock) void k_amb_output(amb_params P, uint8_t* accepted) {
-    for (uint32_t b0 = blockIdx.x * blockDim.x; b0 < P.n_tracks; b0 += gridDim.x * blockDim.x) {
-        const uint32_t t = b0 + threadIdx.x;
-        const bool a = t < P.n_tracks && P.status[t] == kAlive;
-        if (t < P.n_tracks) accepted[t] = a ? 1u : 0u;
-        wave_count(&P.ctl->n_accepted, a);
+    __shared__ append_shared S;
+    uint32_t n = 0u;
+    for (uint32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < P.n_tracks; t += gridDim.x * blockDim.x) {
+        const bool a = P.rec[t].status == kAlive;
+        accepted[t] = a ? 1u : 0u;
+        n += a ? 1u : 0u;
     }
+    block_count(&P.ctl->n_accepted, n, S);
 }
 
 // Per event of a fitted batch: identifiers = event measurement offset +
@@ -406,9 +513,10 @@ __global__ __launch_bounds__(kAmbBlock) void k_amb_fitted_ids(const uint32_t* of
     }
 }
 
+// Two blocks of 1,024 fill a CU's 2,048 lanes; the kernels stride over the rest.
 uint32_t grid_for(uint64_t items) {
     const uint64_t b = (items + kAmbBlock - 1u) / kAmbBlock;
-    return static_cast<uint32_t>(std::max<uint64_t>(1u, std::min<uint64_t>(b, 8192u)));
+    return static_cast<uint32_t>(std::max<uint64_t>(1u, std::min<uint64_t>(b, 512u)));
 }
 
 }  // namespace
@@ -422,11 +530,11 @@ struct ckf_resolver {
     ckf_ambiguity_config cfg{};
     hipStream_t stream = nullptr;
     ckf_resolver_stats stats{};
-    tamd::dbuf status, n_shared, protect, cand0, cand1, n_acc, list_off, fill, list, best_of, hot0,
+    tamd::dbuf rec, protect, cand0, cand1, n_acc, list_off, fill, list, best_of, hot0,
         hot1, sums, ctl, in_off, in_ids, in_pval, out_acc, fit_ids, fit_ev_off;
     tamd::amb_ctl* h_ctl = nullptr;  // pinned
     ~ckf_resolver() {
-        tamd::dbuf* bs[] = {&status, &n_shared, &protect, &cand0,  &cand1,   &n_acc,   &list_off,
+        tamd::dbuf* bs[] = {&rec, &protect, &cand0,  &cand1,   &n_acc,   &list_off,
                             &fill,   &list,     &best_of, &hot0,   &hot1,    &sums,    &ctl,
                             &in_off, &in_ids,   &in_pval, &out_acc, &fit_ids, &fit_ev_off};
         for (tamd::dbuf* b : bs) b->release();
@@ -497,8 +605,7 @@ void resolve_device(ckf_resolver& R, uint32_t n, const uint32_t* d_off, const ui
     using namespace tamd;
     const hipStream_t s = R.stream;
     const uint32_t N = std::max(n, 1u), B = std::max(id_bound, 1u);
-    R.status.ensure(4u * size_t(N));
-    R.n_shared.ensure(4u * size_t(N));
+    R.rec.ensure(sizeof(track_rec) * size_t(N));
     R.protect.ensure(4u * size_t(N));
     R.cand0.ensure(4u * size_t(N));
     R.cand1.ensure(4u * size_t(N));
@@ -523,8 +630,7 @@ void resolve_device(ckf_resolver& R, uint32_t n, const uint32_t* d_off, const ui
     P.off = d_off;
     P.ids = d_ids;
     P.pval = d_pval;
-    P.status = R.status.as<uint32_t>();
-    P.n_shared = R.n_shared.as<uint32_t>();
+    P.rec = R.rec.as<track_rec>();
     P.protect = R.protect.as<uint32_t>();
     P.cand[0] = R.cand0.as<uint32_t>();
     P.cand[1] = R.cand1.as<uint32_t>();
