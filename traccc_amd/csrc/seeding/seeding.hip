@@ -10,17 +10,19 @@
 //                   bin; key (bin << 32 | index)
 //   radix sort      the keys: spacepoints in the reference's grid order
 //                   (bin, then index), the middle order of the seeding
+//   k_sd_place      the spacepoints in that order (16 B each) and the bins'
+//                   bounds, from where neighbouring keys differ
 //   k_sd_doublets   one wave per middle spacepoint: the neighbourhood's
 //                   candidates in zone order, 64 at a time; a ballot keeps
 //                   the compatible ones in order (count pass, scan, fill pass)
-//   k_sd_triplets   one wave per middle: per bottom doublet, the tops 64 at a
-//                   time (count pass, scan, fill pass); every triplet records
-//                   its bottom's segment
-//   k_sd_weights    per triplet: the compatible-seed bonus over its
-//                   segment, in the reference's order
-//   k_sd_filter     one wave per middle: weight bonus, single-seed cut, the
-//                   best maxSeedsPerSpM by (weight, y^2 + z^2 sum, finding
-//                   order), the per-middle cut
+//   k_sd_middle     one wave per middle: its triplets, their weights (the
+//                   compatible-seed bonus over the triplets of the same bottom,
+//                   in the reference's order) and the filter (weight bonus,
+//                   single-seed cut, the best maxSeedsPerSpM by (weight,
+//                   y^2 + z^2 sum, finding order), the per-middle cut), in LDS
+//   k_sd_triplets, k_sd_weights, k_sd_filter
+//                   the same in HBM for the middles whose tops or triplets do
+//                   not fit there
 //   k_sd_compact    the seeds in middle order
 // Every single-precision expression rounds as written (no contraction), as
 // in the oracle, so the cut decisions agree exactly.
@@ -88,8 +90,9 @@ struct sd_params {
     float* phi;
     uint64_t* keys;
     const uint64_t* sorted;
-    uint32_t* bin_count;
+    float4* pts;  // grid order: x, y, z, radius
     uint32_t* bin_off;
+    uint32_t nbins;
     uint32_t* cnt_b;  // per middle (grid order)
     uint32_t* off_b;
     uint32_t* cnt_t;
@@ -105,6 +108,12 @@ struct sd_params {
     seed_rec* seeds;
     sd_ctl* ctl;
 };
+
+// Order this wave's LDS accesses before and after (no other wave shares them).
+__device__ inline void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
 
 __device__ inline float sp_vr(const sd_params& P, uint32_t i) { return P.vr ? P.vr[i] : 0.f; }
 __device__ inline float sp_vz(const sd_params& P, uint32_t i) { return P.vz ? P.vz[i] : 0.f; }
@@ -221,6 +230,18 @@ __device__ inline doublet_rec transform(bool bottom, uint32_t osp, float mx, flo
     return d;
 }
 
+// Whether triplet_ok's first cut, |sqrt(d2) - sqrt(e2)| > sqrt(scat2) with the
+// scattering angle's d2 and its error e2, ends the pair for certain, without its
+// square root: (sqrt(e2) + sqrt(scat2))^2 <= 2 (e2 + scat2), so d2 above that by
+// 1e-4 is above the cut by more than the cut's rounding (4e-7 of d2).  Pairs that
+// this leaves go through triplet_ok.
+__device__ inline bool triplet_scatters(float mvr, float mvz, const doublet_rec& lb, float t_Er, float t_cot,
+                                        float t_iDR, float scat2) {
+    const float error2 = t_Er + lb.Er + 2.f * (lb.cot * t_cot * mvr + mvz) * lb.iDR * t_iDR;
+    const float d = lb.cot - t_cot;
+    return error2 >= 0.f && d * d > 2.0002f * (error2 + scat2);
+}
+
 // triplet_finding_helper.hpp:46-141
 __device__ inline bool triplet_ok(float mr, float mvr, float mvz, const doublet_rec& lb, const doublet_rec& lt,
                                   const ckf_seedfinder_config& c, float iSinTheta2, float scat2, float& curvature,
@@ -282,13 +303,34 @@ __global__ __launch_bounds__(kSdBlock) void k_sd_prep(sd_params P) {
             if (valid) {
                 const uint32_t bin = phi_bin(P.A, phi) + P.A.nphi * z_bin(P.A, z);
                 key = (static_cast<uint64_t>(bin) << 32) | i;
-                atomicAdd(&P.bin_count[bin], 1u);
             }
             P.keys[i] = key;
         }
-        const uint64_t m = wave_ballot(valid);
-        if (m != 0ull && lane() == static_cast<uint32_t>(__builtin_ctzll(m))) {
-            atomicAdd(&P.ctl->n_valid, __popcll(m));
+    }
+}
+
+// The spacepoints in grid order and every bin's first one: where the bin of a
+// sorted key differs from the one before, the bins in between start (counting
+// them with atomics took 140 us for 57,000 spacepoints in 77 bins).  The
+// rejected ones come last, as bin nbins: it starts at the number of valid ones.
+__global__ __launch_bounds__(kSdBlock) void k_sd_place(sd_params P) {
+    for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < P.n_sp; k += gridDim.x * blockDim.x) {
+        const uint64_t key = P.sorted[k];
+        const uint32_t bin = key == ~0ull ? P.nbins : static_cast<uint32_t>(key >> 32);
+        uint32_t from = 0u;
+        if (k > 0u) {
+            const uint64_t below = P.sorted[k - 1u];
+            from = (below == ~0ull ? P.nbins : static_cast<uint32_t>(below >> 32)) + 1u;
+        }
+        for (uint32_t b = from; b <= bin; ++b) P.bin_off[b] = k;
+        if (bin == P.nbins && from <= bin) P.ctl->n_valid = k;
+        if (k + 1u == P.n_sp && bin < P.nbins) {
+            for (uint32_t b = bin + 1u; b <= P.nbins; ++b) P.bin_off[b] = P.n_sp;
+            P.ctl->n_valid = P.n_sp;
+        }
+        if (bin < P.nbins) {
+            const uint32_t i = static_cast<uint32_t>(key);
+            P.pts[k] = make_float4(P.xyz[3 * i], P.xyz[3 * i + 1], P.xyz[3 * i + 2], P.rad[i]);
         }
     }
 }
@@ -303,8 +345,8 @@ __global__ __launch_bounds__(kSdBlock) void k_sd_doublets(sd_params P) {
             continue;  // no bottoms: nothing of this middle is kept
         }
         const uint32_t mi = static_cast<uint32_t>(P.sorted[p]);
-        const float mx = P.xyz[3 * mi], my = P.xyz[3 * mi + 1], mz = P.xyz[3 * mi + 2];
-        const float mr = P.rad[mi];
+        const float4 mid = P.pts[p];
+        const float mx = mid.x, my = mid.y, mz = mid.z, mr = mid.w;
         const float mvr = sp_vr(P, mi), mvz = sp_vz(P, mi);
         const phi_zone pz = make_phi_zone(P.A, P.phi[mi], P.c.neighbor_scope);
         uint32_t za, zc;
@@ -322,16 +364,17 @@ __global__ __launch_bounds__(kSdBlock) void k_sd_doublets(sd_params P) {
                     uint32_t oi = 0u;
                     float ox = 0.f, oy = 0.f, oz = 0.f, orr = 0.f;
                     if (k < s1) {
-                        oi = static_cast<uint32_t>(P.sorted[k]);
-                        ox = P.xyz[3 * oi];
-                        oy = P.xyz[3 * oi + 1];
-                        oz = P.xyz[3 * oi + 2];
-                        orr = P.rad[oi];
+                        const float4 o = P.pts[k];
+                        ox = o.x;
+                        oy = o.y;
+                        oz = o.z;
+                        orr = o.w;
                         isb = doublet_ok(true, mx, my, mz, mr, ox, oy, oz, orr, P.c);
                         ist = doublet_ok(false, mx, my, mz, mr, ox, oy, oz, orr, P.c);
                     }
                     const uint64_t mb = wave_ballot(isb), mt = wave_ballot(ist);
                     if constexpr (kFill) {
+                        if (isb || ist) oi = static_cast<uint32_t>(P.sorted[k]);
                         if (isb) {
                             P.bot[ob + nb + prefix_count(mb)] =
                                 transform(true, oi, mx, my, mz, mr, mvr, mvz, ox, oy, oz, sp_vr(P, oi), sp_vz(P, oi));
@@ -354,39 +397,36 @@ __global__ __launch_bounds__(kSdBlock) void k_sd_doublets(sd_params P) {
     }
 }
 
-// One wave per middle: per bottom doublet, its triplets with the tops.
-template <bool kFill>
+// One wave per middle that k_sd_middle left (cnt_tr): per bottom doublet, its
+// triplets with the tops.
 __global__ __launch_bounds__(kSdBlock) void k_sd_triplets(sd_params P) {
     const uint32_t n_mid = P.ctl->n_valid;
     const uint32_t l = lane();
     const float ss2 = P.c.sigmaScattering * P.c.sigmaScattering;
     for (uint32_t p = blockIdx.x * kSdWaves + threadIdx.x / kWave; p < n_mid; p += gridDim.x * kSdWaves) {
-        const uint32_t nb = P.cnt_b[p], nt = P.cnt_t[p];
-        if (nb == 0u || nt == 0u) {
-            if (!kFill && l == 0u) P.cnt_tr[p] = 0u;
+        if (P.cnt_tr[p] == 0u) {
             continue;
         }
+        const uint32_t nb = P.cnt_b[p], nt = P.cnt_t[p];
         const uint32_t mi = static_cast<uint32_t>(P.sorted[p]);
         const float mr = P.rad[mi], mvr = sp_vr(P, mi), mvz = sp_vz(P, mi);
         const doublet_rec* B = P.bot + P.off_b[p];
         const doublet_rec* T = P.top + P.off_t[p];
-        uint32_t n = kFill ? P.off_tr[p] : 0u;
+        uint32_t n = P.off_tr[p];
         for (uint32_t jb = 0; jb < nb; ++jb) {
             const doublet_rec lb = B[jb];
             const float iSinTheta2 = 1.f + lb.cot * lb.cot;
             float scat2 = P.c.maxScatteringAngle2 * iSinTheta2;
             scat2 *= ss2;
-            // the segment of this bottom: counted first when filling
+            // the segment of this bottom is counted first
             uint32_t seg = 0u;
-            if constexpr (kFill) {
-                for (uint32_t c0 = 0; c0 < nt; c0 += kWave) {
-                    bool ok = false;
-                    if (c0 + l < nt) {
-                        float cv, ip;
-                        ok = triplet_ok(mr, mvr, mvz, lb, T[c0 + l], P.c, iSinTheta2, scat2, cv, ip);
-                    }
-                    seg += __popcll(wave_ballot(ok));
+            for (uint32_t c0 = 0; c0 < nt; c0 += kWave) {
+                bool ok = false;
+                if (c0 + l < nt) {
+                    float cv, ip;
+                    ok = triplet_ok(mr, mvr, mvz, lb, T[c0 + l], P.c, iSinTheta2, scat2, cv, ip);
                 }
+                seg += __popcll(wave_ballot(ok));
             }
             uint32_t w = 0u;
             for (uint32_t c0 = 0; c0 < nt; c0 += kWave) {
@@ -394,23 +434,20 @@ __global__ __launch_bounds__(kSdBlock) void k_sd_triplets(sd_params P) {
                 float cv = 0.f, ip = 0.f;
                 if (c0 + l < nt) ok = triplet_ok(mr, mvr, mvz, lb, T[c0 + l], P.c, iSinTheta2, scat2, cv, ip);
                 const uint64_t m = wave_ballot(ok);
-                if constexpr (kFill) {
-                    if (ok) {
-                        triplet_rec r;
-                        r.b = lb.sp;
-                        r.t = T[c0 + l].sp;
-                        r.curv = cv;
-                        r.w = -ip * P.f.impactWeightFactor;
-                        r.seg0 = n;
-                        r.seg1 = n + seg;
-                        P.trip[n + w + prefix_count(m)] = r;
-                    }
+                if (ok) {
+                    triplet_rec r;
+                    r.b = lb.sp;
+                    r.t = T[c0 + l].sp;
+                    r.curv = cv;
+                    r.w = -ip * P.f.impactWeightFactor;
+                    r.seg0 = n;
+                    r.seg1 = n + seg;
+                    P.trip[n + w + prefix_count(m)] = r;
                 }
                 w += __popcll(m);
             }
             n += w;
         }
-        if (!kFill && l == 0u) P.cnt_tr[p] = n;
     }
 }
 
@@ -466,7 +503,277 @@ __device__ inline bool before(const seed_key& a, const seed_key& b) {
     return a.idx < b.idx;
 }
 
-// seed_filtering.cpp:36-121 for one middle per wave.
+// What k_sd_middle holds in LDS of a middle (16 KB a wave, ten waves a CU):
+// tops, the pairs of 64 bottoms that the first cut leaves, triplets.
+constexpr uint32_t kMidTops = 256;
+constexpr uint32_t kMidPairs = 1024;
+constexpr uint32_t kMidTrips = 256;
+constexpr uint32_t kTopWords = kMidTops / 64u;
+constexpr uint32_t kTripSlots = kMidTrips / kWave;
+
+struct middle_lds {
+    float4 t_Er[kMidTops / 4u], t_cot[kMidTops / 4u], t_iDR[kMidTops / 4u];  // read four at a time
+    float t_U[kMidTops], t_V[kMidTops];
+    uint32_t t_sp[kMidTops];
+    float b_Er[kWave], b_cot[kWave], b_iDR[kWave], b_U[kWave], b_V[kWave];
+    uint32_t b_sp[kWave], b_n[kWave];
+    uint16_t pair[kMidPairs];  // bottom << 8 | top
+    uint32_t b[kMidTrips], t[kMidTrips];
+    float curv[kMidTrips], w[kMidTrips], rt[kMidTrips];
+    uint16_t seg0[kMidTrips], seg1[kMidTrips];  // seg0: the bottom's lane until its segment is known
+};
+
+// The number of a middle's triplets, a bottom per lane, from HBM.
+__device__ __noinline__ uint32_t count_triplets(const sd_params& P, const doublet_rec* B, const doublet_rec* T,
+                                                uint32_t nb, uint32_t nt, float mr, float mvr, float mvz) {
+    const float ss2 = P.c.sigmaScattering * P.c.sigmaScattering;
+    uint32_t n = 0u;
+    for (uint32_t jb = lane(); jb < nb; jb += kWave) {
+        const doublet_rec lb = B[jb];
+        const float iSinTheta2 = 1.f + lb.cot * lb.cot;
+        float scat2 = P.c.maxScatteringAngle2 * iSinTheta2;
+        scat2 *= ss2;
+        for (uint32_t j = 0; j < nt; ++j) {
+            float cv, ip;
+            n += triplet_ok(mr, mvr, mvz, lb, T[j], P.c, iSinTheta2, scat2, cv, ip) ? 1u : 0u;
+        }
+    }
+    return wave_broadcast(wave_inclusive_scan(n), kWave - 1);
+}
+
+// One wave per middle: triplets (triplet_finding.hpp:60-183), weights and
+// filter (seed_filtering.cpp:36-121) without a pass through HBM in between.
+//
+// A lane takes a bottom: the tops come from LDS, the same ones for all lanes, and
+// a test without square root or division ends 98 % of the pairs (9,600 a middle
+// in a 10,000 muon event).  The rest are listed in the reference's order (bottom,
+// then top) and evaluated 64 at a time, so the passing ones are placed by a
+// ballot.  The first test's vector arithmetic and LDS reads bound it.  50,000
+// middles: 624 us; every pair evaluated with lanes on tops, and twice more to
+// count a bottom's segment and the middle's triplets, 4,520 us; a resident grid
+// striding over the middles 1,265 (they differ by a factor of a hundred: one
+// block each, as the hardware places them), tops read one at a time 877.
+__global__ __launch_bounds__(kWave) void k_sd_middle(sd_params P) {
+    __shared__ middle_lds S;
+    float* t_Er = reinterpret_cast<float*>(S.t_Er);
+    float* t_cot = reinterpret_cast<float*>(S.t_cot);
+    float* t_iDR = reinterpret_cast<float*>(S.t_iDR);
+    const uint32_t n_mid = P.ctl->n_valid;
+    const uint32_t l = lane();
+    const ckf_seedfilter_config& f = P.f;
+    const float ss2 = P.c.sigmaScattering * P.c.sigmaScattering;
+    const uint32_t max_s = P.c.maxSeedsPerSpM;
+    for (uint32_t p = blockIdx.x; p < n_mid; p += gridDim.x) {
+        const uint32_t nb = P.cnt_b[p], nt = P.cnt_t[p];
+        if (nb == 0u || nt == 0u) {
+            if (l == 0u) {
+                P.cnt_tr[p] = 0u;
+                P.cnt_s[p] = 0u;
+            }
+            continue;
+        }
+        const uint32_t mi = static_cast<uint32_t>(P.sorted[p]);
+        const float mr = P.pts[p].w, mvr = sp_vr(P, mi), mvz = sp_vz(P, mi);
+        const doublet_rec* B = P.bot + P.off_b[p];
+        const doublet_rec* T = P.top + P.off_t[p];
+        bool fits = nt <= kMidTops;
+        for (uint32_t j = l; fits && j < nt; j += kWave) {
+            const doublet_rec t = T[j];
+            t_Er[j] = t.Er;
+            t_cot[j] = t.cot;
+            t_iDR[j] = t.iDR;
+            S.t_U[j] = t.U;
+            S.t_V[j] = t.V;
+            S.t_sp[j] = t.sp;
+        }
+        uint32_t n = 0u;  // triplets so far
+        for (uint32_t c0 = 0; fits && c0 < nb; c0 += kWave) {
+            const bool has = c0 + l < nb;
+            const doublet_rec own = B[has ? c0 + l : 0u];
+            float own_scat2 = P.c.maxScatteringAngle2 * (1.f + own.cot * own.cot);
+            own_scat2 *= ss2;
+            S.b_Er[l] = own.Er;
+            S.b_cot[l] = own.cot;
+            S.b_iDR[l] = own.iDR;
+            S.b_U[l] = own.U;
+            S.b_V[l] = own.V;
+            S.b_sp[l] = own.sp;
+            S.b_n[l] = 0u;
+            wave_lds_order();
+            uint64_t left[kTopWords];
+            uint32_t mine = 0u;
+#pragma unroll
+            for (uint32_t q = 0; q < kTopWords; ++q) {
+                uint64_t m = 0ull;
+                const uint32_t nq = nt > 64u * q ? (nt - 64u * q < 64u ? nt - 64u * q : 64u) : 0u;
+                for (uint32_t j = 0; j < nq; j += 4u) {
+                    const float4 er = S.t_Er[16u * q + j / 4u], cot = S.t_cot[16u * q + j / 4u],
+                                 idr = S.t_iDR[16u * q + j / 4u];
+                    uint32_t four = 0u;
+                    four |= triplet_scatters(mvr, mvz, own, er.x, cot.x, idr.x, own_scat2) ? 0u : 1u;
+                    four |= triplet_scatters(mvr, mvz, own, er.y, cot.y, idr.y, own_scat2) ? 0u : 2u;
+                    four |= triplet_scatters(mvr, mvz, own, er.z, cot.z, idr.z, own_scat2) ? 0u : 4u;
+                    four |= triplet_scatters(mvr, mvz, own, er.w, cot.w, idr.w, own_scat2) ? 0u : 8u;
+                    m |= static_cast<uint64_t>(four) << j;
+                }
+                // the last four may reach past the tops
+                m = has && nq > 0u ? m & (~0ull >> (64u - nq)) : 0ull;
+                left[q] = m;
+                mine += static_cast<uint32_t>(__popcll(m));
+            }
+            const uint32_t incl = wave_inclusive_scan(mine);
+            const uint32_t pairs = wave_broadcast(incl, kWave - 1);
+            if (pairs > kMidPairs) {
+                fits = false;
+                break;
+            }
+            uint32_t at = incl - mine;
+#pragma unroll
+            for (uint32_t q = 0; q < kTopWords; ++q) {
+                for (uint64_t rest = left[q]; rest != 0ull; rest &= rest - 1ull) {
+                    S.pair[at++] = static_cast<uint16_t>(l << 8 | (64u * q + static_cast<uint32_t>(__builtin_ctzll(rest))));
+                }
+            }
+            wave_lds_order();
+            const uint32_t n0 = n;
+            for (uint32_t k0 = 0; k0 < pairs; k0 += kWave) {
+                const bool in = k0 + l < pairs;
+                const uint32_t pr = S.pair[in ? k0 + l : 0u];
+                const uint32_t jb = pr >> 8, j = pr & 0xffu;
+                const doublet_rec lb{0u, 0.f, S.b_cot[jb], S.b_iDR[jb], S.b_Er[jb], S.b_U[jb], S.b_V[jb]};
+                const doublet_rec lt{0u, 0.f, t_cot[j], t_iDR[j], t_Er[j], S.t_U[j], S.t_V[j]};
+                const float iSinTheta2 = 1.f + lb.cot * lb.cot;
+                float scat2 = P.c.maxScatteringAngle2 * iSinTheta2;
+                scat2 *= ss2;
+                float cv = 0.f, ip = 0.f;
+                const bool ok = in && triplet_ok(mr, mvr, mvz, lb, lt, P.c, iSinTheta2, scat2, cv, ip);
+                const uint64_t m = wave_ballot(ok);
+                const uint32_t pos = n + prefix_count(m);
+                if (ok && pos < kMidTrips) {
+                    S.b[pos] = S.b_sp[jb];
+                    S.t[pos] = S.t_sp[j];
+                    S.curv[pos] = cv;
+                    S.w[pos] = -ip * f.impactWeightFactor;
+                    S.rt[pos] = P.rad[S.t_sp[j]];
+                    S.seg0[pos] = static_cast<uint16_t>(jb);
+                    atomicAdd(&S.b_n[jb], 1u);
+                }
+                n += static_cast<uint32_t>(__popcll(m));
+            }
+            if (n > kMidTrips) {
+                fits = false;
+                break;
+            }
+            wave_lds_order();
+            // the bottoms' segments, and every triplet's
+            const uint32_t bn = S.b_n[l];
+            const uint32_t bi = wave_inclusive_scan(bn);
+            for (uint32_t i0 = n0; i0 < n; i0 += kWave) {
+                const bool in = i0 + l < n;
+                const uint32_t jb = in ? S.seg0[i0 + l] : 0u;
+                const uint32_t end = n0 + __shfl(bi, static_cast<int>(jb), kWave);
+                const uint32_t len = __shfl(bn, static_cast<int>(jb), kWave);
+                if (in) {
+                    S.seg0[i0 + l] = static_cast<uint16_t>(end - len);
+                    S.seg1[i0 + l] = static_cast<uint16_t>(end);
+                }
+            }
+            wave_lds_order();  // the next bottoms write over these
+        }
+        if (!fits) {
+            const uint32_t total = count_triplets(P, B, T, nb, nt, mr, mvr, mvz);
+            if (l == 0u) {
+                P.cnt_tr[p] = total;
+                P.cnt_s[p] = 0u;
+            }
+            continue;
+        }
+        // the weights, then each triplet's sort key (idx kNoSp: none, or cut)
+        seed_key keys[kTripSlots];
+#pragma unroll
+        for (uint32_t q = 0; q < kTripSlots; ++q) {
+            const uint32_t i = q * kWave + l;
+            keys[q] = seed_key{0.f, 0.f, kNoSp};
+            if (i >= n) continue;
+            const float rt = S.rt[i];
+            const float lo = S.curv[i] - f.deltaInvHelixDiameter;
+            const float hi = S.curv[i] + f.deltaInvHelixDiameter;
+            float compat[8];
+            uint32_t nc = 0u;
+            float w = S.w[i];
+            const uint32_t limit = f.compatSeedLimit < 8u ? f.compatSeedLimit : 8u;
+            for (uint32_t j = S.seg0[i]; j < S.seg1[i]; ++j) {
+                if (j == i) continue;
+                const float ro = S.rt[j];
+                const float cj = S.curv[j];
+                const float dr = rt - ro;
+                if (fabsf(dr) < f.deltaRMin) continue;
+                if (cj < lo) continue;
+                if (cj > hi) continue;
+                bool fresh = true;
+#pragma unroll
+                for (uint32_t c = 0; c < 8u; ++c) {
+                    if (c < nc && fabsf(compat[c] - ro) < f.deltaRMin) fresh = false;
+                }
+                if (fresh) {
+#pragma unroll
+                    for (uint32_t c = 0; c < 8u; ++c) {
+                        if (c == nc || (c == 7u && nc > 7u)) compat[c] = ro;
+                    }
+                    ++nc;
+                    w += f.compatSeedWeight;
+                }
+                if (nc >= limit) break;
+            }
+            const uint32_t sb = S.b[i], st = S.t[i];
+            const float rb = P.rad[sb];
+            float bonus = 0;
+            if (rb > f.good_spB_min_radius) bonus = f.good_spB_weight_increase;
+            if (rt < f.good_spT_max_radius) bonus = f.good_spT_weight_increase;
+            w += bonus;
+            if (rb > f.good_spB_min_radius && w < f.good_spB_min_weight) continue;  // single-seed cut
+            const float by = P.xyz[3 * sb + 1], bz = P.xyz[3 * sb + 2];
+            const float ty = P.xyz[3 * st + 1], tz = P.xyz[3 * st + 2];
+            keys[q] = seed_key{w, by * by + bz * bz + ty * ty + tz * tz, i};
+        }
+        uint32_t out = 0u;
+        seed_key last{0.f, 0.f, 0u};
+        for (uint32_t s = 0; s < max_s && s < n; ++s) {
+            seed_key best{0.f, 0.f, kNoSp};
+#pragma unroll
+            for (uint32_t q = 0; q < kTripSlots; ++q) {
+                if (keys[q].idx == kNoSp || (s > 0u && !before(last, keys[q]))) continue;  // none, or taken
+                if (best.idx == kNoSp || before(keys[q], best)) best = keys[q];
+            }
+#pragma unroll
+            for (int d = 32; d >= 1; d >>= 1) {
+                seed_key o;
+                o.w = __shfl_xor(best.w, d, kWave);
+                o.ysum = __shfl_xor(best.ysum, d, kWave);
+                o.idx = __shfl_xor(best.idx, d, kWave);
+                if (o.idx != kNoSp && (best.idx == kNoSp || before(o, best))) best = o;
+            }
+            if (best.idx == kNoSp) break;
+            last = best;
+            const uint32_t sb = S.b[best.idx];
+            // the first is always kept; the others need a heavy seed or a far bottom
+            const bool keep = s == 0u || best.w > f.seed_min_weight || P.rad[sb] > f.spB_min_radius;
+            if (keep) {
+                if (l == 0u) {
+                    P.slots[static_cast<size_t>(p) * max_s + out] = seed_rec{sb, mi, S.t[best.idx], best.w};
+                }
+                ++out;
+            }
+        }
+        if (l == 0u) {
+            P.cnt_tr[p] = 0u;
+            P.cnt_s[p] = out;
+        }
+        wave_lds_order();  // the next middle writes over this one's tables
+    }
+}
+
+// seed_filtering.cpp:36-121, one middle per wave (those of k_sd_triplets).
 __global__ __launch_bounds__(kSdBlock) void k_sd_filter(sd_params P) {
     const uint32_t n_mid = P.ctl->n_valid;
     const uint32_t l = lane();
@@ -474,6 +781,9 @@ __global__ __launch_bounds__(kSdBlock) void k_sd_filter(sd_params P) {
     const uint32_t max_s = P.c.maxSeedsPerSpM;
     for (uint32_t p = blockIdx.x * kSdWaves + threadIdx.x / kWave; p < n_mid; p += gridDim.x * kSdWaves) {
         const uint32_t t0 = P.off_tr[p], nt = P.cnt_tr[p];
+        if (nt == 0u) {
+            continue;  // k_sd_middle's
+        }
         const uint32_t mi = static_cast<uint32_t>(P.sorted[p]);
         uint32_t out = 0u;
         seed_key last{0.f, 0.f, 0u};
@@ -698,11 +1008,11 @@ struct ckf_seeding {
     tamd::sd_axes axes{};
     hipStream_t stream = nullptr;
     uint32_t n_seeds = 0;
-    tamd::dbuf in_xyz, in_vr, in_vz, rad, phi, keys, sorted, sort_tmp, bin_count, bin_off, cnt_b, off_b,
+    tamd::dbuf in_xyz, in_vr, in_vz, rad, phi, keys, sorted, sort_tmp, pts, bin_off, cnt_b, off_b,
         cnt_t, off_t, bot, top, cnt_tr, off_tr, trip, cnt_s, off_s, slots, seeds, sums, ctl;
     tamd::sd_ctl* h_ctl = nullptr;
     ~ckf_seeding() {
-        tamd::dbuf* bs[] = {&in_xyz, &in_vr,  &in_vz,  &rad,   &phi,    &keys,  &sorted, &sort_tmp, &bin_count,
+        tamd::dbuf* bs[] = {&in_xyz, &in_vr,  &in_vz,  &rad,   &phi,    &keys,  &sorted, &sort_tmp, &pts,
                             &bin_off, &cnt_b, &off_b,  &cnt_t, &off_t,  &bot,   &top,    &cnt_tr,   &off_tr,
                             &trip,   &cnt_s,  &off_s,  &slots, &seeds,  &sums,  &ctl};
         for (tamd::dbuf* b : bs) b->release();
@@ -726,15 +1036,14 @@ void run_seeding(ckf_seeding& S, uint32_t n_sp, const float* d_xyz, const float*
     S.phi.ensure(4u * size_t(N));
     S.keys.ensure(8u * size_t(N));
     S.sorted.ensure(8u * size_t(N));
-    S.bin_count.ensure(4u * size_t(nbins));
+    S.pts.ensure(16u * size_t(N));
     S.bin_off.ensure(4u * (size_t(nbins) + 1u));
-    S.sums.ensure(4u * size_t(scan_sums_size(std::max(N, nbins) + 1u)));
+    S.sums.ensure(4u * size_t(scan_sums_size(N + 1u)));
     S.ctl.ensure(sizeof(sd_ctl));
     if (S.h_ctl == nullptr) {
         hip_check(hipHostMalloc(reinterpret_cast<void**>(&S.h_ctl), sizeof(sd_ctl)), "hipHostMalloc");
     }
     hip_check(hipMemsetAsync(S.ctl.p, 0, sizeof(sd_ctl), s), "memset");
-    hip_check(hipMemsetAsync(S.bin_count.p, 0, 4u * size_t(nbins), s), "memset");
     sd_params P{};
     P.c = S.finder;
     P.f = S.filter;
@@ -747,8 +1056,9 @@ void run_seeding(ckf_seeding& S, uint32_t n_sp, const float* d_xyz, const float*
     P.phi = S.phi.as<float>();
     P.keys = S.keys.as<uint64_t>();
     P.sorted = S.sorted.as<uint64_t>();
-    P.bin_count = S.bin_count.as<uint32_t>();
+    P.pts = S.pts.as<float4>();
     P.bin_off = S.bin_off.as<uint32_t>();
+    P.nbins = nbins;
     P.ctl = S.ctl.as<sd_ctl>();
     if (n_sp > 0u) {
         hipLaunchKernelGGL(k_sd_prep, dim3(grid_for(n_sp, kSdBlock)), dim3(kSdBlock), 0, s, P);
@@ -766,7 +1076,10 @@ void run_seeding(ckf_seeding& S, uint32_t n_sp, const float* d_xyz, const float*
                                            end_bit, s),
                   "sort");
     }
-    exclusive_scan(P.bin_count, P.bin_off, S.sums.as<uint32_t>(), nbins, nullptr, s);
+    if (n_sp > 0u) {
+        hipLaunchKernelGGL(k_sd_place, dim3(grid_for(n_sp, kSdBlock)), dim3(kSdBlock), 0, s, P);
+        hip_check(hipGetLastError(), "place");
+    }
     read_ctl(S);
     const uint32_t nm = S.h_ctl->n_valid;
     const uint32_t M = std::max(nm, 1u);
@@ -803,17 +1116,17 @@ void run_seeding(ckf_seeding& S, uint32_t n_sp, const float* d_xyz, const float*
     P.top = S.top.as<doublet_rec>();
     if (nm > 0u) {
         hipLaunchKernelGGL(k_sd_doublets<true>, gw, dim3(kSdBlock), 0, s, P);
-        hipLaunchKernelGGL(k_sd_triplets<false>, gw, dim3(kSdBlock), 0, s, P);
-        hip_check(hipGetLastError(), "triplet count");
+        hipLaunchKernelGGL(k_sd_middle, dim3(std::min(nm, 1u << 20)), dim3(kWave), 0, s, P);
+        hip_check(hipGetLastError(), "triplets");
     }
     exclusive_scan(P.cnt_tr, P.off_tr, S.sums.as<uint32_t>(), nm, &P.ctl->n_trip, s);
     read_ctl(S);
-    S.trip.ensure(sizeof(triplet_rec) * std::max<size_t>(S.h_ctl->n_trip, 1u));
-    P.trip = S.trip.as<triplet_rec>();
-    if (nm > 0u) {
-        hipLaunchKernelGGL(k_sd_triplets<true>, gw, dim3(kSdBlock), 0, s, P);
-        hipLaunchKernelGGL(k_sd_weights, dim3(grid_for(std::max(S.h_ctl->n_trip, 1u), kSdBlock)), dim3(kSdBlock), 0,
-                           s, P);
+    if (S.h_ctl->n_trip > 0u) {
+        // the middles with more tops or triplets than LDS holds
+        S.trip.ensure(sizeof(triplet_rec) * size_t(S.h_ctl->n_trip));
+        P.trip = S.trip.as<triplet_rec>();
+        hipLaunchKernelGGL(k_sd_triplets, gw, dim3(kSdBlock), 0, s, P);
+        hipLaunchKernelGGL(k_sd_weights, dim3(grid_for(S.h_ctl->n_trip, kSdBlock)), dim3(kSdBlock), 0, s, P);
         hipLaunchKernelGGL(k_sd_filter, gw, dim3(kSdBlock), 0, s, P);
         hip_check(hipGetLastError(), "filter");
     }
