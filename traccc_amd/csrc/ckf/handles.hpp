@@ -101,6 +101,27 @@ struct block_cache {
 
 block_cache& result_cache();
 
+// A result's device block, from the result cache and back to it.  Contents are
+// whatever the block held before: the kernels of a result write all of it.
+struct rbuf {
+    void* p = nullptr;
+    size_t bytes = 0;
+    rbuf() = default;
+    rbuf(const rbuf&) = delete;
+    rbuf& operator=(const rbuf&) = delete;
+    ~rbuf() { result_cache().put(p, bytes); }
+    void take(size_t need) {
+        result_cache().put(p, bytes);
+        p = nullptr;
+        p = result_cache().get(need);
+        bytes = need;
+    }
+    template <typename T>
+    T* as() const {
+        return static_cast<T*>(p);
+    }
+};
+
 template <typename T>
 T* dev_copy(const T* src, size_t n) {
     T* d = nullptr;
@@ -163,13 +184,8 @@ struct ckf_device_fitted {
     uint32_t n_tracks = 0, n_states = 0;
     std::vector<uint64_t> ids;            // surface index -> identifier
     std::vector<uint32_t> ev_track_off;   // [n_events + 1] tracks of each event
-    tamd::dbuf outcome, surface, vec, cov, ndf, chi2, pval, nholes, offsets, cons, flt, smt, flags,
+    tamd::rbuf outcome, surface, vec, cov, ndf, chi2, pval, nholes, offsets, cons, flt, smt, flags,
         state_sf;
-    ~ckf_device_fitted() {
-        tamd::dbuf* bs[] = {&outcome, &surface, &vec, &cov, &ndf, &chi2, &pval, &nholes,
-                            &offsets, &cons, &flt, &smt, &flags, &state_sf};
-        for (tamd::dbuf* b : bs) b->release();
-    }
 };
 
 struct ckf_device_tracks {

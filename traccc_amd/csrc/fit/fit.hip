@@ -9,7 +9,8 @@
 // kalman_actor (kalman_actor.hpp) and two_filters_smoother
 // (two_filters_smoother.hpp:38-294).
 //
-// One lane fits one track candidate.  k_fit_forward walks the navigation from
+// One lane fits one track candidate (forward: a team of lanes where there are
+// few candidates).  k_fit_forward walks the navigation from
 // the seed surface: material first, then the gain-matrix update on the
 // candidate's measurement of the surface; any other sensitive surface is a
 // hole (kept in the track's surface sequence when it carries material).
@@ -45,6 +46,13 @@ namespace tamd {
 namespace {
 
 constexpr uint32_t kFitBlock = 128;
+// Lanes per candidate in k_fit_forward.  A candidate is one chain of
+// propagations, updates and propagations again: few candidates are bound by the
+// chain, which a team's navigation shortens (a propagation of one lane takes
+// ~100 us alone, of 8 lanes 55, of 16 lanes 40); many by the lanes, which a team
+// spends on redundant steps.  10,000 muons: 558 us with one lane, 300 with 8.
+constexpr uint32_t kFitTeam16 = 5120u;   // up to here 16 lanes
+constexpr uint32_t kFitTeam8 = 28672u;   // up to here 8, then one
 constexpr uint32_t kSeqState = 0x80000000u;  // sequence entry is a track state
 
 // kalman_fitter_status values (core/include/traccc/fitting/status_codes.hpp:14-29)
@@ -135,18 +143,44 @@ __device__ inline void inflate(float* c, float f) {
     }
 }
 
-__device__ inline void store_rec(float* r, const float* x, const float* c) {
+// A whole record (128 B on its own line): eight 16-byte stores.  A 4-byte
+// access strided by 128 B takes a line per lane, 27 times for a state.
+__device__ inline void store_rec(float* r, const float* x, const float* c, float chi2a, float chi2b) {
+    float v[kRec];
 #pragma unroll
-    for (int k = 0; k < 6; ++k) r[k] = x[k];
+    for (int k = 0; k < 6; ++k) v[k] = x[k];
 #pragma unroll
-    for (int k = 0; k < 21; ++k) r[6 + k] = c[k];
+    for (int k = 0; k < 21; ++k) v[6 + k] = c[k];
+    v[kRecChi2a] = chi2a;
+    v[kRecChi2b] = chi2b;
+#pragma unroll
+    for (int k = kRecChi2b + 1; k < kRec; ++k) v[k] = 0.f;
+    float4* q = reinterpret_cast<float4*>(r);
+#pragma unroll
+    for (int k = 0; k < kRec / 4; ++k) q[k] = make_float4(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
+}
+
+__device__ inline void zero_rec(float* r) {
+    float4* q = reinterpret_cast<float4*>(r);
+#pragma unroll
+    for (int k = 0; k < kRec / 4; ++k) q[k] = make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
 __device__ inline void load_rec(const float* r, float* x, float* c) {
+    const float4* q = reinterpret_cast<const float4*>(r);
+    float v[28];
 #pragma unroll
-    for (int k = 0; k < 6; ++k) x[k] = r[k];
+    for (int k = 0; k < 7; ++k) {
+        const float4 f = q[k];
+        v[4 * k] = f.x;
+        v[4 * k + 1] = f.y;
+        v[4 * k + 2] = f.z;
+        v[4 * k + 3] = f.w;
+    }
 #pragma unroll
-    for (int k = 0; k < 21; ++k) c[k] = r[6 + k];
+    for (int k = 0; k < 6; ++k) x[k] = v[k];
+#pragma unroll
+    for (int k = 0; k < 21; ++k) c[k] = v[6 + k];
 }
 
 // chi2 of residual m - H x against R = V - H C H^T (a filtered or smoothed
@@ -288,10 +322,14 @@ __device__ inline uint32_t smooth_state(const meas_data& m, float* xp, float* cp
     return kSuccess;
 }
 
+template <int kT>
 __global__ __launch_bounds__(kFitBlock) void k_fit_forward(fit_params F, uint32_t iteration) {
     __shared__ nav_tables s_nav;
     stage_nav_tables(s_nav, F.layers, F.n_layers, F.groups, F.n_groups, F.nav.mask_tol_max);
-    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    // the lanes of a team take the same decisions; the first one writes
+    const uint32_t t = (blockIdx.x * blockDim.x + threadIdx.x) / kT;
+    const uint32_t tl = threadIdx.x % kT;
+    const bool leader = tl == 0u;
     if (t >= F.n_tracks) {
         return;
     }
@@ -319,13 +357,14 @@ __global__ __launch_bounds__(kFitBlock) void k_fit_forward(fit_params F, uint32_
         sf = F.meas_sf[moff + F.cons[s0]];
     }
     inflate(c, F.inflation);
-    for (uint32_t k = 0; k < n; ++k) {
+    for (uint32_t k = tl; k < n; k += kT) {
         F.flags[s0 + k] = 0u;
         F.state_sf[s0 + k] = F.meas_sf[moff + F.cons[s0 + k]];
     }
     uint32_t* seq = F.seq + static_cast<size_t>(s0) * F.seq_factor + static_cast<size_t>(t) * F.seq_min;
     const uint32_t cap = max(n * F.seq_factor, F.seq_min);
     uint32_t k = 0u, holes = 0u, n_seq = 0u, status = n > 0u ? kSuccess : kIncomplete;
+    uint32_t filtered = 0u;  // states with a record
     uint32_t next_sf = n > 0u ? F.meas_sf[moff + F.cons[s0]] : 0xffffffffu;
     while (k < n) {
         add_material_sf(F.sfs[sf], F.nav.mass, F.nav.abs_q, x, c);
@@ -337,14 +376,19 @@ __global__ __launch_bounds__(kFitBlock) void k_fit_forward(fit_params F, uint32_
                 status = static_cast<uint32_t>(st);
                 break;
             }
-            float* r = F.flt + static_cast<size_t>(s0 + k) * kRec;
-            store_rec(r, x, c);
-            r[kRecChi2a] = predicted_chi2(md, x, c);
+            const float chi2 = predicted_chi2(md, x, c);
+            if (leader) {
+                store_rec(F.flt + static_cast<size_t>(s0 + k) * kRec, x, c, chi2, 0.f);
+            }
+            filtered = k + 1u;
             if (n_seq == cap) {
                 status = kSequenceOverflow;
                 break;
             }
-            seq[n_seq++] = kSeqState | sf;
+            if (leader) {
+                seq[n_seq] = kSeqState | sf;
+            }
+            ++n_seq;
             if (++k == n) {
                 break;
             }
@@ -364,13 +408,16 @@ __global__ __launch_bounds__(kFitBlock) void k_fit_forward(fit_params F, uint32_
                     status = kSequenceOverflow;
                     break;
                 }
-                seq[n_seq++] = sf;
+                if (leader) {
+                    seq[n_seq] = sf;
+                }
+                ++n_seq;
             }
         }
         uint32_t n_rk = 0u;
         float leg = 0.f;
-        const int nav = transport_bound<1>(G, s_nav.layers, F.nav, x, c, sf, n_rk, leg, 0u,
-                                           &s_nav, F.n_groups);
+        const int nav = transport_bound<kT>(G, s_nav.layers, F.nav, x, c, sf, n_rk, leg, tl,
+                                            &s_nav, F.n_groups);
         if (nav == NAV_EXIT) {
             status = kIncomplete;
             break;
@@ -380,7 +427,23 @@ __global__ __launch_bounds__(kFitBlock) void k_fit_forward(fit_params F, uint32_
             break;
         }
     }
-    F.fw_info[t] = status | (min(holes, 255u) << 8) | (n_seq << 16);
+    // states that the walk did not reach (a later iteration leaves the last one's)
+    for (uint32_t q = filtered + tl; iteration == 0u && q < n; q += kT) {
+        zero_rec(F.flt + static_cast<size_t>(s0 + q) * kRec);
+    }
+    if (leader) {
+        F.fw_info[t] = status | (min(holes, 255u) << 8) | (n_seq << 16);
+    }
+}
+
+// A first iteration that did not end in a fit: what it has not written.
+__device__ inline void zero_unfitted(const fit_params& F, uint32_t t, uint32_t s0, uint32_t unsmoothed) {
+    F.out_surface[t] = 0u;
+#pragma unroll
+    for (int q = 0; q < 6; ++q) F.out_vec[6u * static_cast<size_t>(t) + q] = 0.f;
+#pragma unroll
+    for (int q = 0; q < 21; ++q) F.out_cov[21u * static_cast<size_t>(t) + q] = 0.f;
+    for (uint32_t k = 0; k < unsmoothed; ++k) zero_rec(F.smt + static_cast<size_t>(s0 + k) * kRec);
 }
 
 __global__ __launch_bounds__(kFitBlock) void k_fit_backward(fit_params F, uint32_t iteration) {
@@ -399,15 +462,16 @@ __global__ __launch_bounds__(kFitBlock) void k_fit_backward(fit_params F, uint32
     F.out_ndf[t] = 0.f;
     F.out_chi2[t] = 0.f;
     F.out_pval[t] = 0.f;
+    const uint32_t s0 = F.offsets[t];
+    const uint32_t n = F.offsets[t + 1u] - s0;
     if (fw != kSuccess) {
+        if (iteration == 0u) zero_unfitted(F, t, s0, n);
         F.outcome[t] = fw == kUpdaterSkipped      ? CKF_OUTCOME_FAILURE_NOT_ALL_FITTED
                        : fw == kPropagationFailure ? CKF_OUTCOME_FAILURE_FORWARD_PROPAGATION
                        : (fw == kSequenceOverflow || fw == kIncomplete) ? CKF_OUTCOME_FAILURE_SMOOTHER
                                                                          : CKF_OUTCOME_FAILURE_FITTER;
         return;
     }
-    const uint32_t s0 = F.offsets[t];
-    const uint32_t n = F.offsets[t + 1u] - s0;
     const uint32_t moff = F.ev_meas_off[track_event(F, t)];
     const uint32_t* seq = F.seq + static_cast<size_t>(s0) * F.seq_factor + static_cast<size_t>(t) * F.seq_min;
     const geo_view G{F.sfs, F.n_layers, F.field};
@@ -415,10 +479,8 @@ __global__ __launch_bounds__(kFitBlock) void k_fit_backward(fit_params F, uint32
     // from the inflated filtered state
     float x[6], c[21];
     load_rec(F.flt + static_cast<size_t>(s0 + n - 1u) * kRec, x, c);
-    {
-        float* r = F.smt + static_cast<size_t>(s0 + n - 1u) * kRec;
-        store_rec(r, x, c);
-    }
+    store_rec(F.smt + static_cast<size_t>(s0 + n - 1u) * kRec, x, c, 0.f, 0.f);
+    uint32_t unsmoothed = n - 1u;  // states without a record
     inflate(c, F.inflation);
     uint32_t sf = F.meas_sf[moff + F.cons[s0 + n - 1u]];
     uint32_t j = n;  // states still to smooth: j - 1 is the next
@@ -443,15 +505,14 @@ __global__ __launch_bounds__(kFitBlock) void k_fit_backward(fit_params F, uint32
             if (status != kSuccess) {
                 break;
             }
-            float* r = F.smt + static_cast<size_t>(g) * kRec;
-            store_rec(r, xs, cs);
-            r[kRecChi2a] = chi2_s;
-            r[kRecChi2b] = chi2_b;
+            store_rec(F.smt + static_cast<size_t>(g) * kRec, xs, cs, chi2_s, chi2_b);
+            unsmoothed = min(unsmoothed, j);
             F.flags[g] = CKF_STATE_SMOOTHED;
         }
         add_material_sf(F.sfs[target], F.nav.mass, F.nav.abs_q, x, c);
     }
     if (status != kSuccess) {
+        if (iteration == 0u) zero_unfitted(F, t, s0, unsmoothed);
         F.outcome[t] = status == kSmootherSkipped     ? CKF_OUTCOME_FAILURE_NOT_ALL_SMOOTHED
                        : status == kPropagationFailure ? CKF_OUTCOME_FAILURE_BACKWARD_PROPAGATION
                                                        : CKF_OUTCOME_FAILURE_SMOOTHER;
@@ -595,28 +656,20 @@ ckf_status ckf_fit_tracks(ckf_fitter* f, const ckf_device_detector* det, const c
             R->n_states = ns;
             R->ids = det->ids;
             R->ev_track_off = cand->ev_track_off;
-            R->outcome.ensure(2u * std::max(n, 1u));
-            R->surface.ensure(4u * std::max(n, 1u));
-            R->vec.ensure(24u * std::max(n, 1u));
-            R->cov.ensure(84u * std::max(n, 1u));
-            R->ndf.ensure(4u * std::max(n, 1u));
-            R->chi2.ensure(4u * std::max(n, 1u));
-            R->pval.ensure(4u * std::max(n, 1u));
-            R->nholes.ensure(4u * std::max(n, 1u));
-            R->offsets.ensure(4u * (n + 1u));
-            R->cons.ensure(4u * std::max(ns, 1u));
-            R->flt.ensure(sizeof(float) * tamd::kRec * std::max<size_t>(ns, 1u));
-            R->smt.ensure(sizeof(float) * tamd::kRec * std::max<size_t>(ns, 1u));
-            R->flags.ensure(std::max(ns, 1u));
-            R->state_sf.ensure(4u * std::max(ns, 1u));
-            hip_check(hipMemsetAsync(R->flags.p, 0, R->flags.bytes, s), "memset");
-            hip_check(hipMemsetAsync(R->state_sf.p, 0, R->state_sf.bytes, s), "memset");
-            hip_check(hipMemsetAsync(R->outcome.p, 0, R->outcome.bytes, s), "memset");
-            hip_check(hipMemsetAsync(R->surface.p, 0, R->surface.bytes, s), "memset");
-            hip_check(hipMemsetAsync(R->vec.p, 0, R->vec.bytes, s), "memset");
-            hip_check(hipMemsetAsync(R->cov.p, 0, R->cov.bytes, s), "memset");
-            hip_check(hipMemsetAsync(R->smt.p, 0, R->smt.bytes, s), "memset");
-            hip_check(hipMemsetAsync(R->flt.p, 0, R->flt.bytes, s), "memset");
+            R->outcome.take(2u * std::max(n, 1u));
+            R->surface.take(4u * std::max(n, 1u));
+            R->vec.take(24u * std::max(n, 1u));
+            R->cov.take(84u * std::max(n, 1u));
+            R->ndf.take(4u * std::max(n, 1u));
+            R->chi2.take(4u * std::max(n, 1u));
+            R->pval.take(4u * std::max(n, 1u));
+            R->nholes.take(4u * std::max(n, 1u));
+            R->offsets.take(4u * (n + 1u));
+            R->cons.take(4u * std::max(ns, 1u));
+            R->flt.take(sizeof(float) * tamd::kRec * std::max<size_t>(ns, 1u));
+            R->smt.take(sizeof(float) * tamd::kRec * std::max<size_t>(ns, 1u));
+            R->flags.take(std::max(ns, 1u));
+            R->state_sf.take(4u * std::max(ns, 1u));
             hip_check(hipMemcpyAsync(R->offsets.p, cand->offsets, 4u * (n + 1u),
                                      hipMemcpyDeviceToDevice, s), "copy offsets");
             if (ns > 0u) {
@@ -672,8 +725,16 @@ ckf_status ckf_fit_tracks(ckf_fitter* f, const ckf_device_detector* det, const c
                 F.out_pval = R->pval.as<float>();
                 F.out_nholes = R->nholes.as<uint32_t>();
                 const uint32_t blocks = (n + tamd::kFitBlock - 1u) / tamd::kFitBlock;
+                const uint32_t team = n <= tamd::kFitTeam16 ? 16u : n <= tamd::kFitTeam8 ? 8u : 1u;
+                const dim3 fw((n * team + tamd::kFitBlock - 1u) / tamd::kFitBlock);
                 for (uint32_t it = 0; it < f->cfg.n_iterations; ++it) {
-                    hipLaunchKernelGGL(tamd::k_fit_forward, dim3(blocks), dim3(tamd::kFitBlock), 0, s, F, it);
+                    if (team == 16u) {
+                        hipLaunchKernelGGL(tamd::k_fit_forward<16>, fw, dim3(tamd::kFitBlock), 0, s, F, it);
+                    } else if (team == 8u) {
+                        hipLaunchKernelGGL(tamd::k_fit_forward<8>, fw, dim3(tamd::kFitBlock), 0, s, F, it);
+                    } else {
+                        hipLaunchKernelGGL(tamd::k_fit_forward<1>, fw, dim3(tamd::kFitBlock), 0, s, F, it);
+                    }
                     hip_check(hipGetLastError(), "fit forward");
                     hipLaunchKernelGGL(tamd::k_fit_backward, dim3(blocks), dim3(tamd::kFitBlock), 0, s, F, it);
                     hip_check(hipGetLastError(), "fit backward");
@@ -681,6 +742,7 @@ ckf_status ckf_fit_tracks(ckf_fitter* f, const ckf_device_detector* det, const c
             }
             hip_check(hipStreamSynchronize(s), "fit");
         } catch (...) {
+            (void)hipStreamSynchronize(s);  // the result's blocks may be handed out again
             delete R;
             throw;
         }
