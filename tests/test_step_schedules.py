@@ -93,3 +93,30 @@ def test_duplicate_removal_lengths(minimum):
     assert len(want) < 1.5 * len(again)
     assert np.array_equal(got.offsets, want.offsets)
     assert np.array_equal(got.constituents, want.constituents)
+
+
+@pytest.mark.parametrize("events", [2, 10])  # 6,000 and 30,000 seeds
+def test_progressive_teams_and_window(events):
+    """The progressive filter walks a seed with 16, 8 or one lane by how many
+    seeds there are: an event's tracks are the same alone and in a batch, and with
+    its surfaces' measurements in reverse order (no loc0 window then)."""
+    det, fld, gun = S.workload("C4", n_particles=3000, seed=41)
+    evs = S.generate_events(det, fld, [dataclasses.replace(gun, seed=90 + e) for e in range(events)])
+    cfg = S.finding_config_for("C4")
+    cfg.run_pkf = 1
+    ddet = ckf.DeviceDetector(det, fld)
+    alg = ckf.combinatorial_kalman_filter_algorithm(cfg)
+    one = alg.run_device(ddet, ckf.DeviceEvents(ddet, evs[:1])).download()
+    many = alg.run_device(ddet, ckf.DeviceEvents(ddet, evs)).download()
+    assert len(one) <= 5120 < len(many) and (len(many) > 28672) == (events == 10)
+    assert np.diff(one.offsets.astype(np.int64)).max() > 3
+    for a, b in zip(_columns(one), _columns(many.event(0))):
+        assert np.array_equal(a, b)
+    sl = evs[0].surface_link
+    order = np.lexsort((-np.arange(len(sl)), sl))
+    rev = dataclasses.replace(evs[0], **{f: np.ascontiguousarray(getattr(evs[0], f)[order]) for f in (
+        "local_position", "local_variance", "dimensions", "time", "diameter", "identifier", "surface_link", "subspace",
+        "cluster_index", "meas_particle")}, _keep=[])
+    back = alg.run_device(ddet, ckf.DeviceEvents(ddet, rev)).download()
+    assert np.array_equal(one.offsets, back.offsets) and np.array_equal(one.constituents, order[back.constituents])
+    assert np.array_equal(one.chi2, back.chi2)

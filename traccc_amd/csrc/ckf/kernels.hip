@@ -30,6 +30,7 @@
 #include "../scorer/mlp_device.hpp"
 #include "state_io.hpp"
 #include "wave.hpp"
+#include "window.hpp"
 
 namespace tamd {
 
@@ -62,7 +63,6 @@ constexpr int kFindTeam = 2;
 constexpr int kListTeam = 4;
 // scorer lists: up to kListTeam * kListSlots candidates per input
 constexpr int kListSlots = 4;
-constexpr int kBatch = 4;
 
 // One pass of a team over the surface's measurements [lo, up): the best
 // (chi2, index) candidate after (last_c, last_m) (every candidate when
@@ -128,43 +128,6 @@ struct find_input {
     bool rule0;
 };
 
-// A superset [lo, up) of the surface's measurements whose loc0 can lie in
-// [a, b], for measurements sorted by loc0: cooperative 16-ary narrowing by
-// the team (kT lanes x kBatch probes per round, one memory latency each)
-// of the first index >= a and of the first index > b.
-template <int kT>
-__device__ inline void window_range(const ckf_params& P, float a, float b, uint32_t tl,
-                                    uint32_t& lo, uint32_t& up) {
-    constexpr uint32_t kProbes = kT * kBatch;
-    for (int bound = 0; bound < 2; ++bound) {
-        const float key = bound == 0 ? a : b;
-        uint32_t L = lo, H = up;  // the wanted index lies in [L, H]
-        while (H - L > kProbes) {
-            const uint32_t span = H - L;
-            uint32_t below = 0u;
-#pragma unroll
-            for (int u = 0; u < kBatch; ++u) {
-                const uint32_t k = static_cast<uint32_t>(u * kT) + tl;
-                const uint32_t pos = L + ((k + 1u) * span) / (kProbes + 1u);
-                const float v = P.meas_pos[pos].x;
-                below += (bound == 0 ? (v < key) : !(v > key)) ? 1u : 0u;
-            }
-#pragma unroll
-            for (int d = kT / 2; d >= 1; d >>= 1) below += __shfl_xor(below, d, kT);
-            // probes are sorted: `below` of them precede the wanted index
-            const uint32_t nL = below == 0u ? L : L + (below * span) / (kProbes + 1u) + 1u;
-            const uint32_t nH = below == kProbes ? H : L + ((below + 1u) * span) / (kProbes + 1u);
-            L = nL;
-            H = nH;
-        }
-        if (bound == 0) {
-            lo = L;
-        } else {
-            up = H;
-        }
-    }
-}
-
 // Candidates of one input in (chi2, index) order from a single pass over the
 // surface's measurements (its loc0 window when the event allows one): every
 // lane keeps the kLaneKeep best passing candidates of its share in registers
@@ -199,16 +162,10 @@ __device__ __forceinline__ void stream_init(const ckf_params& P, const find_inpu
         S.lm[j] = kInvalid;
     }
     uint32_t np = 0u;
-    // a measurement passing the cut has r0^2 <= chi2_max (P00 + V00)
-    // (chi2 >= r0^2 / R00 for any 2x2 SPD R): outside that loc0 window none
-    // can pass, so on a dense surface sorted by loc0 only the window is read
+    // on a dense surface sorted by loc0 only the window of measurements that
+    // can pass is read
     uint32_t lo = in.lo, up = in.up;
-    if (in.win_var >= 0.f && up - lo > static_cast<uint32_t>(kT * kBatch)) {
-        const float w = sqrtf(P.chi2_max * (in.c[sym_idx(0, 0)] + in.win_var)) * 1.01f + 1e-3f;
-        if (w == w) {
-            window_range<kT>(P, in.x[e_loc0] - w, in.x[e_loc0] + w, tl, lo, up);
-        }
-    }
+    narrow_to_window<kT>(P, in.win_var, in.x[e_loc0], in.c[sym_idx(0, 0)], tl, lo, up);
     for (uint32_t m0 = lo + tl; m0 < up; m0 += kT * kBatch) {
         meas_data mb[kBatch];
 #pragma unroll

@@ -6,9 +6,10 @@
 //   measurement_updater actor      core/include/traccc/finding/actors/measurement_kalman_updater.hpp:94-260
 //   find_optimal_measurement       core/include/traccc/finding/measurement_selector.hpp:224-264
 //
-// There is no step structure: one lane walks one seed through the detector in
-// a single persistent kernel (waves take 64-seed partitions from a ticket
-// queue), writing its measurements into a fixed per-seed slot range.  A scan
+// There is no step structure: a team of lanes (one lane where there are many
+// seeds) walks one seed through the detector in a single persistent kernel
+// (waves take partitions of seeds from a ticket queue), writing its measurements
+// into a fixed per-seed slot range.  A scan
 // with decoupled look-back then lays the tracks out in seed order, one entry
 // per seed as the reference does (an empty entry where no track survived).
 #include <hip/hip_runtime.h>
@@ -21,6 +22,7 @@
 #include "kernels.hpp"
 #include "state_io.hpp"
 #include "wave.hpp"
+#include "window.hpp"
 
 namespace tamd {
 
@@ -34,9 +36,56 @@ __device__ inline bool momentum_above(const ckf_params& P, const float* x, float
     return pT > P.nav.min_pT / div && p > P.nav.min_p / div;
 }
 
-// One seed's walk through the detector.
+// The best measurement of [lo, up) by a team: find_optimal_measurement takes
+// them in order, keeps the lowest chi2 (the first index on ties) and stops at
+// one within eps of zero, which is the first such index: both are the minimum of
+// (chi2, zero within eps; index).  Only a measurement within the cut is used, so
+// the loc0 window's are enough.
+template <int kT>
+__device__ inline uint32_t best_measurement(const ckf_params& P, const float* x, const float* c, float win_var,
+                                            uint32_t lo, uint32_t up, float eps, uint32_t tl, float& chi2_out) {
+    narrow_to_window<kT>(P, win_var, x[e_loc0], c[sym_idx(0, 0)], tl, lo, up);
+    uint32_t best = kInvalid;
+    float key = FLT_MAX;
+    for (uint32_t m0 = lo + tl; m0 < up; m0 += kT * kBatch) {
+        meas_data mb[kBatch];
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u) {
+            const uint32_t m = m0 + static_cast<uint32_t>(u * kT);
+            mb[u] = load_meas(P.meas_pos, P.meas_var, P.meas_info, m < up ? m : lo);
+        }
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u) {
+            const uint32_t m = m0 + static_cast<uint32_t>(u * kT);
+            const float chi2 = predicted_chi2(mb[u], x, c);
+            const float k = chi2 <= eps ? 0.f : chi2;
+            if (m < up && chi2 >= 0.f && (k < key || (k == key && m < best))) {
+                best = m;
+                key = k;
+            }
+        }
+    }
+#pragma unroll
+    for (int d = kT / 2; d >= 1; d >>= 1) {
+        const float ok = __shfl_xor(key, d, kT);
+        const uint32_t om = __shfl_xor(best, d, kT);
+        if (om != kInvalid && (ok < key || (ok == key && om < best))) {
+            best = om;
+            key = ok;
+        }
+    }
+    chi2_out = FLT_MAX;
+    if (best != kInvalid) {
+        chi2_out = predicted_chi2(load_meas(P.meas_pos, P.meas_var, P.meas_info, best), x, c);
+    }
+    return best;
+}
+
+// One seed's walk through the detector (the team's lanes take it together;
+// the first one writes).
+template <int kT>
 __device__ inline void walk_seed(const ckf_params& P, const pkf_params& Q, const nav_tables& s_nav,
-                                 const nav_config<float>& leg_cfg, uint32_t s) {
+                                 const nav_config<float>& leg_cfg, uint32_t s, uint32_t tl) {
     const float eps = FLT_EPSILON;
     float x[6], c[21];
     uint32_t sf = 0u;
@@ -47,25 +96,13 @@ __device__ inline void walk_seed(const ckf_params& P, const pkf_params& Q, const
     if (momentum_above(P, x, 10.f)) {
         const uint32_t ev = P.seed_event[s];
         const uint32_t* rg = P.meas_ranges + static_cast<size_t>(ev) * (P.n_surfaces + 1u);
+        const float win_var = P.event_win_var[ev];
         uint32_t* states = Q.states + static_cast<size_t>(s) * Q.max_states;
         for (;;) {
             add_material(P, sf, x, c);
             // find_optimal_measurement: lowest chi2, first index on ties
-            const uint32_t lo = rg[sf];
-            const uint32_t up = rg[sf + 1u];
-            uint32_t best = kInvalid;
             float best_chi2 = FLT_MAX;
-            for (uint32_t m = lo; m < up; ++m) {
-                const meas_data md = load_meas(P.meas_pos, P.meas_var, P.meas_info, m);
-                const float chi2 = predicted_chi2(md, x, c);
-                if (chi2 < best_chi2 && chi2 >= 0.f) {
-                    best = m;
-                    best_chi2 = chi2;
-                    if (best_chi2 <= eps) {
-                        break;
-                    }
-                }
-            }
+            const uint32_t best = best_measurement<kT>(P, x, c, win_var, rg[sf], rg[sf + 1u], eps, tl, best_chi2);
             int res = CKF_FIT_ERROR_OTHER;
             if (best != kInvalid && best_chi2 <= P.chi2_max) {
                 const meas_data md = load_meas(P.meas_pos, P.meas_var, P.meas_info, best);
@@ -84,7 +121,9 @@ __device__ inline void walk_seed(const ckf_params& P, const pkf_params& Q, const
                 ++consec;
                 exit = holes > P.max_skip || consec > P.max_consec;
             } else {
-                states[n_states] = best;
+                if (tl == 0u) {
+                    states[n_states] = best;
+                }
                 ++n_states;
                 consec = 0u;
                 ndf += P.meas_info[best] & 0xffu;
@@ -97,8 +136,8 @@ __device__ inline void walk_seed(const ckf_params& P, const pkf_params& Q, const
             }
             uint32_t n_rk = 0u;
             float leg = 0.f;
-            const int status = transport_state(P, s_nav.layers, leg_cfg, x, c, sf, n_rk, leg, 0u,
-                                               &s_nav, P.n_groups);
+            const int status = transport_state<kT>(P, s_nav.layers, leg_cfg, x, c, sf, n_rk, leg, tl,
+                                                   &s_nav, P.n_groups);
             path += leg;
             if (status == NAV_EXIT) {
                 good = true;  // left the detector
@@ -111,12 +150,22 @@ __device__ inline void walk_seed(const ckf_params& P, const pkf_params& Q, const
         good = good && momentum_above(P, x, 1.f) && n_states >= P.min_cands &&
                static_cast<int>(ndf) - 5 >= 0;
     }
-    Q.n_states[s] = good ? n_states : 0u;
-    Q.chi2[s] = chi2_sum;
-    Q.ndf[s] = ndf;
-    Q.holes[s] = holes;
+    if (tl == 0u) {
+        Q.n_states[s] = good ? n_states : 0u;
+        Q.chi2[s] = chi2_sum;
+        Q.ndf[s] = ndf;
+        Q.holes[s] = holes;
+    }
 }
 
+// A seed is one chain of searches, updates and propagations through the whole
+// detector: up to kTeam16 seeds 16 lanes take one together, up to kTeam8 seeds
+// 8, then the lanes are worth more than the chain (10,000 muons: 1,064 us with one
+// lane that also read every measurement of its surfaces, 319 with 8).
+constexpr uint32_t kTeam16 = 5120u;
+constexpr uint32_t kTeam8 = 28672u;
+
+template <int kT>
 __global__ __launch_bounds__(kBlock) void k_pkf(ckf_params P, pkf_params Q) {
     // the navigation layers and groups live in LDS for the whole kernel
     __shared__ nav_tables s_nav;
@@ -128,15 +177,16 @@ __global__ __launch_bounds__(kBlock) void k_pkf(ckf_params P, pkf_params Q) {
     leg_cfg.min_step_length = 0.f;
     leg_cfg.max_steps = 0x7fffffffu;
     const uint32_t n = P.n_seeds;
-    const uint32_t n_parts = (n + kWave - 1) / kWave;
+    constexpr uint32_t kPerWave = kWave / kT;
+    const uint32_t n_parts = (n + kPerWave - 1) / kPerWave;
     for (;;) {
         const uint32_t p = wave_ticket(&ctl->ticket[0].v);
         if (p >= n_parts) {
             break;
         }
-        const uint32_t s = p * kWave + lane();
+        const uint32_t s = p * kPerWave + lane() / kT;
         if (s < n) {
-            walk_seed(P, Q, s_nav, leg_cfg, s);
+            walk_seed<kT>(P, Q, s_nav, leg_cfg, s, lane() % kT);
         }
     }
 }
@@ -214,7 +264,16 @@ __global__ __launch_bounds__(kBlock) void k_pkf_write(ckf_params P, pkf_params Q
 hipError_t launch_pkf(const ckf_params& P, const pkf_params& Q, uint32_t n_cu, hipStream_t stream) {
     const uint32_t parts = (P.n_seeds + kWave - 1u) / kWave;
     const uint32_t blocks = std::max(1u, std::min((parts + 3u) / 4u, n_cu * 8u));
-    hipLaunchKernelGGL(k_pkf, dim3(blocks), dim3(kBlock), 0, stream, P, Q);
+    const uint32_t team = P.n_seeds <= kTeam16 ? 16u : P.n_seeds <= kTeam8 ? 8u : 1u;
+    const uint64_t lanes = uint64_t(P.n_seeds) * team;
+    const dim3 walk(static_cast<uint32_t>(std::max<uint64_t>(1u, std::min<uint64_t>((lanes + kBlock - 1u) / kBlock, n_cu * 8u))));
+    if (team == 16u) {
+        hipLaunchKernelGGL(k_pkf<16>, walk, dim3(kBlock), 0, stream, P, Q);
+    } else if (team == 8u) {
+        hipLaunchKernelGGL(k_pkf<8>, walk, dim3(kBlock), 0, stream, P, Q);
+    } else {
+        hipLaunchKernelGGL(k_pkf<1>, walk, dim3(kBlock), 0, stream, P, Q);
+    }
     hipLaunchKernelGGL(k_pkf_scan, dim3(blocks), dim3(kBlock), 0, stream, P, Q);
     return hipGetLastError();
 }
