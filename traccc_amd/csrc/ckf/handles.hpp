@@ -8,6 +8,7 @@
 #include <algorithm>
 #include <cstdint>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <vector>
 
@@ -122,6 +123,9 @@ struct rbuf {
     }
 };
 
+// Surface index -> identifier, made once per detector and held by its results.
+using id_table = std::shared_ptr<const std::vector<uint64_t>>;
+
 template <typename T>
 T* dev_copy(const T* src, size_t n) {
     T* d = nullptr;
@@ -138,7 +142,7 @@ T* dev_copy(const T* src, size_t n) {
 struct ckf_device_detector {
     std::vector<ckf_surface> h_sfs;
     std::vector<ckf_layer> h_layers;
-    std::vector<uint64_t> ids;
+    tamd::id_table ids;
     ckf_bfield field{};
     ckf_surface* d_sfs = nullptr;
     ckf_layer* d_layers = nullptr;
@@ -182,7 +186,7 @@ struct ckf_device_event {
 // per-state filtered / smoothed records.
 struct ckf_device_fitted {
     uint32_t n_tracks = 0, n_states = 0;
-    std::vector<uint64_t> ids;            // surface index -> identifier
+    tamd::id_table ids;
     std::vector<uint32_t> ev_track_off;   // [n_events + 1] tracks of each event
     tamd::rbuf outcome, surface, vec, cov, ndf, chi2, pval, nholes, offsets, cons, flt, smt, flags,
         state_sf;
@@ -191,7 +195,7 @@ struct ckf_device_fitted {
 struct ckf_device_tracks {
     uint32_t n_events = 0, n_tracks = 0, n_const = 0;
     std::vector<uint32_t> ev_track_off, ev_const_off;
-    std::vector<uint64_t> ids;
+    tamd::id_table ids;
     uint16_t* outcome = nullptr;
     uint32_t* surface = nullptr;
     float* vec = nullptr;

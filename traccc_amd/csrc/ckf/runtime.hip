@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "../common/errors.hpp"
+#include "../common/readback.hpp"
 #include "handles.hpp"
 #include "kernels.hpp"
 #include "traccc_amd/ckf.h"
@@ -475,7 +476,6 @@ uint32_t run_steps(ckf_algorithm& A, const tamd::ckf_params& P, const tamd::laun
     if (P.verdict_n != nullptr) {
         hip_check(hipMemsetAsync(P.verdict_n, 0, 4u, A.stream), "memset");
     }
-    hip_check(hipStreamSynchronize(A.stream), "sync");
 
     if (A.timing) {
         return run_steps_timed(A, P, s);
@@ -733,10 +733,12 @@ ckf_device_tracks* find_tracks_pkf(ckf_algorithm& A, const ckf_device_detector& 
         if (ns > 0u) {
             hip_check(tamd::launch_pkf_write(P, Q, static_cast<uint32_t>(A.n_cu), A.stream),
                       "pkf write");
-            hip_check(hipMemcpyAsync(T->ev_const_off.data(), P.event_const_off,
-                                     4u * ev.n_events, hipMemcpyDeviceToHost, A.stream),
-                      "offsets");
+            const tamd::pinned_block off(4u * size_t(ev.n_events));
+            const hipError_t copied = hipMemcpyAsync(off.p, P.event_const_off, 4u * size_t(ev.n_events),
+                                                     hipMemcpyDeviceToHost, A.stream);
             hip_check(hipStreamSynchronize(A.stream), "pkf write sync");
+            hip_check(copied, "offsets");
+            std::memcpy(T->ev_const_off.data(), off.p, 4u * size_t(ev.n_events));
         } else {
             hip_check(hipMemcpyAsync(T->offsets, T->ev_const_off.data(), 4u, hipMemcpyHostToDevice,
                                      A.stream),
@@ -871,13 +873,16 @@ ckf_device_tracks* find_tracks(ckf_algorithm& A, const ckf_device_detector& D,
         }
         T->ev_track_off.resize(ev.n_events + 1u);
         T->ev_const_off.resize(ev.n_events + 1u);
-        hip_check(hipMemcpyAsync(T->ev_track_off.data(), track_off, 4u * (ev.n_events + 1u),
-                                 hipMemcpyDeviceToHost, A.stream),
-                  "offsets");
-        hip_check(hipMemcpyAsync(T->ev_const_off.data(), const_off, 4u * (ev.n_events + 1u),
-                                 hipMemcpyDeviceToHost, A.stream),
-                  "offsets");
+        const size_t off_bytes = 4u * (size_t(ev.n_events) + 1u);
+        const tamd::pinned_block off(2u * off_bytes);
+        char* const h_off = static_cast<char*>(off.p);
+        const hipError_t copied[2] = {
+            hipMemcpyAsync(h_off, track_off, off_bytes, hipMemcpyDeviceToHost, A.stream),
+            hipMemcpyAsync(h_off + off_bytes, const_off, off_bytes, hipMemcpyDeviceToHost, A.stream)};
         hip_check(hipStreamSynchronize(A.stream), "build write sync");
+        for (const hipError_t e : copied) hip_check(e, "offsets");
+        std::memcpy(T->ev_track_off.data(), h_off, off_bytes);
+        std::memcpy(T->ev_const_off.data(), h_off + off_bytes, off_bytes);
         if (votes) {
             T->n_tracks = T->ev_track_off[ev.n_events];
             T->n_const = T->ev_const_off[ev.n_events];
@@ -895,6 +900,7 @@ ckf_device_event* upload_event(const ckf_device_detector& D, const ckf_measureme
         throw ckf_error(CKF_ERR_INVALID_ARGUMENT, "null event input");
     }
     const uint32_t S = static_cast<uint32_t>(D.h_sfs.size());
+    const std::vector<uint64_t>& ids = *D.ids;
     auto* E = new ckf_device_event();
     try {
         E->n_events = n_events;
@@ -943,7 +949,7 @@ ckf_device_event* upload_event(const ckf_device_detector& D, const ckf_measureme
             uint32_t* row = ranges.data() + size_t(e) * (S + 1u);
             row[0] = off;
             for (uint32_t s = 0; s < S; ++s) {
-                const uint64_t id = D.ids[s];
+                const uint64_t id = ids[s];
                 const uint64_t* b = M.surface_link;
                 const uint32_t ub = static_cast<uint32_t>(std::upper_bound(b, b + M.size, id) - b);
                 row[s + 1u] = off + ub;
@@ -956,7 +962,7 @@ ckf_device_event* upload_event(const ckf_device_detector& D, const ckf_measureme
                 throw ckf_error(CKF_ERR_INVALID_ARGUMENT, "measurement on an unknown surface");
             }
             for (uint32_t i = 0; i < M.size; ++i) {
-                if (D.ids[meas_sf[off + i]] != M.surface_link[i]) {
+                if (ids[meas_sf[off + i]] != M.surface_link[i]) {
                     throw ckf_error(CKF_ERR_INVALID_ARGUMENT, "measurement on an unknown surface");
                 }
             }
@@ -985,11 +991,11 @@ ckf_device_event* upload_event(const ckf_device_detector& D, const ckf_measureme
             for (uint32_t i = 0; i < B.size; ++i) {
                 const uint32_t g = E->seed_off[e] + i;
                 seed_event[g] = e;
-                const auto it = std::lower_bound(D.ids.begin(), D.ids.end(), B.surface_link[i]);
-                if (it == D.ids.end() || *it != B.surface_link[i]) {
+                const auto it = std::lower_bound(ids.begin(), ids.end(), B.surface_link[i]);
+                if (it == ids.end() || *it != B.surface_link[i]) {
                     throw ckf_error(CKF_ERR_INVALID_ARGUMENT, "seed on an unknown surface");
                 }
-                seed_surface[g] = static_cast<uint32_t>(it - D.ids.begin());
+                seed_surface[g] = static_cast<uint32_t>(it - ids.begin());
                 std::memcpy(&seed_vec[6u * size_t(g)], B.vector + 6u * size_t(i), 24u);
                 std::memcpy(&seed_cov[36u * size_t(g)], B.covariance + 36u * size_t(i), 144u);
             }
@@ -1031,10 +1037,10 @@ ckf_device_detector* upload_detector(const ckf_detector* det, const ckf_bfield* 
     try {
         D->h_sfs.assign(det->surfaces, det->surfaces + det->n_surfaces);
         D->h_layers.assign(det->layers, det->layers + det->n_layers);
-        D->ids.resize(det->n_surfaces);
+        std::vector<uint64_t> ids(det->n_surfaces);
         for (uint32_t i = 0; i < det->n_surfaces; ++i) {
-            D->ids[i] = det->surfaces[i].identifier;
-            if (i > 0u && D->ids[i] <= D->ids[i - 1u]) {
+            ids[i] = det->surfaces[i].identifier;
+            if (i > 0u && ids[i] <= ids[i - 1u]) {
                 throw ckf_error(CKF_ERR_INVALID_ARGUMENT,
                                 "surface identifiers must increase with the index");
             }
@@ -1042,6 +1048,7 @@ ckf_device_detector* upload_detector(const ckf_detector* det, const ckf_bfield* 
                 throw ckf_error(CKF_ERR_INVALID_ARGUMENT, "surface refers to an unknown layer");
             }
         }
+        D->ids = std::make_shared<const std::vector<uint64_t>>(std::move(ids));
         D->field = *field;
         D->d_sfs = dev_copy(det->surfaces, det->n_surfaces);
         D->d_layers = dev_copy(det->layers, det->n_layers);
@@ -1187,14 +1194,15 @@ ckf_status ckf_find_tracks_logged(ckf_algorithm* alg, const ckf_device_detector*
             const uint32_t n = static_cast<uint32_t>(A.stats.n_links);
             const tamd::ckf_params P = make_params(A, *det, *ev);
             const uint32_t blocks = (n + 1023u) / 1024u;
-            std::vector<uint32_t> counts(blocks + 1u, 0u);
             uint32_t total = 0u;
             if (blocks > 0u) {
-                uint32_t* d_cnt = nullptr;
-                hip_check(hipMalloc(&d_cnt, 4u * (blocks + 1u)), "log buffers");
+                tamd::rbuf d_cnt;
+                d_cnt.take(4u * (blocks + 1u));
+                const tamd::pinned_block h_cnt(4u * size_t(blocks));
+                uint32_t* const counts = static_cast<uint32_t*>(h_cnt.p);
                 try {
-                    hip_check(tamd::launch_log_count(P, n, d_cnt, A.stream), "log count");
-                    hip_check(hipMemcpyAsync(counts.data(), d_cnt, 4u * blocks, hipMemcpyDeviceToHost,
+                    hip_check(tamd::launch_log_count(P, n, d_cnt.as<uint32_t>(), A.stream), "log count");
+                    hip_check(hipMemcpyAsync(counts, d_cnt.p, 4u * size_t(blocks), hipMemcpyDeviceToHost,
                                              A.stream), "log count");
                     hip_check(hipStreamSynchronize(A.stream), "log count");
                     for (uint32_t b = 0; b < blocks; ++b) {
@@ -1202,18 +1210,17 @@ ckf_status ckf_find_tracks_logged(ckf_algorithm* alg, const ckf_device_detector*
                         counts[b] = total;
                         total += c;
                     }
-                    hip_check(hipMemcpyAsync(d_cnt, counts.data(), 4u * blocks, hipMemcpyHostToDevice,
+                    hip_check(hipMemcpyAsync(d_cnt.p, counts, 4u * size_t(blocks), hipMemcpyHostToDevice,
                                              A.stream), "log offsets");
                     if (capacity > 0u) {
-                        hip_check(tamd::launch_log_write(P, n, d_cnt, d_features, d_labels, capacity,
-                                                         A.stream), "log write");
+                        hip_check(tamd::launch_log_write(P, n, d_cnt.as<uint32_t>(), d_features, d_labels,
+                                                         capacity, A.stream), "log write");
                     }
                     hip_check(hipStreamSynchronize(A.stream), "log write");
                 } catch (...) {
-                    (void)hipFree(d_cnt);
+                    (void)hipStreamSynchronize(A.stream);  // the blocks may be handed out again
                     throw;
                 }
-                (void)hipFree(d_cnt);
             }
             *n_samples = total;
         } catch (...) {
@@ -1273,31 +1280,20 @@ ckf_status ckf_tracks_download(const ckf_device_tracks* trk, ckf_track_candidate
         const size_t nt = trk->n_tracks, nc = trk->n_const;
         out->n_tracks = trk->n_tracks;
         out->n_constituents = trk->n_const;
-        auto d2h = [](void* dst, const void* src, size_t bytes) {
-            if (dst != nullptr && bytes > 0) {
-                hip_check(hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost), "download");
-            }
-        };
-        d2h(out->fit_outcome, trk->outcome, 2u * nt);
-        d2h(out->params_vector, trk->vec, 24u * nt);
-        d2h(out->params_covariance, trk->cov, 144u * nt);
-        d2h(out->ndf, trk->ndf, 4u * nt);
-        d2h(out->chi2, trk->chi2, 4u * nt);
-        d2h(out->pval, trk->pval, 4u * nt);
-        d2h(out->nholes, trk->nholes, 4u * nt);
-        d2h(out->constituent_index, trk->cons, 4u * nc);
-        if (out->constituent_offsets != nullptr) {
-            // offsets index the whole (all-event) constituent array
-            d2h(out->constituent_offsets, trk->offsets, 4u * (nt + 1u));
-        }
-        if (out->params_surface_link != nullptr && nt > 0) {
-            std::vector<uint32_t> sf(nt);
-            d2h(sf.data(), trk->surface, 4u * nt);
-            for (size_t i = 0; i < nt; ++i) {
-                // an empty progressive-filter entry has no surface
-                out->params_surface_link[i] = sf[i] < trk->ids.size() ? trk->ids[sf[i]] : ~0ull;
-            }
-        }
+        tamd::readback rb;
+        rb.bytes(out->fit_outcome, trk->outcome, 2u * nt);
+        rb.bytes(out->params_vector, trk->vec, 24u * nt);
+        rb.bytes(out->params_covariance, trk->cov, 144u * nt);
+        rb.bytes(out->ndf, trk->ndf, 4u * nt);
+        rb.bytes(out->chi2, trk->chi2, 4u * nt);
+        rb.bytes(out->pval, trk->pval, 4u * nt);
+        rb.bytes(out->nholes, trk->nholes, 4u * nt);
+        rb.bytes(out->constituent_index, trk->cons, 4u * nc);
+        // offsets index the whole (all-event) constituent array
+        rb.bytes(out->constituent_offsets, trk->offsets, 4u * (nt + 1u));
+        // an empty progressive-filter entry has no surface
+        rb.identifiers(out->params_surface_link, trk->surface, nt, *trk->ids);
+        rb.run();
         if (out->constituent_type != nullptr) {
             std::fill(out->constituent_type, out->constituent_type + nc, uint16_t(0));
         }
@@ -1460,7 +1456,10 @@ ckf_status ckf_debug_kernel_times(const ckf_algorithm* alg, double* ms_find, dou
 }
 
 ckf_status ckf_release_cached_memory(void) {
-    return guarded([&] { result_cache().release(); });
+    return guarded([&] {
+        result_cache().release();
+        tamd::staging_cache().release();
+    });
 }
 
 ckf_status ckf_debug_set_verdict_log(ckf_algorithm* alg, uint32_t capacity) {

@@ -40,6 +40,7 @@
 #include "../ckf/kalman_device.hpp"
 #include "../ckf/state_io.hpp"
 #include "../common/errors.hpp"
+#include "../common/readback.hpp"
 #include "traccc_amd/fitting.h"
 
 namespace tamd {
@@ -600,13 +601,6 @@ tamd::nav_config<float> fit_nav(const ckf_fitting_config& c) {
     return n;
 }
 
-template <typename T>
-void d2h(T* dst, const void* src, size_t n, hipStream_t s) {
-    if (dst != nullptr && n > 0u) {
-        hip_check(hipMemcpyAsync(dst, src, n * sizeof(T), hipMemcpyDeviceToHost, s), "download");
-    }
-}
-
 }  // namespace
 
 extern "C" {
@@ -765,52 +759,31 @@ ckf_status ckf_fitted_download(const ckf_device_fitted* r, ckf_fitted_tracks* o)
             throw ckf_error(CKF_ERR_INVALID_ARGUMENT, "output sized for another result");
         }
         const uint32_t n = r->n_tracks, ns = r->n_states;
-        const hipStream_t s = nullptr;
-        std::vector<uint32_t> sfs(n), cons(ns), state_sf(ns);
-        std::vector<float> cov21(21u * size_t(n)), flt(size_t(ns) * tamd::kRec),
-            smt(size_t(ns) * tamd::kRec);
-        d2h(o->fit_outcome, r->outcome.p, n, s);
-        d2h(sfs.data(), r->surface.p, n, s);
-        d2h(o->params_vector, r->vec.p, 6u * size_t(n), s);
-        d2h(cov21.data(), r->cov.p, 21u * size_t(n), s);
-        d2h(o->ndf, r->ndf.p, n, s);
-        d2h(o->chi2, r->chi2.p, n, s);
-        d2h(o->pval, r->pval.p, n, s);
-        d2h(o->nholes, r->nholes.p, n, s);
-        d2h(o->state_offsets, r->offsets.p, n + 1u, s);
-        d2h(o->state_flags, r->flags.p, ns, s);
-        d2h(cons.data(), r->cons.p, ns, s);
-        d2h(state_sf.data(), r->state_sf.p, ns, s);
-        d2h(flt.data(), r->flt.p, flt.size(), s);
-        d2h(smt.data(), r->smt.p, smt.size(), s);
-        hip_check(hipStreamSynchronize(s), "download");
-        auto unpack = [](const float* c21, float* c36) {
-            for (int i = 0; i < 6; ++i)
-                for (int j = 0; j < 6; ++j) c36[6 * i + j] = c21[tamd::sym_idx(i, j)];
-        };
-        for (uint32_t t = 0; t < n; ++t) {
-            if (o->params_surface_link) {
-                const uint16_t oc = o->fit_outcome ? o->fit_outcome[t] : CKF_OUTCOME_SUCCESS;
-                o->params_surface_link[t] = (oc == CKF_OUTCOME_SUCCESS && sfs[t] < r->ids.size())
-                                                ? r->ids[sfs[t]] : ~0ull;
-            }
-            if (o->params_covariance) unpack(&cov21[21u * size_t(t)], o->params_covariance + 36u * size_t(t));
-        }
-        for (uint32_t g = 0; g < ns; ++g) {
-            const float* fr = &flt[size_t(g) * tamd::kRec];
-            const float* sr = &smt[size_t(g) * tamd::kRec];
-            if (o->filtered_chi2) o->filtered_chi2[g] = fr[tamd::kRecChi2a];
-            if (o->smoothed_chi2) o->smoothed_chi2[g] = sr[tamd::kRecChi2a];
-            if (o->backward_chi2) o->backward_chi2[g] = sr[tamd::kRecChi2b];
-            if (o->filtered_vector) std::memcpy(o->filtered_vector + 6u * size_t(g), fr, 24u);
-            if (o->smoothed_vector) std::memcpy(o->smoothed_vector + 6u * size_t(g), sr, 24u);
-            if (o->filtered_covariance) unpack(fr + 6, o->filtered_covariance + 36u * size_t(g));
-            if (o->smoothed_covariance) unpack(sr + 6, o->smoothed_covariance + 36u * size_t(g));
-            if (o->measurement_index) o->measurement_index[g] = cons[g];
-            if (o->state_surface_link) {
-                o->state_surface_link[g] = state_sf[g] < r->ids.size() ? r->ids[state_sf[g]] : ~0ull;
-            }
-        }
+        const float* flt = r->flt.as<float>();
+        const float* smt = r->smt.as<float>();
+        tamd::readback rb;
+        rb.bytes(o->fit_outcome, r->outcome.p, 2u * size_t(n));
+        // an identifier where the caller sees a successful fit
+        rb.identifiers(o->params_surface_link, r->surface.as<uint32_t>(), n, *r->ids,
+                       o->fit_outcome ? r->outcome.as<uint16_t>() : nullptr, CKF_OUTCOME_SUCCESS);
+        rb.bytes(o->params_vector, r->vec.p, 24u * size_t(n));
+        rb.symmetric(o->params_covariance, r->cov.p, n, 21u, 0u);
+        rb.bytes(o->ndf, r->ndf.p, 4u * size_t(n));
+        rb.bytes(o->chi2, r->chi2.p, 4u * size_t(n));
+        rb.bytes(o->pval, r->pval.p, 4u * size_t(n));
+        rb.bytes(o->nholes, r->nholes.p, 4u * size_t(n));
+        rb.bytes(o->state_offsets, r->offsets.p, 4u * (size_t(n) + 1u));
+        rb.bytes(o->state_flags, r->flags.p, ns);
+        rb.words(o->filtered_chi2, flt, ns, tamd::kRec, tamd::kRecChi2a, 1u);
+        rb.words(o->smoothed_chi2, smt, ns, tamd::kRec, tamd::kRecChi2a, 1u);
+        rb.words(o->backward_chi2, smt, ns, tamd::kRec, tamd::kRecChi2b, 1u);
+        rb.identifiers(o->state_surface_link, r->state_sf.as<uint32_t>(), ns, *r->ids);
+        rb.words(o->filtered_vector, flt, ns, tamd::kRec, 0u, 6u);
+        rb.symmetric(o->filtered_covariance, flt, ns, tamd::kRec, 6u);
+        rb.words(o->smoothed_vector, smt, ns, tamd::kRec, 0u, 6u);
+        rb.symmetric(o->smoothed_covariance, smt, ns, tamd::kRec, 6u);
+        rb.bytes(o->measurement_index, r->cons.p, 4u * size_t(ns));
+        rb.run();
     });
 }
 

@@ -38,6 +38,7 @@
 #include "../ckf/handles.hpp"
 #include "../ckf/wave.hpp"
 #include "../common/errors.hpp"
+#include "../common/readback.hpp"
 #include "../common/scan.hpp"
 #include "../core/geometry.hpp"
 #include "traccc_amd/seeding.h"
@@ -1232,17 +1233,13 @@ ckf_status ckf_seeding_result_download(const ckf_seeding* s, ckf_seeds* out) {
     return guarded([&] {
         if (s == nullptr || out == nullptr) throw ckf_error(CKF_ERR_INVALID_ARGUMENT, "null argument");
         if (out->size < s->n_seeds) throw ckf_error(CKF_ERR_INVALID_ARGUMENT, "output smaller than the seeds");
-        std::vector<tamd::seed_rec> h(s->n_seeds);
-        if (s->n_seeds > 0u) {
-            hip_check(hipMemcpy(h.data(), s->seeds.p, sizeof(tamd::seed_rec) * h.size(), hipMemcpyDeviceToHost),
-                      "download");
-        }
-        for (uint32_t i = 0; i < s->n_seeds; ++i) {
-            if (out->bottom) out->bottom[i] = h[i].b;
-            if (out->middle) out->middle[i] = h[i].m;
-            if (out->top) out->top[i] = h[i].t;
-            if (out->weight) out->weight[i] = h[i].w;
-        }
+        static_assert(sizeof(tamd::seed_rec) == 16u, "a seed is four words: bottom, middle, top, weight");
+        tamd::readback rb;
+        rb.words(out->bottom, s->seeds.p, s->n_seeds, 4u, 0u, 1u);
+        rb.words(out->middle, s->seeds.p, s->n_seeds, 4u, 1u, 1u);
+        rb.words(out->top, s->seeds.p, s->n_seeds, 4u, 2u, 1u);
+        rb.words(out->weight, s->seeds.p, s->n_seeds, 4u, 3u, 1u);
+        rb.run();
     });
 }
 
@@ -1256,43 +1253,41 @@ ckf_status ckf_spacepoint_formation(const ckf_device_detector* det, const ckf_de
         }
         const uint32_t m0 = ev->meas_off[event], nm = ev->meas_off[event + 1] - m0;
         const hipStream_t s = nullptr;
-        tamd::dbuf flag, off, sums, xyz, midx;
+        tamd::rbuf flag, off, sums, d_total, xyz, midx;
         const uint32_t N = std::max(nm, 1u);
-        flag.ensure(4u * size_t(N));
-        off.ensure(4u * (size_t(N) + 1u));
-        sums.ensure(4u * size_t(tamd::scan_sums_size(N)));
-        uint32_t* d_total = nullptr;
-        hip_check(hipMalloc(reinterpret_cast<void**>(&d_total), 4), "hipMalloc");
+        flag.take(4u * size_t(N));
+        off.take(4u * (size_t(N) + 1u));
+        sums.take(4u * size_t(tamd::scan_sums_size(N)));
+        d_total.take(4u);
+        const tamd::pinned_block h_total(4u);
         try {
             if (nm > 0u) {
                 hipLaunchKernelGGL(tamd::k_sd_sp_flag, dim3(tamd::grid_for(nm, tamd::kSdBlock)), dim3(tamd::kSdBlock),
                                    0, s, ev->d_info, m0, nm, flag.as<uint32_t>());
                 hip_check(hipGetLastError(), "spacepoint flags");
             }
-            tamd::exclusive_scan(flag.as<uint32_t>(), off.as<uint32_t>(), sums.as<uint32_t>(), nm, d_total, s);
-            uint32_t total = 0;
-            hip_check(hipMemcpy(&total, d_total, 4, hipMemcpyDeviceToHost), "readback");
+            tamd::exclusive_scan(flag.as<uint32_t>(), off.as<uint32_t>(), sums.as<uint32_t>(), nm,
+                                 d_total.as<uint32_t>(), s);
+            hip_check(hipMemcpyAsync(h_total.p, d_total.p, 4u, hipMemcpyDeviceToHost, s), "readback");
+            hip_check(hipStreamSynchronize(s), "readback");
+            const uint32_t total = *static_cast<const uint32_t*>(h_total.p);
             *n = total;
             if ((global != nullptr || measurement_index != nullptr) && total > 0u) {
-                xyz.ensure(12u * size_t(total));
-                midx.ensure(4u * size_t(total));
+                xyz.take(12u * size_t(total));
+                midx.take(4u * size_t(total));
                 hipLaunchKernelGGL(tamd::k_sd_sp_form, dim3(tamd::grid_for(nm, tamd::kSdBlock)), dim3(tamd::kSdBlock), 0,
                                    s, det->d_sfs, ev->d_pos, ev->d_meas_sf, m0, nm, flag.as<uint32_t>(),
                                    off.as<uint32_t>(), xyz.as<float>(), midx.as<uint32_t>());
                 hip_check(hipGetLastError(), "spacepoints");
-                if (global) hip_check(hipMemcpy(global, xyz.p, 12u * size_t(total), hipMemcpyDeviceToHost), "download");
-                if (measurement_index) {
-                    hip_check(hipMemcpy(measurement_index, midx.p, 4u * size_t(total), hipMemcpyDeviceToHost),
-                              "download");
-                }
+                tamd::readback rb;
+                rb.bytes(global, xyz.p, 12u * size_t(total));
+                rb.bytes(measurement_index, midx.p, 4u * size_t(total));
+                rb.run();
             }
         } catch (...) {
-            (void)hipFree(d_total);
-            for (tamd::dbuf* b : {&flag, &off, &sums, &xyz, &midx}) b->release();
+            (void)hipStreamSynchronize(s);  // the blocks may be handed out again
             throw;
         }
-        (void)hipFree(d_total);
-        for (tamd::dbuf* b : {&flag, &off, &sums, &xyz, &midx}) b->release();
     });
 }
 
@@ -1307,53 +1302,59 @@ ckf_status ckf_estimate_track_params(const ckf_track_params_estimation_config* c
             !meas->local_position || !meas->surface_link) {
             throw ckf_error(CKF_ERR_INVALID_ARGUMENT, "null seed, spacepoint or measurement arrays");
         }
-        // the bottom spacepoint's measurement: local position and surface (host gather)
-        std::vector<float> bl(2u * size_t(n));
+        // One pinned block holds what the kernel needs: the seeds' indices, the
+        // bottom spacepoint's local position (gathered here, with its surface)
+        // and the spacepoints.  A copy from the caller's own arrays would cost
+        // 10 to 100 us each, for the same reasons as on the way back.
+        const size_t np = sp->size, in_bytes = 20u * size_t(n) + 12u * np;
+        const tamd::pinned_block h_in(in_bytes);
+        uint32_t* const hi = static_cast<uint32_t*>(h_in.p);
+        float* const hb = reinterpret_cast<float*>(hi + 3u * size_t(n));
         for (uint32_t i = 0; i < n; ++i) {
             const uint32_t b = seeds->bottom[i];
-            if (seeds->bottom[i] >= sp->size || seeds->middle[i] >= sp->size || seeds->top[i] >= sp->size) {
+            if (b >= np || seeds->middle[i] >= np || seeds->top[i] >= np) {
                 throw ckf_error(CKF_ERR_INVALID_ARGUMENT, "seed spacepoint index out of range");
             }
             const uint32_t m = sp->measurement_index_1[b];
             if (m >= meas->size) throw ckf_error(CKF_ERR_INVALID_ARGUMENT, "spacepoint measurement index out of range");
-            bl[2 * i] = meas->local_position[2 * m];
-            bl[2 * i + 1] = meas->local_position[2 * m + 1];
+            hb[2u * size_t(i)] = meas->local_position[2u * size_t(m)];
+            hb[2u * size_t(i) + 1u] = meas->local_position[2u * size_t(m) + 1u];
             if (surface_link) surface_link[i] = meas->surface_link[m];
         }
-        tamd::dbuf d_xyz, d_idx, d_bl, d_vec, d_cov;
-        d_xyz.ensure(12u * size_t(sp->size));
-        d_idx.ensure(12u * size_t(n));
-        d_bl.ensure(8u * size_t(n));
-        d_vec.ensure(24u * size_t(n));
-        d_cov.ensure(144u * size_t(n));
+        std::memcpy(hi, seeds->bottom, 4u * size_t(n));
+        std::memcpy(hi + n, seeds->middle, 4u * size_t(n));
+        std::memcpy(hi + 2u * size_t(n), seeds->top, 4u * size_t(n));
+        std::memcpy(hb + 2u * size_t(n), sp->global, 12u * np);
+        tamd::rbuf d_in, d_vec, d_cov;
+        d_in.take(in_bytes);
+        d_vec.take(24u * size_t(n));
+        d_cov.take(144u * size_t(n));
         try {
-            hip_check(hipMemcpy(d_xyz.p, sp->global, 12u * size_t(sp->size), hipMemcpyHostToDevice), "upload");
-            uint32_t* di = d_idx.as<uint32_t>();
-            hip_check(hipMemcpy(di, seeds->bottom, 4u * size_t(n), hipMemcpyHostToDevice), "upload");
-            hip_check(hipMemcpy(di + n, seeds->middle, 4u * size_t(n), hipMemcpyHostToDevice), "upload");
-            hip_check(hipMemcpy(di + 2u * n, seeds->top, 4u * size_t(n), hipMemcpyHostToDevice), "upload");
-            hip_check(hipMemcpy(d_bl.p, bl.data(), 8u * size_t(n), hipMemcpyHostToDevice), "upload");
+            hip_check(hipMemcpyAsync(d_in.p, h_in.p, in_bytes, hipMemcpyHostToDevice, nullptr), "upload");
+            const uint32_t* di = d_in.as<uint32_t>();
             tamd::tp_params P{};
             P.cfg = *cfg;
             for (int k = 0; k < 3; ++k) P.b[k] = bfield[k];
             P.n = n;
-            P.xyz = d_xyz.as<float>();
             P.sb = di;
             P.sm = di + n;
-            P.st = di + 2u * n;
-            P.bottom_local = d_bl.as<float>();
+            P.st = di + 2u * size_t(n);
+            P.bottom_local = d_in.as<float>() + 3u * size_t(n);
+            P.xyz = P.bottom_local + 2u * size_t(n);
             P.vec = d_vec.as<float>();
             P.cov = d_cov.as<float>();
             hipLaunchKernelGGL(tamd::k_track_params, dim3(tamd::grid_for(n, tamd::kSdBlock)), dim3(tamd::kSdBlock), 0,
                                nullptr, P);
             hip_check(hipGetLastError(), "track parameters");
-            if (vector) hip_check(hipMemcpy(vector, d_vec.p, 24u * size_t(n), hipMemcpyDeviceToHost), "download");
-            if (covariance) hip_check(hipMemcpy(covariance, d_cov.p, 144u * size_t(n), hipMemcpyDeviceToHost), "download");
+            tamd::readback rb;
+            rb.bytes(vector, d_vec.p, 24u * size_t(n));
+            rb.bytes(covariance, d_cov.p, 144u * size_t(n));
+            rb.run();
+            hip_check(hipStreamSynchronize(nullptr), "track parameters");
         } catch (...) {
-            for (tamd::dbuf* b : {&d_xyz, &d_idx, &d_bl, &d_vec, &d_cov}) b->release();
+            (void)hipStreamSynchronize(nullptr);  // the blocks may be handed out again
             throw;
         }
-        for (tamd::dbuf* b : {&d_xyz, &d_idx, &d_bl, &d_vec, &d_cov}) b->release();
     });
 }
 
