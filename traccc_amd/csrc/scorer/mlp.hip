@@ -5,10 +5,10 @@
 // pass as in mlp_device.hpp; the backward pass forms
 //   dW3 = H2^T dS,  dZ2 = dS W3^T * GELU'(Z2),  dW2 = H1^T dZ2,
 //   dZ1 = (dZ2 W2^T) * GELU'(Z1),  dW1 = X^T dZ1
-// with dZ2 / dZ1 rounded to BF16 as MFMA operands.  Every wave writes its
-// tile's full gradient to its own slot; the step kernel sums the slots in a
+// with dZ2 / dZ1 rounded to BF16 as MFMA operands.  Every block writes the
+// gradient of its rows to its own slot; the step kernel sums the slots in a
 // fixed order (16 waves per 64 parameters, each over a fixed stride of
-// tiles, combined in wave order), so training is bitwise reproducible, and
+// slots, combined in wave order), so training is bitwise reproducible, and
 // applies AdamW and writes the BF16 views of its parameters in the same
 // pass.  The batch index, the Adam step count and the epoch's permutation
 // live on the device, so a run of steps is one captured graph replayed.
@@ -32,16 +32,18 @@ namespace tamd {
 namespace {
 
 constexpr int kWavesPerBlock = 4;
-// LDS per wave of the gradient kernel: the forward pass's X and H1 tiles,
-// then H1^T [64][kHStride], X^T [16][kHStride] and the tile's 64 labels (FP32)
-constexpr int kGradLdsPerWave = kMlpLdsPerWave + 64 * kHStride + 16 * kHStride + 128;
 constexpr int kBlock = 64 * kWavesPerBlock;
 
 // Pseudo-random bijection of [0, n): i -> (a i + b) mod n, gcd(a, n) = 1.
+// inv = floor(2^64 / n) (at most 2^64 - 1): the quotient from it is exact or one
+// too small for every 64-bit dividend, and a 64-bit division, 120 instructions
+// of which a third at a quarter of the rate, stays out of each row's chain.
 struct perm_map {
-    uint64_t a, b, n;
+    uint64_t a, b, n, inv;
     __device__ uint32_t operator()(uint64_t i) const {
-        return static_cast<uint32_t>((a * i + b) % n);
+        const uint64_t x = a * i + b;
+        const uint64_t r = x - __umul64hi(x, inv) * n;
+        return static_cast<uint32_t>(r >= n ? r - n : r);
     }
 };
 
@@ -108,191 +110,318 @@ __global__ __launch_bounds__(kBlock) void k_mlp_infer(mlp_dev W, const float* fe
     }
 }
 
-// Gradient of one 64-sample tile per wave into grad_part[tile][kMlpParams],
-// for the batch the training state names.
-__global__ __launch_bounds__(kBlock) void k_mlp_grad(mlp_dev W, const float* feats,
-                                                      const uint8_t* labels,
-                                                      const train_state* state, uint32_t n,
-                                                      uint32_t batch, float pos_weight,
-                                                      float* grad_part, float* loss_part) {
-    __shared__ short lds[kWavesPerBlock * kGradLdsPerWave];
+// The gradient kernel's rows per block and iteration: 16 per wave.  With 16
+// waves a block's partial gradient covers 256 rows, so the step kernel reads a
+// quarter of the bytes, and a batch of 65,536 rows is one block on every CU with
+// four waves on every SIMD; below kWideRows that leaves CUs idle and blocks of
+// four waves are used.  An optimiser step with 16 / 4 waves: 19.5 / 16.1 us at
+// 8,192 rows, 20.0 / 18.3 at 16,384, 20.6 / 22.3 at 24,576, 24.6 / 30.0 at 65,536.
+constexpr uint32_t kWideRows = 20480u;
+constexpr uint32_t kWideParts = 256u;    // blocks at most: one per CU, then they loop
+constexpr uint32_t kNarrowParts = 320u;  // 20,480 rows
+constexpr uint32_t kMaxParts = kNarrowParts > kWideParts ? kNarrowParts : kWideParts;
+
+// How a batch of `batch` rows is split into partial gradients.
+struct grad_split {
+    uint32_t wide, part_rows, max_parts;
+};
+__host__ inline grad_split split_batch(uint32_t batch) {
+    grad_split g;
+    g.wide = batch >= kWideRows ? 1u : 0u;
+    g.part_rows = g.wide ? 256u : 64u;
+    const uint32_t tiles = (batch + g.part_rows - 1u) / g.part_rows;
+    g.max_parts = std::min(tiles, g.wide ? kWideParts : kNarrowParts);
+    return g;
+}
+
+// Keeps a value computed here: the compiler otherwise moves sums and
+// activations to their last use and holds all their operands until then (twice
+// the registers, which 16 waves of a block don't have).
+__device__ inline void pin(float& v) { __asm__ volatile("" : "+v"(v)); }
+template <int kN>
+__device__ inline void pin(float (&v)[kN]) {
+#pragma unroll
+    for (int k = 0; k < kN; ++k) pin(v[k]);
+}
+
+// Lane exchange within rows of 16 lanes, by mirror images: of the row (15 - i),
+// of its halves, of its quarters, and of its pairs.
+template <int kCtrl>
+__device__ inline float mirrored(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), kCtrl, 0xf, 0xf, true));
+}
+constexpr int kMirrorRow = 0x140, kMirrorHalf = 0x141, kMirrorQuad = 0x1b, kMirrorPair = 0xb1;
+
+// One exchange of the sum below: half of the values stay, the mirror lane's
+// other half is added.
+template <int kCtrl, int kN>
+__device__ inline void fold16(float (&v)[16], bool upper) {
+#pragma unroll
+    for (int k = 0; k < kN; ++k) {
+        const float keep = upper ? v[k + kN] : v[k], give = upper ? v[k] : v[k + kN];
+        v[k] = keep + mirrored<kCtrl>(give);
+    }
+}
+
+// Sixteen values per lane, summed over the 16 lanes of a row: lane r of the row
+// gets the sum of v[r] (45 instructions; a full sum of each value takes 64).
+__device__ inline float row_sums(float (&v)[16], uint32_t r16) {
+    fold16<kMirrorRow, 8>(v, (r16 & 8u) != 0u);
+    fold16<kMirrorHalf, 4>(v, (r16 & 4u) != 0u);
+    fold16<kMirrorQuad, 2>(v, (r16 & 2u) != 0u);
+    fold16<kMirrorPair, 1>(v, (r16 & 1u) != 0u);
+    return v[0];
+}
+
+// Gradient of the batch the training state names: block b takes the row tiles
+// b, b + gridDim.x, ... of 16 kW rows and writes their sum to grad_part[b].
+//
+// Each wave takes 16 rows through the forward and backward pass on its own, all
+// transposed: Z1^T = W1^T X^T, Z2^T = W2^T H1^T, dH1^T = W2 dZ2^T.  A D fragment
+// (lane: one row, four units) is then the next product's B operand as it stands,
+// and a lane has one row's logit.  The activations, dZ2 and dZ1 go to the block's
+// LDS, and after one barrier each wave forms its own 16 x 16 tiles of dW2 and dW1
+// over all rows of the block, in accumulators that live for the whole kernel: no
+// sum over waves, no gradient in memory before the end.
+//
+// What bounds it: the chain of one tile (state, permutation, row, weights, two
+// layers and back) and the GELUs on the vector units (128 per row, each with one
+// exponential and one reciprocal, evaluated once with their derivatives).  With
+// a 64-row tile and its whole gradient per wave, one wave per SIMD, two
+// evaluations of each GELU and 20 KB written per 64 rows, a batch of 65,536 rows
+// took 35.8 us and the step kernel's sum over 1,024 partials 10.5; now 19.4 and 4.7
+// (8,192 rows: 31.0 and 7.2, now 11.4 and 4.6).
+template <int kW>
+__global__ __launch_bounds__(64 * kW) void k_mlp_grad(mlp_dev W, const float* feats, const uint8_t* labels,
+                                                      const train_state* state, uint32_t n, uint32_t batch,
+                                                      float pos_weight, float* grad_part, float* loss_part) {
+    constexpr uint32_t kRows = 16u * kW;
+    // an operand row (one hidden unit or feature, all rows of the block): 16
+    // bytes of padding spread a fragment's 16 operand rows over the banks
+    constexpr uint32_t kRs = kRows + 8u;
+    constexpr int kTiles = 16 / kW;  // of dW2, per wave
+    __shared__ mlp_vecs s_v;
+    __shared__ bf16x4 s_w[36][64];   // fragments of W1^T (4), W2^T (16), W2 (16)
+    __shared__ __align__(16) short s_ht[kMlpHidden * kRs];   // H1^T
+    __shared__ __align__(16) short s_z2[kMlpHidden * kRs];   // dZ2^T
+    __shared__ __align__(16) short s_z1[kMlpHidden * kRs];   // dZ1^T
+    __shared__ __align__(16) short s_xt[kMlpInPad * kRs];    // X^T
     const train_state ts = *state;
-    const perm_map perm = ts.perm;
     const uint32_t row0 = ts.batch_idx * batch;
     const uint32_t rows = batch_rows(ts, n, batch);
-    const float inv_norm = rows > 0u ? 1.f / static_cast<float>(rows) : 0.f;
+    const uint32_t n_tiles = (rows + kRows - 1u) / kRows;
+    if (blockIdx.x >= n_tiles) {
+        return;  // whole blocks; the step kernel counts the same partials
+    }
+    const float inv_norm = 1.f / static_cast<float>(rows);
     const uint32_t wave = threadIdx.x / 64u;
-    short* lds_x = lds + wave * kGradLdsPerWave;
-    short* lds_h = lds_x + 64 * kMlpInPad;
-    short* lds_ht = lds_h + 64 * kHStride;
-    short* lds_xt = lds_ht + 64 * kHStride;
-    float* lds_y = reinterpret_cast<float*>(lds_xt + 16 * kHStride);
-    const uint32_t tile = blockIdx.x * kWavesPerBlock + wave;
     const uint32_t l = __lane_id();
     const uint32_t r16 = l % 16u;
     const uint32_t g4 = 4u * (l / 16u);
-    if (tile * 64u >= rows) {
-        return;  // whole waves only: no wave-level operation is left half-done
-    }
-    float* gp = grad_part + static_cast<size_t>(tile) * kMlpParams;
+    const uint32_t own = 16u * wave + r16;  // the lane's row in the block's tile
+    const bool pieces = (reinterpret_cast<uintptr_t>(feats) & 15u) == 0u;  // rows are 48 B
 
-    const uint32_t i = tile * 64u + l;
-    const bool valid = i < rows;
-    // the lane's row: its features, and its label into the wave's LDS for
-    // the lanes that hold the row's logit below (the permutation is
-    // evaluated once per row)
-    float f[kMlpIn];
-    {
-        const uint32_t row = valid ? perm(row0 + i) : 0u;
+    // lane: features g4 .. g4 + 3 of its row (the B fragment), and the label
+    auto load_row = [&](uint32_t tile, float (&x)[4]) {
+        const uint32_t i = tile * kRows + own;
+        const bool valid = i < rows;
+        const size_t row = valid ? ts.perm(row0 + i) : 0u;
 #pragma unroll
-        for (int k = 0; k < kMlpIn; ++k) f[k] = valid ? feats[static_cast<size_t>(row) * kMlpIn + k] : 0.f;
-        lds_y[l] = (valid && labels[row]) ? 1.f : 0.f;
+        for (int e = 0; e < 4; ++e) x[e] = 0.f;
+        if (valid && g4 < static_cast<uint32_t>(kMlpIn)) {
+            const float* f = feats + row * kMlpIn + g4;
+            if (pieces) {
+                const float4 v = *reinterpret_cast<const float4*>(f);
+                x[0] = v.x, x[1] = v.y, x[2] = v.z, x[3] = v.w;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[e] = f[e];
+            }
+        }
+        return (valid && labels[row]) ? 1.f : 0.f;
+    };
+    float x[4];
+    float y = load_row(blockIdx.x, x);
+    for (uint32_t i = threadIdx.x; i < 36u * 64u; i += 64u * kW) {
+        const uint32_t k = i / 64u, fl = i % 64u, fr = fl % 16u, fg = 4u * (fl / 16u);
+        const uint32_t nt = (k - 4u) / 4u % 4u, kt = k % 4u;
+        s_w[k][fl] = k < 4u ? load4(W.w1t + (16u * k + fr) * kMlpInPad + fg)
+                            : load4((k < 20u ? W.w2t : W.w2) + (16u * nt + fr) * kMlpHidden + 16u * kt + fg);
     }
-    float z1[4][4][4], z2[4][4][4], s[4][4];
-    mlp_tile_layers(W, f, valid, lds_x, lds_h, z1, z2, lds_xt, lds_ht);
-    mlp_tile_output(W, z2, s);
+    mlp_fill_vecs(W, s_v, threadIdx.x, 64u * kW);
 
-    // loss and dL/ds for the rows this lane holds
-    float ds[4][4];
-    float loss = 0.f;
+    f32x4 dw2[kTiles], dw1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt) {
+    for (int j = 0; j < kTiles; ++j) dw2[j] = {0.f, 0.f, 0.f, 0.f};
+    // of unit 16 (r16 / 4) + g4 + r16 % 4 (row_sums)
+    float db1 = 0.f, db2 = 0.f, dw3 = 0.f;
+    float db3 = 0.f, loss = 0.f;
+
+    for (uint32_t tile = blockIdx.x;;) {
+        // the weights are there; the last tile's operands are done with
+        __syncthreads();
+        const bool valid = tile * kRows + own < rows;
+        bf16x4 xb;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const uint32_t pos = tile * 64u + 16u * mt + g4 + e;
-            const float y = lds_y[16u * mt + g4 + e];
-            ds[mt][e] = 0.f;
-            if (pos < rows) {
-                const float w = (y > 0.5f ? pos_weight : 1.f) * inv_norm;
-                const float x = s[mt][e];
-                const float sig = 1.f / (1.f + expf(-x));
-                ds[mt][e] = w * (sig - y);
-                if (r16 == 0u) {
-                    loss += w * (fmaxf(x, 0.f) - x * y + log1pf(expf(-fabsf(x))));
-                }
-            }
+            const bool real = valid && g4 + e < static_cast<uint32_t>(kMlpIn);
+            xb[e] = f2bf(real ? (x[e] - s_v.mean[g4 + e]) * s_v.inv_std[g4 + e] : 0.f);
+            s_xt[(g4 + e) * kRs + own] = xb[e];
         }
-    }
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) loss += __shfl_xor(loss, d, 64);
-    if (l == 0u) loss_part[tile] = loss;
-
-    float w3[4];
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) w3[nt] = W.w3[16 * nt + r16];
-    // db3 = sum_r dS[r]
-    {
-        float db3 = 0.f;
-#pragma unroll
-        for (int mt = 0; mt < 4; ++mt) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) db3 += ds[mt][e];
-        }
-        db3 = (r16 == 0u) ? db3 : 0.f;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) db3 += __shfl_xor(db3, d, 64);
-        if (l == 0u) gp[kOffB3] = db3;
-    }
-    // dW3[c] = sum_r H2[r][c] dS[r]; dZ2 = dS W3^T * GELU'(Z2) (in place of
-    // z2) and db2, from one GELU evaluation per entry
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-        float accw = 0.f, accb = 0.f;
-#pragma unroll
-        for (int mt = 0; mt < 4; ++mt) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                float h, gg;
-                gelu_and_grad(z2[mt][nt][e], h, gg);
-                accw += h * ds[mt][e];
-                z2[mt][nt][e] = ds[mt][e] * w3[nt] * gg;
-                accb += z2[mt][nt][e];
-            }
-        }
-        accw += __shfl_xor(accw, 16, 64);
-        accw += __shfl_xor(accw, 32, 64);
-        accb += __shfl_xor(accb, 16, 64);
-        accb += __shfl_xor(accb, 32, 64);
-        if (l < 16u) {
-            gp[kOffW3 + 16 * nt + r16] = accw;
-            gp[kOffB2 + 16 * nt + r16] = accb;
-        }
-    }
-    // dW2 = H1^T dZ2: A = H1^T (the transposed tile in LDS), B = dZ2 in D layout
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-        bf16x4 b[4];
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) b[kt][e] = f2bf(z2[kt][nt][e]);
-        }
-#pragma unroll
-        for (int mi = 0; mi < 4; ++mi) {
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int kt = 0; kt < 4; ++kt) {
-                const bf16x4 a = load4(lds_ht + (16 * mi + r16) * kHStride + 16 * kt + g4);
-                acc = mfma16(a, b[kt], acc);
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) gp[kOffW2 + (16 * mi + g4 + e) * kMlpHidden + 16 * nt + r16] = acc[e];
-        }
-    }
-    // dZ2 -> LDS (A layout for dH1), replacing H1
-    wave_lds_sync();
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt) {
+        // layer 1: H1^T = GELU(W1^T X^T + b1), with the derivatives
+        bf16x4 h[4];
+        float g1[16];
 #pragma unroll
         for (int nt = 0; nt < 4; ++nt) {
+            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+            acc = mfma16(s_w[nt][l], xb, acc);
+            const f32x4 b = *reinterpret_cast<const f32x4*>(&s_v.b1[16 * nt + g4]);
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                lds_h[(16 * mt + g4 + e) * kHStride + 16 * nt + r16] = f2bf(z2[mt][nt][e]);
+                float a;
+                gelu_and_grad(acc[e] + b[e], a, g1[4 * nt + e]);
+                pin(g1[4 * nt + e]);
+                h[nt][e] = f2bf(a);
+                s_ht[(16 * nt + g4 + e) * kRs + own] = h[nt][e];
             }
         }
-    }
-    wave_lds_sync();
-    // dH1 = dZ2 W2^T, dZ1 = dH1 * GELU'(Z1) (in place of z1), db1
+        // layer 2 the same way, and the logit
+        float h2[16], g2[16], s = 0.f;
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-        bf16x4 b[4];
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt) b[kt] = load4(W.w2 + (16 * nt + r16) * kMlpHidden + 16 * kt + g4);
-        float accb = 0.f;
-#pragma unroll
-        for (int mt = 0; mt < 4; ++mt) {
+        for (int nt = 0; nt < 4; ++nt) {
             f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int kt = 0; kt < 4; ++kt) {
-                const bf16x4 a = load4(lds_h + (16 * mt + r16) * kHStride + 16 * kt + g4);
-                acc = mfma16(a, b[kt], acc);
-            }
+            for (int kt = 0; kt < 4; ++kt) acc = mfma16(s_w[4 + 4 * nt + kt][l], h[kt], acc);
+            const f32x4 b = *reinterpret_cast<const f32x4*>(&s_v.b2[16 * nt + g4]);
+            const f32x4 w = *reinterpret_cast<const f32x4*>(&s_v.w3[16 * nt + g4]);
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                z1[mt][nt][e] = acc[e] * gelu_grad(z1[mt][nt][e]);
-                accb += z1[mt][nt][e];
+                const int k = 4 * nt + e;
+                gelu_and_grad(acc[e] + b[e], h2[k], g2[k]);
+                s += h2[k] * w[e];
+                pin(h2[k]);
+                pin(g2[k]);
+            }
+            pin(s);
+        }
+        s += __shfl_xor(s, 16, 64);
+        s += __shfl_xor(s, 32, 64);
+        s += s_v.b3;
+        // loss and dL/ds; the row's four lanes hold the same
+        const float wt = valid ? (y > 0.5f ? pos_weight : 1.f) * inv_norm : 0.f;
+        const float ds = wt * (1.f / (1.f + expf(-s)) - y);
+        loss += valid ? wt * (fmaxf(s, 0.f) - s * y + log1pf(expf(-fabsf(s)))) : 0.f;
+        db3 += ds;
+        // dW3, dZ2 = dS W3^T * GELU'(Z2), db2
+#pragma unroll
+        for (int k = 0; k < 16; ++k) h2[k] *= ds;
+        dw3 += row_sums(h2, r16);
+        pin(dw3);
+        bf16x4 z[4];
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt) {
+            const f32x4 w = *reinterpret_cast<const f32x4*>(&s_v.w3[16 * nt + g4]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int k = 4 * nt + e;
+                g2[k] = ds * w[e] * g2[k];
+                z[nt][e] = f2bf(g2[k]);
+                s_z2[(16 * nt + g4 + e) * kRs + own] = z[nt][e];
             }
         }
-        accb += __shfl_xor(accb, 16, 64);
-        accb += __shfl_xor(accb, 32, 64);
-        if (l < 16u) gp[kOffB1 + 16 * nt + r16] = accb;
-    }
-    // dW1 = X^T dZ1: A = X^T (the transposed tile in LDS), B = dZ1 in D layout
+        db2 += row_sums(g2, r16);
+        pin(db2);
+        // dZ1 = (dZ2 W2^T) * GELU'(Z1), db1
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        for (int nt = 0; nt < 4; ++nt) {
+            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int kt = 0; kt < 4; ++kt) {
-            const bf16x4 a = load4(lds_xt + r16 * kHStride + 16 * kt + g4);
-            bf16x4 b;
+            for (int kt = 0; kt < 4; ++kt) acc = mfma16(s_w[20 + 4 * nt + kt][l], z[kt], acc);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) b[e] = f2bf(z1[kt][nt][e]);
-            acc = mfma16(a, b, acc);
+            for (int e = 0; e < 4; ++e) {
+                const int k = 4 * nt + e;
+                g1[k] = acc[e] * g1[k];
+                s_z1[(16 * nt + g4 + e) * kRs + own] = f2bf(g1[k]);
+            }
         }
+        db1 += row_sums(g1, r16);
+        pin(db1);
+        const uint32_t next = tile + gridDim.x;
+        if (next < n_tiles) y = load_row(next, x);
+        __syncthreads();
+        // dW2 += H1^T dZ2 (tiles 4 nt + mi) and dW1 += X^T dZ1 (one per wave of
+        // the first four) over the block's rows
+        const uint32_t t0 = wave * kTiles, nt = t0 / 4u;
+#pragma unroll 4
+        for (uint32_t kt = 0; kt < static_cast<uint32_t>(kW); ++kt) {
+            const bf16x4 b = load4(s_z2 + (16u * nt + r16) * kRs + 16u * kt + g4);
+#pragma unroll
+            for (int j = 0; j < kTiles; ++j) {
+                const bf16x4 a = load4(s_ht + (16u * ((t0 + j) % 4u) + r16) * kRs + 16u * kt + g4);
+                dw2[j] = mfma16(a, b, dw2[j]);
+            }
+        }
+        if (wave < 4u) {
+#pragma unroll 4
+            for (uint32_t kt = 0; kt < static_cast<uint32_t>(kW); ++kt) {
+                dw1 = mfma16(load4(s_xt + r16 * kRs + 16u * kt + g4),
+                             load4(s_z1 + (16u * wave + r16) * kRs + 16u * kt + g4), dw1);
+            }
+        }
+        if (next >= n_tiles) {
+            break;
+        }
+        tile = next;
+    }
+
+    float* gp = grad_part + static_cast<size_t>(blockIdx.x) * kMlpParams;
+#pragma unroll
+    for (int j = 0; j < kTiles; ++j) {
+        const uint32_t t = wave * kTiles + j, nt = t / 4u, mi = t % 4u;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) gp[kOffW2 + (16u * mi + g4 + e) * kMlpHidden + 16u * nt + r16] = dw2[j][e];
+    }
+    if (wave < 4u) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const uint32_t fi = g4 + e;
-            if (fi < static_cast<uint32_t>(kMlpIn)) gp[kOffW1 + fi * kMlpHidden + 16 * nt + r16] = acc[e];
+            if (g4 + e < static_cast<uint32_t>(kMlpIn)) gp[kOffW1 + (g4 + e) * kMlpHidden + 16u * wave + r16] = dw1[e];
+        }
+    }
+    // the vectors' gradients over the waves in order; the last tile's operands
+    // are done with
+    __syncthreads();
+    float* s_sum = reinterpret_cast<float*>(s_ht);  // [kW][3 * 64 + 2]
+    constexpr uint32_t kSums = 3u * kMlpHidden + 2u;
+    static_assert(sizeof(float) * kW * kSums <= sizeof(s_ht), "the sums fit over the operand");
+#pragma unroll
+    for (int d = 1; d < 16; d <<= 1) {
+        loss += __shfl_xor(loss, d, 64);
+        db3 += __shfl_xor(db3, d, 64);
+    }
+    const uint32_t unit = 16u * (r16 / 4u) + g4 + r16 % 4u;
+    s_sum[wave * kSums + unit] = db1;
+    s_sum[wave * kSums + kMlpHidden + unit] = db2;
+    s_sum[wave * kSums + 2 * kMlpHidden + unit] = dw3;
+    if (l == 0u) {
+        s_sum[wave * kSums + 3 * kMlpHidden] = db3;
+        s_sum[wave * kSums + 3 * kMlpHidden + 1] = loss;
+    }
+    __syncthreads();
+    for (uint32_t k = threadIdx.x; k < kSums; k += 64u * kW) {
+        float v = 0.f;
+#pragma unroll
+        for (uint32_t w = 0; w < static_cast<uint32_t>(kW); ++w) v += s_sum[w * kSums + k];
+        const uint32_t c = k % kMlpHidden;
+        if (k < 1u * kMlpHidden) {
+            gp[kOffB1 + c] = v;
+        } else if (k < 2u * kMlpHidden) {
+            gp[kOffB2 + c] = v;
+        } else if (k < 3u * kMlpHidden) {
+            gp[kOffW3 + c] = v;
+        } else if (k == 3u * kMlpHidden) {
+            gp[kOffB3] = v;
+        } else {
+            loss_part[blockIdx.x] = v;
         }
     }
 }
@@ -302,13 +431,13 @@ struct adam_hyper {
 };
 
 // One optimiser step.  Block b owns parameters 64 b .. 64 b + 63 (one per
-// lane): its 16 waves each sum a fixed stride of the batch's tile gradients
+// lane): its 16 waves each sum a fixed stride of the batch's partial gradients
 // (coalesced 256 B rows), the block combines them in wave order, then --
 // with apply != 0 -- AdamW updates the parameter and writes its BF16 / FP32
-// views (the k_mlp_pack layouts).  Block 0 also sums the tile losses into
+// views (the k_mlp_pack layouts).  Block 0 also sums the partial losses into
 // losses[batch_idx].  The last block to finish advances the training state.
 constexpr int kStepWaves = 16;
-constexpr int kStepLoads = 32;
+constexpr int kStepLoads = 16;
 
 __device__ inline void pack_param(uint32_t p, float w, short* w1t, short* w2, short* w2t,
                                   float* b1, float* b2, float* w3, float* b3) {
@@ -331,46 +460,60 @@ __device__ inline void pack_param(uint32_t p, float w, short* w1t, short* w2, sh
 }
 
 __global__ __launch_bounds__(64 * kStepWaves) void k_mlp_step(
-    const float* grad_part, const float* loss_part, uint32_t n, uint32_t batch,
+    const float* grad_part, const float* loss_part, uint32_t n, uint32_t batch, grad_split split,
     train_state* state, int apply, adam_hyper h, float* params, float* m, float* v,
     float* grad_out, float* losses, short* w1t, short* w2, short* w2t, float* b1, float* b2,
     float* w3, float* b3) {
     __shared__ float s_part[kStepWaves][64];
     const train_state ts = *state;
     const uint32_t rows = batch_rows(ts, n, batch);
-    const uint32_t tiles = (rows + 63u) / 64u;
+    const uint32_t parts = min((rows + split.part_rows - 1u) / split.part_rows, split.max_parts);
     const uint32_t wave = threadIdx.x / 64u;
     const uint32_t l = __lane_id();
     const uint32_t p = blockIdx.x * 64u + l;
     const bool real = p < static_cast<uint32_t>(kMlpParams);
-    // the wave's tiles in batches of kStepLoads loads in flight, added in
-    // tile order (the same sum as one load at a time)
+    // the parameter's state while the partials are on their way; the bias
+    // corrections by another wave than the one that needs them
+    __shared__ float s_bc[2];
+    if (apply && wave == 2u) {
+        const float t = static_cast<float>(ts.adam_t + 1u);
+        const float bc = 1.f - powf(l == 0u ? h.beta1 : h.beta2, t);
+        if (l < 2u) s_bc[l] = bc;
+    }
+    float pm = 0.f, pv = 0.f, pw = 0.f;
+    if (apply && wave == 0u && real) {
+        pm = m[p];
+        pv = v[p];
+        pw = params[p];
+    }
+    // the wave's partials in batches of kStepLoads loads in flight, added in
+    // their order (the same sum as one load at a time)
     float acc = 0.f;
-    for (uint32_t t0 = wave; t0 < tiles; t0 += kStepWaves * kStepLoads) {
+    for (uint32_t t0 = wave; t0 < parts; t0 += kStepWaves * kStepLoads) {
         float g[kStepLoads];
 #pragma unroll
         for (int k = 0; k < kStepLoads; ++k) {
             const uint32_t t = t0 + static_cast<uint32_t>(k) * kStepWaves;
-            g[k] = (real && t < tiles) ? grad_part[static_cast<size_t>(t) * kMlpParams + p] : 0.f;
+            g[k] = (real && t < parts) ? grad_part[static_cast<size_t>(t) * kMlpParams + p] : 0.f;
         }
 #pragma unroll
         for (int k = 0; k < kStepLoads; ++k) {
-            if (t0 + static_cast<uint32_t>(k) * kStepWaves < tiles) acc += g[k];
+            if (t0 + static_cast<uint32_t>(k) * kStepWaves < parts) acc += g[k];
         }
     }
     s_part[wave][l] = acc;
     if (blockIdx.x == 0u && wave == 1u) {
         float lo = 0.f;
-        for (uint32_t t0 = l; t0 < tiles; t0 += 64u * kStepLoads) {
+        for (uint32_t t0 = l; t0 < parts; t0 += 64u * kStepLoads) {
             float x[kStepLoads];
 #pragma unroll
             for (int k = 0; k < kStepLoads; ++k) {
                 const uint32_t t = t0 + 64u * static_cast<uint32_t>(k);
-                x[k] = t < tiles ? loss_part[t] : 0.f;
+                x[k] = t < parts ? loss_part[t] : 0.f;
             }
 #pragma unroll
             for (int k = 0; k < kStepLoads; ++k) {
-                if (t0 + 64u * static_cast<uint32_t>(k) < tiles) lo += x[k];
+                if (t0 + 64u * static_cast<uint32_t>(k) < parts) lo += x[k];
             }
         }
 #pragma unroll
@@ -384,24 +527,19 @@ __global__ __launch_bounds__(64 * kStepWaves) void k_mlp_step(
         for (int w = 0; w < kStepWaves; ++w) g += s_part[w][l];
         if (grad_out != nullptr) grad_out[p] = g;
         if (apply) {
-            const float t = static_cast<float>(ts.adam_t + 1u);
-            const float bc1 = 1.f - powf(h.beta1, t);
-            const float bc2 = 1.f - powf(h.beta2, t);
-            const float mm = h.beta1 * m[p] + (1.f - h.beta1) * g;
-            const float vv = h.beta2 * v[p] + (1.f - h.beta2) * g * g;
+            const float mm = h.beta1 * pm + (1.f - h.beta1) * g;
+            const float vv = h.beta2 * pv + (1.f - h.beta2) * g * g;
             m[p] = mm;
             v[p] = vv;
-            const float w = params[p] - h.lr * ((mm / bc1) / (sqrtf(vv / bc2) + h.eps) +
-                                                h.wd * params[p]);
+            const float w = pw - h.lr * ((mm / s_bc[0]) / (sqrtf(vv / s_bc[1]) + h.eps) + h.wd * pw);
             params[p] = w;
             pack_param(p, w, w1t, w2, w2t, b1, b2, w3, b3);
         }
     }
     // the last block to finish moves the state to the next batch (every
-    // block read the state at its start, before counting itself)
-    __syncthreads();
+    // block has read the state, its waves having passed the barrier above,
+    // before it counts itself; what the blocks wrote is for the next kernel)
     if (threadIdx.x == 0u) {
-        __threadfence();
         const uint32_t before = atomicAdd(&state->done_blocks, 1u);
         if (before + 1u == gridDim.x) {
             state->done_blocks = 0u;
@@ -521,12 +659,10 @@ __global__ void k_mfma_layout(const float* A, const float* B, float* D) {
 }  // namespace
 
 // Scratch of the allocation-free gradient (ckf_scorer_gradient_noalloc): the
-// per-tile partial gradients and losses of up to kNoAllocMaxSamples samples
-// (1,024 tiles x 5,057 parameters + 1,024 losses, 20.7 MB).  Every GPU the
-// library runs on holds its own copy until the process ends.
+// partial gradients and losses of a batch (320 x 5,058 words, 6.5 MB).  Every
+// GPU the library runs on holds its own copy until the process ends.
 constexpr uint32_t kNoAllocMaxSamples = CKF_SCORER_NOALLOC_MAX_SAMPLES;
-constexpr uint32_t kNoAllocTiles = kNoAllocMaxSamples / 64u;
-static __device__ __align__(256) float scratch[size_t(kNoAllocTiles) * kMlpParams + kNoAllocTiles];
+static __device__ __align__(256) float scratch[size_t(kMaxParts) * kMlpParams + kMaxParts];
 
 }  // namespace tamd
 
@@ -600,12 +736,14 @@ uint64_t splitmix(uint64_t& x) {
 }
 
 tamd::perm_map make_perm(uint64_t n, uint64_t& rng, bool identity) {
-    if (identity || n <= 1) return tamd::perm_map{1, 0, n ? n : 1};
+    if (n <= 1) return tamd::perm_map{1, 0, 1, ~uint64_t(0)};
+    const uint64_t inv = ~uint64_t(0) / n + ((n & (n - 1)) == 0 ? 1 : 0);
+    if (identity) return tamd::perm_map{1, 0, n, inv};
     uint64_t a = 0;
     do {
         a = splitmix(rng) % n;
     } while (a == 0 || gcd64(a, n) != 1);
-    return tamd::perm_map{a, splitmix(rng) % n, n};
+    return tamd::perm_map{a, splitmix(rng) % n, n, inv};
 }
 
 // Device address of `scratch` on the current device, looked up (with that
@@ -634,19 +772,23 @@ void set_state(ckf_scorer& S, const tamd::perm_map& perm, uint32_t batch_idx, hi
     hip_check(hipStreamSynchronize(st), "scorer state");
 }
 
-// One optimiser step on the batch the device state names: the tile
+// One optimiser step on the batch the device state names: the partial
 // gradients, then their fixed-order sum with (apply) the AdamW update and the
 // BF16 views; the state moves to the next batch.
 void launch_step(ckf_scorer& S, const float* feats, const uint8_t* labels, uint32_t n,
                  uint32_t batch, float pos_weight, int apply, const tamd::adam_hyper& h,
                  float* part, float* loss_part, float* losses, float* grad_out, hipStream_t st) {
-    const uint32_t tiles = (batch + 63u) / 64u;
-    const uint32_t blocks = (tiles + tamd::kWavesPerBlock - 1) / tamd::kWavesPerBlock;
-    hipLaunchKernelGGL(tamd::k_mlp_grad, dim3(blocks), dim3(tamd::kBlock), 0, st, S.view(), feats,
-                       labels, S.state, n, batch, pos_weight, part, loss_part);
+    const tamd::grad_split split = tamd::split_batch(batch);
+    if (split.wide) {
+        hipLaunchKernelGGL(tamd::k_mlp_grad<16>, dim3(split.max_parts), dim3(1024), 0, st, S.view(), feats,
+                           labels, S.state, n, batch, pos_weight, part, loss_part);
+    } else {
+        hipLaunchKernelGGL(tamd::k_mlp_grad<4>, dim3(split.max_parts), dim3(256), 0, st, S.view(), feats,
+                           labels, S.state, n, batch, pos_weight, part, loss_part);
+    }
     hip_check(hipGetLastError(), "scorer grad");
     hipLaunchKernelGGL(tamd::k_mlp_step, dim3((tamd::kMlpParams + 63) / 64),
-                       dim3(64 * tamd::kStepWaves), 0, st, part, loss_part, n, batch, S.state,
+                       dim3(64 * tamd::kStepWaves), 0, st, part, loss_part, n, batch, split, S.state,
                        apply, h, S.params, S.m, S.v, grad_out, losses, S.w1t, S.w2, S.w2t, S.b1,
                        S.b2, S.w3, S.b3);
     hip_check(hipGetLastError(), "scorer step");
@@ -811,15 +953,15 @@ ckf_status ckf_scorer_gradient(const ckf_scorer* s, const float* d_features,
     return guarded([&] {
         if (!s || !d_features || !d_labels || n == 0) throw ckf_error(CKF_ERR_INVALID_ARGUMENT, "invalid argument");
         hipStream_t st = static_cast<hipStream_t>(stream);
-        const uint32_t tiles = (n + 63u) / 64u;
+        const uint32_t parts = tamd::split_batch(n).max_parts;
         float* part = nullptr;
-        hip_check(hipMalloc(&part, (size_t(tiles) * tamd::kMlpParams + tiles) * 4), "scorer grad");
+        hip_check(hipMalloc(&part, (size_t(parts) * tamd::kMlpParams + parts) * 4), "scorer grad");
         ckf_scorer& S = const_cast<ckf_scorer&>(*s);
         try {
             uint64_t rng = 0;
             set_state(S, make_perm(n, rng, true), 0u, st);
             launch_step(S, d_features, d_labels, n, n, pos_weight, 0, tamd::adam_hyper{},
-                        part, part + size_t(tiles) * tamd::kMlpParams, S.loss, S.grad, st);
+                        part, part + size_t(parts) * tamd::kMlpParams, S.loss, S.grad, st);
             if (grad) hip_check(hipMemcpyAsync(grad, s->grad, tamd::kMlpParams * 4, hipMemcpyDeviceToHost, st), "grad");
             if (loss) hip_check(hipMemcpyAsync(loss, s->loss, 4, hipMemcpyDeviceToHost, st), "loss");
             hip_check(hipStreamSynchronize(st), "scorer grad sync");
@@ -844,14 +986,13 @@ ckf_status ckf_scorer_gradient_noalloc(const ckf_scorer* s, const float* d_featu
         }
         hipStream_t st = static_cast<hipStream_t>(stream);
         float* part = noalloc_scratch();
-        const uint32_t tiles = (n + 63u) / 64u;
         ckf_scorer& S = const_cast<ckf_scorer&>(*s);
         uint64_t rng = 0;
         hipLaunchKernelGGL(tamd::k_set_state, dim3(1), dim3(64), 0, st, S.state,
                            make_perm(n, rng, true), 0u, static_cast<uint32_t>(S.adam_t));
         hip_check(hipGetLastError(), "scorer state");
         launch_step(S, d_features, d_labels, n, n, pos_weight, 0, tamd::adam_hyper{}, part,
-                    part + size_t(tiles) * tamd::kMlpParams, d_loss, d_grad, st);
+                    part + size_t(tamd::kMaxParts) * tamd::kMlpParams, d_loss, d_grad, st);
     });
 }
 
@@ -878,16 +1019,16 @@ ckf_status ckf_scorer_train(ckf_scorer* s, const float* d_features, const uint8_
             }
         } own_guard{own};
         const uint32_t batch = std::min(cfg->batch, ((n + 63u) / 64u) * 64u);
-        const uint32_t tiles = (batch + 63u) / 64u;
+        const uint32_t parts = tamd::split_batch(batch).max_parts;
         const uint32_t n_batches = (n + batch - 1) / batch;
         // steps per captured graph: the step kernels read their batch from
         // the device state, so one capture serves every replay
         constexpr uint32_t kGraphSteps = 32;
         float* part = nullptr;
-        hip_check(hipMalloc(&part, (size_t(tiles) * tamd::kMlpParams + tiles + n_batches) * 4),
+        hip_check(hipMalloc(&part, (size_t(parts) * tamd::kMlpParams + parts + n_batches) * 4),
                   "scorer train");
-        float* loss_part = part + size_t(tiles) * tamd::kMlpParams;
-        float* losses = loss_part + tiles;
+        float* loss_part = part + size_t(parts) * tamd::kMlpParams;
+        float* losses = loss_part + parts;
         hipEvent_t e0 = nullptr, e1 = nullptr;
         hipGraphExec_t graph = nullptr;
         try {
