@@ -93,7 +93,7 @@ ckf_status ckf_scorer_train(ckf_scorer* s, const float* d_features, const uint8_
  * reference; for callers that cannot allocate (code under HIP graph
  * capture, training loops that forbid hipMalloc).  Same gradient and loss,
  * bit for bit, into caller DEVICE memory: d_grad [ckf_scorer_n_params()]
- * floats, d_loss [1] float.  The per-tile partial gradients go to a fixed
+ * floats, d_loss [1] float.  The batch's partial gradients go to a fixed
  * device array of the library (6.5 MB per GPU, held until the process
  * ends), so n is limited to CKF_SCORER_NOALLOC_MAX_SAMPLES
  * (CKF_ERR_INVALID_ARGUMENT above it).  Ordered on the stream, no host

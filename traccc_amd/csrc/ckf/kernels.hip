@@ -1,15 +1,15 @@
 // CKF step kernels for CDNA (gfx950).
 //
 // Per step (counts live in the device step control block):
-//   k_find        one lane per input branch: chi2 over the surface's
+//   k_find        two lanes per input branch: chi2 over the surface's
 //                 measurements, best-N selection by (chi2, measurement index),
 //                 gain-matrix update, hole links; links are compacted in input
 //                 order with a wave scan + decoupled look-back
 //                 (traccc host: details/combinatorial_kalman_filter.hpp:174-364)
-//   k_dedup_mark  duplicate removal grouped by last measurement (the groups'
+//   k_dedup_mark  duplicate removal grouped by latest measurements (the groups'
 //                 lists are made where the links are, in k_find_emit)
 //                 (traccc host :371-488)
-//   k_propagate   one lane per link: per-seed cap, hole limits, RK4 transport
+//   k_propagate   one lane or a team per link: per-seed cap, hole limits, RK4 transport
 //                 to the next sensitive surface, tips; next-step inputs and
 //                 tips compacted with ballots + look-back (traccc host :493-627)
 //   k_advance     one lane: advances the control block
