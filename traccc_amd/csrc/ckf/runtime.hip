@@ -156,9 +156,8 @@ void ensure_buffers(ckf_algorithm& A, const ckf_device_event& ev) {
     const uint32_t N = A.cfg.max_num_branches_per_surface;
     A.flt_cap = static_cast<uint32_t>(std::min<uint64_t>(uint64_t(A.in_cap) * N, 0x3fffffffu));
     A.state_cap = A.flt_cap;
-    // look-back partitions: k_find_emit takes 64 inputs per wave,
-    // k_propagate 64 / team links per wave (teams of up to 16 lanes), the
-    // other kernels 64 items per wave (the 16-input bound is kept as slack)
+    // look-back words: the compactions' partitions hold 256 items or more, so
+    // these bounds leave ample slack
     A.lb_cap = std::max({(A.in_cap + 15u) / 16u, (A.state_cap + 3u) / 4u, parts(A.tip_cap)}) + 1u;
     const size_t st = size_t(tamd::kStateCols) * 4u;
     A.state[0].ensure(st * A.state_cap);
