@@ -13,11 +13,11 @@
 
 #include "../core/propagator.hpp"
 #include "../scorer/mlp_view.hpp"
+#include "step_ctl.hpp"
 
 namespace tamd {
 
 constexpr int kStateCols = 28;  // 6 + 21 + 1
-constexpr int kTickets = 9;     // work queues of the control block
 constexpr int kLookbacks = 4;   // compactions with their own look-back words:
                                 // find emit, dedup, propagate emit, build
 constexpr uint32_t kInvalid = 0xffffffffu;
@@ -84,22 +84,6 @@ TAMD_HD uint32_t pack_link(uint32_t step, uint32_t skipped, uint32_t consec) {
            ((consec > 255u ? 255u : consec) << 24);
 }
 
-// A counter alone on its 128-byte cache line.  The work-queue counters take
-// an atomic per partition from every wave of a grid; counters sharing a line
-// (with each other, or with the fields every wave reads at kernel start) are
-// served one after another by that line's L2 channel.
-struct alignas(128) line_u32 {
-    uint32_t v;
-};
-struct alignas(128) line_u64 {
-    uint64_t v;
-};
-static_assert(sizeof(line_u32) == 128 && sizeof(line_u64) == 128, "one counter per line");
-
-// Step control block in device memory; the step loop reads and advances it
-// without host round trips.  The fields every wave reads at kernel start
-// share the first line; each counter that waves hammer with atomics has its
-// own.
 // A deferred propagation: link, visited layers (2 words), RK steps, path,
 // the free state (11 words), the transport Jacobian (31 words), state ref.
 constexpr uint32_t kDeferWords = 48u;
@@ -109,34 +93,6 @@ constexpr uint32_t kDeferWords = 48u;
 // + 72 deferred; 285,989 268 and 229 + 74; 323,274 285 and 245 + 79 (the 40 us
 // grow with the links, the 80 do not).
 constexpr uint32_t kDeferLinks = 700000u;
-
-struct step_ctl {
-    uint32_t step;        // current CKF step
-    uint32_t epoch;       // tag of this step's look-back descriptors
-    uint32_t n_in;        // inputs of this step
-    uint32_t link_base;   // global index of this step's first link
-    uint32_t n_links;     // links made this step (written by find)
-    uint32_t n_live;      // inputs of the next step (written by propagate)
-    uint32_t n_tips;      // tips recorded before this step
-    uint32_t n_tips_step; // tips recorded this step (written by propagate)
-    uint32_t overflow;    // bit 0 links, bit 1 per-step states, bit 2 filtered, bit 3 tips, bit 4 inputs
-    uint32_t done;
-    uint32_t n_steps_run;
-    uint32_t n_tracks;
-    uint32_t n_constituents;
-    uint32_t prev_link_base;  // global index of the previous step's first link
-    uint64_t n_links_total;
-    uint64_t n_scored;        // scorer rows of the finished steps
-    line_u32 ticket[kTickets];  // work-queue tickets: [0] progressive filter, [1] votes /
-                                // progressive filter, [2] free, [3] build, [4] find emit,
-                                // [5] propagate emit, [6] free, [7] resume, [8] free
-    line_u32 exit_count;  // blocks of k_prop_emit that have finished this step
-    line_u32 n_rows;      // scorer rows scored this step (added up by k_score_update)
-    line_u64 n_props;     // propagations so far
-    line_u32 n_defer;     // links whose propagation k_propagate_resume continues (this step)
-    line_u32 xcd_ticket[4][8];  // per-XCD work queues (one counter per XCD): find, scorer
-                                // list, propagate, dedup mark
-};
 
 struct ckf_params {
     // detector + field

@@ -369,19 +369,8 @@ __device__ inline dlink staged_link(const stage_head& h, const stage_cand& c, ui
 // one wave walking a partition of 1,024 items chunk by chunk, a step of 90,000
 // inputs kept 88 waves of the chip busy and its compaction took 50 us, four
 // times what the bytes and one look-back cost.
-constexpr uint32_t kEmitChunks = 4;
 constexpr uint32_t kEmitWaves = kBlock / kWave;
-
-// Chunks per partition for n items: one until there are `parts` partitions,
-// then more, at most kEmitChunks.  A look-back round trip covers 64 partitions,
-// so that many keep its chain at a round (k_prop_emit, 200,000 links: 12 us, 24
-// with 512); k_find_emit, whose items cost more than the chain, takes two for
-// every CU (with duplicate lists to make, 160,000 inputs: 38 us, 60 with 64).
-constexpr uint32_t kLightParts = 64u, kHeavyParts = 512u;
-__device__ inline uint32_t emit_chunks(uint32_t n, uint32_t parts) {
-    const uint32_t c = n / (kBlock * parts);
-    return c < 1u ? 1u : (c > kEmitChunks ? kEmitChunks : c);
-}
+static_assert(kBlock == kEmitBlock, "a chunk is an item per thread of a block");
 
 struct emit_shared {
     uint32_t ticket;
@@ -975,6 +964,7 @@ __global__ __launch_bounds__(kBlock) void k_find_emit(ckf_params P) {
         const uint32_t base = lo32(block_lookback(P.lb_lo[0], nullptr, p, epoch, pack2(total, 0u), S));
         if (p == n_parts - 1u && threadIdx.x == 0u) {
             ctl->n_links = base + total;
+            ctl->emit_links = base + total;
         }
 #pragma unroll
         for (uint32_t ch = 0; ch < kEmitChunks; ++ch) {
@@ -1037,23 +1027,6 @@ __global__ __launch_bounds__(kBlock) void k_find_emit(ckf_params P) {
     }
 }
 
-// Overflow bits raised by k_find (links, filtered states).  Later kernels of
-// the step only read these: the bits k_propagate raises itself must not change
-// the partition count its waves see mid-kernel.
-constexpr uint32_t kFindOverflow = 1u | 4u;
-
-// Links of this step that exist: a step whose find kernel overflowed a buffer
-// is abandoned (the host regrows and re-runs), so nothing walks missing links.
-__device__ inline uint32_t links_this_step(const ckf_params& P, const step_ctl* ctl) {
-    if ((ctl->overflow & kFindOverflow) != 0u) {
-        return 0u;
-    }
-    uint32_t n = ctl->n_links;
-    n = n < P.state_cap ? n : P.state_cap;
-    const uint32_t room = P.link_cap > ctl->link_base ? P.link_cap - ctl->link_base : 0u;
-    return n < room ? n : room;
-}
-
 namespace {
 // Is track `a` dominated by `b` (identical measurement history down to a's
 // first link)?  traccc host :431-471.  Two links with the same previous link
@@ -1084,7 +1057,7 @@ __global__ __launch_bounds__(kBlock) void k_dedup_mark(ckf_params P) {
     if (ctl->done || ctl->step < P.dup_min_len || (ctl->overflow & kFindOverflow) != 0u) {
         return;
     }
-    const uint32_t n = links_this_step(P, ctl);
+    const uint32_t n = step_links(*ctl, P.state_cap, P.link_cap);
     const uint32_t base = ctl->link_base;
     const uint32_t epoch = ctl->epoch;
     const uint32_t n_parts = (n + kWave - 1) / kWave;
@@ -1205,7 +1178,7 @@ __global__ __launch_bounds__(kBlock) void k_propagate(ckf_params P, uint32_t fro
     if (ctl->done) {
         return;
     }
-    const uint32_t n = links_this_step(P, ctl);
+    const uint32_t n = step_links(*ctl, P.state_cap, P.link_cap);
     // the grid is sized for the largest step: a block without a partition leaves
     if (n < from || n >= below || static_cast<uint64_t>(blockIdx.x) * kBlock >= static_cast<uint64_t>(n) * kT) {
         return;
@@ -1382,13 +1355,12 @@ __global__ __launch_bounds__(kBlock) void k_prop_emit(ckf_params P, int fused_ad
     if (ctl->done) {
         return;
     }
-    const uint32_t n = links_this_step(P, ctl);
+    const emit_extent extent = emit_extent_of(*ctl);
+    const uint32_t n = extent.n, kc = extent.chunks, n_parts = extent.parts;
+    const uint32_t part = kBlock * kc;
     const uint32_t base = ctl->link_base;
     const uint32_t epoch = ctl->epoch;
     const uint32_t tip_base = ctl->n_tips;
-    const uint32_t kc = emit_chunks(n, kLightParts);
-    const uint32_t part = kBlock * kc;
-    const uint32_t n_parts = (n + part - 1u) / part;
     if (blockIdx.x >= n_parts) {
         // a step abandoned by an overflow has no links and no partition that
         // could end it
@@ -1446,15 +1418,12 @@ __global__ __launch_bounds__(kBlock) void k_prop_emit(ckf_params P, int fused_ad
         // The block that finishes the last partition advances the step: every
         // partition counts itself once it is written (counting every block of
         // the grid instead cost a 1,024-block grid 15 us of atomics on one
-        // word).  A block that starts after the advance does nothing: it finds
-        // done, or no links, or (with the step's old counts) a spent queue,
-        // which k_find_emit clears in the next step.  The step's totals come
-        // from the last partition's look-back words, which carry their own
-        // visibility; the overflow bits that other blocks raise are read with a
-        // device-scope atomic load (the bits they set with atomicOr live at the
-        // device's coherence point); everything else the advance reads was
-        // written by earlier kernels, and its own stores reach the next kernel
-        // at the launch boundary.
+        // word).  A block that starts during or after the advance does nothing
+        // (emit_extent).  The step's totals come from the last partition's
+        // look-back words, which carry their own visibility; the overflow bits
+        // that other blocks raise are read with a device-scope atomic load;
+        // everything else the advance reads was written by earlier kernels, and
+        // its own stores reach the next kernel at the launch boundary.
         __syncthreads();
         if (threadIdx.x == 0u) {
             const uint32_t before = atomicAdd(&ctl->exit_count.v, 1u);
@@ -1468,36 +1437,10 @@ __global__ __launch_bounds__(kBlock) void k_prop_emit(ckf_params P, int fused_ad
     }
 }
 
-// Step advance: move the control block to the next step.  Run by one lane
-// once the step's propagation and its compaction have finished (k_advance,
-// or the last block to leave k_prop_emit).
+// The advance by k_advance, or by the block that ends k_prop_emit: the overflow
+// bits that other blocks raised with atomicOr live at the device's coherence point.
 __device__ void advance_step(const ckf_params& P, step_ctl* ctl) {
-    const uint32_t n_links = ctl->n_links;
-    ctl->n_links_total += n_links;
-    ctl->n_tips += ctl->n_tips_step;
-    ctl->n_tips_step = 0u;
-    ctl->prev_link_base = ctl->link_base;
-    ctl->link_base += n_links;
-    ctl->n_in = ctl->n_live;
-    ctl->n_live = 0u;
-    ctl->n_links = 0u;
-    ctl->n_scored += ctl->n_rows.v;
-    ctl->n_rows.v = 0u;
-    ctl->step += 1u;
-    ctl->n_steps_run = ctl->step;
-    ctl->epoch += 1u;
-    for (int k = 0; k < kTickets; ++k) {
-        if (k != 5) ctl->ticket[k].v = 0u;  // [5] is still being taken from: see k_find_emit
-    }
-    ctl->n_defer.v = 0u;
-    for (int q = 0; q < 4; ++q) {
-        for (uint32_t x = 0; x < kXcds; ++x) ctl->xcd_ticket[q][x].v = 0u;
-    }
-    const uint32_t overflow =
-        __hip_atomic_load(&ctl->overflow, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (ctl->n_in == 0u || ctl->step >= P.max_cands || overflow != 0u) {
-        ctl->done = 1u;
-    }
+    advance_ctl(ctl, P.max_cands, __hip_atomic_load(&ctl->overflow, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
 }
 
 __global__ void k_advance(ckf_params P) {
