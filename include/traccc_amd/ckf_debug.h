@@ -50,6 +50,16 @@ ckf_status ckf_debug_set_kernel_timing(ckf_algorithm* alg, int enable);
 ckf_status ckf_debug_set_schedule(ckf_algorithm* alg, uint32_t lanes_per_link);
 ckf_status ckf_debug_get_schedule(const ckf_algorithm* alg, uint32_t* lanes_per_link);
 
+/* Deferred propagations (one lane per link): in steps of from_links links and
+ * more, a propagation that needs a second layer search is written to a buffer
+ * of at most `capacity` entries and continued by a kernel of its own; past the
+ * buffer it continues in place.  CKF_DEBUG_DEFERRAL_RULE for either leaves it
+ * to the library's rule (the default).  *n receives how many propagations of
+ * the last call asked for it. */
+#define CKF_DEBUG_DEFERRAL_RULE 0xffffffffu
+ckf_status ckf_debug_set_deferral(ckf_algorithm* alg, uint32_t from_links, uint32_t capacity);
+ckf_status ckf_debug_get_deferred(const ckf_algorithm* alg, uint64_t* n);
+
 /* One 16x16x16 BF16 matrix-core product D = A B (row-major FP32 host arrays,
  * inputs rounded to BF16) through the fragment layout the scorer kernels
  * use; checks that layout on the device. */

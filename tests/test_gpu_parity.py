@@ -340,9 +340,10 @@ def test_measurement_on_unknown_surface_rejected(where):
 def test_propagation_schedules_identical(workload, n):
     """Every propagation schedule (lanes per link 1, 2, 4, 8, 16) gives the same
     tracks: the same measurements bit for bit, chi2 and parameters to 1e-5
-    relative (one lane per link continues a propagation that needs a second
-    layer search in its own kernel, whose compiled arithmetic may fuse
-    multiply-adds differently); the autotuned default is one of them."""
+    relative (the compiled arithmetic of the team sizes may fuse multiply-adds
+    differently); so does the default, which goes by each step's links.
+    (Propagations that are deferred, in steps of far more links, have
+    test_deferred_propagation.py.)"""
     det, fld, gun = S.workload(workload, n_particles=n, seed=17)
     ev = S.generate_event(det, fld, gun)
     cfg = S.finding_config_for(workload)

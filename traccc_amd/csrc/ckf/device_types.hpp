@@ -91,7 +91,11 @@ constexpr uint32_t kDeferWords = 48u;
 // the continuing kernel's own chain (50-80 us for a few waves) costs more than
 // the divergence it takes out of the others: 84,815 links 124 us in place, 101
 // + 72 deferred; 285,989 268 and 229 + 74; 323,274 285 and 245 + 79 (the 40 us
-// grow with the links, the 80 do not).
+// grow with the links, the 80 do not).  All propagations of a call, events of
+// 60,000 pions with three branches: four events, deferring its four steps of
+// 350,000 to 500,000 links 4.57 -> 4.62 ms; six events, its steps of 700,000 to
+// 1,000,000 links 6.32 -> 6.19; twelve, those of 1,400,000 to 2,000,000 11.54 ->
+// 11.06; in between (500,000 to 700,000) no difference.
 constexpr uint32_t kDeferLinks = 700000u;
 
 struct ckf_params {
@@ -105,6 +109,7 @@ struct ckf_params {
     // words per entry, word w of entry k at defer[w * defer_cap + k]
     uint32_t* defer;
     uint32_t defer_cap;
+    uint32_t defer_links;         // steps of so many links and more defer (kDeferLinks)
     uint32_t n_surfaces;
     field_view<float> field;
     nav_config<float> nav;

@@ -1161,7 +1161,7 @@ __device__ inline uint8_t finish_link(const ckf_params& P, const navigator<float
 
 // kT lanes propagate one link together (team navigator); 64 / kT links per
 // wave partition.  The team leader writes the results.  With one lane per
-// link and kDeferLinks links or more, a propagation that needs a second layer
+// link and defer_links links or more, a propagation that needs a second layer
 // search (a few % of them, but nearly every wave has one) is written to the
 // defer buffer and continued by k_propagate_resume, so the wave does not run a
 // second search, approach and window for one or two of its lanes.
@@ -1194,7 +1194,7 @@ __global__ __launch_bounds__(kBlock) void k_propagate(ckf_params P, uint32_t fro
     const bool dedup = step >= P.dup_min_len;
     const uint32_t tl = lane() % kT;
     const bool leader = (tl == 0u);
-    const bool defer = (kT == 1) && P.defer_cap > 0u && n >= kDeferLinks;
+    const bool defer = (kT == 1) && P.defer_cap > 0u && n >= P.defer_links;
 
     xcd_ticket_run queue(&ctl->xcd_ticket[2][0].v, n_parts, 1u);
     for (;;) {

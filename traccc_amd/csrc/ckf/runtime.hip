@@ -100,6 +100,9 @@ struct ckf_algorithm {
     // propagations deferred to k_propagate_resume (one lane per link)
     dbuf defer;
     uint32_t defer_cap = 0;
+    uint32_t defer_links_set = CKF_DEBUG_DEFERRAL_RULE;  // diagnostics: see ckf_debug_set_deferral
+    uint32_t defer_cap_set = CKF_DEBUG_DEFERRAL_RULE;
+    uint64_t n_deferred = 0;  // of the last call
     bool logging = false;
     // candidate-verdict log of scored calls (diagnostics)
     dbuf verdict_log, verdict_n;
@@ -120,6 +123,10 @@ struct ckf_algorithm {
     double t_find = 0.0, t_dedup = 0.0, t_prop = 0.0, t_other = 0.0, t_find_work = 0.0,
            t_find_emit = 0.0, t_prop_work = 0.0, t_prop_emit = 0.0;
     uint32_t n_prop_launches = 0;
+
+    uint32_t defer_links() const {
+        return defer_links_set != CKF_DEBUG_DEFERRAL_RULE ? defer_links_set : tamd::kDeferLinks;
+    }
 
     ~ckf_algorithm() {
         for (auto& g : graph) {
@@ -171,9 +178,13 @@ void ensure_buffers(ckf_algorithm& A, const ckf_device_event& ev) {
     A.prop_flag.ensure(size_t(A.state_cap));
     // a propagation that needs a second layer search (a few % of them)
     // continues in its own kernel where a step may hold enough links for that
-    // to pay (some seeds branch: half of kDeferLinks seeds); beyond the buffer
+    // to pay (some seeds branch: half as many seeds); beyond the buffer
     // it continues in place
-    A.defer_cap = ev.n_seeds >= tamd::kDeferLinks / 2u ? std::max<uint32_t>(A.state_cap / 8u, 1024u) : 0u;
+    const uint32_t from = A.defer_links();
+    A.defer_cap = ev.n_seeds >= from / 2u ? std::max<uint32_t>(A.state_cap / 8u, 1024u) : 0u;
+    if (A.defer_cap_set != CKF_DEBUG_DEFERRAL_RULE) {
+        A.defer_cap = std::min(A.defer_cap, A.defer_cap_set);
+    }
     A.defer.ensure(4u * size_t(tamd::kDeferWords) * A.defer_cap);
     A.tips.ensure(4u * size_t(A.tip_cap));
     A.seed_first.ensure(4u * size_t(std::max(ev.n_seeds, 1u)));
@@ -261,6 +272,7 @@ tamd::ckf_params make_params(ckf_algorithm& A, const ckf_device_detector& D,
     P.n_groups = static_cast<uint32_t>(D.h_groups.size());
     P.defer = A.defer.as<uint32_t>();
     P.defer_cap = A.defer_cap;
+    P.defer_links = A.defer_links();
     P.n_surfaces = static_cast<uint32_t>(D.h_sfs.size());
     P.field = tamd::make_field_view<float>(D.field, D.d_map);
     P.nav = tamd::make_nav_config<float>(c);
@@ -668,6 +680,7 @@ ckf_device_tracks* find_tracks_pkf(ckf_algorithm& A, const ckf_device_detector& 
                   "hipHostMalloc");
     }
     A.stats = ckf_run_stats{};
+    A.n_deferred = 0u;
     tamd::ckf_params P = make_params(A, D, ev);
     tamd::pkf_params Q{};
     Q.states = A.pkf_states.as<uint32_t>();
@@ -803,6 +816,7 @@ ckf_device_tracks* find_tracks(ckf_algorithm& A, const ckf_device_detector& D,
     A.stats.n_propagations = done.n_props.v;
     A.stats.n_tips = done.n_tips;
     A.stats.n_scored = done.n_scored;
+    A.n_deferred = done.n_deferred;
 
     // build_tracks: count, size, fill (the build marks logged links on tracks)
     if (A.logging) {
@@ -1439,6 +1453,21 @@ ckf_status ckf_debug_get_schedule(const ckf_algorithm* alg, uint32_t* lanes_per_
             throw ckf_error(CKF_ERR_INVALID_ARGUMENT, "null argument");
         }
         *lanes_per_link = alg->schedule_override;
+    });
+}
+
+ckf_status ckf_debug_set_deferral(ckf_algorithm* alg, uint32_t from_links, uint32_t capacity) {
+    return guarded([&] {
+        if (alg == nullptr) throw ckf_error(CKF_ERR_INVALID_ARGUMENT, "null algorithm");
+        alg->defer_links_set = from_links;
+        alg->defer_cap_set = capacity;
+    });
+}
+
+ckf_status ckf_debug_get_deferred(const ckf_algorithm* alg, uint64_t* n) {
+    return guarded([&] {
+        if (alg == nullptr || n == nullptr) throw ckf_error(CKF_ERR_INVALID_ARGUMENT, "null argument");
+        *n = alg->n_deferred;
     });
 }
 

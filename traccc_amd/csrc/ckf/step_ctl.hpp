@@ -46,6 +46,7 @@ struct step_ctl {
     uint32_t emit_links;  // n_links for k_prop_emit: written by find, left alone by the advance
     uint64_t n_links_total;
     uint64_t n_scored;        // scorer rows of the finished steps
+    uint64_t n_deferred;      // propagations of the finished steps that asked to be deferred
     line_u32 ticket[kTickets];  // work-queue tickets: [0] progressive filter, [1] votes /
                                 // progressive filter, [2] free, [3] build, [4] find emit,
                                 // [5] propagate emit, [6] free, [7] resume, [8] free
@@ -135,6 +136,7 @@ TAMD_HD void advance_ctl(step_ctl* ctl, uint32_t max_cands, uint32_t overflow) {
     for (int k = 0; k < kTickets; ++k) {
         if (k != 5) ctl->ticket[k].v = 0u;  // [5] is still being taken from: see emit_extent
     }
+    ctl->n_deferred += ctl->n_defer.v;
     ctl->n_defer.v = 0u;
     for (int q = 0; q < 4; ++q) {
         for (uint32_t x = 0; x < kCtlXcds; ++x) ctl->xcd_ticket[q][x].v = 0u;
