@@ -1,0 +1,103 @@
+// Host harness: result blocks and read-backs on the host runtime's devices.
+#include <cstring>
+
+#include "ckf/handles.hpp"
+#include "common/readback.hpp"
+
+namespace tamd {
+block_cache& result_cache() {
+    static block_cache c;
+    return c;
+}
+std::string& last_error() {
+    static thread_local std::string s;
+    return s;
+}
+}  // namespace tamd
+
+using host_runtime::rt;
+
+// Blocks returned on one device are handed out on that one only, whichever
+// device the thread that returns or takes them is on.  0, or a step's number.
+extern "C" int cache_keeps_devices_apart() {
+    using namespace tamd;
+    (void)hipSetDevice(1);
+    void* first = nullptr;
+    {
+        rbuf b;
+        b.take(1000);
+        first = b.p;
+        if (rt().blocks[first].first != 1) return 1;
+        (void)hipSetDevice(0);  // the block goes back from here
+    }
+    {
+        rbuf b;
+        b.take(1000);
+        if (b.p == first || rt().blocks[b.p].first != 0) return 2;
+    }
+    (void)hipSetDevice(1);
+    {
+        rbuf b;
+        b.take(1000);
+        if (b.p != first) return 3;
+    }
+    ckf_device_tracks* t = new ckf_device_tracks();
+    t->vec = static_cast<float*>(result_cache().get(5000));
+    t->track_bytes[2] = 5000;
+    void* vec = t->vec;
+    (void)hipSetDevice(2);
+    delete t;
+    void* other = result_cache().get(5000);
+    if (other == vec || rt().blocks[other].first != 2) return 4;
+    result_cache().put(other, 5000, 2);
+    (void)hipSetDevice(0);
+    result_cache().release();
+    return rt().blocks.empty() ? 0 : 5;
+}
+
+// A result of n records (6 words, a triangle of 21, flags, identifiers) on
+// `device`, read back by a thread on device 0.  0, or what is wrong.
+extern "C" int read_back_from(int device, uint32_t n) {
+    using namespace tamd;
+    (void)hipSetDevice(device);
+    rbuf rec, flag, surface;
+    rec.take(128u * size_t(n));
+    flag.take(size_t(n) + 3u);
+    surface.take(4u * size_t(n));
+    for (size_t i = 0; i < 32u * size_t(n); ++i) rec.as<uint32_t>()[i] = static_cast<uint32_t>(i * 2654435761u);
+    for (uint32_t i = 0; i < n; ++i) {
+        flag.as<uint8_t>()[i] = static_cast<uint8_t>(i * 7u);
+        surface.as<uint32_t>()[i] = i % 5u;
+    }
+    const std::vector<uint64_t> ids = {11, 22, 33, 44};
+    (void)hipSetDevice(0);
+    uint64_t before[host_runtime::kDevices];
+    std::memcpy(before, rt().launches, sizeof(before));
+    std::vector<float> vec(6u * size_t(n)), cov(36u * size_t(n));
+    std::vector<uint8_t> flags(n);
+    std::vector<uint64_t> links(n);
+    readback rb(device);
+    rb.words(vec.data(), rec.p, n, 32u, 0u, 6u);
+    rb.symmetric(cov.data(), rec.p, n, 32u, 6u);
+    rb.bytes(flags.data(), flag.p, n);
+    rb.identifiers(links.data(), surface.as<uint32_t>(), n, ids);
+    rb.run();
+    if (host_runtime::device != 0) return 1;  // the caller's device is his own
+    for (int d = 0; d < host_runtime::kDevices; ++d) {
+        if ((rt().launches[d] > before[d]) != (d == device)) return 2;
+    }
+    const uint32_t* r = rec.as<uint32_t>();
+    for (uint32_t i = 0; i < n; ++i) {
+        if (std::memcmp(&vec[6u * size_t(i)], r + 32u * size_t(i), 24u) != 0) return 3;
+        for (uint32_t a = 0, k = 0; a < 6u; ++a) {
+            for (uint32_t b = a; b < 6u; ++b, ++k) {
+                const uint32_t* want = r + 32u * size_t(i) + 6u + k;
+                if (std::memcmp(&cov[36u * size_t(i) + 6u * a + b], want, 4u) != 0) return 4;
+                if (std::memcmp(&cov[36u * size_t(i) + 6u * b + a], want, 4u) != 0) return 5;
+            }
+        }
+        if (flags[i] != static_cast<uint8_t>(i * 7u)) return 6;
+        if (links[i] != (i % 5u < 4u ? ids[i % 5u] : ~0ull)) return 7;
+    }
+    return 0;
+}

@@ -10,8 +10,10 @@
 #include <map>
 #include <memory>
 #include <mutex>
+#include <utility>
 #include <vector>
 
+#include "../common/device.hpp"
 #include "../common/errors.hpp"
 #include "traccc_amd/ckf.h"
 #include "../core/geometry.hpp"
@@ -49,25 +51,26 @@ struct dbuf {
 };
 
 // Process-wide cache of device blocks for per-call results: freed blocks are
-// kept by power-of-two size class and handed out again, so a steady stream of
-// operator calls does not call hipMalloc / hipFree.  At most kMaxHeld bytes
-// are kept (a returned block beyond that is freed); release() frees them all
-// (ckf_release_cached_memory).
+// kept by device and power-of-two size class and handed out again, so a steady
+// stream of operator calls does not call hipMalloc / hipFree.  At most kMaxHeld
+// bytes are kept (a returned block beyond that is freed); release() frees them
+// all (ckf_release_cached_memory).
 struct block_cache {
     static constexpr size_t kMaxHeld = size_t(4) << 30;
     std::mutex mu;
-    std::map<size_t, std::vector<void*>> free_blocks;
+    std::map<std::pair<int, size_t>, std::vector<void*>> free_blocks;  // (device, class)
     size_t held = 0;
     static size_t size_class(size_t bytes) {
         size_t c = 256;
         while (c < bytes) c <<= 1;
         return c;
     }
+    // A block on the calling thread's current device.
     void* get(size_t bytes) {
         const size_t c = size_class(std::max<size_t>(bytes, 1));
         {
             std::lock_guard<std::mutex> lk(mu);
-            auto it = free_blocks.find(c);
+            auto it = free_blocks.find({current_device(), c});
             if (it != free_blocks.end() && !it->second.empty()) {
                 void* p = it->second.back();
                 it->second.pop_back();
@@ -79,7 +82,8 @@ struct block_cache {
         tamd::hip_check(hipMalloc(&p, c), "hipMalloc");
         return p;
     }
-    void put(void* p, size_t bytes) {
+    // Back to the cache, from whichever thread: `device` is where get() was called.
+    void put(void* p, size_t bytes, int device) {
         if (p == nullptr) return;
         const size_t c = size_class(std::max<size_t>(bytes, 1));
         std::lock_guard<std::mutex> lk(mu);
@@ -87,7 +91,7 @@ struct block_cache {
             (void)hipFree(p);
             return;
         }
-        free_blocks[c].push_back(p);
+        free_blocks[{device, c}].push_back(p);
         held += c;
     }
     void release() {
@@ -107,13 +111,15 @@ block_cache& result_cache();
 struct rbuf {
     void* p = nullptr;
     size_t bytes = 0;
+    int device = 0;
     rbuf() = default;
     rbuf(const rbuf&) = delete;
     rbuf& operator=(const rbuf&) = delete;
-    ~rbuf() { result_cache().put(p, bytes); }
+    ~rbuf() { result_cache().put(p, bytes, device); }
     void take(size_t need) {
-        result_cache().put(p, bytes);
+        result_cache().put(p, bytes, device);
         p = nullptr;
+        device = current_device();
         p = result_cache().get(need);
         bytes = need;
     }
@@ -186,6 +192,7 @@ struct ckf_device_event {
 // per-state filtered / smoothed records.
 struct ckf_device_fitted {
     uint32_t n_tracks = 0, n_states = 0;
+    int device = tamd::current_device();
     tamd::id_table ids;
     std::vector<uint32_t> ev_track_off;   // [n_events + 1] tracks of each event
     tamd::rbuf outcome, surface, vec, cov, ndf, chi2, pval, nholes, offsets, cons, flt, smt, flags,
@@ -194,6 +201,7 @@ struct ckf_device_fitted {
 
 struct ckf_device_tracks {
     uint32_t n_events = 0, n_tracks = 0, n_const = 0;
+    int device = tamd::current_device();
     std::vector<uint32_t> ev_track_off, ev_const_off;
     tamd::id_table ids;
     uint16_t* outcome = nullptr;
@@ -209,7 +217,7 @@ struct ckf_device_tracks {
     size_t track_bytes[10] = {};
     ~ckf_device_tracks() {
         void* ps[] = {outcome, surface, vec, cov, ndf, chi2, pval, nholes, offsets, cons};
-        for (int i = 0; i < 10; ++i) tamd::result_cache().put(ps[i], track_bytes[i]);
+        for (int i = 0; i < 10; ++i) tamd::result_cache().put(ps[i], track_bytes[i], device);
     }
 };
 

@@ -1293,7 +1293,7 @@ ckf_status ckf_tracks_download(const ckf_device_tracks* trk, ckf_track_candidate
         const size_t nt = trk->n_tracks, nc = trk->n_const;
         out->n_tracks = trk->n_tracks;
         out->n_constituents = trk->n_const;
-        tamd::readback rb;
+        tamd::readback rb(trk->device);
         rb.bytes(out->fit_outcome, trk->outcome, 2u * nt);
         rb.bytes(out->params_vector, trk->vec, 24u * nt);
         rb.bytes(out->params_covariance, trk->cov, 144u * nt);

@@ -17,6 +17,7 @@
 #include <cstring>
 #include <thread>
 
+#include "device.hpp"
 #include "errors.hpp"
 
 namespace tamd {
@@ -199,6 +200,8 @@ void readback::deliver(const char* staged, size_t begin, size_t end) const {
 
 void readback::run() {
     if (total_ == 0u) return;
+    const device_scope on(device_);
+    hip_check(on.status, "hipSetDevice");
     const size_t n_chunks = (total_ + kChunk - 1u) / kChunk;
     const size_t slots = std::min<size_t>(n_chunks, kSlots);
     const size_t block = n_chunks == 1u ? total_ : slots * kChunk;

@@ -46,6 +46,8 @@ struct pinned_block {
 // of a multiple of four bytes is needed, which every device block here is.
 class readback {
 public:
+    // `device`: where the sources are (the caller's thread may be on another one)
+    explicit readback(int device) : device_(device) {}
     // `bytes` bytes as they are
     void bytes(void* dst, const void* src, size_t bytes);
     // words [base, base + width) of every record of `stride` words
@@ -56,7 +58,7 @@ public:
     // item, may be null) is not `value`
     void identifiers(uint64_t* dst, const uint32_t* src, size_t n, const std::vector<uint64_t>& ids,
                      const uint16_t* only_if = nullptr, uint16_t value = 0);
-    // On the null stream; returns when every host array is written.
+    // On the device's null stream; returns when every host array is written.
     void run();
 
     static constexpr uint32_t kMaxColumns = 20;
@@ -82,6 +84,7 @@ private:
     void add(column c);
     void deliver(const char* staged, size_t begin, size_t end) const;
     hipError_t launch(void* staged, size_t begin, size_t end) const;
+    const int device_;
     column cols_[kMaxColumns];
     uint32_t n_ = 0;
     size_t total_ = 0;

@@ -773,7 +773,7 @@ ckf_status ckf_fitted_download(const ckf_device_fitted* r, ckf_fitted_tracks* o)
         const uint32_t n = r->n_tracks, ns = r->n_states;
         const float* flt = r->flt.as<float>();
         const float* smt = r->smt.as<float>();
-        tamd::readback rb;
+        tamd::readback rb(r->device);
         rb.bytes(o->fit_outcome, r->outcome.p, 2u * size_t(n));
         // an identifier where the caller sees a successful fit
         rb.identifiers(o->params_surface_link, r->surface.as<uint32_t>(), n, *r->ids,

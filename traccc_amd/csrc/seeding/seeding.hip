@@ -1009,6 +1009,7 @@ struct ckf_seeding {
     tamd::sd_axes axes{};
     hipStream_t stream = nullptr;
     uint32_t n_seeds = 0;
+    int device = 0;  // where the seeds of the last run are
     tamd::dbuf in_xyz, in_vr, in_vz, rad, phi, keys, sorted, sort_tmp, pts, bin_off, cnt_b, off_b,
         cnt_t, off_t, bot, top, cnt_tr, off_tr, trip, cnt_s, off_s, slots, seeds, sums, ctl;
     tamd::sd_ctl* h_ctl = nullptr;
@@ -1031,6 +1032,7 @@ void read_ctl(ckf_seeding& S) {
 void run_seeding(ckf_seeding& S, uint32_t n_sp, const float* d_xyz, const float* d_vr, const float* d_vz) {
     using namespace tamd;
     const hipStream_t s = S.stream;
+    S.device = current_device();
     const uint32_t nbins = S.axes.nphi * S.axes.nz;
     const uint32_t N = std::max(n_sp, 1u);
     S.rad.ensure(4u * size_t(N));
@@ -1234,7 +1236,7 @@ ckf_status ckf_seeding_result_download(const ckf_seeding* s, ckf_seeds* out) {
         if (s == nullptr || out == nullptr) throw ckf_error(CKF_ERR_INVALID_ARGUMENT, "null argument");
         if (out->size < s->n_seeds) throw ckf_error(CKF_ERR_INVALID_ARGUMENT, "output smaller than the seeds");
         static_assert(sizeof(tamd::seed_rec) == 16u, "a seed is four words: bottom, middle, top, weight");
-        tamd::readback rb;
+        tamd::readback rb(s->device);
         rb.words(out->bottom, s->seeds.p, s->n_seeds, 4u, 0u, 1u);
         rb.words(out->middle, s->seeds.p, s->n_seeds, 4u, 1u, 1u);
         rb.words(out->top, s->seeds.p, s->n_seeds, 4u, 2u, 1u);
@@ -1279,7 +1281,7 @@ ckf_status ckf_spacepoint_formation(const ckf_device_detector* det, const ckf_de
                                    s, det->d_sfs, ev->d_pos, ev->d_meas_sf, m0, nm, flag.as<uint32_t>(),
                                    off.as<uint32_t>(), xyz.as<float>(), midx.as<uint32_t>());
                 hip_check(hipGetLastError(), "spacepoints");
-                tamd::readback rb;
+                tamd::readback rb(tamd::current_device());
                 rb.bytes(global, xyz.p, 12u * size_t(total));
                 rb.bytes(measurement_index, midx.p, 4u * size_t(total));
                 rb.run();
@@ -1346,7 +1348,7 @@ ckf_status ckf_estimate_track_params(const ckf_track_params_estimation_config* c
             hipLaunchKernelGGL(tamd::k_track_params, dim3(tamd::grid_for(n, tamd::kSdBlock)), dim3(tamd::kSdBlock), 0,
                                nullptr, P);
             hip_check(hipGetLastError(), "track parameters");
-            tamd::readback rb;
+            tamd::readback rb(tamd::current_device());
             rb.bytes(vector, d_vec.p, 24u * size_t(n));
             rb.bytes(covariance, d_cov.p, 144u * size_t(n));
             rb.run();
