@@ -19,7 +19,7 @@ namespace tamd {
 
 constexpr int kStateCols = 28;  // 6 + 21 + 1
 constexpr int kLookbacks = 4;   // compactions with their own look-back words:
-                                // find emit, dedup, propagate emit, build
+                                // find emit, votes, propagate emit, build
 constexpr uint32_t kInvalid = 0xffffffffu;
 
 // state_ref encoding: where a link's (filtered) state lives
@@ -60,12 +60,16 @@ struct stage_cand {
 };
 static_assert(sizeof(stage_head) == 32 && sizeof(stage_cand) == 8, "stage record sizes");
 
-// A link's measurement history in short: its four latest measurements, a hash
-// of all, the first two and how many (a root's: zeros).
-struct alignas(16) link_history {
-    uint4 last;
-    uint32_t all, first, second, count;
+// A link's measurement history in short (a root's: zeros).  20 bytes a link, as
+// a 16-byte piece and a word in columns of their own: two steps of them are in
+// memory for every slot of a step.
+struct link_history {
+    uint32_t m0, m1;  // its two latest measurements
+    uint32_t tail;    // 16-bit hashes of the two before them
+    uint32_t all;     // hash of all
+    uint32_t ends;    // 12-bit hashes of the first two, how many (255: or more)
 };
+constexpr uint32_t kHistoryBytes = 20u;
 
 // A link in its duplicate-removal list.
 struct alignas(16) dedup_node {
@@ -73,8 +77,10 @@ struct alignas(16) dedup_node {
     float p;        // the link's p-value
     uint32_t hash;  // of its latest measurements
     uint32_t head;  // its list
-    uint32_t all, first, second, count;  // of its history
+    uint32_t all, ends;  // of its history
+    uint32_t pad[2];
 };
+static_assert(sizeof(dedup_node) <= 4u * kStateCols, "a step's nodes lie in its states' memory");
 
 TAMD_HD uint32_t link_step(const dlink& l) { return l.packed & 0xffffu; }
 TAMD_HD uint32_t link_skipped(const dlink& l) { return (l.packed >> 16) & 0xffu; }
@@ -106,8 +112,7 @@ struct ckf_params {
     const layer_group* groups;  // build_layer_groups of the layers
     uint32_t n_groups;
     // propagations deferred at their second layer search: kDeferWords
-    // words per entry, word w of entry k at defer[w * defer_cap + k]
-    uint32_t* defer;
+    // words per entry, word w of entry k at defer_words(P, step)[w * defer_cap + k]
     uint32_t defer_cap;
     uint32_t defer_links;         // steps of so many links and more defer (kDeferLinks)
     uint32_t n_surfaces;
@@ -147,10 +152,10 @@ struct ckf_params {
     uint32_t* tips;               // [tip_cap] global link indices
     uint32_t tip_cap;
     uint32_t* seed_first;         // [n_seeds] local index of the seed's first link this step
-    link_history* history[2];     // [state_cap] each link's history, by step parity
+    uint4* history[2];            // [state_cap] each link's history but for `ends`, by step parity,
+                                  // then `ends` [state_cap]
     uint64_t* alive_bits;         // [state_cap / 64 + 1] surviving links, a bit each (dedup steps)
     uint64_t* dedup_head;         // [n_meas + 1] epoch << 32 | link (epoch-tagged list heads)
-    dedup_node* dedup_nodes;      // [state_cap]
     uint64_t* lb_lo[kLookbacks];  // look-back words per compaction: low counter channel
     uint64_t* lb_hi[kLookbacks];  // and high counter channel
     uint32_t lb_cap;
@@ -210,5 +215,25 @@ struct ckf_params {
     uint32_t* verdict_n;          // records written (may exceed verdict_cap)
     uint32_t verdict_cap;
 };
+
+// Memory that a step uses between its kernels.  The states of the step's parity are
+// written by its propagation; until then they are the last step but one's, which
+// nothing reads, and hold the step's duplicate-removal nodes (k_find_emit to
+// k_dedup_mark).  The histories of the other parity are read last by the step's
+// k_find_emit and hold the deferred propagations from k_propagate to
+// k_propagate_resume; the next step's k_find_emit writes them anew.
+TAMD_HD dedup_node* dedup_nodes(const ckf_params& P, uint32_t step) {
+    return reinterpret_cast<dedup_node*>(P.state[step & 1u]);
+}
+TAMD_HD uint32_t* history_ends(const ckf_params& P, uint32_t parity) {
+    return reinterpret_cast<uint32_t*>(P.history[parity] + P.state_cap);
+}
+TAMD_HD uint32_t* defer_words(const ckf_params& P, uint32_t step) {
+    return reinterpret_cast<uint32_t*>(P.history[(step + 1u) & 1u]);
+}
+// Entries that fit there: a propagation in ten, where a few percent ask.
+TAMD_HD uint32_t defer_entries(uint32_t state_cap) {
+    return static_cast<uint32_t>(static_cast<uint64_t>(state_cap) * kHistoryBytes / (4u * kDeferWords));
+}
 
 }  // namespace tamd

@@ -858,27 +858,46 @@ __global__ __launch_bounds__(kBlock) void k_find(ckf_params P) {
 // states it, held 50 and more links in dense events, and the branches of a seed
 // that parted early agree in all that follows: a chain of dependent loads of
 // 50-110 us a step, however few links the step had.)
+__device__ inline uint32_t hash16(uint32_t m) { return (m * 0x85ebca77u) >> 16; }
+__device__ inline uint32_t hash12(uint32_t m) { return (m * 0x9e3779b1u) >> 20; }
+
 __device__ inline link_history extend_history(const link_history& h, uint32_t meas) {
     link_history r = h;
     if (meas != kInvalid) {
-        r.last = make_uint4(meas, h.last.x, h.last.y, h.last.z);
-        uint32_t f = (h.all ^ meas) * 0x9e3779b1u;
+        r.m0 = meas;
+        r.m1 = h.m0;
+        r.tail = hash16(h.m1) | (h.tail << 16);
+        const uint32_t f = (h.all ^ meas) * 0x9e3779b1u;
         r.all = f ^ (f >> 15);
-        r.first = h.count == 0u ? meas : h.first;
-        r.second = h.count == 1u ? meas : h.second;
-        r.count = h.count + 1u;
+        const uint32_t count = h.ends >> 24;
+        r.ends = (h.ends & 0xffffffu) | (count < 255u ? count + 1u : 255u) << 24;
+        if (count < 2u) r.ends |= hash12(meas) << (12u * count);
     }
     return r;
 }
 
-__device__ inline uint32_t latest_hash(const ckf_params& P, const uint4& r) {
-    uint32_t h = r.x * 0x9e3779b1u;
+__device__ inline link_history load_history(const ckf_params& P, uint32_t parity, uint32_t i) {
+    const uint4 q = P.history[parity][i];
+    return {q.x, q.y, q.z, q.w, history_ends(P, parity)[i]};
+}
+
+__device__ inline void store_history(const ckf_params& P, uint32_t parity, uint32_t i, const link_history& h) {
+    P.history[parity][i] = make_uint4(h.m0, h.m1, h.tail, h.all);
+    history_ends(P, parity)[i] = h.ends;
+}
+
+// Hash of the latest measurements that duplicates share: dup_min_len + 1 of them,
+// up to four.  Where holes may outnumber what a link counts of them, a link that
+// counts as long enough may have fewer: only the latest one is sure.
+__device__ inline uint32_t latest_hash(const ckf_params& P, const link_history& r) {
+    const uint32_t more = P.max_skip < 255u ? P.dup_min_len : 0u;
+    uint32_t h = r.m0 * 0x9e3779b1u;
     h ^= h >> 15;
-    if (P.dup_min_len >= 1u) h = (h ^ r.y) * 0x85ebca77u;
+    if (more >= 1u) h = (h ^ r.m1) * 0x85ebca77u;
     h ^= h >> 13;
-    if (P.dup_min_len >= 2u) h = (h ^ r.z) * 0xc2b2ae3du;
+    if (more >= 2u) h = (h ^ (r.tail & 0xffffu)) * 0xc2b2ae3du;
     h ^= h >> 16;
-    if (P.dup_min_len >= 3u) h = (h ^ r.w) * 0x27d4eb2fu;
+    if (more >= 3u) h = (h ^ (r.tail >> 16)) * 0x27d4eb2fu;
     return h ^ (h >> 15);
 }
 
@@ -891,11 +910,11 @@ constexpr uint32_t kDedupShort = 0xffffffffu;
 __device__ inline void dedup_insert(const ckf_params& P, const dlink& L, const link_history& r, uint32_t i,
                                     uint32_t step, uint32_t epoch) {
     if (step + 1u - link_skipped(L) <= P.dup_min_len) {
-        P.dedup_nodes[i].head = kDedupShort;
+        dedup_nodes(P, step)[i].head = kDedupShort;
         return;
     }
     dedup_node node;
-    node.hash = latest_hash(P, r.last);
+    node.hash = latest_hash(P, r);
     node.head = static_cast<uint32_t>((static_cast<uint64_t>(node.hash) * (P.n_meas + 1u)) >> 32);
     // list heads carry the step's epoch: a head from an earlier step reads as empty
     const unsigned long long tagged = (static_cast<unsigned long long>(epoch) << 32) | i;
@@ -904,18 +923,19 @@ __device__ inline void dedup_insert(const ckf_params& P, const dlink& L, const l
     node.next = (static_cast<uint32_t>(old >> 32) == epoch) ? static_cast<uint32_t>(old) : kInvalid;
     node.p = prob_chi2(L.chi2_sum, static_cast<float>(L.ndf_sum - 5u));
     node.all = r.all;
-    node.first = r.first;
-    node.second = r.second;
-    node.count = r.count;
-    P.dedup_nodes[i] = node;
+    node.ends = r.ends;
+    node.pad[0] = node.pad[1] = 0u;
+    dedup_nodes(P, step)[i] = node;
 }
 
 // Can a's history be contained in b's?  Equal numbers of measurements: the
 // whole histories agree.  One more in b: a's first is b's second.
 __device__ inline bool may_contain(const dedup_node& a, const dedup_node& b) {
-    if (a.count == b.count) return a.all == b.all;
-    if (a.count + 1u == b.count) return a.first == b.second;
-    return a.count < b.count;
+    const uint32_t na = a.ends >> 24, nb = b.ends >> 24;
+    if (na == 255u || nb == 255u) return true;
+    if (na == nb) return a.all == b.all;
+    if (na + 1u == nb) return (a.ends & 0xfffu) == ((b.ends >> 12) & 0xfffu);
+    return na < nb;
 }
 
 // Links of the step, after k_find: the inputs' link counts (kept branches, or
@@ -987,7 +1007,7 @@ __global__ __launch_bounds__(kBlock) void k_find_emit(ckf_params P) {
             // the previous link's history (a hole's state reference names its slot)
             link_history before{};
             if (step > 0u) {
-                before = P.history[(step + 1u) & 1u][h.hole_ref & kRefMask];
+                before = load_history(P, (step + 1u) & 1u, h.hole_ref & kRefMask);
             }
             for (uint32_t k = 0; k < n_out[ch]; ++k) {
                 const uint32_t slot = flt_slot(P, i, k);
@@ -999,7 +1019,7 @@ __global__ __launch_bounds__(kBlock) void k_find_emit(ckf_params P) {
                 if (g < P.link_cap && at + k < P.state_cap) {
                     P.links[g] = L;
                     const link_history r = extend_history(before, L.meas);
-                    P.history[step & 1u][at + k] = r;
+                    store_history(P, step & 1u, at + k, r);
                     if (dedup) {
                         dedup_insert(P, L, r, at + k, step, epoch);
                     }
@@ -1061,6 +1081,7 @@ __global__ __launch_bounds__(kBlock) void k_dedup_mark(ckf_params P) {
     const uint32_t base = ctl->link_base;
     const uint32_t epoch = ctl->epoch;
     const uint32_t n_parts = (n + kWave - 1) / kWave;
+    const dedup_node* nodes = dedup_nodes(P, ctl->step);
     xcd_ticket_run queue(&ctl->xcd_ticket[3][0].v, n_parts, 1u);
     for (;;) {
         const uint32_t p = queue.next();
@@ -1071,13 +1092,13 @@ __global__ __launch_bounds__(kBlock) void k_dedup_mark(ckf_params P) {
         bool alive = i < n;
         dedup_node own{};
         if (alive) {
-            own = P.dedup_nodes[i];
+            own = nodes[i];
         }
         if (alive && own.head != kDedupShort) {
             const uint64_t h = P.dedup_head[own.head];
             uint32_t j = (static_cast<uint32_t>(h >> 32) == epoch) ? static_cast<uint32_t>(h) : kInvalid;
             while (j != kInvalid) {
-                const dedup_node node = P.dedup_nodes[j];
+                const dedup_node node = nodes[j];
                 const bool better = own.p != node.p ? node.p >= own.p : j < i;
                 if (j != i && node.hash == own.hash && better && may_contain(own, node)) {
                     const dlink Li = load_link(P, base + i);
@@ -1263,7 +1284,7 @@ __global__ __launch_bounds__(kBlock) void k_propagate(ckf_params P, uint32_t fro
                             w[47] = L.state_ref;
 #pragma unroll
                             for (uint32_t e = 0; e < kDeferWords; ++e) {
-                                P.defer[static_cast<size_t>(e) * P.defer_cap + k] = w[e];
+                                defer_words(P, step)[static_cast<size_t>(e) * P.defer_cap + k] = w[e];
                             }
                             deferred = true;
                         } else {
@@ -1317,7 +1338,7 @@ __global__ __launch_bounds__(kBlock) void k_propagate_resume(ckf_params P) {
         uint32_t w[kDeferWords];
 #pragma unroll
         for (uint32_t e = 0; e < kDeferWords; ++e) {
-            w[e] = P.defer[static_cast<size_t>(e) * P.defer_cap + k];
+            w[e] = defer_words(P, step)[static_cast<size_t>(e) * P.defer_cap + k];
         }
         const geo_view G{P.sfs, P.n_layers, P.field};
         navigator<float, true, 1> nav = make_navigator<1>(G, s_nav.layers, P.nav, 0u, &s_nav, P.n_groups);

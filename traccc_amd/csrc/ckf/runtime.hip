@@ -89,7 +89,7 @@ struct ckf_algorithm {
     uint32_t seed_cap = 0, meas_cap = 0, seg_cap = 0, ev_cap = 0;
     // work buffers
     dbuf state[2], flt, stage_in, stage_slot, links, live, tips, seed_first;
-    dbuf history[2], alive_bits, dedup_head, dedup_nodes, lb_lo[tamd::kLookbacks], lb_hi[tamd::kLookbacks], ctl;
+    dbuf history[2], alive_bits, dedup_head, lb_lo[tamd::kLookbacks], lb_hi[tamd::kLookbacks], ctl;
     dbuf tip_keep, tip_rank, tip_cprefix, seg_count, seg_ccount, seg_base, seg_cbase, seg_off,
         seg_coff, ev_toff, ev_coff;
     // measurement votes (max_num_tracks_per_measurement > 0)
@@ -98,7 +98,6 @@ struct ckf_algorithm {
     dbuf feat_slot, log_feat, log_label, seed_best, list_m, list_c, list_n, list_row,
         find_count, seed_run_min, list_seed, prop_flag;
     // propagations deferred to k_propagate_resume (one lane per link)
-    dbuf defer;
     uint32_t defer_cap = 0;
     uint32_t defer_links_set = CKF_DEBUG_DEFERRAL_RULE;  // diagnostics: see ckf_debug_set_deferral
     uint32_t defer_cap_set = CKF_DEBUG_DEFERRAL_RULE;
@@ -133,14 +132,14 @@ struct ckf_algorithm {
             if (g) (void)hipGraphExecDestroy(g);
         }
         dbuf* all[] = {&state[0], &state[1], &flt, &stage_in, &stage_slot, &links, &live, &tips,
-                       &seed_first, &history[0], &history[1], &alive_bits, &dedup_head, &dedup_nodes, &ctl,
+                       &seed_first, &history[0], &history[1], &alive_bits, &dedup_head, &ctl,
                        &tip_keep, &tip_rank, &tip_cprefix, &seg_count, &seg_ccount, &seg_base,
                        &seg_cbase, &seg_off, &seg_coff, &ev_toff, &ev_coff, &vote_slots,
                        &vote_key, &vote_keep, &vote_rank, &vote_cpos, &vote_misc,
                        &pkf_states, &pkf_n, &pkf_chi2, &pkf_ndf, &pkf_holes, &pkf_cpos,
                        &pkf_lb_lo, &feat_slot, &log_feat,
                        &log_label, &seed_best, &list_m, &list_c, &list_n, &list_row, &find_count,
-                       &seed_run_min, &list_seed, &prop_flag, &verdict_log, &verdict_n, &defer};
+                       &seed_run_min, &list_seed, &prop_flag, &verdict_log, &verdict_n};
         for (dbuf* b : all) b->release();
         for (int k = 0; k < tamd::kLookbacks; ++k) {
             lb_lo[k].release();
@@ -163,9 +162,11 @@ void ensure_buffers(ckf_algorithm& A, const ckf_device_event& ev) {
     const uint32_t N = A.cfg.max_num_branches_per_surface;
     A.flt_cap = static_cast<uint32_t>(std::min<uint64_t>(uint64_t(A.in_cap) * N, 0x3fffffffu));
     A.state_cap = A.flt_cap;
-    // look-back words: the compactions' partitions hold 256 items or more, so
-    // these bounds leave ample slack
-    A.lb_cap = std::max({(A.in_cap + 15u) / 16u, (A.state_cap + 3u) / 4u, parts(A.tip_cap)}) + 1u;
+    // look-back words, one a partition: the step's and the build's partitions
+    // hold kEmitBlock items or more, those of the votes (kept tracks, of which
+    // there may be as many as tips) 64
+    const uint32_t most = std::max(A.in_cap, A.state_cap);
+    A.lb_cap = std::max((most + tamd::kEmitBlock - 1u) / tamd::kEmitBlock, parts(A.tip_cap)) + 1u;
     const size_t st = size_t(tamd::kStateCols) * 4u;
     A.state[0].ensure(st * A.state_cap);
     A.state[1].ensure(st * A.state_cap);
@@ -181,15 +182,14 @@ void ensure_buffers(ckf_algorithm& A, const ckf_device_event& ev) {
     // to pay (some seeds branch: half as many seeds); beyond the buffer
     // it continues in place
     const uint32_t from = A.defer_links();
-    A.defer_cap = ev.n_seeds >= from / 2u ? std::max<uint32_t>(A.state_cap / 8u, 1024u) : 0u;
+    A.defer_cap = ev.n_seeds >= from / 2u ? tamd::defer_entries(A.state_cap) : 0u;
     if (A.defer_cap_set != CKF_DEBUG_DEFERRAL_RULE) {
         A.defer_cap = std::min(A.defer_cap, A.defer_cap_set);
     }
-    A.defer.ensure(4u * size_t(tamd::kDeferWords) * A.defer_cap);
     A.tips.ensure(4u * size_t(A.tip_cap));
     A.seed_first.ensure(4u * size_t(std::max(ev.n_seeds, 1u)));
-    A.history[0].ensure(sizeof(tamd::link_history) * size_t(A.state_cap));
-    A.history[1].ensure(sizeof(tamd::link_history) * size_t(A.state_cap));
+    A.history[0].ensure(tamd::kHistoryBytes * size_t(A.state_cap));
+    A.history[1].ensure(tamd::kHistoryBytes * size_t(A.state_cap));
     A.alive_bits.ensure(8u * (size_t(A.state_cap) / 64u + 1u));
     {
         const size_t old = A.dedup_head.bytes;
@@ -199,7 +199,6 @@ void ensure_buffers(ckf_algorithm& A, const ckf_device_event& ev) {
             hip_check(hipMemsetAsync(A.dedup_head.p, 0, A.dedup_head.bytes, A.stream), "memset");
         }
     }
-    A.dedup_nodes.ensure(sizeof(tamd::dedup_node) * size_t(A.state_cap));
     for (int k = 0; k < tamd::kLookbacks; ++k) {
         for (dbuf* w : {&A.lb_lo[k], &A.lb_hi[k]}) {
             const size_t old = w->bytes;
@@ -270,7 +269,6 @@ tamd::ckf_params make_params(ckf_algorithm& A, const ckf_device_detector& D,
     P.n_layers = static_cast<uint32_t>(D.h_layers.size());
     P.groups = D.d_groups;
     P.n_groups = static_cast<uint32_t>(D.h_groups.size());
-    P.defer = A.defer.as<uint32_t>();
     P.defer_cap = A.defer_cap;
     P.defer_links = A.defer_links();
     P.n_surfaces = static_cast<uint32_t>(D.h_sfs.size());
@@ -311,11 +309,10 @@ tamd::ckf_params make_params(ckf_algorithm& A, const ckf_device_detector& D,
     P.tips = A.tips.as<uint32_t>();
     P.tip_cap = A.tip_cap;
     P.seed_first = A.seed_first.as<uint32_t>();
-    P.history[0] = A.history[0].as<tamd::link_history>();
-    P.history[1] = A.history[1].as<tamd::link_history>();
+    P.history[0] = A.history[0].as<uint4>();
+    P.history[1] = A.history[1].as<uint4>();
     P.alive_bits = A.alive_bits.as<uint64_t>();
     P.dedup_head = A.dedup_head.as<uint64_t>();
-    P.dedup_nodes = A.dedup_nodes.as<tamd::dedup_node>();
     for (int k = 0; k < tamd::kLookbacks; ++k) {
         P.lb_lo[k] = A.lb_lo[k].as<uint64_t>();
         P.lb_hi[k] = A.lb_hi[k].as<uint64_t>();
