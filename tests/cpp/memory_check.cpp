@@ -43,13 +43,12 @@ extern "C" int cache_keeps_devices_apart() {
     }
     ckf_device_tracks* t = new ckf_device_tracks();
     t->vec = static_cast<float*>(result_cache().get(5000));
-    t->track_bytes[2] = 5000;
     void* vec = t->vec;
     (void)hipSetDevice(2);
     delete t;
     void* other = result_cache().get(5000);
     if (other == vec || rt().blocks[other].first != 2) return 4;
-    result_cache().put(other, 5000, 2);
+    result_cache().put(other, 2);
     (void)hipSetDevice(0);
     result_cache().release();
     return rt().blocks.empty() ? 0 : 5;
@@ -100,4 +99,68 @@ extern "C" int read_back_from(int device, uint32_t n) {
         if (links[i] != (i % 5u < 4u ? ids[i % 5u] : ~0ull)) return 7;
     }
     return 0;
+}
+
+// Device bytes that a result's blocks take beyond what it needs.
+extern "C" uint64_t bytes_over(const uint64_t* need, uint32_t n) {
+    using namespace tamd;
+    result_cache().release();
+    const size_t before = rt().device_bytes;
+    uint64_t sum = 0;
+    std::vector<rbuf> blocks(n);
+    for (uint32_t i = 0; i < n; ++i) {
+        blocks[i].take(need[i]);
+        sum += need[i];
+    }
+    return rt().device_bytes - before - sum;
+}
+
+// Allocations of `calls` results one after another, their sizes around `bytes`.
+extern "C" uint64_t allocations_of(uint64_t bytes, uint32_t calls) {
+    using namespace tamd;
+    result_cache().release();
+    const size_t before = rt().allocations;
+    uint32_t r = 12345u;
+    for (uint32_t k = 0; k < calls; ++k) {
+        r = r * 1664525u + 1013904223u;
+        rbuf a, b;
+        a.take(bytes * 8 / 10 + bytes * 4 / 10 * (r >> 16) / 65536);
+        b.take(bytes / 3);
+    }
+    result_cache().release();
+    return rt().allocations - before;
+}
+
+// On a device that holds `limit` bytes: a result of `idle` bytes goes to the cache,
+// then a result and a work buffer of `want` bytes each are asked for.
+// 0, or the step that fails.
+extern "C" int room_from_the_cache(uint64_t limit, uint64_t idle, uint64_t want) {
+    using namespace tamd;
+    result_cache().release();
+    rt().device_limit = rt().device_bytes + limit;
+    int step = 0;
+    dbuf work;
+    try {
+        {
+            rbuf b;
+            b.take(idle);
+        }
+        step = 1;
+        {
+            rbuf b;
+            b.take(want);
+        }
+        step = 2;
+        work.ensure(want);
+        step = 3;
+        rbuf b;
+        b.take(limit);  // does not fit beside it
+        step = 4;
+    } catch (const ckf_error& e) {
+        if (step == 3 && e.code == CKF_ERR_OUT_OF_MEMORY) step = 0;
+    }
+    work.release();
+    result_cache().release();
+    rt().device_limit = ~size_t(0);
+    return step;
 }

@@ -51,3 +51,20 @@ def test_step_buffers(branches):
     inputs = branches ** 2
     want = 376 * inputs * branches + 40 * inputs + 32 * 100 + 20 * 25 + 8 * one.n_meas / one.n_seeds
     assert held / dev.n_seeds < 1.02 * want
+
+
+def test_fit_results():
+    """A fit's columns: 134 B a track, 267 B a state at most, and a sixteenth for their blocks."""
+    from traccc_amd import fitting as FT
+    det, fld, gun = S.workload("C2", n_particles=1000, seed=3)
+    one = S.generate_event(det, fld, gun)
+    ddet = ckf.DeviceDetector(det, fld)
+    cfg = S.finding_config_for("C2")
+    dev = ckf.DeviceEvents(ddet, [one] * 360)
+    tracks = ckf.combinatorial_kalman_filter_algorithm(cfg).run_device(ddet, dev)
+    fitter = FT.kalman_fitting_algorithm(FT.fitting_config(cfg))
+    first = fitter.run_device(ddet, dev, tracks)  # the fitter's own buffers
+    held, fitted = _held(lambda: fitter.run_device(ddet, dev, tracks))
+    n, states = fitted.sizes()
+    assert first.sizes() == (n, states) and states > 1500000
+    assert held < (134 * n + 267 * states) * 17 / 16 + 14 * (2 << 20)

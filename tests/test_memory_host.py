@@ -28,6 +28,32 @@ def test_cached_blocks_stay_on_their_device(lib):
     assert lib.cache_keeps_devices_apart() == 0
 
 
+def test_large_results_take_what_they_need(lib):
+    """A fit's columns for 3.8 million tracks of 37 million states, and a small one's."""
+    lib.bytes_over.restype = C.c_uint64
+    for tracks, states in ((3840000, 37300000), (20000, 106000)):
+        need = [2 * tracks, 4 * tracks, 24 * tracks, 84 * tracks, 4 * tracks, 4 * states, 128 * states, 128 * states, states]
+        over = lib.bytes_over((C.c_uint64 * len(need))(*need), len(need))
+        # a sixteenth where a block is below 1 GiB, 2 MiB beyond
+        assert over < sum(n // 16 if n < 1 << 30 else 2 << 20 for n in need) + len(need) * (2 << 20)
+    small = [1, 255, 256, 257, 4000, 100000]
+    assert lib.bytes_over((C.c_uint64 * len(small))(*small), len(small)) <= sum(small) + 256 * len(small)
+
+
+@pytest.mark.parametrize("size", [1000, 300000, 5000000, 90000000])
+def test_events_of_different_sizes_reuse_blocks(lib, size):
+    lib.allocations_of.restype = C.c_uint64
+    lib.allocations_of.argtypes = [C.c_uint64, C.c_uint32]
+    # sizes spread over 0.8 to 1.2: a larger one than ever before may need a new block
+    assert lib.allocations_of(size, 200) <= 14
+
+
+def test_a_full_device_gets_the_cached_blocks_back(lib):
+    lib.room_from_the_cache.argtypes = [C.c_uint64] * 3
+    assert lib.room_from_the_cache(100 << 20, 70 << 20, 34 << 20) == 0
+    assert lib.room_from_the_cache(100 << 20, 70 << 20, 80 << 20) == 0
+
+
 # one chunk, two, and more than are on their way at once (copied by threads)
 @pytest.mark.parametrize("n", [1, 777, 15000, 120000])
 @pytest.mark.parametrize("device", [0, 1, 2])

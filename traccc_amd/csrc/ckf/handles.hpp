@@ -20,6 +20,95 @@
 
 namespace tamd {
 
+// Process-wide cache of device blocks for per-call results: freed blocks are
+// kept by device and size and handed out again, so a steady stream of operator
+// calls does not call hipMalloc / hipFree.  At most kMaxHeld bytes are kept (a
+// returned block beyond that is freed); release() frees them all
+// (ckf_release_cached_memory), and so does an allocation that finds the device
+// full.
+//
+// New blocks have a power of two up to kGrain, up to kLarge a sixteenth of the
+// power of two below them as a step (results of nearly the same size find each
+// other's blocks: a fit that allocates takes 0.4 ms longer), and from there on
+// what they need: rounded up to a power of two, the fit of 37 million states took
+// 16 GiB for records of 9.6.  A request is served by the smallest free block that
+// is at most twice its size, so events of different sizes find blocks all the same.
+struct block_cache {
+    static constexpr size_t kMaxHeld = size_t(4) << 30;
+    static constexpr size_t kGrain = size_t(2) << 20;
+    static constexpr size_t kLarge = size_t(1) << 30;
+    std::mutex mu;
+    std::map<std::pair<int, size_t>, std::vector<void*>> free_blocks;  // (device, size)
+    std::map<void*, size_t> out;  // sizes of the blocks handed out
+    size_t held = 0;
+    static size_t block_size(size_t bytes) {
+        size_t c = 256;
+        while (c < bytes) c <<= 1;
+        if (c <= kGrain) return c;
+        const size_t step = c > kLarge ? kGrain : c / 32;
+        return (bytes + step - 1) / step * step;
+    }
+    // A block on the calling thread's current device.
+    void* get(size_t bytes) {
+        const size_t c = block_size(bytes);
+        const int device = current_device();
+        std::unique_lock<std::mutex> lk(mu);
+        for (auto it = free_blocks.lower_bound({device, c});
+             it != free_blocks.end() && it->first.first == device && it->first.second <= 2 * c; ++it) {
+            if (it->second.empty()) continue;
+            void* p = it->second.back();
+            it->second.pop_back();
+            held -= it->first.second;
+            out[p] = it->first.second;
+            return p;
+        }
+        lk.unlock();
+        void* p = allocate(c);
+        lk.lock();
+        out[p] = c;
+        return p;
+    }
+    // Back to the cache, from whichever thread: `device` is where get() was called.
+    void put(void* p, int device) {
+        if (p == nullptr) return;
+        std::lock_guard<std::mutex> lk(mu);
+        const auto it = out.find(p);
+        const size_t c = it->second;
+        out.erase(it);
+        if (held + c > kMaxHeld) {
+            (void)hipFree(p);
+            return;
+        }
+        free_blocks[{device, c}].push_back(p);
+        held += c;
+    }
+    // hipMalloc; where the device is full, once more without the cached blocks.
+    void* allocate(size_t bytes) {
+        void* p = nullptr;
+        hipError_t e = hipMalloc(&p, bytes);
+        if (e == hipErrorOutOfMemory) {
+            (void)hipGetLastError();
+            release();
+            e = hipMalloc(&p, bytes);
+        }
+        hip_check(e, "hipMalloc");
+        return p;
+    }
+    void release() {
+        std::lock_guard<std::mutex> lk(mu);
+        for (auto& kv : free_blocks) {
+            for (void* p : kv.second) (void)hipFree(p);
+        }
+        free_blocks.clear();
+        held = 0;
+    }
+};
+
+block_cache& result_cache();
+
+// Device memory that is no result: the cached results' make room for it.
+inline void* device_alloc(size_t bytes) { return result_cache().allocate(bytes); }
+
 // Device allocation that grows by doubling and is reused across calls.
 struct dbuf {
     void* p = nullptr;
@@ -34,7 +123,7 @@ struct dbuf {
         }
         size_t nb = std::max<size_t>(need, bytes * 2);
         nb = (nb + 255) & ~size_t(255);
-        tamd::hip_check(hipMalloc(&p, nb), "hipMalloc");
+        p = device_alloc(nb);
         bytes = nb;
     }
     void release() {
@@ -50,78 +139,20 @@ struct dbuf {
     }
 };
 
-// Process-wide cache of device blocks for per-call results: freed blocks are
-// kept by device and power-of-two size class and handed out again, so a steady
-// stream of operator calls does not call hipMalloc / hipFree.  At most kMaxHeld
-// bytes are kept (a returned block beyond that is freed); release() frees them
-// all (ckf_release_cached_memory).
-struct block_cache {
-    static constexpr size_t kMaxHeld = size_t(4) << 30;
-    std::mutex mu;
-    std::map<std::pair<int, size_t>, std::vector<void*>> free_blocks;  // (device, class)
-    size_t held = 0;
-    static size_t size_class(size_t bytes) {
-        size_t c = 256;
-        while (c < bytes) c <<= 1;
-        return c;
-    }
-    // A block on the calling thread's current device.
-    void* get(size_t bytes) {
-        const size_t c = size_class(std::max<size_t>(bytes, 1));
-        {
-            std::lock_guard<std::mutex> lk(mu);
-            auto it = free_blocks.find({current_device(), c});
-            if (it != free_blocks.end() && !it->second.empty()) {
-                void* p = it->second.back();
-                it->second.pop_back();
-                held -= c;
-                return p;
-            }
-        }
-        void* p = nullptr;
-        tamd::hip_check(hipMalloc(&p, c), "hipMalloc");
-        return p;
-    }
-    // Back to the cache, from whichever thread: `device` is where get() was called.
-    void put(void* p, size_t bytes, int device) {
-        if (p == nullptr) return;
-        const size_t c = size_class(std::max<size_t>(bytes, 1));
-        std::lock_guard<std::mutex> lk(mu);
-        if (held + c > kMaxHeld) {
-            (void)hipFree(p);
-            return;
-        }
-        free_blocks[{device, c}].push_back(p);
-        held += c;
-    }
-    void release() {
-        std::lock_guard<std::mutex> lk(mu);
-        for (auto& kv : free_blocks) {
-            for (void* p : kv.second) (void)hipFree(p);
-        }
-        free_blocks.clear();
-        held = 0;
-    }
-};
-
-block_cache& result_cache();
-
 // A result's device block, from the result cache and back to it.  Contents are
 // whatever the block held before: the kernels of a result write all of it.
 struct rbuf {
     void* p = nullptr;
-    size_t bytes = 0;
     int device = 0;
     rbuf() = default;
     rbuf(const rbuf&) = delete;
     rbuf& operator=(const rbuf&) = delete;
-    ~rbuf() { result_cache().put(p, bytes, device); }
+    ~rbuf() { result_cache().put(p, device); }
     void take(size_t need) {
-        result_cache().put(p, bytes, device);
+        result_cache().put(p, device);
         p = nullptr;
         device = current_device();
         p = result_cache().get(need);
-        bytes = need;
     }
     template <typename T>
     T* as() const {
@@ -134,9 +165,7 @@ using id_table = std::shared_ptr<const std::vector<uint64_t>>;
 
 template <typename T>
 T* dev_copy(const T* src, size_t n) {
-    T* d = nullptr;
-    const size_t bytes = std::max<size_t>(n, 1) * sizeof(T);
-    tamd::hip_check(hipMalloc(&d, bytes), "hipMalloc");
+    T* d = static_cast<T*>(device_alloc(std::max<size_t>(n, 1) * sizeof(T)));
     if (n > 0 && src != nullptr) {
         tamd::hip_check(hipMemcpy(d, src, n * sizeof(T), hipMemcpyHostToDevice), "hipMemcpy H2D");
     }
@@ -214,10 +243,9 @@ struct ckf_device_tracks {
     uint32_t* nholes = nullptr;
     uint32_t* offsets = nullptr;
     uint32_t* cons = nullptr;
-    size_t track_bytes[10] = {};
     ~ckf_device_tracks() {
         void* ps[] = {outcome, surface, vec, cov, ndf, chi2, pval, nholes, offsets, cons};
-        for (int i = 0; i < 10; ++i) tamd::result_cache().put(ps[i], track_bytes[i], device);
+        for (void* p : ps) tamd::result_cache().put(p, device);
     }
 };
 

@@ -585,7 +585,6 @@ void run_votes(ckf_algorithm& A, const tamd::ckf_params& P, const ckf_device_eve
                         reinterpret_cast<void**>(&K2.offsets), reinterpret_cast<void**>(&K2.cons)};
     for (int i = 0; i < 10; ++i) {
         *slots[i] = result_cache().get(sizes[i]);
-        K2.track_bytes[i] = sizes[i];
     }
 
     tamd::vote_params V{};
@@ -637,7 +636,6 @@ void run_votes(ckf_algorithm& A, const tamd::ckf_params& P, const ckf_device_eve
     std::swap(T.nholes, K2.nholes);
     std::swap(T.offsets, K2.offsets);
     std::swap(T.cons, K2.cons);
-    for (int i = 0; i < 10; ++i) std::swap(T.track_bytes[i], K2.track_bytes[i]);
 }
 
 // The operator's dispatch (core/src/finding/combinatorial_kalman_filter_algorithm.cpp:47-57):
@@ -723,7 +721,6 @@ ckf_device_tracks* find_tracks_pkf(ckf_algorithm& A, const ckf_device_detector& 
                             reinterpret_cast<void**>(&T->offsets), reinterpret_cast<void**>(&T->cons)};
         for (int i = 0; i < 10; ++i) {
             *slots[i] = result_cache().get(sizes[i]);
-            T->track_bytes[i] = sizes[i];
         }
         P.out_outcome = T->outcome;
         P.out_surface = T->surface;
@@ -850,7 +847,6 @@ ckf_device_tracks* find_tracks(ckf_algorithm& A, const ckf_device_detector& D,
                             reinterpret_cast<void**>(&T->offsets), reinterpret_cast<void**>(&T->cons)};
         for (int i = 0; i < 10; ++i) {
             *slots[i] = result_cache().get(sizes[i]);
-            T->track_bytes[i] = sizes[i];
         }
         P.out_outcome = T->outcome;
         P.out_surface = T->surface;
