@@ -25,28 +25,28 @@ extern "C" int cache_keeps_devices_apart() {
     void* first = nullptr;
     {
         rbuf b;
-        b.take(1000);
+        b.take(1000, current_device());
         first = b.p;
         if (rt().blocks[first].first != 1) return 1;
         (void)hipSetDevice(0);  // the block goes back from here
     }
     {
         rbuf b;
-        b.take(1000);
+        b.take(1000, current_device());
         if (b.p == first || rt().blocks[b.p].first != 0) return 2;
     }
     (void)hipSetDevice(1);
     {
         rbuf b;
-        b.take(1000);
+        b.take(1000, current_device());
         if (b.p != first) return 3;
     }
     ckf_device_tracks* t = new ckf_device_tracks();
-    t->vec = static_cast<float*>(result_cache().get(5000));
+    t->vec = static_cast<float*>(result_cache().get(5000, current_device()));
     void* vec = t->vec;
     (void)hipSetDevice(2);
     delete t;
-    void* other = result_cache().get(5000);
+    void* other = result_cache().get(5000, current_device());
     if (other == vec || rt().blocks[other].first != 2) return 4;
     result_cache().put(other, 2);
     (void)hipSetDevice(0);
@@ -60,9 +60,9 @@ extern "C" int read_back_from(int device, uint32_t n) {
     using namespace tamd;
     (void)hipSetDevice(device);
     rbuf rec, flag, surface;
-    rec.take(128u * size_t(n));
-    flag.take(size_t(n) + 3u);
-    surface.take(4u * size_t(n));
+    rec.take(128u * size_t(n), current_device());
+    flag.take(size_t(n) + 3u, current_device());
+    surface.take(4u * size_t(n), current_device());
     for (size_t i = 0; i < 32u * size_t(n); ++i) rec.as<uint32_t>()[i] = static_cast<uint32_t>(i * 2654435761u);
     for (uint32_t i = 0; i < n; ++i) {
         flag.as<uint8_t>()[i] = static_cast<uint8_t>(i * 7u);
@@ -109,7 +109,7 @@ extern "C" uint64_t bytes_over(const uint64_t* need, uint32_t n) {
     uint64_t sum = 0;
     std::vector<rbuf> blocks(n);
     for (uint32_t i = 0; i < n; ++i) {
-        blocks[i].take(need[i]);
+        blocks[i].take(need[i], current_device());
         sum += need[i];
     }
     return rt().device_bytes - before - sum;
@@ -124,8 +124,8 @@ extern "C" uint64_t allocations_of(uint64_t bytes, uint32_t calls) {
     for (uint32_t k = 0; k < calls; ++k) {
         r = r * 1664525u + 1013904223u;
         rbuf a, b;
-        a.take(bytes * 8 / 10 + bytes * 4 / 10 * (r >> 16) / 65536);
-        b.take(bytes / 3);
+        a.take(bytes * 8 / 10 + bytes * 4 / 10 * (r >> 16) / 65536, current_device());
+        b.take(bytes / 3, current_device());
     }
     result_cache().release();
     return rt().allocations - before;
@@ -143,18 +143,18 @@ extern "C" int room_from_the_cache(uint64_t limit, uint64_t idle, uint64_t want)
     try {
         {
             rbuf b;
-            b.take(idle);
+            b.take(idle, current_device());
         }
         step = 1;
         {
             rbuf b;
-            b.take(want);
+            b.take(want, current_device());
         }
         step = 2;
         work.ensure(want);
         step = 3;
         rbuf b;
-        b.take(limit);  // does not fit beside it
+        b.take(limit, current_device());  // does not fit beside it
         step = 4;
     } catch (const ckf_error& e) {
         if (step == 3 && e.code == CKF_ERR_OUT_OF_MEMORY) step = 0;
@@ -163,4 +163,28 @@ extern "C" int room_from_the_cache(uint64_t limit, uint64_t idle, uint64_t want)
     result_cache().release();
     rt().device_limit = ~size_t(0);
     return step;
+}
+
+// Blocks for transfers of `bytes` from a pool that may pin `limit` bytes more; the
+// result: the largest block pinned since the last call.
+extern "C" uint64_t staging(uint64_t bytes, uint64_t limit) {
+    using namespace tamd;
+    staging_cache().release();
+    rt().pinned_limit = rt().pinned_bytes + limit;
+    rt().largest_pinned = 0;
+    {
+        const staging_block b(bytes);
+        std::memset(b.p, 7, bytes);
+    }
+    rt().pinned_limit = ~size_t(0);
+    return rt().largest_pinned;
+}
+
+extern "C" int read_back_without_pinned_memory(uint32_t n) {
+    using namespace tamd;
+    staging_cache().release();
+    rt().pinned_limit = rt().pinned_bytes;
+    const int r = read_back_from(1, n);
+    rt().pinned_limit = ~size_t(0);
+    return r;
 }

@@ -59,3 +59,17 @@ def test_a_full_device_gets_the_cached_blocks_back(lib):
 @pytest.mark.parametrize("device", [0, 1, 2])
 def test_read_back_runs_where_the_result_is(lib, device, n):
     assert lib.read_back_from(device, n) == 0
+
+
+@pytest.mark.parametrize("n", [1, 777, 15000, 120000])
+def test_read_back_without_pinned_memory(lib, n):
+    assert lib.read_back_without_pinned_memory(n) == 0
+
+
+def test_large_transfers_pin_no_block_of_their_own(lib):
+    lib.staging.restype, lib.staging.argtypes = C.c_uint64, [C.c_uint64] * 2
+    mb = 1 << 20
+    assert lib.staging(5000, 100 * mb) == 8192
+    assert lib.staging(32 * mb, 100 * mb) == 32 * mb
+    assert lib.staging(32 * mb + 1, 100 * mb) == 0
+    assert lib.staging(5000, 0) == 0

@@ -66,3 +66,36 @@ def test_rejected_spacepoints():
     assert _same(outside) == 0
     assert _same(xyz[:1]) == 0
     assert _same(np.zeros((0, 3), np.float32)) == 0
+
+
+def test_parameters_of_more_seeds_than_a_pinned_block_holds():
+    """Past 32 MiB of indices and spacepoints the arrays are copied one by one: the
+    parameters are those of the same seeds in smaller calls."""
+    import ctypes as C
+    from traccc_amd import simulation as S
+    lib = SD._lib()
+    r = np.random.default_rng(8)
+    det, fld, gun = S.workload("C2", n_particles=500, seed=3)
+    ev = S.generate_event(det, fld, gun)
+    meas, cfg, field = ev.measurements_struct(), SD.track_params_estimation_config(), (C.c_float * 3)(0, 0, 2 * SD.TESLA)
+    points, seeds = 50000, 1680000
+    xyz = r.normal(0, 100, (points, 3)).astype(np.float32)
+    index = r.integers(0, ev.n_meas, points).astype(np.uint32)
+    b, m, t = (r.integers(0, points, seeds).astype(np.uint32) for _ in range(3))
+    w = np.zeros(seeds, np.float32)
+    sp = SD.Spacepoints(points, xyz.ctypes.data, None, None, index.ctypes.data)
+
+    def estimate(lo, hi):
+        part = [v[lo:hi] for v in (b, m, t, w)]
+        struct = SD.Seeds(hi - lo, *[v.ctypes.data for v in part])
+        out = np.zeros(hi - lo, np.uint64), np.zeros((hi - lo, 6), np.float32), np.zeros((hi - lo, 36), np.float32)
+        assert lib.ckf_estimate_track_params(C.byref(cfg), C.byref(sp), C.byref(struct), C.byref(meas), C.byref(field),
+                                             *[v.ctypes.data for v in out]) == 0
+        return out
+
+    assert 20 * seeds + 12 * points > 32 << 20 > 20 * (seeds // 2) + 12 * points
+    whole = estimate(0, seeds)
+    for lo, hi in ((0, seeds // 2), (seeds // 2, seeds)):
+        for a, part in zip(whole, estimate(lo, hi)):
+            assert np.array_equal(a[lo:hi].view(np.uint32), part.view(np.uint32))
+    assert np.isfinite(whole[1]).mean() > 0.9

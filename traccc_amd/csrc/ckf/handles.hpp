@@ -48,10 +48,9 @@ struct block_cache {
         const size_t step = c > kLarge ? kGrain : c / 32;
         return (bytes + step - 1) / step * step;
     }
-    // A block on the calling thread's current device.
-    void* get(size_t bytes) {
+    // A block on the calling thread's current device, `device`.
+    void* get(size_t bytes, int device) {
         const size_t c = block_size(bytes);
-        const int device = current_device();
         std::unique_lock<std::mutex> lk(mu);
         for (auto it = free_blocks.lower_bound({device, c});
              it != free_blocks.end() && it->first.first == device && it->first.second <= 2 * c; ++it) {
@@ -68,7 +67,7 @@ struct block_cache {
         out[p] = c;
         return p;
     }
-    // Back to the cache, from whichever thread: `device` is where get() was called.
+    // Back to the cache, from whichever thread.
     void put(void* p, int device) {
         if (p == nullptr) return;
         std::lock_guard<std::mutex> lk(mu);
@@ -148,11 +147,11 @@ struct rbuf {
     rbuf(const rbuf&) = delete;
     rbuf& operator=(const rbuf&) = delete;
     ~rbuf() { result_cache().put(p, device); }
-    void take(size_t need) {
+    void take(size_t need, int on) {
         result_cache().put(p, device);
         p = nullptr;
-        device = current_device();
-        p = result_cache().get(need);
+        device = on;
+        p = result_cache().get(need, on);
     }
     template <typename T>
     T* as() const {

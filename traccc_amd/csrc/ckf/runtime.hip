@@ -584,7 +584,7 @@ void run_votes(ckf_algorithm& A, const tamd::ckf_params& P, const ckf_device_eve
                         reinterpret_cast<void**>(&K2.pval), reinterpret_cast<void**>(&K2.nholes),
                         reinterpret_cast<void**>(&K2.offsets), reinterpret_cast<void**>(&K2.cons)};
     for (int i = 0; i < 10; ++i) {
-        *slots[i] = result_cache().get(sizes[i]);
+        *slots[i] = result_cache().get(sizes[i], K2.device);
     }
 
     tamd::vote_params V{};
@@ -720,7 +720,7 @@ ckf_device_tracks* find_tracks_pkf(ckf_algorithm& A, const ckf_device_detector& 
                             reinterpret_cast<void**>(&T->pval), reinterpret_cast<void**>(&T->nholes),
                             reinterpret_cast<void**>(&T->offsets), reinterpret_cast<void**>(&T->cons)};
         for (int i = 0; i < 10; ++i) {
-            *slots[i] = result_cache().get(sizes[i]);
+            *slots[i] = result_cache().get(sizes[i], T->device);
         }
         P.out_outcome = T->outcome;
         P.out_surface = T->surface;
@@ -739,7 +739,7 @@ ckf_device_tracks* find_tracks_pkf(ckf_algorithm& A, const ckf_device_detector& 
         if (ns > 0u) {
             hip_check(tamd::launch_pkf_write(P, Q, static_cast<uint32_t>(A.n_cu), A.stream),
                       "pkf write");
-            const tamd::pinned_block off(4u * size_t(ev.n_events));
+            const tamd::staging_block off(4u * size_t(ev.n_events));
             const hipError_t copied = hipMemcpyAsync(off.p, P.event_const_off, 4u * size_t(ev.n_events),
                                                      hipMemcpyDeviceToHost, A.stream);
             hip_check(hipStreamSynchronize(A.stream), "pkf write sync");
@@ -759,6 +759,7 @@ ckf_device_tracks* find_tracks_pkf(ckf_algorithm& A, const ckf_device_detector& 
             }
         }
     } catch (...) {
+        (void)hipStreamSynchronize(A.stream);  // the result's blocks may be handed out again
         delete T;
         throw;
     }
@@ -846,7 +847,7 @@ ckf_device_tracks* find_tracks(ckf_algorithm& A, const ckf_device_detector& D,
                             reinterpret_cast<void**>(&T->pval), reinterpret_cast<void**>(&T->nholes),
                             reinterpret_cast<void**>(&T->offsets), reinterpret_cast<void**>(&T->cons)};
         for (int i = 0; i < 10; ++i) {
-            *slots[i] = result_cache().get(sizes[i]);
+            *slots[i] = result_cache().get(sizes[i], T->device);
         }
         P.out_outcome = T->outcome;
         P.out_surface = T->surface;
@@ -880,7 +881,7 @@ ckf_device_tracks* find_tracks(ckf_algorithm& A, const ckf_device_detector& D,
         T->ev_track_off.resize(ev.n_events + 1u);
         T->ev_const_off.resize(ev.n_events + 1u);
         const size_t off_bytes = 4u * (size_t(ev.n_events) + 1u);
-        const tamd::pinned_block off(2u * off_bytes);
+        const tamd::staging_block off(2u * off_bytes);
         char* const h_off = static_cast<char*>(off.p);
         const hipError_t copied[2] = {
             hipMemcpyAsync(h_off, track_off, off_bytes, hipMemcpyDeviceToHost, A.stream),
@@ -894,6 +895,7 @@ ckf_device_tracks* find_tracks(ckf_algorithm& A, const ckf_device_detector& D,
             T->n_const = T->ev_const_off[ev.n_events];
         }
     } catch (...) {
+        (void)hipStreamSynchronize(A.stream);  // the result's blocks may be handed out again
         delete T;
         throw;
     }
@@ -1203,8 +1205,8 @@ ckf_status ckf_find_tracks_logged(ckf_algorithm* alg, const ckf_device_detector*
             uint32_t total = 0u;
             if (blocks > 0u) {
                 tamd::rbuf d_cnt;
-                d_cnt.take(4u * (blocks + 1u));
-                const tamd::pinned_block h_cnt(4u * size_t(blocks));
+                d_cnt.take(4u * (blocks + 1u), T->device);
+                const tamd::staging_block h_cnt(4u * size_t(blocks));
                 uint32_t* const counts = static_cast<uint32_t*>(h_cnt.p);
                 try {
                     hip_check(tamd::launch_log_count(P, n, d_cnt.as<uint32_t>(), A.stream), "log count");

@@ -29,6 +29,7 @@ size_t pinned_cache::size_class(size_t bytes) {
 }
 
 void* pinned_cache::get(size_t bytes) {
+    if (bytes > kMaxBlock) return nullptr;
     const size_t c = size_class(bytes);
     {
         std::lock_guard<std::mutex> lk(mu);
@@ -41,7 +42,10 @@ void* pinned_cache::get(size_t bytes) {
         }
     }
     void* p = nullptr;
-    hip_check(hipHostMalloc(&p, c, hipHostMallocPortable | hipHostMallocMapped), "hipHostMalloc");
+    if (hipHostMalloc(&p, c, hipHostMallocPortable | hipHostMallocMapped) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
     return p;
 }
 
@@ -72,6 +76,15 @@ pinned_cache& staging_cache() {
 }
 
 namespace {
+
+struct pinned_scope {
+    void* const p;
+    const size_t bytes;
+    explicit pinned_scope(size_t n) : p(staging_cache().get(n)), bytes(n) {}
+    pinned_scope(const pinned_scope&) = delete;
+    pinned_scope& operator=(const pinned_scope&) = delete;
+    ~pinned_scope() { staging_cache().put(p, bytes); }
+};
 
 enum : uint8_t { kPlain = 0, kWords = 1, kSymmetric = 2, kMasked = 3 };
 
@@ -198,6 +211,24 @@ void readback::deliver(const char* staged, size_t begin, size_t end) const {
     }
 }
 
+// Without pinned memory: each chunk through a device block, copied as the runtime
+// copies to any memory.
+void readback::run_pageable() {
+    const size_t block = std::min(total_, kChunk);
+    const std::unique_ptr<char[]> host(new char[block]);
+    void* dev = nullptr;
+    hip_check(hipMalloc(&dev, block), "hipMalloc");
+    hipError_t e = hipSuccess;
+    for (size_t begin = 0; begin < total_ && e == hipSuccess; begin += block) {
+        const size_t end = std::min(total_, begin + block);
+        e = launch(dev, begin, end);
+        if (e == hipSuccess) e = hipMemcpy(host.get(), dev, end - begin, hipMemcpyDeviceToHost);
+        if (e == hipSuccess) deliver(host.get(), begin, end);
+    }
+    (void)hipFree(dev);
+    hip_check(e, "download");
+}
+
 void readback::run() {
     if (total_ == 0u) return;
     const device_scope on(device_);
@@ -205,7 +236,11 @@ void readback::run() {
     const size_t n_chunks = (total_ + kChunk - 1u) / kChunk;
     const size_t slots = std::min<size_t>(n_chunks, kSlots);
     const size_t block = n_chunks == 1u ? total_ : slots * kChunk;
-    const pinned_block held(block);
+    const pinned_scope held(block);
+    if (held.p == nullptr) {
+        run_pageable();
+        return;
+    }
     char* const staged = static_cast<char*>(held.p);
     auto begin = [&](size_t c) { return c * kChunk; };
     auto end = [&](size_t c) { return std::min(total_, (c + 1u) * kChunk); };

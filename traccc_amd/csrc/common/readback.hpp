@@ -7,6 +7,7 @@
 #include <cstddef>
 #include <cstdint>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <vector>
 
@@ -14,9 +15,12 @@ namespace tamd {
 
 // Process-wide pool of pinned host blocks, in power-of-two size classes.  At
 // most kMaxHeld bytes are kept (a returned block beyond that is freed);
-// release() frees them all (ckf_release_cached_memory).
+// release() frees them all (ckf_release_cached_memory).  get() gives none above
+// kMaxBlock, which would be pinned and freed again by every call (a 128 MiB
+// block: 10 ms of an estimation of 3 million seeds), nor where none is to be had.
 struct pinned_cache {
     static constexpr size_t kMaxHeld = size_t(64) << 20;
+    static constexpr size_t kMaxBlock = size_t(32) << 20;
     std::mutex mu;
     std::map<size_t, std::vector<void*>> free_blocks;
     size_t held = 0;
@@ -28,15 +32,24 @@ struct pinned_cache {
 
 pinned_cache& staging_cache();
 
-// A pinned block from the pool and back to it.  Whoever lets a transfer use it
-// waits for the transfer before the block goes.
-struct pinned_block {
-    void* const p;
+// A host block for transfers: a pinned one from the pool and back to it, or
+// ordinary memory, which a copy takes as well (a kernel does not).  Whoever lets
+// a transfer use it waits for the transfer before the block goes.
+struct staging_block {
+    void* const pinned;
     const size_t bytes;
-    explicit pinned_block(size_t n) : p(staging_cache().get(n)), bytes(n) {}
-    pinned_block(const pinned_block&) = delete;
-    pinned_block& operator=(const pinned_block&) = delete;
-    ~pinned_block() { staging_cache().put(p, bytes); }
+    explicit staging_block(size_t n)
+        : pinned(staging_cache().get(n)), bytes(n), pageable_(pinned == nullptr ? new char[n] : nullptr),
+          p(pinned != nullptr ? pinned : pageable_.get()) {}
+    staging_block(const staging_block&) = delete;
+    staging_block& operator=(const staging_block&) = delete;
+    ~staging_block() { staging_cache().put(pinned, bytes); }
+
+private:
+    const std::unique_ptr<char[]> pageable_;
+
+public:
+    void* const p;
 };
 
 // One read-back: the columns are declared, then run() fills the host arrays.
@@ -84,6 +97,7 @@ private:
     void add(column c);
     void deliver(const char* staged, size_t begin, size_t end) const;
     hipError_t launch(void* staged, size_t begin, size_t end) const;
+    void run_pageable();
     const int device_;
     column cols_[kMaxColumns];
     uint32_t n_ = 0;

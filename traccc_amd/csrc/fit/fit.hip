@@ -662,20 +662,20 @@ ckf_status ckf_fit_tracks(ckf_fitter* f, const ckf_device_detector* det, const c
             R->n_states = ns;
             R->ids = det->ids;
             R->ev_track_off = cand->ev_track_off;
-            R->outcome.take(2u * std::max(n, 1u));
-            R->surface.take(4u * std::max(n, 1u));
-            R->vec.take(24u * std::max(n, 1u));
-            R->cov.take(84u * std::max(n, 1u));
-            R->ndf.take(4u * std::max(n, 1u));
-            R->chi2.take(4u * std::max(n, 1u));
-            R->pval.take(4u * std::max(n, 1u));
-            R->nholes.take(4u * std::max(n, 1u));
-            R->offsets.take(4u * (n + 1u));
-            R->cons.take(4u * std::max(ns, 1u));
-            R->flt.take(sizeof(float) * tamd::kRec * std::max<size_t>(ns, 1u));
-            R->smt.take(sizeof(float) * tamd::kRec * std::max<size_t>(ns, 1u));
-            R->flags.take(std::max(ns, 1u));
-            R->state_sf.take(4u * std::max(ns, 1u));
+            R->outcome.take(2u * std::max(n, 1u), R->device);
+            R->surface.take(4u * std::max(n, 1u), R->device);
+            R->vec.take(24u * std::max(n, 1u), R->device);
+            R->cov.take(84u * std::max(n, 1u), R->device);
+            R->ndf.take(4u * std::max(n, 1u), R->device);
+            R->chi2.take(4u * std::max(n, 1u), R->device);
+            R->pval.take(4u * std::max(n, 1u), R->device);
+            R->nholes.take(4u * std::max(n, 1u), R->device);
+            R->offsets.take(4u * (n + 1u), R->device);
+            R->cons.take(4u * std::max(ns, 1u), R->device);
+            R->flt.take(sizeof(float) * tamd::kRec * std::max<size_t>(ns, 1u), R->device);
+            R->smt.take(sizeof(float) * tamd::kRec * std::max<size_t>(ns, 1u), R->device);
+            R->flags.take(std::max(ns, 1u), R->device);
+            R->state_sf.take(4u * std::max(ns, 1u), R->device);
             hip_check(hipMemcpyAsync(R->offsets.p, cand->offsets, 4u * (n + 1u),
                                      hipMemcpyDeviceToDevice, s), "copy offsets");
             if (ns > 0u) {

@@ -1255,13 +1255,14 @@ ckf_status ckf_spacepoint_formation(const ckf_device_detector* det, const ckf_de
         }
         const uint32_t m0 = ev->meas_off[event], nm = ev->meas_off[event + 1] - m0;
         const hipStream_t s = nullptr;
+        const int device = tamd::current_device();
         tamd::rbuf flag, off, sums, d_total, xyz, midx;
         const uint32_t N = std::max(nm, 1u);
-        flag.take(4u * size_t(N));
-        off.take(4u * (size_t(N) + 1u));
-        sums.take(4u * size_t(tamd::scan_sums_size(N)));
-        d_total.take(4u);
-        const tamd::pinned_block h_total(4u);
+        flag.take(4u * size_t(N), device);
+        off.take(4u * (size_t(N) + 1u), device);
+        sums.take(4u * size_t(tamd::scan_sums_size(N)), device);
+        d_total.take(4u, device);
+        const tamd::staging_block h_total(4u);
         try {
             if (nm > 0u) {
                 hipLaunchKernelGGL(tamd::k_sd_sp_flag, dim3(tamd::grid_for(nm, tamd::kSdBlock)), dim3(tamd::kSdBlock),
@@ -1275,13 +1276,13 @@ ckf_status ckf_spacepoint_formation(const ckf_device_detector* det, const ckf_de
             const uint32_t total = *static_cast<const uint32_t*>(h_total.p);
             *n = total;
             if ((global != nullptr || measurement_index != nullptr) && total > 0u) {
-                xyz.take(12u * size_t(total));
-                midx.take(4u * size_t(total));
+                xyz.take(12u * size_t(total), device);
+                midx.take(4u * size_t(total), device);
                 hipLaunchKernelGGL(tamd::k_sd_sp_form, dim3(tamd::grid_for(nm, tamd::kSdBlock)), dim3(tamd::kSdBlock), 0,
                                    s, det->d_sfs, ev->d_pos, ev->d_meas_sf, m0, nm, flag.as<uint32_t>(),
                                    off.as<uint32_t>(), xyz.as<float>(), midx.as<uint32_t>());
                 hip_check(hipGetLastError(), "spacepoints");
-                tamd::readback rb(tamd::current_device());
+                tamd::readback rb(device);
                 rb.bytes(global, xyz.p, 12u * size_t(total));
                 rb.bytes(measurement_index, midx.p, 4u * size_t(total));
                 rb.run();
@@ -1304,14 +1305,18 @@ ckf_status ckf_estimate_track_params(const ckf_track_params_estimation_config* c
             !meas->local_position || !meas->surface_link) {
             throw ckf_error(CKF_ERR_INVALID_ARGUMENT, "null seed, spacepoint or measurement arrays");
         }
-        // One pinned block holds what the kernel needs: the seeds' indices, the
+        // What the kernel needs, in one device block: the seeds' indices, the
         // bottom spacepoint's local position (gathered here, with its surface)
-        // and the spacepoints.  A copy from the caller's own arrays would cost
-        // 10 to 100 us each, for the same reasons as on the way back.
+        // and the spacepoints.  One pinned block holds it on the host: a copy from
+        // the caller's own arrays would cost 10 to 100 us each, for the same
+        // reasons as on the way back.  Past the largest pinned block the copies are
+        // the lesser cost (3 million seeds: 52 ms with a block of 128 MiB pinned
+        // for the call, 42 with four copies and column by column back).
         const size_t np = sp->size, in_bytes = 20u * size_t(n) + 12u * np;
-        const tamd::pinned_block h_in(in_bytes);
+        const bool staged = in_bytes <= tamd::pinned_cache::kMaxBlock;
+        const tamd::staging_block h_in(staged ? in_bytes : 8u * size_t(n));
         uint32_t* const hi = static_cast<uint32_t*>(h_in.p);
-        float* const hb = reinterpret_cast<float*>(hi + 3u * size_t(n));
+        float* const hb = reinterpret_cast<float*>(hi + (staged ? 3u * size_t(n) : 0u));
         for (uint32_t i = 0; i < n; ++i) {
             const uint32_t b = seeds->bottom[i];
             if (b >= np || seeds->middle[i] >= np || seeds->top[i] >= np) {
@@ -1323,17 +1328,28 @@ ckf_status ckf_estimate_track_params(const ckf_track_params_estimation_config* c
             hb[2u * size_t(i) + 1u] = meas->local_position[2u * size_t(m) + 1u];
             if (surface_link) surface_link[i] = meas->surface_link[m];
         }
-        std::memcpy(hi, seeds->bottom, 4u * size_t(n));
-        std::memcpy(hi + n, seeds->middle, 4u * size_t(n));
-        std::memcpy(hi + 2u * size_t(n), seeds->top, 4u * size_t(n));
-        std::memcpy(hb + 2u * size_t(n), sp->global, 12u * np);
+        if (staged) {
+            std::memcpy(hi, seeds->bottom, 4u * size_t(n));
+            std::memcpy(hi + n, seeds->middle, 4u * size_t(n));
+            std::memcpy(hi + 2u * size_t(n), seeds->top, 4u * size_t(n));
+            std::memcpy(hb + 2u * size_t(n), sp->global, 12u * np);
+        }
+        const int device = tamd::current_device();
         tamd::rbuf d_in, d_vec, d_cov;
-        d_in.take(in_bytes);
-        d_vec.take(24u * size_t(n));
-        d_cov.take(144u * size_t(n));
+        d_in.take(in_bytes, device);
+        d_vec.take(24u * size_t(n), device);
+        d_cov.take(144u * size_t(n), device);
         try {
-            hip_check(hipMemcpyAsync(d_in.p, h_in.p, in_bytes, hipMemcpyHostToDevice, nullptr), "upload");
-            const uint32_t* di = d_in.as<uint32_t>();
+            uint32_t* const di = d_in.as<uint32_t>();
+            if (staged) {
+                hip_check(hipMemcpyAsync(di, h_in.p, in_bytes, hipMemcpyHostToDevice, nullptr), "upload");
+            } else {
+                hip_check(hipMemcpy(di, seeds->bottom, 4u * size_t(n), hipMemcpyHostToDevice), "upload");
+                hip_check(hipMemcpy(di + n, seeds->middle, 4u * size_t(n), hipMemcpyHostToDevice), "upload");
+                hip_check(hipMemcpy(di + 2u * size_t(n), seeds->top, 4u * size_t(n), hipMemcpyHostToDevice), "upload");
+                hip_check(hipMemcpy(di + 3u * size_t(n), hb, 8u * size_t(n), hipMemcpyHostToDevice), "upload");
+                hip_check(hipMemcpy(di + 5u * size_t(n), sp->global, 12u * np, hipMemcpyHostToDevice), "upload");
+            }
             tamd::tp_params P{};
             P.cfg = *cfg;
             for (int k = 0; k < 3; ++k) P.b[k] = bfield[k];
@@ -1348,7 +1364,7 @@ ckf_status ckf_estimate_track_params(const ckf_track_params_estimation_config* c
             hipLaunchKernelGGL(tamd::k_track_params, dim3(tamd::grid_for(n, tamd::kSdBlock)), dim3(tamd::kSdBlock), 0,
                                nullptr, P);
             hip_check(hipGetLastError(), "track parameters");
-            tamd::readback rb(tamd::current_device());
+            tamd::readback rb(device);
             rb.bytes(vector, d_vec.p, 24u * size_t(n));
             rb.bytes(covariance, d_cov.p, 144u * size_t(n));
             rb.run();
