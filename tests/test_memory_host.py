@@ -34,8 +34,9 @@ def test_large_results_take_what_they_need(lib):
     for tracks, states in ((3840000, 37300000), (20000, 106000)):
         need = [2 * tracks, 4 * tracks, 24 * tracks, 84 * tracks, 4 * tracks, 4 * states, 128 * states, 128 * states, states]
         over = lib.bytes_over((C.c_uint64 * len(need))(*need), len(need))
-        # a sixteenth where a block is below 1 GiB, 2 MiB beyond
-        assert over < sum(n // 16 if n < 1 << 30 else 2 << 20 for n in need) + len(need) * (2 << 20)
+        # an eighth and a sixteenth up to 256 MiB, a sixteenth up to 1 GiB, 2 MiB beyond
+        assert over < sum(3 * n // 16 if n <= 256 << 20 else n // 16 if n <= 1 << 30 else 2 << 20
+                          for n in need) + len(need) * (2 << 20)
     small = [1, 255, 256, 257, 4000, 100000]
     assert lib.bytes_over((C.c_uint64 * len(small))(*small), len(small)) <= sum(small) + 256 * len(small)
 
@@ -44,8 +45,8 @@ def test_large_results_take_what_they_need(lib):
 def test_events_of_different_sizes_reuse_blocks(lib, size):
     lib.allocations_of.restype = C.c_uint64
     lib.allocations_of.argtypes = [C.c_uint64, C.c_uint32]
-    # sizes spread over 0.8 to 1.2: a larger one than ever before may need a new block
-    assert lib.allocations_of(size, 200) <= 14
+    # sizes spread over 0.8 to 1.2: one that is an eighth larger than any before needs a new block
+    assert lib.allocations_of(size, 200) <= 8
 
 
 def test_a_full_device_gets_the_cached_blocks_back(lib):
