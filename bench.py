@@ -346,10 +346,10 @@ def propagate_roofline(ctx, kt, workload_tag):
     launches = max(kt["steps"], 1)
     lanes = kt["lanes"]
     fld = ctx["fld"]
-    # per link its 32 B record and 4 B alive-prefix word read and 1 B outcome
-    # flag written; per propagated branch the 112 B filtered state read and
-    # the 112 B propagated state written; once per launch the field map
-    # (2 x 4 B per (r, z) node) when the field is a map
+    # per link its 32 B record and its seed's first link (4 B; its alive bit is
+    # 1/8 B) read and 1 B outcome flag written; per propagated branch the 112 B
+    # filtered state read and the 112 B propagated state written; once per
+    # launch the field map (2 x 4 B per (r, z) node) when the field is a map
     field_bytes = 0
     if fld.struct.kind == 1:
         field_bytes = 8 * fld.struct.n_r * fld.struct.n_z
@@ -358,11 +358,11 @@ def propagate_roofline(ctx, kt, workload_tag):
     avg_ms = kt["propagate_kernel"] / launches
     per_launch = alg_bytes / launches
     achieved = per_launch / (avg_ms * 1e-3) / 1e9 if avg_ms > 0 else 0.0
-    # one "launch" is the propagation step: k_propagate with one lane per
-    # link or, for steps of few links, a team of eight, and the
-    # k_propagate_resume that continues the deferred links of large steps
-    # (the HIP events bracket all)
-    kernels = [f"k_propagate<{lanes}>"] if lanes else ["k_propagate<1>", "k_propagate<8>", "k_propagate_resume"]
+    # one "launch" is the propagation step: k_propagate at the lanes per link
+    # of the call's largest steps and, with one, a team of eight for steps of
+    # few links and the k_propagate_resume that continues the deferred links of
+    # large ones (the HIP events bracket all)
+    kernels = [f"k_propagate<{lanes}>"] + (["k_propagate<8>", "k_propagate_resume"] if lanes == 1 else [])
     kernel = " + ".join(kernels)
     traffic = None
     tpath = os.path.join(ROOT, "profiles", f"hbm_traffic_{workload_tag}.json")

@@ -46,9 +46,14 @@ ckf_status ckf_debug_set_kernel_timing(ckf_algorithm* alg, int enable);
 
 /* Propagation schedule: lanes that navigate one link together in the
  * propagation kernel (1, 2, 4, 8 or 16; 0 = chosen for each step by how many
- * links it has, the default).  *lanes receives the setting. */
+ * links it has, the default).  *lanes receives the schedule of the last call: the
+ * lanes of its largest steps. */
 ckf_status ckf_debug_set_schedule(ckf_algorithm* alg, uint32_t lanes_per_link);
 ckf_status ckf_debug_get_schedule(const ckf_algorithm* alg, uint32_t* lanes_per_link);
+/* The propagation launches of the last call's steps: launch k runs lanes[k]
+ * lanes per link (0: there is none) where a step has from[k] links or more (the
+ * second one below the first one's). */
+ckf_status ckf_debug_get_launches(const ckf_algorithm* alg, uint32_t lanes[2], uint32_t from[2]);
 
 /* Deferred propagations (one lane per link): in steps of from_links links and
  * more, a propagation that needs a second layer search is written to a buffer

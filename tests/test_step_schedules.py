@@ -120,3 +120,30 @@ def test_progressive_teams_and_window(events):
     back = alg.run_device(ddet, ckf.DeviceEvents(ddet, rev)).download()
     assert np.array_equal(one.offsets, back.offsets) and np.array_equal(one.constituents, order[back.constituents])
     assert np.array_equal(one.chi2, back.chi2)
+
+
+def test_small_event_after_a_large_one():
+    """The launches of a call go by its own seeds, not by the buffers that an
+    earlier, larger call of the same object left."""
+    det, fld, gun = S.workload("C4", n_particles=9000, seed=43)
+    large, small = S.generate_events(det, fld, [gun, dataclasses.replace(gun, n_particles=40, seed=44)])
+    cfg = S.finding_config_for("C4")
+    cfg.max_num_branches_per_surface = 3
+    lib = F.load_library(ckf.LIB)
+    lib.ckf_debug_get_launches.argtypes = [C.c_void_p, C.POINTER(C.c_uint32), C.POINTER(C.c_uint32)]
+    ddet = ckf.DeviceDetector(det, fld)
+
+    def run(alg, ev):
+        tracks = alg.run_device(ddet, ckf.DeviceEvents(ddet, ev)).download()
+        lanes, since = (C.c_uint32 * 2)(), (C.c_uint32 * 2)()
+        assert lib.ckf_debug_get_launches(alg._h, lanes, since) == 0
+        return tracks, list(lanes), list(since)
+
+    want, lanes, since = run(ckf.combinatorial_kalman_filter_algorithm(cfg), small)
+    assert lanes == [16, 0] and since[0] == 0
+    alg = ckf.combinatorial_kalman_filter_algorithm(cfg)
+    assert run(alg, large)[1] == [1, 8]
+    got, again, _ = run(alg, small)
+    assert again == lanes
+    for a, b in zip(_columns(got), _columns(want)):
+        assert np.array_equal(a, b)

@@ -4,14 +4,9 @@
 #include <hip/hip_runtime.h>
 
 #include "device_types.hpp"
+#include "teams.hpp"
 
 namespace tamd {
-
-// One launch of k_propagate: `team` lanes per link (1, 2, 4, 8 or 16; 0: no
-// launch) for steps of [from, below) links.
-struct prop_launch {
-    uint32_t team, from, below, blocks;
-};
 
 struct launch_shape {
     uint32_t find_blocks;

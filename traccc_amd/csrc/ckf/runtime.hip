@@ -118,6 +118,7 @@ struct ckf_algorithm {
     // per-kernel event timing (diagnostics; the step loop then runs uncaptured)
     uint32_t last_steps = 0;  // steps the previous call ran (sizes the first launch)
     uint32_t schedule_override = 0;   // fixed lanes per link, 0 = by each step's links
+    tamd::prop_launch launches[2] = {{1u, 0u, 0xffffffffu, 0u}, {}};  // of the last call
     bool timing = false;
     double t_find = 0.0, t_dedup = 0.0, t_prop = 0.0, t_other = 0.0, t_find_work = 0.0,
            t_find_emit = 0.0, t_prop_work = 0.0, t_prop_emit = 0.0;
@@ -153,8 +154,6 @@ struct ckf_algorithm {
 namespace {
 
 constexpr uint32_t kStepsPerChunk = 4u;
-// k_propagate's registers allow two waves per SIMD, four SIMDs per CU
-constexpr uint32_t kPropWavesPerCu = 8u;
 
 uint32_t parts(uint32_t n) { return (n + 63u) / 64u; }
 
@@ -362,45 +361,7 @@ tamd::ckf_params make_params(ckf_algorithm& A, const ckf_device_detector& D,
     return P;
 }
 
-// The launches of k_propagate in a step, by how many links a step of this call
-// can have (`bound`; with one branch per surface a step never has more links
-// than seeds).  W = the waves the chip holds (two per SIMD, what the kernel's
-// registers allow): a team is worth its redundant steps while its waves all
-// run at once.  us per step (1 without deferral / 2 / 4 / 8 / 16 lanes):
-// 285,989 links 268 / 416 / 518 / 693 / 1011; 84,815 124 / 156 / 188 / 288 /
-// 416; 54,417 117 / 106 / 131 / 187 / 264; 29,559 107 / 93 / 75 / 107 / 176;
-// 11,089 89 / 86 / 60 / 54 / 68; 3,435 93 / 79 / 55 / 44 / 40; 335 66 / 73 /
-// 48 / 36 / 30.  A call whose steps all fit one team's range runs one launch
-// (a second one costs ~3 us a step to find that it has nothing to do).
-void propagate_schedule(const ckf_algorithm& A, uint64_t bound, tamd::launch_shape& s) {
-    const uint64_t lanes = uint64_t(A.n_cu) * kPropWavesPerCu * 64u;
-    const uint32_t max_blocks = static_cast<uint32_t>(A.n_cu) * kPropWavesPerCu / 4u;
-    auto entry = [&](int k, uint32_t team, uint32_t from, uint32_t below) {
-        const uint64_t most = std::min<uint64_t>(bound, below);
-        const uint64_t blocks = (most * team + 255u) / 256u;
-        s.prop[k] = tamd::prop_launch{team, from, below, static_cast<uint32_t>(std::max<uint64_t>(
-                                                             1u, std::min<uint64_t>(blocks, max_blocks)))};
-    };
-    constexpr uint32_t kAll = 0xffffffffu;
-    s.prop[0] = s.prop[1] = tamd::prop_launch{};
-    if (A.schedule_override != 0u) {
-        entry(0, A.schedule_override, 0u, kAll);  // fixed (diagnostics)
-    } else if (bound * 16u <= lanes * 5u / 8u) {
-        entry(0, 16u, 0u, kAll);
-    } else if (bound * 8u <= lanes) {
-        entry(0, 8u, 0u, kAll);
-    } else if (bound * 4u <= lanes) {
-        const uint32_t t = static_cast<uint32_t>(lanes / 16u);  // 8,192 on 256 CUs
-        entry(0, 4u, t, kAll);
-        entry(1, 16u, 0u, t);
-    } else {
-        const uint32_t t = static_cast<uint32_t>(lanes * 27u / 128u);  // 27,648 on 256 CUs
-        entry(0, bound * 2u <= lanes * 7u / 8u ? 2u : 1u, t, kAll);
-        entry(1, 8u, 0u, t);
-    }
-}
-
-tamd::launch_shape make_shape(const ckf_algorithm& A, uint32_t n_seeds) {
+tamd::launch_shape make_shape(const ckf_algorithm& A, uint32_t n_seeds, bool regrown) {
     const uint32_t max_blocks = static_cast<uint32_t>(A.n_cu) * 8u;
     auto blocks = [&](uint32_t cap) {
         const uint32_t b = (parts(cap) + 3u) / 4u;
@@ -412,7 +373,10 @@ tamd::launch_shape make_shape(const ckf_algorithm& A, uint32_t n_seeds) {
     // (its two-lane teams hold 32, the scored update 64).
     s.find_blocks = std::max(1u, std::min((((A.in_cap + 15u) / 16u) + 3u) / 4u, max_blocks));
     s.dedup_blocks = blocks(A.state_cap);
-    propagate_schedule(A, A.cfg.max_num_branches_per_surface == 1u ? n_seeds : A.state_cap, s);
+    tamd::propagate_launches(static_cast<uint32_t>(A.n_cu),
+                             tamd::step_bound(n_seeds, A.cfg.max_num_branches_per_surface,
+                                              A.cfg.max_num_branches_per_seed, A.state_cap, regrown),
+                             A.schedule_override, s.prop);
     s.resume_blocks = A.defer_cap == 0u ? 0u : std::max(1u, std::min((parts(A.defer_cap) + 3u) / 4u, max_blocks));
     // scorer-pruned finding: 16 inputs per wave listing, 64 per scoring wave
     s.list_blocks = std::max(1u, std::min((((A.in_cap + 15u) / 16u) + 3u) / 4u, max_blocks));
@@ -774,11 +738,9 @@ ckf_device_tracks* find_tracks(ckf_algorithm& A, const ckf_device_detector& D,
     }
     // initial capacities; grown and re-run on overflow
     const uint32_t ns = std::max(ev.n_seeds, 1u);
-    const uint64_t branchy = std::min<uint64_t>(c.max_num_branches_per_seed,
-                                                uint64_t(c.max_num_branches_per_surface) *
-                                                    c.max_num_branches_per_surface);
     A.in_cap = std::max<uint32_t>(A.in_cap, static_cast<uint32_t>(std::min<uint64_t>(
-                                                uint64_t(ns) * std::max<uint64_t>(branchy, 1u),
+                                                tamd::input_bound(ns, c.max_num_branches_per_surface,
+                                                                  c.max_num_branches_per_seed),
                                                 0x3fffffffu)));
     A.link_cap = std::max<uint32_t>(A.link_cap, static_cast<uint32_t>(std::min<uint64_t>(
                                                     uint64_t(ns) * c.initial_links_per_seed,
@@ -792,7 +754,8 @@ ckf_device_tracks* find_tracks(ckf_algorithm& A, const ckf_device_detector& D,
         for (int attempt = 0;; ++attempt) {
             ensure_buffers(A, ev);
             P = make_params(A, D, ev);
-            shape = make_shape(A, ev.n_seeds);
+            shape = make_shape(A, ev.n_seeds, attempt > 0);
+            std::copy(shape.prop, shape.prop + 2, A.launches);
             const uint32_t ovf = run_steps(A, P, shape, ev);
             if (ovf == 0u) {
                 break;
@@ -1447,7 +1410,19 @@ ckf_status ckf_debug_get_schedule(const ckf_algorithm* alg, uint32_t* lanes_per_
         if (alg == nullptr || lanes_per_link == nullptr) {
             throw ckf_error(CKF_ERR_INVALID_ARGUMENT, "null argument");
         }
-        *lanes_per_link = alg->schedule_override;
+        *lanes_per_link = alg->launches[0].team;
+    });
+}
+
+ckf_status ckf_debug_get_launches(const ckf_algorithm* alg, uint32_t lanes[2], uint32_t from[2]) {
+    return guarded([&] {
+        if (alg == nullptr || lanes == nullptr || from == nullptr) {
+            throw ckf_error(CKF_ERR_INVALID_ARGUMENT, "null argument");
+        }
+        for (int k = 0; k < 2; ++k) {
+            lanes[k] = alg->launches[k].team;
+            from[k] = alg->launches[k].from;
+        }
     });
 }
 
