@@ -16,3 +16,5 @@ extern "C" uint64_t step_bound(uint32_t n_seeds, uint32_t per_surface, uint32_t 
                                int regrown) {
     return tamd::step_bound(n_seeds, per_surface, per_seed, state_cap, regrown != 0);
 }
+
+extern "C" uint32_t chain_team(uint64_t n, uint32_t n_cu) { return tamd::chain_team(n, n_cu); }

@@ -23,6 +23,7 @@ def lib(tmp_path_factory):
     lib = C.CDLL(str(out))
     lib.propagate_launches.argtypes = [C.c_uint32, C.c_uint64, C.c_uint32, C.POINTER(C.c_uint32)]
     lib.step_bound.restype = C.c_uint64
+    lib.chain_team.argtypes = [C.c_uint64, C.c_uint32]
     return lib
 
 
@@ -58,3 +59,11 @@ def test_a_large_call_before_changes_nothing(lib, seeds, surface, seed):
     # a call that has outgrown its first buffers goes by what they are now
     assert lib.step_bound(seeds, surface, seed, 4 * own, 1) == 4 * own
     assert lib.step_bound(seeds, 1, seed, 4 * own, 1) == seeds
+
+
+@pytest.mark.parametrize("n,want", [(0, 16), (1, 16), (5120, 16), (5121, 8), (28672, 8), (28673, 1), (1 << 32, 1)])
+def test_chain_teams_follow_the_cus(lib, n, want):
+    """The fit's and the progressive filter's teams: on an eighth of the chip an
+    eighth of the chains fill it."""
+    assert lib.chain_team(n, 256) == want
+    assert lib.chain_team(-(-n // 8), 32) == want

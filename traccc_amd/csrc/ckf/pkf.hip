@@ -159,12 +159,9 @@ __device__ inline void walk_seed(const ckf_params& P, const pkf_params& Q, const
 }
 
 // A seed is one chain of searches, updates and propagations through the whole
-// detector: up to kTeam16 seeds 16 lanes take one together, up to kTeam8 seeds
-// 8, then the lanes are worth more than the chain (10,000 muons: 1,064 us with one
-// lane that also read every measurement of its surfaces, 319 with 8).
-constexpr uint32_t kTeam16 = 5120u;
-constexpr uint32_t kTeam8 = 28672u;
-
+// detector, which 16, 8 or one lane take by how many seeds there are (chain_team;
+// 10,000 muons: 1,064 us with one lane that also read every measurement of its
+// surfaces, 319 with 8).
 template <int kT>
 __global__ __launch_bounds__(kBlock) void k_pkf(ckf_params P, pkf_params Q) {
     // the navigation layers and groups live in LDS for the whole kernel
@@ -264,7 +261,7 @@ __global__ __launch_bounds__(kBlock) void k_pkf_write(ckf_params P, pkf_params Q
 hipError_t launch_pkf(const ckf_params& P, const pkf_params& Q, uint32_t n_cu, hipStream_t stream) {
     const uint32_t parts = (P.n_seeds + kWave - 1u) / kWave;
     const uint32_t blocks = std::max(1u, std::min((parts + 3u) / 4u, n_cu * 8u));
-    const uint32_t team = P.n_seeds <= kTeam16 ? 16u : P.n_seeds <= kTeam8 ? 8u : 1u;
+    const uint32_t team = chain_team(P.n_seeds, n_cu);
     const uint64_t lanes = uint64_t(P.n_seeds) * team;
     const dim3 walk(static_cast<uint32_t>(std::max<uint64_t>(1u, std::min<uint64_t>((lanes + kBlock - 1u) / kBlock, n_cu * 8u))));
     if (team == 16u) {

@@ -71,4 +71,22 @@ inline void propagate_launches(uint32_t n_cu, uint64_t bound, uint32_t fixed, pr
     }
 }
 
+// Lanes that take one chain together in a kernel without steps (the fit's forward
+// pass: a candidate's propagations and updates one after another; the progressive
+// filter: a seed's walk through the detector): few chains are bound by the chain,
+// which a team's navigation shortens (a propagation takes ~100 us on one lane
+// alone, 55 on 8, 40 on 16), many by the lanes, which a team spends on redundant
+// steps.  So the lines lie at chains per CU.  Whole calls, us, with 1 / 8 / 16
+// lanes on 256 CUs:
+//                fit of candidates         progressive filter of seeds
+//    5,000   1,084 /   795 /   724       787 /   394 /   388
+//   10,000   1,263 /   998 / 1,026       875 /   490 /   529
+//   28,000   2,115 / 1,935 / 2,078     1,003 /   858 / 1,014
+//   36,000   2,477 / 2,450 / 2,601     1,016 /   903 / 1,125
+//   56,000   3,431 / 3,488 / 3,805     1,121 / 1,292 / 1,568
+inline uint32_t chain_team(uint64_t n, uint32_t n_cu) {
+    if (n <= uint64_t(n_cu) * 20u) return 16u;  // 5,120 on 256 CUs
+    return n <= uint64_t(n_cu) * 112u ? 8u : 1u;  // 28,672
+}
+
 }  // namespace tamd

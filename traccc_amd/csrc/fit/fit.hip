@@ -39,6 +39,7 @@
 #include "../ckf/handles.hpp"
 #include "../ckf/kalman_device.hpp"
 #include "../ckf/state_io.hpp"
+#include "../ckf/teams.hpp"
 #include "../common/errors.hpp"
 #include "../common/readback.hpp"
 #include "traccc_amd/fitting.h"
@@ -59,13 +60,8 @@ constexpr uint32_t kFitBlock = 64;
 __device__ inline uint32_t fit_track(uint32_t n_tracks, uint32_t i) {
     return i < n_tracks ? n_tracks - 1u - i : n_tracks;
 }
-// Lanes per candidate in k_fit_forward.  A candidate is one chain of
-// propagations, updates and propagations again: few candidates are bound by the
-// chain, which a team's navigation shortens (a propagation of one lane takes
-// ~100 us alone, of 8 lanes 55, of 16 lanes 40); many by the lanes, which a team
-// spends on redundant steps.  10,000 muons: 558 us with one lane, 268 with 8.
-constexpr uint32_t kFitTeam16 = 5120u;   // up to here 16 lanes
-constexpr uint32_t kFitTeam8 = 28672u;   // up to here 8, then one
+// Lanes per candidate in k_fit_forward: 16, 8 or one by how many there are
+// (chain_team; 10,000 muons: 558 us with one lane, 268 with 8).
 constexpr uint32_t kSeqState = 0x80000000u;  // sequence entry is a track state
 
 // kalman_fitter_status values (core/include/traccc/fitting/status_codes.hpp:14-29)
@@ -569,6 +565,7 @@ using tamd::hip_check;
 struct ckf_fitter {
     ckf_fitting_config cfg{};
     hipStream_t stream = nullptr;
+    uint32_t n_cu = 256;
     tamd::dbuf seq, fw_info, ev_track_off;
 };
 
@@ -623,6 +620,11 @@ ckf_status ckf_fitter_create(const ckf_fitting_config* cfg, ckf_fitter** out) {
         validate(*cfg);
         auto* f = new ckf_fitter();
         f->cfg = *cfg;
+        int n_cu = 0;
+        if (hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, tamd::current_device()) == hipSuccess &&
+            n_cu > 0) {
+            f->n_cu = static_cast<uint32_t>(n_cu);
+        }
         *out = f;
     });
 }
@@ -731,7 +733,7 @@ ckf_status ckf_fit_tracks(ckf_fitter* f, const ckf_device_detector* det, const c
                 F.out_pval = R->pval.as<float>();
                 F.out_nholes = R->nholes.as<uint32_t>();
                 const uint32_t blocks = (n + tamd::kFitBlock - 1u) / tamd::kFitBlock;
-                const uint32_t team = n <= tamd::kFitTeam16 ? 16u : n <= tamd::kFitTeam8 ? 8u : 1u;
+                const uint32_t team = tamd::chain_team(n, f->n_cu);
                 const dim3 fw((n * team + tamd::kFitBlock - 1u) / tamd::kFitBlock);
                 for (uint32_t it = 0; it < f->cfg.n_iterations; ++it) {
                     if (team == 16u) {
