@@ -42,13 +42,14 @@ extern "C" int cache_keeps_devices_apart() {
         if (b.p != first) return 3;
     }
     ckf_device_tracks* t = new ckf_device_tracks();
-    t->vec = static_cast<float*>(result_cache().get(5000, current_device()));
+    t->blocks[2] = result_cache().get(5000, current_device());
+    t->vec = static_cast<float*>(t->blocks[2].p);
     void* vec = t->vec;
     (void)hipSetDevice(2);
     delete t;
-    void* other = result_cache().get(5000, current_device());
-    if (other == vec || rt().blocks[other].first != 2) return 4;
-    result_cache().put(other, 2);
+    const device_block other = result_cache().get(5000, current_device());
+    if (other.p == vec || rt().blocks[other.p].first != 2) return 4;
+    result_cache().put(other);
     (void)hipSetDevice(0);
     result_cache().release();
     return rt().blocks.empty() ? 0 : 5;

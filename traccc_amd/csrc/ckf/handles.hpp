@@ -20,6 +20,13 @@
 
 namespace tamd {
 
+// A device block of the cache: its own size, and the device it is on.
+struct device_block {
+    void* p = nullptr;
+    size_t size = 0;
+    int device = 0;
+};
+
 // Process-wide cache of device blocks for per-call results: freed blocks are
 // kept by device and size and handed out again, so a steady stream of operator
 // calls does not call hipMalloc / hipFree.  At most kMaxHeld bytes are kept (a
@@ -41,7 +48,6 @@ struct block_cache {
     static constexpr size_t kLarge = size_t(1) << 30;
     std::mutex mu;
     std::map<std::pair<int, size_t>, std::vector<void*>> free_blocks;  // (device, size)
-    std::map<void*, size_t> out;  // sizes of the blocks handed out
     size_t held = 0;
     static size_t block_size(size_t bytes) {
         size_t c = 256;
@@ -52,7 +58,7 @@ struct block_cache {
         return (bytes + step - 1) / step * step;
     }
     // A block on the calling thread's current device, `device`.
-    void* get(size_t bytes, int device) {
+    device_block get(size_t bytes, int device) {
         const size_t c = block_size(bytes);
         std::unique_lock<std::mutex> lk(mu);
         for (auto it = free_blocks.lower_bound({device, bytes});
@@ -61,28 +67,21 @@ struct block_cache {
             void* p = it->second.back();
             it->second.pop_back();
             held -= it->first.second;
-            out[p] = it->first.second;
-            return p;
+            return {p, it->first.second, device};
         }
         lk.unlock();
-        void* p = allocate(c);
-        lk.lock();
-        out[p] = c;
-        return p;
+        return {allocate(c), c, device};
     }
     // Back to the cache, from whichever thread.
-    void put(void* p, int device) {
-        if (p == nullptr) return;
+    void put(const device_block& b) {
+        if (b.p == nullptr) return;
         std::lock_guard<std::mutex> lk(mu);
-        const auto it = out.find(p);
-        const size_t c = it->second;
-        out.erase(it);
-        if (held + c > kMaxHeld) {
-            (void)hipFree(p);
+        if (held + b.size > kMaxHeld) {
+            (void)hipFree(b.p);
             return;
         }
-        free_blocks[{device, c}].push_back(p);
-        held += c;
+        free_blocks[{b.device, b.size}].push_back(b.p);
+        held += b.size;
     }
     // hipMalloc; where the device is full, once more without the cached blocks.
     void* allocate(size_t bytes) {
@@ -145,21 +144,23 @@ struct dbuf {
 // whatever the block held before: the kernels of a result write all of it.
 struct rbuf {
     void* p = nullptr;
-    int device = 0;
     rbuf() = default;
     rbuf(const rbuf&) = delete;
     rbuf& operator=(const rbuf&) = delete;
-    ~rbuf() { result_cache().put(p, device); }
-    void take(size_t need, int on) {
-        result_cache().put(p, device);
-        p = nullptr;
-        device = on;
-        p = result_cache().get(need, on);
+    ~rbuf() { result_cache().put(block_); }
+    void take(size_t need, int device) {
+        result_cache().put(block_);
+        block_ = {};
+        block_ = result_cache().get(need, device);
+        p = block_.p;
     }
     template <typename T>
     T* as() const {
         return static_cast<T*>(p);
     }
+
+private:
+    device_block block_;
 };
 
 // Surface index -> identifier, made once per detector and held by its results.
@@ -245,9 +246,9 @@ struct ckf_device_tracks {
     uint32_t* nholes = nullptr;
     uint32_t* offsets = nullptr;
     uint32_t* cons = nullptr;
+    tamd::device_block blocks[10];  // of the columns, in that order
     ~ckf_device_tracks() {
-        void* ps[] = {outcome, surface, vec, cov, ndf, chi2, pval, nholes, offsets, cons};
-        for (void* p : ps) tamd::result_cache().put(p, device);
+        for (const tamd::device_block& b : blocks) tamd::result_cache().put(b);
     }
 };
 

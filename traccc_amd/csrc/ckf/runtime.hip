@@ -548,7 +548,8 @@ void run_votes(ckf_algorithm& A, const tamd::ckf_params& P, const ckf_device_eve
                         reinterpret_cast<void**>(&K2.pval), reinterpret_cast<void**>(&K2.nholes),
                         reinterpret_cast<void**>(&K2.offsets), reinterpret_cast<void**>(&K2.cons)};
     for (int i = 0; i < 10; ++i) {
-        *slots[i] = result_cache().get(sizes[i], K2.device);
+        K2.blocks[i] = result_cache().get(sizes[i], K2.device);
+        *slots[i] = K2.blocks[i].p;
     }
 
     tamd::vote_params V{};
@@ -600,6 +601,7 @@ void run_votes(ckf_algorithm& A, const tamd::ckf_params& P, const ckf_device_eve
     std::swap(T.nholes, K2.nholes);
     std::swap(T.offsets, K2.offsets);
     std::swap(T.cons, K2.cons);
+    std::swap(T.blocks, K2.blocks);
 }
 
 // The operator's dispatch (core/src/finding/combinatorial_kalman_filter_algorithm.cpp:47-57):
@@ -684,7 +686,8 @@ ckf_device_tracks* find_tracks_pkf(ckf_algorithm& A, const ckf_device_detector& 
                             reinterpret_cast<void**>(&T->pval), reinterpret_cast<void**>(&T->nholes),
                             reinterpret_cast<void**>(&T->offsets), reinterpret_cast<void**>(&T->cons)};
         for (int i = 0; i < 10; ++i) {
-            *slots[i] = result_cache().get(sizes[i], T->device);
+            T->blocks[i] = result_cache().get(sizes[i], T->device);
+            *slots[i] = T->blocks[i].p;
         }
         P.out_outcome = T->outcome;
         P.out_surface = T->surface;
@@ -810,7 +813,8 @@ ckf_device_tracks* find_tracks(ckf_algorithm& A, const ckf_device_detector& D,
                             reinterpret_cast<void**>(&T->pval), reinterpret_cast<void**>(&T->nholes),
                             reinterpret_cast<void**>(&T->offsets), reinterpret_cast<void**>(&T->cons)};
         for (int i = 0; i < 10; ++i) {
-            *slots[i] = result_cache().get(sizes[i], T->device);
+            T->blocks[i] = result_cache().get(sizes[i], T->device);
+            *slots[i] = T->blocks[i].p;
         }
         P.out_outcome = T->outcome;
         P.out_surface = T->surface;
