@@ -34,8 +34,8 @@ def test_large_results_take_what_they_need(lib):
     for tracks, states in ((3840000, 37300000), (20000, 106000)):
         need = [2 * tracks, 4 * tracks, 24 * tracks, 84 * tracks, 4 * tracks, 4 * states, 128 * states, 128 * states, states]
         over = lib.bytes_over((C.c_uint64 * len(need))(*need), len(need))
-        # an eighth and a sixteenth up to 256 MiB, a sixteenth up to 1 GiB, 2 MiB beyond
-        assert over < sum(3 * n // 16 if n <= 256 << 20 else n // 16 if n <= 1 << 30 else 2 << 20
+        # an eighth up to 256 MiB, a sixteenth up to 1 GiB, and a step of a sixteenth; 2 MiB beyond
+        assert over < sum(n // 5 if n <= 256 << 20 else n // 7 if n <= 1 << 30 else 2 << 20
                           for n in need) + len(need) * (2 << 20)
     small = [1, 255, 256, 257, 4000, 100000]
     assert lib.bytes_over((C.c_uint64 * len(small))(*small), len(small)) <= sum(small) + 256 * len(small)

@@ -34,13 +34,14 @@ struct device_block {
 // (ckf_release_cached_memory), and so does an allocation that finds the device
 // full.
 //
-// New blocks are a power of two up to kGrain, an eighth larger than asked for up
-// to kMedium (the next event's result, a few percent larger, finds it then: the
-// first seeding of another 10,000 muons takes 2,600 us, 2,650 where it allocates),
-// and in steps of a sixteenth up to kLarge; from there on they are what is asked
-// for: rounded up to a power of two, the fit of 37 million states took 16 GiB for
-// records of 9.6.  A request is served by the smallest free block that holds it and
-// is at most twice what a new one would be.
+// New blocks are a power of two up to kGrain, then an eighth larger than asked
+// for up to kMedium and a sixteenth up to kLarge, in steps of a sixteenth of the
+// power of two below: the next event's result, a few percent larger, finds them
+// then.  (First call on other events, us: seeding of 10,000 muons 2,600, 2,650
+// where it allocates; fit and resolution of 2 x 60,000 pions 5,650 and 6,200.)
+// From kLarge on they are what is asked for: rounded up to a power of two, the fit
+// of 37 million states took 16 GiB for records of 9.6.  A request is served by the
+// smallest free block that holds it and is at most twice what a new one would be.
 struct block_cache {
     static constexpr size_t kMaxHeld = size_t(4) << 30;
     static constexpr size_t kGrain = size_t(2) << 20;
@@ -54,7 +55,7 @@ struct block_cache {
         while (c < bytes) c <<= 1;
         if (c <= kGrain) return c;
         const size_t step = c > kLarge ? kGrain : c / 32;
-        if (bytes <= kMedium) bytes += bytes / 8;
+        if (bytes <= kLarge) bytes += bytes <= kMedium ? bytes / 8 : bytes / 16;
         return (bytes + step - 1) / step * step;
     }
     // A block on the calling thread's current device, `device`.
