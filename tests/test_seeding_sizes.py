@@ -45,6 +45,14 @@ def test_middles_of_every_size(bottoms, middles, tops):
     assert _same(_fan(bottoms, middles, tops)) >= 1
 
 
+@pytest.mark.parametrize("bottoms,middles,tops", [
+    (3, 40, 300), (64, 9, 300), (65, 9, 300), (300, 9, 65),  # counted with lanes on tops or on bottoms
+    (3, 40, 200), (16, 5, 17), (130, 5, 3), (70, 5, 256)])   # more triplets than fit: the first bottoms, or later ones
+def test_middles_that_do_not_fit(bottoms, middles, tops):
+    assert _same(_fan(bottoms, middles, tops)) >= 1
+    assert _same(_fan(bottoms, middles, tops, spread=2.0)) >= 1
+
+
 def test_small_and_large_middles_together():
     """Some middles through LDS, some through HBM, one run: the seeds keep the
     middles' order."""

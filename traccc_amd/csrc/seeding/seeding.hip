@@ -524,11 +524,26 @@ struct middle_lds {
     uint16_t seg0[kMidTrips], seg1[kMidTrips];  // seg0: the bottom's lane until its segment is known
 };
 
-// The number of a middle's triplets, a bottom per lane, from HBM.
+// The number of a middle's triplets, from HBM: a lane takes a bottom, or a top
+// where that takes fewer turns (3 bottoms with 300 tops: 15 turns for 300; 3,000
+// such middles in 1,918 us for 2,361).
 __device__ __noinline__ uint32_t count_triplets(const sd_params& P, const doublet_rec* B, const doublet_rec* T,
                                                 uint32_t nb, uint32_t nt, float mr, float mvr, float mvz) {
     const float ss2 = P.c.sigmaScattering * P.c.sigmaScattering;
     uint32_t n = 0u;
+    if (uint64_t(nb) * ((nt + kWave - 1u) / kWave) < uint64_t(nt) * ((nb + kWave - 1u) / kWave)) {
+        for (uint32_t jb = 0; jb < nb; ++jb) {
+            const doublet_rec lb = B[jb];
+            const float iSinTheta2 = 1.f + lb.cot * lb.cot;
+            float scat2 = P.c.maxScatteringAngle2 * iSinTheta2;
+            scat2 *= ss2;
+            for (uint32_t j = lane(); j < nt; j += kWave) {
+                float cv, ip;
+                n += triplet_ok(mr, mvr, mvz, lb, T[j], P.c, iSinTheta2, scat2, cv, ip) ? 1u : 0u;
+            }
+        }
+        return wave_broadcast(wave_inclusive_scan(n), kWave - 1);
+    }
     for (uint32_t jb = lane(); jb < nb; jb += kWave) {
         const doublet_rec lb = B[jb];
         const float iSinTheta2 = 1.f + lb.cot * lb.cot;
@@ -661,11 +676,10 @@ __global__ __launch_bounds__(kWave) void k_sd_middle(sd_params P) {
                 }
                 n += static_cast<uint32_t>(__popcll(m));
             }
-            if (n > kMidTrips) {
-                fits = false;
-                break;
-            }
             wave_lds_order();
+            if (n > kMidTrips) {
+                continue;  // the rest is only counted
+            }
             // the bottoms' segments, and every triplet's
             const uint32_t bn = S.b_n[l];
             const uint32_t bi = wave_inclusive_scan(bn);
@@ -681,8 +695,8 @@ __global__ __launch_bounds__(kWave) void k_sd_middle(sd_params P) {
             }
             wave_lds_order();  // the next bottoms write over these
         }
-        if (!fits) {
-            const uint32_t total = count_triplets(P, B, T, nb, nt, mr, mvr, mvz);
+        if (!fits || n > kMidTrips) {
+            const uint32_t total = fits ? n : count_triplets(P, B, T, nb, nt, mr, mvr, mvz);
             if (l == 0u) {
                 P.cnt_tr[p] = total;
                 P.cnt_s[p] = 0u;
