@@ -189,3 +189,24 @@ extern "C" int read_back_without_pinned_memory(uint32_t n) {
     rt().pinned_limit = ~size_t(0);
     return r;
 }
+
+// Allocations of `calls` results of two blocks after one call's blocks of `stale`
+// bytes in all have gone to the cache.
+extern "C" uint64_t allocations_after(uint64_t stale, uint64_t bytes, uint32_t calls) {
+    using namespace tamd;
+    result_cache().release();
+    {
+        rbuf a, b;
+        a.take(stale / 4 * 3, current_device());
+        b.take(stale / 4, current_device());
+    }
+    const size_t before = rt().allocations;
+    for (uint32_t k = 0; k < calls; ++k) {
+        rbuf a, b;
+        a.take(bytes, current_device());
+        b.take(bytes / 10, current_device());
+    }
+    const bool bounded = result_cache().held <= block_cache::kMaxHeld;
+    result_cache().release();
+    return bounded ? rt().allocations - before : ~uint64_t(0);
+}

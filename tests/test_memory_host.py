@@ -49,6 +49,14 @@ def test_events_of_different_sizes_reuse_blocks(lib, size):
     assert lib.allocations_of(size, 200) <= 8
 
 
+def test_blocks_of_a_larger_call_before_do_not_keep_later_ones_out(lib):
+    lib.allocations_after.restype = C.c_uint64
+    lib.allocations_after.argtypes = [C.c_uint64, C.c_uint64, C.c_uint32]
+    gb = 1 << 30
+    for stale in (gb, int(3.9 * gb), 9 * gb):
+        assert lib.allocations_after(stale, gb, 50) <= 2
+
+
 def test_a_full_device_gets_the_cached_blocks_back(lib):
     lib.room_from_the_cache.argtypes = [C.c_uint64] * 3
     assert lib.room_from_the_cache(100 << 20, 70 << 20, 34 << 20) == 0
