@@ -210,3 +210,23 @@ extern "C" uint64_t allocations_after(uint64_t stale, uint64_t bytes, uint32_t c
     result_cache().release();
     return bounded ? rt().allocations - before : ~uint64_t(0);
 }
+
+// A work buffer whose growth failed holds nothing: a smaller request allocates.
+extern "C" int buffer_after_a_failed_growth() {
+    using namespace tamd;
+    result_cache().release();
+    dbuf b;
+    b.ensure(3 << 20);
+    rt().device_limit = rt().device_bytes + (1 << 20);
+    int step = 1;
+    try {
+        b.ensure(50 << 20);
+    } catch (const ckf_error& e) {
+        step = e.code == CKF_ERR_OUT_OF_MEMORY ? 2 : 3;
+    }
+    rt().device_limit = ~size_t(0);
+    b.ensure(2 << 20);
+    const bool there = b.p != nullptr && b.bytes >= (2 << 20);
+    b.release();
+    return step == 2 && there ? 0 : step;
+}

@@ -63,6 +63,11 @@ def test_a_full_device_gets_the_cached_blocks_back(lib):
     assert lib.room_from_the_cache(100 << 20, 70 << 20, 80 << 20) == 0
 
 
+def test_a_buffer_whose_growth_failed_is_empty(lib):
+    """A call that runs out of memory leaves an object that the next, smaller call can use."""
+    assert lib.buffer_after_a_failed_growth() == 0
+
+
 # one chunk, two, and more than are on their way at once (copied by threads)
 @pytest.mark.parametrize("n", [1, 777, 15000, 120000])
 @pytest.mark.parametrize("device", [0, 1, 2])

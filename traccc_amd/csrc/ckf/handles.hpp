@@ -143,6 +143,7 @@ struct dbuf {
             p = nullptr;
         }
         size_t nb = std::max<size_t>(need, bytes * 2);
+        bytes = 0;  // of nothing, should the allocation fail
         nb = (nb + 255) & ~size_t(255);
         p = device_alloc(nb);
         bytes = nb;
