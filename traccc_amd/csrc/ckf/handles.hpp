@@ -53,7 +53,7 @@ struct block_cache {
         void* p;
         uint64_t since;
     };
-    std::map<std::pair<int, size_t>, std::vector<waiting>> free_blocks;  // (device, size)
+    std::map<std::pair<int, size_t>, std::vector<waiting>> free_blocks;  // (device, size); none empty
     size_t held = 0;
     uint64_t puts = 0;
     static size_t block_size(size_t bytes) {
@@ -68,13 +68,13 @@ struct block_cache {
     device_block get(size_t bytes, int device) {
         const size_t c = block_size(bytes);
         std::unique_lock<std::mutex> lk(mu);
-        for (auto it = free_blocks.lower_bound({device, bytes});
-             it != free_blocks.end() && it->first.first == device && it->first.second <= 2 * c; ++it) {
-            if (it->second.empty()) continue;
-            void* p = it->second.back().p;
+        const auto it = free_blocks.lower_bound({device, bytes});
+        if (it != free_blocks.end() && it->first.first == device && it->first.second <= 2 * c) {
+            const device_block b{it->second.back().p, it->first.second, device};
             it->second.pop_back();
-            held -= it->first.second;
-            return {p, it->first.second, device};
+            held -= b.size;
+            if (it->second.empty()) free_blocks.erase(it);
+            return b;
         }
         lk.unlock();
         return {allocate(c), c, device};
@@ -95,7 +95,6 @@ struct block_cache {
     void drop_oldest() {
         auto oldest = free_blocks.end();
         for (auto it = free_blocks.begin(); it != free_blocks.end(); ++it) {
-            if (it->second.empty()) continue;
             if (oldest == free_blocks.end() || it->second.front().since < oldest->second.front().since) oldest = it;
         }
         (void)hipFree(oldest->second.front().p);

@@ -795,6 +795,7 @@ ckf_device_tracks* find_tracks(ckf_algorithm& A, const ckf_device_detector& D,
     hip_check(hipStreamSynchronize(A.stream), "build sync");
     A.epoch_next = A.h_ctl->epoch + 2u;
 
+    ckf_device_tracks built;  // blocks the vote kernels read, released after the sync (the handler's too)
     auto* T = new ckf_device_tracks();
     try {
         const uint32_t nt = A.h_ctl->n_tracks;
@@ -839,7 +840,6 @@ ckf_device_tracks* find_tracks(ckf_algorithm& A, const ckf_device_detector& D,
         hip_check(tamd::launch_build_write(P, shape, A.h_ctl->n_tips, A.stream), "build write");
         const uint32_t* track_off = P.event_track_off;
         const uint32_t* const_off = P.event_const_off;
-        ckf_device_tracks built;  // blocks the vote kernels read, released after the sync
         if (votes) {
             run_votes(A, P, ev, *T, built);
             track_off = A.vote_misc.as<uint32_t>() + 2u;
