@@ -1,7 +1,7 @@
 """Ambiguity resolution at the edges of its kernels' blocks, identifier chunks
-and list batches (GPU): blocks of 1,024 threads, up to 512 of them; a track's
-identifiers eight at a time; a shared identifier's tracks four at a time.  The
-kept tracks are the oracle's."""
+and list batches (GPU): blocks of 256 threads up to 131,072 tracks or identifiers,
+then of 1,024, up to 512 of them; a track's identifiers eight at a time; a shared
+identifier's tracks four at a time.  The kept tracks are the oracle's."""
 import numpy as np
 import pytest
 
@@ -27,7 +27,9 @@ def _tracks(seed, n, longest, n_ids, repeat):
 
 @pytest.mark.parametrize("n,longest,n_ids,repeat", [
     (1023, 8, 900, False), (1024, 9, 5000, True), (1025, 17, 3000, True), (700, 40, 60, True),
-    (3000, 7, 20, False), (524289, 6, 2000000, True)])
+    (3000, 7, 20, False), (524289, 6, 2000000, True),
+    (255, 8, 300, False), (256, 8, 300, True), (257, 8, 300, False),
+    (131072, 5, 131073, True), (131073, 5, 131072, False)])
 def test_blocks_chunks_and_lists(n, longest, n_ids, repeat):
     from traccc_amd import ambiguity as AMB
     off, ids, pv = _tracks(n, n, longest, n_ids, repeat)

@@ -63,7 +63,14 @@ namespace {
 // atomic per block and pass.  All waves of a grid end on the same few words, so
 // with an atomic per wave of 64 those words bounded every kernel here (1 M
 // tracks, 5 M identifiers: k_amb_hot0 629 us for 20 MB, k_amb_output 179 us).
+// Up to kAmbSmall items (512 blocks of 256) the atomics are few either way, and
+// blocks of 256 spread the items over four times as many CUs.  Whole calls, us,
+// with 1,024 / 256 threads: 30,000 tracks with 60,000 identifiers 931 / 720 (910
+// with 256 and an atomic per wave), 100,000 tracks 488 / 456, 200,000 628 / 653,
+// 1 M 1,378 / 1,546.
 constexpr uint32_t kAmbBlock = 1024;
+constexpr uint32_t kAmbSmallBlock = 256;
+constexpr uint32_t kAmbSmall = 131072;
 constexpr uint32_t kAmbWaves = kAmbBlock / kWave;
 constexpr uint32_t kSeqBlock = 1024;
 // identifiers of a track held in registers at a time
@@ -168,8 +175,9 @@ __device__ inline void block_append(uint32_t* counter, uint32_t* list, bool take
     uint32_t before = 0u, total = 0u;
 #pragma unroll
     for (uint32_t q = 0; q < kAmbWaves; ++q) {
-        before += q < w ? S.tot[q] : 0u;
-        total += S.tot[q];
+        const uint32_t n = q < blockDim.x / kWave ? S.tot[q] : 0u;
+        before += q < w ? n : 0u;
+        total += n;
     }
     if (threadIdx.x == 0u) S.base = total > 0u ? atomicAdd(counter, total) : 0u;
     __syncthreads();
@@ -185,7 +193,7 @@ __device__ inline void block_count(uint32_t* counter, uint32_t n, append_shared&
     __syncthreads();
     if (threadIdx.x == 0u) {
         uint32_t total = 0u;
-        for (uint32_t q = 0; q < kAmbWaves; ++q) total += S.tot[q];
+        for (uint32_t q = 0; q < blockDim.x / kWave; ++q) total += S.tot[q];
         if (total > 0u) atomicAdd(counter, total);
     }
 }
@@ -525,9 +533,18 @@ __global__ __launch_bounds__(kAmbBlock) void k_amb_fitted_ids(const uint32_t* of
 }
 
 // Two blocks of 1,024 fill a CU's 2,048 lanes; the kernels stride over the rest.
-uint32_t grid_for(uint64_t items) {
-    const uint64_t b = (items + kAmbBlock - 1u) / kAmbBlock;
-    return static_cast<uint32_t>(std::max<uint64_t>(1u, std::min<uint64_t>(b, 512u)));
+struct amb_grid {
+    dim3 blocks, threads;
+};
+amb_grid grid_for(uint64_t items) {
+    const uint32_t t = items <= kAmbSmall ? kAmbSmallBlock : kAmbBlock;
+    const uint64_t b = (items + t - 1u) / t;
+    return {dim3(static_cast<uint32_t>(std::max<uint64_t>(1u, std::min<uint64_t>(b, 512u)))), dim3(t)};
+}
+
+template <typename... K, typename... A>
+void launch(void (*kernel)(K...), const amb_grid& g, hipStream_t s, A... args) {
+    hipLaunchKernelGGL(kernel, g.blocks, g.threads, 0, s, static_cast<K>(args)...);
 }
 
 }  // namespace
@@ -569,7 +586,7 @@ void setup(ckf_resolver& R, tamd::amb_params& P, uint32_t n_entries) {
     hip_check(hipMemsetAsync(R.ctl.p, 0, sizeof(amb_ctl), s), "memset");
     hip_check(hipMemsetAsync(P.n_acc, 0, 4u * size_t(B), s), "memset");
     hip_check(hipMemsetAsync(P.best_of, 0xff, 4u * size_t(B), s), "memset");
-    hipLaunchKernelGGL(k_amb_count, dim3(grid_for(P.n_tracks)), dim3(kAmbBlock), 0, s, P);
+    launch(k_amb_count, grid_for(P.n_tracks), s, P);
     hip_check(hipGetLastError(), "count");
     exclusive_scan(P.n_acc, P.list_off, R.sums.as<uint32_t>(), B, &P.ctl->scan_total, s);
     read_ctl(R);
@@ -582,8 +599,8 @@ void setup(ckf_resolver& R, tamd::amb_params& P, uint32_t n_entries) {
     if (R.h_ctl->scan_total > n_entries) {
         throw ckf_error(CKF_ERR_INTERNAL, "identifier lists exceed the constituents");
     }
-    hipLaunchKernelGGL(k_amb_fill, dim3(grid_for(P.n_tracks)), dim3(kAmbBlock), 0, s, P);
-    hipLaunchKernelGGL(k_amb_hot0, dim3(grid_for(B)), dim3(kAmbBlock), 0, s, P);
+    launch(k_amb_fill, grid_for(P.n_tracks), s, P);
+    launch(k_amb_hot0, grid_for(B), s, P);
     hip_check(hipGetLastError(), "fill");
 }
 
@@ -591,12 +608,12 @@ void run_rounds(ckf_resolver& R, tamd::amb_params& P) {
     using namespace tamd;
     const hipStream_t s = R.stream;
     // a round's grid covers its lists (they only shrink); kernels stride over the rest
-    const uint32_t gb = grid_for(std::max(P.id_bound, 1u));
-    const uint32_t gr = grid_for(std::max(P.n_tracks, 1u));
+    const amb_grid gb = grid_for(std::max(P.id_bound, 1u));
+    const amb_grid gr = grid_for(std::max(P.n_tracks, 1u));
     constexpr uint32_t kChunk = 4;
     for (uint32_t r = 0;; ++r) {
-        hipLaunchKernelGGL(k_amb_best, dim3(gb), dim3(kAmbBlock), 0, s, P, r);
-        hipLaunchKernelGGL(k_amb_remove, dim3(gr), dim3(kAmbBlock), 0, s, P, r);
+        launch(k_amb_best, gb, s, P, r);
+        launch(k_amb_remove, gr, s, P, r);
         hip_check(hipGetLastError(), "round");
         if (r % kChunk == kChunk - 1u) {
             read_ctl(R);
@@ -673,7 +690,7 @@ void resolve_device(ckf_resolver& R, uint32_t n, const uint32_t* d_off, const ui
                            R.cfg.max_iterations);
         hip_check(hipGetLastError(), "sequential");
     }
-    hipLaunchKernelGGL(k_amb_output, dim3(grid_for(N)), dim3(kAmbBlock), 0, s, P, d_accepted);
+    launch(k_amb_output, grid_for(N), s, P, d_accepted);
     hip_check(hipGetLastError(), "output");
     read_ctl(R);
     st.n_candidates = R.h_ctl->n_candidates;
@@ -833,7 +850,7 @@ ckf_status ckf_resolve_fitted(ckf_resolver* r, const ckf_device_event* ev,
                                  4u * fitted->ev_track_off.size(), hipMemcpyHostToDevice, s),
                   "event offsets");
         const uint32_t* d_off = fitted->offsets.as<uint32_t>();
-        hipLaunchKernelGGL(tamd::k_amb_fitted_ids, dim3(tamd::grid_for(n)), dim3(tamd::kAmbBlock), 0, s,
+        tamd::launch(tamd::k_amb_fitted_ids, tamd::grid_for(n), s,
                            d_off, fitted->cons.as<uint32_t>(), r->fit_ev_off.as<uint32_t>(),
                            ev->d_meas_off, ev->n_events, n, r->fit_ids.as<uint32_t>());
         hip_check(hipGetLastError(), "identifiers");
